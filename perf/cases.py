@@ -53,36 +53,36 @@ PRESETS = {
 def listed():
     return [
         # The smallest call: the plug-in module with its default settings on a short ragged sequence; launches and host work.
-        dict(name="plug-in, short", kind="plug", B=1, H=8, L=1000, D=64, block_n=64, ratios="default", mode="topk", dtype="bf16"),
+        dict(name="plug-in short", kind="plug", B=1, H=8, L=1000, D=64, block_n=64, ratios="default", mode="topk", dtype="bf16"),
         # A small fp32 layer (the benchmark's small workload): every stage computes in fp32.
-        dict(name="plug-in, fp32", kind="plug", B=1, H=2, L=4096, D=64, block_m=64, block_n=64, tile_n=16, ratios="bound80",
+        dict(name="plug-in fp32", kind="plug", B=1, H=2, L=4096, D=64, block_m=64, block_n=64, tile_n=16, ratios="bound80",
              mode="thresholdbound", dtype="fp32"),
         # The plug-in module with its default settings at an ordinary size, half precision, ragged length.
-        dict(name="plug-in, fp16", kind="plug", B=2, H=16, L=8200, D=128, block_n=64, ratios="default", mode="topk", dtype="fp16"),
+        dict(name="plug-in fp16", kind="plug", B=2, H=16, L=8200, D=128, block_n=64, ratios="default", mode="topk", dtype="fp16"),
         # Wan2.1 1.3B at 832 x 480, 81 frames: a sparse step under the preset with the similarity cap and the token re-ordering.
-        dict(name="video, 128-token blocks", kind="video", preset="Wan2.1_1.3b/psa_balanced", B=1, H=12, width=52, height=30, depth=21,
+        dict(name="video 128-token blocks", kind="video", preset="Wan2.1_1.3b/psa_balanced", B=1, H=12, width=52, height=30, depth=21,
              D=128, dtype="bf16"),
         # The same model under its fixed-quota preset with 32-token kv-blocks.
-        dict(name="video, 32-token blocks", kind="video", preset="Wan2.1_1.3b/psa_topk", B=1, H=12, width=52, height=30, depth=21,
+        dict(name="video 32-token blocks", kind="video", preset="Wan2.1_1.3b/psa_topk", B=1, H=12, width=52, height=30, depth=21,
              D=128, dtype="bf16"),
         # The dense warm-up steps (15 of 50 under that model's presets).
-        dict(name="video, warm-up step", kind="dense", preset="Wan2.1_1.3b/psa_balanced", B=1, H=12, width=52, height=30, depth=21,
+        dict(name="video warm-up step", kind="dense", preset="Wan2.1_1.3b/psa_balanced", B=1, H=12, width=52, height=30, depth=21,
              D=128, dtype="bf16"),
         # CogVideoX-5B, guidance batch of 2, 720 x 480, 49 frames, joint text + video tokens, head dim 64, the 4-step preset.
-        dict(name="video + text, head dim 64", kind="video", preset="CogVideo_5b/psa_4steps", B=2, H=48, width=45, height=30, depth=13,
+        dict(name="video and text head dim 64", kind="video", preset="CogVideo_5b/psa_4steps", B=2, H=48, width=45, height=30, depth=13,
              D=64, dtype="bf16"),
         # CogVideoX1.5-5B at 1360 x 768, 81 frames: the longest sequence, 32-token kv-blocks, head dim 64.
-        dict(name="long video, head dim 64", kind="video", preset="CogVideo1.5_5b/psa_balanced", B=1, H=48, width=85, height=48, depth=11,
+        dict(name="long video head dim 64", kind="video", preset="CogVideo1.5_5b/psa_balanced", B=1, H=48, width=85, height=48, depth=11,
              D=64, dtype="bf16"),
         # One fine-tuning step of the attention layer at the Wan2.1 1.3B shape (the benchmark's training workload).
         dict(name="training", kind="train", B=1, H=12, L=32760, D=128, ratios="bound85", mode="thresholdbound", dtype="bf16"),
         # The same for a head-dim-64 model and a shorter clip, fixed quotas (tuning for the 4-step preset).
-        dict(name="training, head dim 64", kind="train", B=1, H=48, L=8776, D=64, ratios="default", mode="topk", dtype="bf16"),
+        dict(name="training head dim 64", kind="train", B=1, H=48, L=8776, D=64, ratios="default", mode="topk", dtype="bf16"),
         # Prefill of a vision-language decoder (28 query heads on 4 kv heads), 1024 text tokens before a long video.
         dict(name="causal prefill", kind="causal", B=1, H=28, Hkv=4, L=32768, D=128, text=1024, stride=8, ratios="bound80",
              mode="energybound", dtype="bf16"),
         # Prefill of the same decoder on one picture: a short ragged prompt.
-        dict(name="causal prefill, short", kind="causal", B=1, H=28, Hkv=4, L=2345, D=128, text=512, stride=8, ratios="bound80",
+        dict(name="causal prefill short", kind="causal", B=1, H=28, Hkv=4, L=2345, D=128, text=512, stride=8, ratios="bound80",
              mode="energybound", dtype="bf16"),
     ]
 
