@@ -232,6 +232,12 @@ int psa_fwd_indexed(psa_tensor4 q, const int32_t* q_index, psa_tensor4 k, psa_te
  * reference src/psa_triton/utils/transfer_attn_to_mask.py:510-544. */
 int psa_density(const void* map, int map_elem_bytes, int64_t bh, int Mq, int Nk, int causal,
                 float* density_out, psa_stream_t stream);
+/* The same with the maps of B * H (batch, head) pairs counted by several workgroups each (workspace:
+ * psa_density_stats_workspace_bytes bytes, 4-byte aligned) and the figures a caller logs per layer in the same pass:
+ * stats_out: B * H densities | their mean | 1 - mean | H means over the batches (B * H + 2 + H floats). */
+int64_t psa_density_stats_workspace_bytes(int map_elem_bytes, int B, int H, int Mq, int Nk);
+int psa_density_stats(const void* map, int map_elem_bytes, int B, int H, int Mq, int Nk, int causal, void* workspace,
+                      float* stats_out, psa_stream_t stream);
 
 /* Sparse attention forward from a level map.  out [B, Hq, L, D] in the type of q / k / v (bf16, fp16 or fp32); lse (may be NULL)
  * [B, Hq, L] fp32 = natural-log softmax denominator incl. the +ln(level) bias; map == NULL means

@@ -345,15 +345,24 @@ __device__ __forceinline__ float est_reduce_row(const EstParams& p, float* s_e, 
     for (int e = 0; e < 4; ++e) m[e] = fmaxf(m[e], x[e]);
   }
   const float* rt = p.rt + (int64_t)bh * p.n_d * p.Ms_pad + r0;
-  for (int j0 = wave * per_iter; j0 < p.n_d; j0 += 4 * per_iter) {
-    const int j = j0 + sub;
-    float v = -INFINITY;
-    if (j < p.n_d) {
-      const f32x4 x = *(const f32x4*)(rt + (int64_t)j * p.Ms_pad);
-      v = fmaxf(fmaxf(x[0] - m[0], x[1] - m[1]), fmaxf(x[2] - m[2], x[3] - m[3]));
-    }
+  auto group = [&](int j, const f32x4& x) __attribute__((always_inline)) {
+    float v = fmaxf(fmaxf(x[0] - m[0], x[1] - m[1]), fmaxf(x[2] - m[2], x[3] - m[3]));
     for (int o = (1 << lpg_log2) >> 1; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
     if (quad == 0 && j < p.n_d) s_e[j] = fast_exp2(v);
+  };
+  // four loads in flight per lane while there are that many key groups left for the wave, then one at a time
+  constexpr int UN = 4;
+  int j0 = wave * per_iter;
+  for (; j0 + (UN - 1) * 4 * per_iter + per_iter <= p.n_d; j0 += UN * 4 * per_iter) {
+    f32x4 x[UN];
+#pragma unroll
+    for (int u = 0; u < UN; ++u) x[u] = *(const f32x4*)(rt + (int64_t)(j0 + u * 4 * per_iter + sub) * p.Ms_pad);
+#pragma unroll
+    for (int u = 0; u < UN; ++u) group(j0 + u * 4 * per_iter + sub, x[u]);
+  }
+  for (; j0 < p.n_d; j0 += 4 * per_iter) {
+    const int j = j0 + sub;
+    group(j, *(const f32x4*)(rt + (int64_t)(j < p.n_d ? j : p.n_d - 1) * p.Ms_pad));
   }
   __syncthreads();
   // row sum in a fixed order: per-thread strided partials, wave butterfly, four wave partials
@@ -438,7 +447,7 @@ int launch_est(EstParams& p, int B, hipStream_t stream, const LevelMapParams* lp
     hipLaunchKernelGGL(psa_est_reduce_kernel, rgrid, dim3(256), (size_t)p.n_d * sizeof(float), stream, p);
     return psa_check_launch("psa_estimate_sampled (reduction)");
   }
-  const size_t lm_bytes = (level_map_lds_bytes(lp->Nk) + 15) & ~(size_t)15;
+  const size_t lm_bytes = (level_map_lds_bytes(*lp) + 15) & ~(size_t)15;
   const size_t shmem = lm_bytes + (size_t)p.n_d * sizeof(float);
   if (shmem > 150 * 1024) {
     // very wide maps: the row of scores and the level-map scratch do not fit into LDS together - two kernels

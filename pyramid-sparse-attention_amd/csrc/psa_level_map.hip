@@ -29,7 +29,7 @@ extern "C" int psa_level_map(const float* scores, void* map_out, int map_elem_by
   const int rc = level_map_fill_params(p, Nk, mode, n_items, item_level, item_hi, align_div, text_blocks, min_full_attn_ratio);
   if (rc != PSA_OK) return rc;
   p.scores = scores; p.map_out = map_out; p.list_out = list_out; p.map_elem = map_elem_bytes;
-  size_t shmem = level_map_lds_bytes(Nk);
+  size_t shmem = level_map_lds_bytes(p);
   if (shmem > 48 * 1024) {
     hipError_t e = hipFuncSetAttribute((const void*)psa_level_map_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
     PSA_REQUIRE(e == hipSuccess, PSA_ERR_LAUNCH, "psa_level_map: cannot reserve %zu bytes of LDS", shmem);
@@ -271,64 +271,145 @@ extern "C" int psa_map_min_cap(void* map, int map_elem_bytes, const int32_t* cap
 // ---------------------------------------------------------------------------------------
 // density = mean(1/level)
 // ---------------------------------------------------------------------------------------
-__global__ __launch_bounds__(1024) void psa_density_kernel(const void* map, int map_elem, int Mq, int Nk, int causal, int BH,
-                                                           float* out) {
-  __shared__ float s_part[16];
+// Kernel 1 counts, in eighths (8 / level: exact integers), a share of one (batch, head) map per workgroup; kernel 2 adds the
+// shares of every map and forms the means in a fixed order (deterministic).  One workgroup per map used B * H of the 256
+// CUs, and a map that does not start on a 16-byte boundary was read byte by byte: 48 maps of 353 x 1410 bytes 259 -> 10 us,
+// 12 maps of 256 x 256 bytes 12 -> 5 us (the mean kernel: 5 us, its launch).
+constexpr int DENS_UNITS = 4096;   // 16-byte units per workgroup: 16 per thread
+constexpr int DENS_MAX_SHARES = 64;
+
+// eighths of the four map bytes in w: a byte counts when it is exactly 1, 2, 4 or 8
+__device__ __forceinline__ int density_eighths4(uint32_t w) {
+  const uint32_t one = 0x01010101u;
+  const uint32_t b1 = w & one, b2 = (w >> 1) & one, b4 = (w >> 2) & one, b8 = (w >> 3) & one;
+  uint32_t ok = one;
+  // (rare) some byte has several bits set, or one above the fourth
+  if (__builtin_expect((((b1 + b2 + b4 + b8) & 0x06060606u) | (w & 0xf0f0f0f0u)) != 0, 0)) {
+    ok = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t v = (w >> (8 * e)) & 0xffu;
+      ok |= (uint32_t)(v == 1 || v == 2 || v == 4 || v == 8) << (8 * e);
+    }
+  }
+  return 8 * __popc(b1 & ok) + 4 * __popc(b2 & ok) + 2 * __popc(b4 & ok) + __popc(b8 & ok);
+}
+__device__ __forceinline__ int density_eighths1(int lv) {
+  return lv == 1 ? 8 : lv == 2 ? 4 : lv == 4 ? 2 : lv == 8 ? 1 : 0;
+}
+
+__global__ __launch_bounds__(256) void psa_density_kernel(const void* map, int map_elem, int Mq, int Nk, int causal, int32_t* part) {
+  __shared__ int s_part[4];
   const int64_t bh = blockIdx.x;
   const int64_t n = (int64_t)Mq * Nk;
-  const int tid = threadIdx.x;
-  // counts per level are exact integers; 1/level sums are exact in fp32 up to 2^24/8 blocks
-  int c1 = 0, c2 = 0, c4 = 0, c8 = 0;
-  auto count = [&](int lv, int64_t idx) {
-    if (causal) {
-      const int64_t r = idx / Nk, c = idx - r * Nk;
-      if (c > r) return;
-    }
-    c1 += lv == 1; c2 += lv == 2; c4 += lv == 4; c8 += lv == 8;
-  };
+  const int tid = threadIdx.x, shares = gridDim.y;
   const unsigned char* base = (const unsigned char*)map + bh * n * map_elem;
   const int epu = 16 / map_elem;  // map entries per 16-byte load
-  const int64_t units = (((uintptr_t)base & 15) == 0) ? n / epu : 0;
-  for (int64_t u = tid; u < units; u += 1024) {
-    const u32x4 w = *(const u32x4*)(base + u * 16);
-    if (map_elem == 1) {
+  // entries in front of the first 16-byte boundary (maps of odd sizes start anywhere) and behind the last one: one by one
+  const int64_t to_16 = (int64_t)((16 - ((uintptr_t)base & 15)) & 15) / map_elem;
+  const int64_t head = to_16 < n ? to_16 : n;
+  const int64_t units = (n - head) / epu;
+  const unsigned char* body = base + head * map_elem;
+  int acc = 0;
+  for (int64_t u = (int64_t)blockIdx.y * 256 + tid; u < units; u += (int64_t)shares * 256) {
+    const u32x4 w = *(const u32x4*)(body + u * 16);
+    if (causal) {
+      const int64_t i0 = head + u * epu;
+      int64_t r = i0 / Nk;
+      int c = (int)(i0 - r * Nk);
+      for (int e = 0; e < epu; ++e) {
+        const int lv = map_elem == 1 ? (int)(signed char)((w[e >> 2] >> ((e & 3) * 8)) & 0xff) : (int)w[e & 3];
+        acc += c <= r ? density_eighths1(lv) : 0;
+        if (++c == Nk) {
+          c = 0;
+          ++r;
+        }
+      }
+    } else if (map_elem == 1) {
 #pragma unroll
-      for (int e = 0; e < 16; ++e) count((int)(signed char)((w[e >> 2] >> ((e & 3) * 8)) & 0xff), u * 16 + e);
+      for (int e = 0; e < 4; ++e) acc += density_eighths4(w[e]);
     } else {
 #pragma unroll
-      for (int e = 0; e < 4; ++e) count((int)w[e], u * 4 + e);
+      for (int e = 0; e < 4; ++e) acc += density_eighths1((int)w[e]);
     }
   }
-  for (int64_t idx = units * epu + tid; idx < n; idx += 1024) count(load_map(map, bh * n + idx, map_elem), idx);
-  float v = (float)c1 + 0.5f * (float)c2 + 0.25f * (float)c4 + 0.125f * (float)c8;
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  if ((tid & 63) == 0) s_part[tid >> 6] = v;
+  const int64_t singles = n - units * epu;
+  for (int64_t i = (int64_t)blockIdx.y * 256 + tid; i < singles; i += (int64_t)shares * 256) {
+    const int64_t idx = i < head ? i : i + units * epu;
+    const int64_t r = idx / Nk;
+    if (!causal || idx - r * Nk <= r) acc += density_eighths1(load_map(map, bh * n + idx, map_elem));
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
+  if ((tid & 63) == 0) s_part[tid >> 6] = acc;
   __syncthreads();
+  if (tid == 0) part[bh * shares + blockIdx.y] = s_part[0] + s_part[1] + s_part[2] + s_part[3];
+}
+
+// out: the BH densities, then their mean (summed in index order); with H > 0 also 1 - mean and the H per-head means over the
+// BH / H batches.  One workgroup.  (With one share per map the counts may lie in out[] itself.)
+__global__ __launch_bounds__(256) void psa_density_mean_kernel(const int32_t* part, int shares, int BH, int H, double cells, float* out) {
+  __shared__ float s_d[256];
+  const int tid = threadIdx.x;
+  double acc = 0.0;
+  for (int i0 = 0; i0 < BH; i0 += 256) {
+    const int i = i0 + tid;
+    if (i < BH) {
+      int64_t t = 0;
+      for (int s = 0; s < shares; ++s) t += part[(int64_t)i * shares + s];
+      s_d[tid] = out[i] = (float)((double)t * 0.125 / cells);
+    }
+    __syncthreads();
+    if (tid == 0)
+      for (int e = 0; e < 256 && i0 + e < BH; ++e) acc += (double)s_d[e];
+    __syncthreads();
+  }
   if (tid == 0) {
-    float tot = 0.f;
-    for (int w = 0; w < 16; ++w) tot += s_part[w];  // exact: multiples of 1/8 below 2^21
-    const double cnt = causal ? ((double)(Mq < Nk ? Mq : Nk) * ((Mq < Nk ? Mq : Nk) + 1) / 2.0 +
-                                 (Mq > Nk ? (double)(Mq - Nk) * Nk : 0.0))
-                              : (double)n;
-    const float d = (float)((double)tot / cnt);
-    out[bh] = d;
+    const float mean = (float)(acc / (double)BH);
+    out[BH] = mean;
+    if (H > 0) out[BH + 1] = 1.0f - mean;
+  }
+  for (int h = tid; h < H; h += 256) {
+    float sum = 0.f;
+    for (int b = 0; b * H + h < BH; ++b) sum += out[b * H + h];
+    out[BH + 2 + h] = sum / (float)(BH / H);
   }
 }
 
-// overall mean in a fixed order (deterministic)
-__global__ void psa_density_mean_kernel(float* out, int BH) {
-  double acc = 0.0;
-  for (int i = 0; i < BH; ++i) acc += (double)out[i];
-  out[BH] = (float)(acc / (double)BH);
-}
-
-extern "C" int psa_density(const void* map, int map_elem_bytes, int64_t bh, int Mq, int Nk, int causal, float* density_out,
-                           psa_stream_t stream) {
-  PSA_REQUIRE(map && density_out, PSA_ERR_ARG, "psa_density: null pointer");
+static int density_run(const void* map, int map_elem_bytes, int64_t bh, int H, int Mq, int Nk, int causal, int shares, int32_t* part,
+                       float* out, psa_stream_t stream) {
+  PSA_REQUIRE(map && out && part, PSA_ERR_ARG, "psa_density: null pointer");
   PSA_REQUIRE(map_elem_bytes == 1 || map_elem_bytes == 4, PSA_ERR_ARG, "psa_density: map_elem_bytes must be 1 or 4");
   PSA_REQUIRE(bh > 0 && bh < (1 << 30) && Mq > 0 && Nk > 0, PSA_ERR_ARG, "psa_density: bad sizes");
-  hipLaunchKernelGGL(psa_density_kernel, dim3((unsigned)bh), dim3(1024), 0, (hipStream_t)stream, map, map_elem_bytes, Mq,
-                     Nk, causal, (int)bh, density_out);
-  hipLaunchKernelGGL(psa_density_mean_kernel, dim3(1), dim3(1), 0, (hipStream_t)stream, density_out, (int)bh);
+  const int sq = Mq < Nk ? Mq : Nk;
+  const double cells = causal ? (double)sq * (sq + 1) / 2.0 + (Mq > Nk ? (double)(Mq - Nk) * Nk : 0.0) : (double)Mq * Nk;
+  hipLaunchKernelGGL(psa_density_kernel, dim3((unsigned)bh, (unsigned)shares), dim3(256), 0, (hipStream_t)stream, map, map_elem_bytes, Mq,
+                     Nk, causal, part);
+  hipLaunchKernelGGL(psa_density_mean_kernel, dim3(1), dim3(256), 0, (hipStream_t)stream, part, shares, (int)bh, H, cells, out);
   return psa_check_launch("psa_density");
+}
+
+// (no workspace: one share per map)
+extern "C" int psa_density(const void* map, int map_elem_bytes, int64_t bh, int Mq, int Nk, int causal, float* density_out,
+                           psa_stream_t stream) {
+  return density_run(map, map_elem_bytes, bh, 0, Mq, Nk, causal, 1, (int32_t*)density_out, density_out, stream);
+}
+
+static int density_shares(int map_elem_bytes, int64_t bh, int Mq, int Nk) {
+  const int64_t units = ((int64_t)Mq * Nk * map_elem_bytes + 15) / 16;
+  int64_t s = (units + DENS_UNITS - 1) / DENS_UNITS;
+  // at least about two workgroups per CU, down to one 16-byte unit per thread
+  while (s * bh < 512 && s * 256 < units) s *= 2;
+  return (int)(s < 1 ? 1 : (s > DENS_MAX_SHARES ? DENS_MAX_SHARES : s));
+}
+extern "C" int64_t psa_density_stats_workspace_bytes(int map_elem_bytes, int B, int H, int Mq, int Nk) {
+  if (B <= 0 || H <= 0 || Mq <= 0 || Nk <= 0) return 0;
+  return (int64_t)B * H * density_shares(map_elem_bytes, (int64_t)B * H, Mq, Nk) * (int64_t)sizeof(int32_t);
+}
+extern "C" int psa_density_stats(const void* map, int map_elem_bytes, int B, int H, int Mq, int Nk, int causal, void* workspace,
+                                 float* stats_out, psa_stream_t stream) {
+  PSA_REQUIRE(B > 0 && H > 0, PSA_ERR_ARG, "psa_density_stats: B and H must be positive");
+  PSA_REQUIRE(Mq > 0 && Nk > 0, PSA_ERR_ARG, "psa_density_stats: bad sizes");
+  return density_run(map, map_elem_bytes, (int64_t)B * H, H, Mq, Nk, causal, density_shares(map_elem_bytes, (int64_t)B * H, Mq, Nk),
+                     (int32_t*)workspace, stats_out, stream);
 }

@@ -16,6 +16,10 @@ struct LevelMapParams {
   float thr[PSA_MAX_LEVEL_ITEMS];     // thresholdbound: fp32(hi + 1e-6)
   int fixed_s[PSA_MAX_LEVEL_ITEMS];   // topk: row-independent intervals
   int fixed_e[PSA_MAX_LEVEL_ITEMS];
+  // topk: the same intervals as cuts of the rank axis: ranks cut[s - 1] .. cut[s] - 1 get seg_level[s] (cut[-1] = 0)
+  int n_cuts;
+  int cut[2 * PSA_MAX_LEVEL_ITEMS];
+  int seg_level[2 * PSA_MAX_LEVEL_ITEMS + 1];
   int min_index;                      // thresholdbound: floor for the level-1 interval
   int text_blocks;
 };
@@ -110,11 +114,159 @@ __device__ __forceinline__ void row_prefix_sums(double* wide, const float* sw, f
   __syncthreads();
 }
 
-// One row of the level map.  `src` = the row's N scores (global memory or LDS), `smem` = level_map_lds_bytes(N) bytes
+// Levels by fixed quotas need no sorted row: the level of a column follows from how many of the `n_cuts` keys of rank
+// cut[0], cut[1], .. its own key reaches.  A histogram of the keys (SEL_BINS bins, 16 per octave below the row's best
+// score) finds the bin of every cut, the few keys in that bin are ranked by counting, and one pass compares each key
+// with the cut keys.  A bin that holds more than SEL_CAP keys (ties, scores more than 64 octaves below the best) is
+// resolved by building the cut key bit by bit instead.  Measured with the reduction of the estimator's workspace, which the
+// launch also does and which now bounds it: 3072 rows of 1024 scores 157 -> 105 us (403 MB read), 16944 rows of 1410 scores
+// 1480 -> 585 us (3.05 GB read, 5.2 TB/s), against the bitonic network.  Below RANK_SORT_MAX ranking by counting is as fast
+// and also serves the other modes.
+// LDS: (SEL_BINS + 2 * SEL_MAX_CUTS * SEL_CAP + 8 * SEL_MAX_CUTS) 4-byte words.  256 threads.
+constexpr int SEL_BINS = 1024, SEL_SHIFT = 19, SEL_CAP = 64, SEL_MAX_CUTS = 8;
+constexpr size_t SEL_LDS_BYTES = (SEL_BINS + 2 * SEL_MAX_CUTS * SEL_CAP + 8 * SEL_MAX_CUTS) * 4;
+__host__ __device__ inline bool level_map_selects(int mode, int n_cuts, int Nk) {
+  return mode == PSA_MODE_TOPK && n_cuts <= SEL_MAX_CUTS && Nk > RANK_SORT_MAX;
+}
+__device__ __forceinline__ void level_map_row_select(const LevelMapParams& p, const float* src, int64_t row, unsigned char* smem, int tid) {
+  constexpr int NT = 256, PER = SEL_BINS / NT;
+  uint64_t* cand = (uint64_t*)smem;                       // [cut][SEL_CAP] keys of the bin that holds the cut
+  uint64_t* cut_key = cand + SEL_MAX_CUTS * SEL_CAP;      // [cut] key of rank cut[c]
+  int* hist = (int*)(cut_key + SEL_MAX_CUTS);             // [SEL_BINS]
+  int* bin_of = hist + SEL_BINS;                          // [cut] bin that holds the cut
+  int* before = bin_of + SEL_MAX_CUTS;                    // [cut] keys in earlier bins
+  int* n_in = before + SEL_MAX_CUTS;                      // [cut] keys in that bin
+  int* fill = n_in + SEL_MAX_CUTS;                        // [cut] keys collected so far
+  int* wsum = fill + SEL_MAX_CUTS;                        // [8] partial results of the waves
+  const int N = p.Nk, lane = tid & 63, wave = tid >> 6, C = p.n_cuts;
+
+  for (int i = tid; i < SEL_BINS; i += NT) hist[i] = 0;
+  if (tid < SEL_MAX_CUTS) fill[tid] = 0;
+  uint32_t kmin = 0xffffffffu;
+  for (int j = tid; j < N; j += NT) {
+    const uint32_t k = desc_key(src[j]);
+    kmin = k < kmin ? k : kmin;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const uint32_t other = (uint32_t)__shfl_xor((int)kmin, o, 64);
+    kmin = other < kmin ? other : kmin;
+  }
+  if (lane == 0) wsum[wave] = (int)kmin;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < NT / 64; ++w) {
+    const uint32_t k = (uint32_t)wsum[w];
+    kmin = k < kmin ? k : kmin;
+  }
+  auto bin_at = [&](uint32_t k) __attribute__((always_inline)) {
+    const uint32_t b = (k - kmin) >> SEL_SHIFT;
+    return (int)(b < SEL_BINS - 1 ? b : SEL_BINS - 1);
+  };
+  for (int j = tid; j < N; j += NT) atomicAdd(&hist[bin_at(desc_key(src[j]))], 1);
+  __syncthreads();
+  {
+    int c[PER], sum = 0;
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+      c[e] = hist[tid * PER + e];
+      sum += c[e];
+    }
+    int incl = sum;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int up = __shfl_up(incl, d, 64);
+      incl += lane >= d ? up : 0;
+    }
+    if (lane == 63) wsum[4 + wave] = incl;
+    __syncthreads();
+    int run = incl - sum;
+#pragma unroll
+    for (int w = 0; w < NT / 64; ++w) run += w < wave ? wsum[4 + w] : 0;
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+      if (c[e] > 0)
+        for (int t = 0; t < C; ++t)
+          if (p.cut[t] >= run && p.cut[t] < run + c[e]) {
+            bin_of[t] = tid * PER + e;
+            before[t] = run;
+            n_in[t] = c[e];
+          }
+      run += c[e];
+    }
+  }
+  __syncthreads();
+  int cut_bin[SEL_MAX_CUTS];
+#pragma unroll
+  for (int t = 0; t < SEL_MAX_CUTS; ++t) cut_bin[t] = t < C ? bin_of[t] : -1;
+  for (int j = tid; j < N; j += NT) {
+    const uint32_t k = desc_key(src[j]);
+    const int b = bin_at(k);
+#pragma unroll
+    for (int t = 0; t < SEL_MAX_CUTS; ++t)
+      if (b == cut_bin[t]) {
+        const int at = atomicAdd(&fill[t], 1);
+        if (at < SEL_CAP) cand[t * SEL_CAP + at] = ((uint64_t)k << 32) | (uint32_t)j;
+      }
+  }
+  __syncthreads();
+  bool crowded = false;
+#pragma unroll
+  for (int t = 0; t < SEL_MAX_CUTS; ++t)
+    if (t < C) {
+      const int n = n_in[t];
+      if (n > SEL_CAP) {
+        crowded = true;
+      } else if ((t & 3) == wave) {
+        const uint64_t mine = lane < n ? cand[t * SEL_CAP + lane] : ~0ull;
+        int rank = 0;
+        for (int i = 0; i < n; ++i) rank += cand[t * SEL_CAP + i] < mine ? 1 : 0;
+        if (lane < n && rank == p.cut[t] - before[t]) cut_key[t] = mine;
+      }
+    }
+  if (crowded) {  // uniform: the counts are the same for every thread
+    for (int t = 0; t < C; ++t) {
+      if (n_in[t] <= SEL_CAP) continue;
+      uint64_t k0 = 0;
+      for (int bit = 63; bit >= 0; --bit) {
+        if (bit == 31) bit = 15;  // columns have 16 bits
+        const uint64_t probe = k0 | (1ull << bit);
+        int below = 0;
+        for (int j0 = 0; j0 < N; j0 += NT) {
+          const int j = j0 + tid;
+          below += __popcll(__ballot(j < N && (((uint64_t)desc_key(src[j < N ? j : 0]) << 32) | (uint32_t)j) < probe));
+        }
+        __syncthreads();
+        if (lane == 0) wsum[wave] = below;
+        __syncthreads();
+        if (wsum[0] + wsum[1] + wsum[2] + wsum[3] <= p.cut[t]) k0 = probe;
+      }
+      if (tid == 0) cut_key[t] = k0;
+    }
+  }
+  __syncthreads();
+  uint64_t ck[SEL_MAX_CUTS];
+#pragma unroll
+  for (int t = 0; t < SEL_MAX_CUTS; ++t) ck[t] = t < C ? cut_key[t] : ~0ull;
+  for (int j = tid; j < N; j += NT) {
+    const uint64_t k = ((uint64_t)desc_key(src[j]) << 32) | (uint32_t)j;
+    int lv = p.seg_level[0];
+#pragma unroll
+    for (int t = 0; t < SEL_MAX_CUTS; ++t) lv = k >= ck[t] ? p.seg_level[t + 1] : lv;
+    if (j >= N - p.text_blocks) lv = 1;
+    store_map(p.map_out, row * N + j, p.map_elem, lv);
+  }
+}
+
+// One row of the level map.  `src` = the row's N scores (global memory or LDS), `smem` = level_map_lds_bytes(p) bytes
 // of 16-byte aligned LDS, s_cnt / s_iv = PSA_MAX_LEVEL_ITEMS (x2) ints of LDS; called by all nt threads of the workgroup.
 __device__ __forceinline__ void level_map_row(const LevelMapParams& p, const float* src, int64_t row, unsigned char* smem,
                                               int* s_cnt, int (*s_iv)[2], int tid, int nt) {
   const int N = p.Nk;
+  if (p.list_out == nullptr && level_map_selects(p.mode, p.n_cuts, N)) {
+    level_map_row_select(p, src, row, smem, tid);
+    return;
+  }
   uint64_t* key = (uint64_t*)smem;            // [sort_pad(N)]
   float* sw = (float*)(key + sort_pad(N));    // [N] scores in sorted order
   int* sidx = (int*)(sw + N);                 // [N] column of sorted position
@@ -259,7 +411,30 @@ static inline int level_map_fill_params(LevelMapParams& p, int Nk, int mode, int
       }
     }
   }
+  p.n_cuts = 0;
+  for (int t = 0; t < 2 * PSA_MAX_LEVEL_ITEMS; ++t) p.cut[t] = 0;
+  for (int t = 0; t <= 2 * PSA_MAX_LEVEL_ITEMS; ++t) p.seg_level[t] = 0;
+  if (mode == PSA_MODE_TOPK) {
+    // the intervals are disjoint and in ascending order; ranks outside all of them are skipped (level 0)
+    int at = 0, lvl = 0;  // level of the ranks from `at` on
+    auto open = [&](int rank, int level) {
+      if (level == lvl && rank > 0) return;
+      if (rank > at) p.cut[p.n_cuts++] = rank;
+      p.seg_level[p.n_cuts] = level;
+      at = rank;
+      lvl = level;
+    };
+    for (int t = 0; t < n_items; ++t)
+      if (p.fixed_s[t] < p.fixed_e[t]) {
+        open(p.fixed_s[t], p.level[t]);
+        if (p.fixed_e[t] < Nk) open(p.fixed_e[t], 0);
+      }
+  }
   return PSA_OK;
 }
 
-static inline size_t level_map_lds_bytes(int Nk) { return (size_t)sort_pad(Nk) * 8 + (size_t)Nk * (4 + 4 + 4); }
+// LDS scratch of level_map_row: of the selection where it serves the call (dense maps by quotas), else of the sort
+static inline size_t level_map_lds_bytes(const LevelMapParams& p) {
+  if (p.list_out == nullptr && level_map_selects(p.mode, p.n_cuts, p.Nk)) return SEL_LDS_BYTES;
+  return (size_t)sort_pad(p.Nk) * 8 + (size_t)p.Nk * (4 + 4 + 4);
+}

@@ -97,8 +97,8 @@ def adaptive_block_sparse_attn(q, k, v, config: AttentionConfig, sparse_attentio
     out = sparse_attention_fn(q, k, v, mask, None)
     if not compute_stats:
         return out, 0.0, []
-    d = ops.density(mask, causal=config.causal_main)  # stays on the device
-    return out, 1 - d[-1], d[:-1].view(q.shape[0], q.shape[1]).mean(0)
+    _, sparsity, per_head = ops.density_stats(mask, causal=config.causal_main)  # stays on the device
+    return out, sparsity, per_head
 
 
 class PyramidAdaptiveBlockSparseAttnTrain(nn.Module):

@@ -453,16 +453,25 @@ def map_min_cap(level_map_: torch.Tensor, cap: torch.Tensor) -> torch.Tensor:
     return level_map_
 
 
-def density(level_map_: torch.Tensor, causal: bool = False) -> torch.Tensor:
-    """Device-side mean(1/level): returns a float32 tensor [B*H + 1] (per (b,h), then the overall
-    mean) without synchronising the host."""
+def density_stats(level_map_: torch.Tensor, causal: bool = False) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """Device-side mean(1/level), no host synchronisation: (densities fp32 [B*H + 1]: per (b,h), then the overall mean;
+    sparsity = 1 - that mean, a scalar tensor; per-head means over the batch [H])."""
     _require_gpu(level_map_)
     m = level_map_.contiguous()
     B, H, Mq, Nk = m.shape
-    out = torch.empty(B * H + 1, dtype=torch.float32, device=m.device)
+    n_ws = lib.psa_density_stats_workspace_bytes(m.element_size(), B, H, Mq, Nk) // 4
+    BH = B * H
+    out = torch.empty(BH + 2 + H + n_ws, dtype=torch.float32, device=m.device)
     with torch.cuda.device(m.device):
-        check(lib.psa_density(_ptr(m), m.element_size(), B * H, Mq, Nk, int(causal), _ptr(out), _stream(m)), "psa_density")
-    return out
+        check(lib.psa_density_stats(_ptr(m), m.element_size(), B, H, Mq, Nk, int(causal), ctypes.c_void_p(out.data_ptr() + 4 * (BH + 2 + H)),
+                                    _ptr(out), _stream(m)), "psa_density_stats")
+    return out[:BH + 1], out[BH + 1], out[BH + 2:BH + 2 + H]
+
+
+def density(level_map_: torch.Tensor, causal: bool = False) -> torch.Tensor:
+    """Device-side mean(1/level): returns a float32 tensor [B*H + 1] (per (b,h), then the overall
+    mean) without synchronising the host."""
+    return density_stats(level_map_, causal)[0]
 
 
 # ----------------------------------------------------------------------------- attention forward

@@ -110,9 +110,7 @@ def adaptive_block_sparse_attn(q, k, v, config, sparse_attention_fn, compute_sta
     if compute_stats:
         if dense is None:
             dense = mask if config.attn_impl == "old_mask_type" else ops.map_from_list(mask, -(-k.shape[2] // config.block_n))
-        d = ops.density(dense)  # [B*H + 1] on the device
-        sparsity = 1 - d[-1]
-        per_head = d[:-1].view(q.shape[0], q.shape[1]).mean(0)
+        _, sparsity, per_head = ops.density_stats(dense)  # on the device
     else:
         sparsity, per_head = 0.0, []
     return out, sparsity, per_head, sim_cap
@@ -220,8 +218,8 @@ class PyramidSparseAttention(nn.Module):
             token_index=self.rearranger.token_index(q.device) if through_index else None,
             sim_thresholds=thr, return_map=True, return_cap=True)
         if compute_stats:
-            d = ops.density(mp)  # [B*H + 1] on the device
-            return out, 1 - d[-1], d[:-1].view(B, H).mean(0), cap
+            _, sparsity, per_head = ops.density_stats(mp)  # on the device
+            return out, sparsity, per_head, cap
         return out, 0.0, [], cap
 
     def close_logger(self):
