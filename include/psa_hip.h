@@ -283,6 +283,15 @@ int psa_fwd_scheduled(psa_tensor4 q, const int32_t* q_index, psa_tensor4 k, psa_
                       float* lse, int B, int Hq, int Hkv, int L, int D, int block_m, int block_n, float sm_scale,
                       int causal, psa_stream_t stream);
 
+/* The same for every block_n the forward serves (32, 64, 128; D = 64 or 128, block_m = 128; psa_walk_bytes returns 0
+ * otherwise): what a call that has its map once builds for itself.  A call on such a walk gives the bits of psa_fwd. */
+int64_t psa_walk_bytes(int B, int Hq, int Hkv, int L, int D, int block_m, int block_n);
+int psa_build_walk(const void* map, int map_elem_bytes, void* walk, int B, int Hq, int Hkv, int L, int D, int block_m,
+                   int block_n, int causal, psa_stream_t stream);
+int psa_fwd_walk(psa_tensor4 q, const int32_t* q_index, psa_tensor4 k, psa_tensor4 v, const void* k_pool, const void* v_pool,
+                 const void* map, int map_elem_bytes, const void* walk, psa_tensor4 out, float* lse, int B, int Hq, int Hkv,
+                 int L, int D, int block_m, int block_n, float sm_scale, int causal, psa_stream_t stream);
+
 /* psa_fwd without a workspace argument and without any allocation: the row-ordering scratch is a fixed array inside
  * the library (one copy per GPU, about 0.5 MiB, held until the process ends).  This entry point has no counterpart in
  * the reference; it exists for callers that cannot allocate device memory around the call - code under HIP graph

@@ -83,7 +83,78 @@ struct FwdParams {
   const u32x4* sched_rec;
   const int32_t* sched_tiles;
   int rec_stride;
+  const uint16_t* sched_fine;  // block ids of the fine tiles (64- / 32-key blocks), fine_stride tiles per row
+  int fine_stride;
 };
+
+// Where a walk takes its tiles from.
+//   WALK_MAP      the workgroup compacts its map row and looks block ids up per lane and tile
+//   WALK_REC      prebuilt records (psa_schedule.h), 128-key blocks, K / V rows D elements apart
+//   WALK_REC_ANY  prebuilt records, any block size and row stride
+//   WALK_DENSE    no map: every key at level 0, the records are computed; any row stride (one-row kernel)
+// Measured against WALK_MAP: head dim 64 5 - 7 % of the layer (48 heads of 17776 tokens x 2, 128-key blocks, and of 45106
+// tokens, 32-key blocks); head dim 128, bound by power, 0 - 2 %.
+enum { WALK_MAP = 0, WALK_REC = 1, WALK_REC_ANY = 2, WALK_DENSE = 3 };
+
+// The word of tile t of a dense row (the form psa_schedule.h gives the records), for quarter g; scalar arithmetic only.
+__device__ __forceinline__ uint32_t dense_word(int t, int T, int g, int L, bool causal, int q_first_row) {
+  const int r0 = (t < T ? t : T - 1) * TK;
+  const int left = L - r0, nvalid = left < TK ? left : TK;
+  const bool masked = nvalid < TK || (causal && r0 + TK - 1 > q_first_row);
+  return (uint32_t)(r0 + 16 * g) | ((nvalid < TK ? psa_sched::REC_CODE_RAGGED : 0u) << psa_sched::REC_CODE_SHIFT) |
+         ((uint32_t)masked << psa_sched::REC_MASKED_BIT) | ((uint32_t)nvalid << psa_sched::REC_NVALID_SHIFT);
+}
+// tiles of a dense row whose keys end at block jmax
+__device__ __forceinline__ int dense_tiles(int jmax, int bn_log2, int L) {
+  const int64_t end = (int64_t)jmax << bn_log2;
+  return (int)(((end < L ? end : L) + TK - 1) / TK);
+}
+
+// Block ids of the fine tiles of a row, 4 per quarter (one per 4 tile rows), read through the scalar cache.
+using fine_ptr = const __attribute__((address_space(4))) uint64_t*;
+// first of the lane's consecutive source rows of a fine tile: ids = the quarter's 4 block ids, lane_row = first of its rows
+__device__ __forceinline__ uint32_t fine_row(uint64_t ids, int lane, int lane_row, int sbs_log2) {
+  const uint32_t pair = (lane & 32) ? (uint32_t)(ids >> 32) : (uint32_t)ids;
+  return (((pair >> (lane & 16)) & 0xffffu) << sbs_log2) + (uint32_t)(lane_row & ((1 << sbs_log2) - 1));
+}
+
+// Logits of the slots of tile t that hold no key or a key the row may not see: -inf.  w: the word of this wave's record.
+template <int WALK>
+__device__ __forceinline__ void mask_words(f32x16 (&s)[2], uint32_t w, int t, const __attribute__((address_space(4))) u32x4* recs,
+                                           fine_ptr fine, int bn_log2, bool causal, int q_idx, int hh) {
+  const int lv = psa_sched::rec_level(w);
+  const int nvalid = psa_sched::rec_nvalid(w);
+  const int qlim = (q_idx + 1) >> lv;
+  u32x4 r4 = {0u, 0u, 0u, 0u};
+  if constexpr (WALK != WALK_DENSE)
+    if (causal) r4 = recs[t];  // the source rows of all four quarters (rare path: fetched on demand)
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int r0 = c * 32 + g * 8 + hh * 4;
+      int keep = nvalid - r0;
+      if (causal) {
+        // slots r0 .. r0+3 lie in quarter 2c + g/2 of the tile, whose source rows are consecutive (fine tiles: in one run
+        // of 4 rows of it)
+        int src0;
+        if constexpr (WALK == WALK_DENSE) {
+          src0 = t * TK + r0;
+        } else {
+          src0 = psa_sched::rec_src(r4[c * 2 + (g >> 1)]) + (g & 1) * 8 + hh * 4;
+          if constexpr (WALK == WALK_REC_ANY)
+            if (psa_sched::rec_code(w) >= psa_sched::REC_CODE_FINE) {
+              const int sbs_log2 = bn_log2 - lv;
+              const uint32_t pair = (uint32_t)(fine[psa_sched::rec_src(w) * 4 + c * 2 + (g >> 1)] >> ((g & 1) * 32));
+              src0 = (int)(((pair >> (hh * 16)) & 0xffffu) << sbs_log2) + (r0 & ((1 << sbs_log2) - 1));
+            }
+        }
+        keep = keep < qlim - src0 ? keep : qlim - src0;
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s[c][g * 4 + e] = e < keep ? s[c][g * 4 + e] : -INFINITY;
+    }
+}
 
 constexpr int F_ISTR = psa_tiles::LT_ISTR;  // bytes between the blocks of a tile
 
@@ -94,10 +165,11 @@ constexpr int F_ISTR = psa_tiles::LT_ISTR;  // bytes between the blocks of a til
     __syncthreads();                        \
   } while (0)
 
-// GS: the row's tiles come from a prebuilt schedule (psa_schedule.h) as in the two-group kernel below: one scalar word
-// per wave and tile instead of a per-lane look-up, copies addressed from scalar registers.
-template <int D, int NW, bool GS, class ET>
-__global__ __launch_bounds__(NW * 64, 2) void psa_fwd_lds_kernel(FwdParams p) {
+// GS: the row's tiles come from records (psa_schedule.h) as in the two-group kernel below: one scalar word per wave and
+// tile instead of a per-lane look-up, copies addressed from scalar registers.
+template <int D, int NW, int WALK, class ET>
+__global__ __launch_bounds__(NW * 64, (D == 64 && WALK != WALK_MAP) ? 4 : 2) void psa_fwd_lds_kernel(FwdParams p) {
+  constexpr bool GS = WALK != WALK_MAP, ANY_STRIDE = WALK >= WALK_REC_ANY;
   using x8 = typename ET::x8;
   using G = psa_tiles::LtGeom<D>;
   constexpr int F_TILE = G::TILE;  // bytes of one K or V tile
@@ -153,9 +225,13 @@ __global__ __launch_bounds__(NW * 64, 2) void psa_fwd_lds_kernel(FwdParams p) {
   using w_ptr = const __attribute__((address_space(4))) uint32_t*;
   using rec_ptr = const __attribute__((address_space(4))) u32x4*;
   rec_ptr recs = nullptr;
+  fine_ptr fine = nullptr;  // WALK_REC_ANY: block ids of the row's fine tiles
   int T;
-  if constexpr (GS) {
+  if constexpr (WALK == WALK_DENSE) {
+    T = dense_tiles(jmax, P_bn_log2, P_L);
+  } else if constexpr (GS) {
     recs = (rec_ptr)(uintptr_t)(p.sched_rec + (int64_t)logical * p.rec_stride);
+    if constexpr (WALK == WALK_REC_ANY) fine = (fine_ptr)(uintptr_t)(p.sched_fine + (int64_t)logical * p.fine_stride * psa_sched::FINE_RUNS);
     T = __builtin_amdgcn_readfirstlane(p.sched_tiles[logical]);
   } else {
     T = psa_tiles::build_row_schedule<NT>(p.map, p.map_elem, ((int64_t)bh * p.Mq + I) * p.Nk, p.Nk, jmax, P_bn_log2, P_L,
@@ -198,26 +274,7 @@ __global__ __launch_bounds__(NW * 64, 2) void psa_fwd_lds_kernel(FwdParams p) {
     else d = __builtin_amdgcn_readfirstlane(tdesc[t][0]);
     const int lv = d & 3;
     if constexpr (GS) {
-      if (d & 4) {
-        const int nvalid = psa_sched::rec_nvalid(w_cur);
-        const int qlim = (q_idx + 1) >> lv;
-        u32x4 r4 = {0u, 0u, 0u, 0u};
-        if (P_causal) r4 = recs[t];  // the source rows of all four quarters (rare path: fetched on demand)
-#pragma unroll
-        for (int c = 0; c < 2; ++c)
-#pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            const int r0 = c * 32 + g * 8 + hh * 4;
-            int keep = nvalid - r0;
-            if (P_causal) {
-              // slots r0 .. r0+3 lie in quarter 2c + g/2 of the tile, whose source rows are consecutive
-              const int src0 = psa_sched::rec_src(r4[c * 2 + (g >> 1)]) + (g & 1) * 8 + hh * 4;
-              keep = keep < qlim - src0 ? keep : qlim - src0;
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) s_cur[c][g * 4 + e] = e < keep ? s_cur[c][g * 4 + e] : -INFINITY;
-          }
-      }
+      if (d & 4) mask_words<WALK>(s_cur, w_cur, t, recs, fine, P_bn_log2, P_causal != 0, q_idx, hh);
     } else if (d & 4) {
       // Partly empty tile and/or causal diagonal.  Valid slots are a prefix of the tile (nvalid), and a
       // pooled key of level lv is visible to query i once its last token is: ((src + 1) << lv) - 1 <= i, i.e.
@@ -352,29 +409,44 @@ __global__ __launch_bounds__(NW * 64, 2) void psa_fwd_lds_kernel(FwdParams p) {
   struct Stream {  // where one tensor's tiles currently come from: a level's rows (the level changes 3 times per row)
     const char* base;
     uint32_t code;
+    uint32_t str, voff;  // ANY_STRIDE: bytes between rows, this lane's offset
   };
-  Stream st_k = {kb0, 0u}, st_v = {vb0, 0u};
-  auto issue_tile = [&](Stream& st, bool is_k, uint32_t w, auto lds_byte) __attribute__((always_inline)) {
+  Stream st_k = {kb0, 0u, P_k_strb, (uint32_t)lane_row * P_k_strb + f_chunk}, st_v = {vb0, 0u, P_v_strb, (uint32_t)lane_row * P_v_strb + f_chunk};
+  auto issue_tile = [&](Stream& st, bool is_k, uint32_t w, uint64_t fids, auto lds_byte) __attribute__((always_inline)) {
     const uint32_t code = psa_sched::rec_code(w);
-    bool rag = false;
+    bool rag = false, is_fine = false;
     if (code != st.code) {
       const int lv = (int)(code & 3u);
-      st.code = code & 3u;  // (a ragged tile comes back here for every tile)
+      st.code = code & 3u;  // (a ragged or fine tile comes back here for every tile)
       const uint16_t* pool = is_k ? P_kp : P_vp;
       st.base = lv == 0 ? (is_k ? kb0 : vb0) : pool_base(pool, lv);
+      if constexpr (ANY_STRIDE) {
+        st.str = lv == 0 ? (is_k ? P_k_strb : P_v_strb) : (uint32_t)(D * 2);
+        st.voff = (uint32_t)lane_row * st.str + f_chunk;
+      }
       rag = code == psa_sched::REC_CODE_RAGGED;
+      if constexpr (WALK == WALK_REC_ANY) is_fine = code >= psa_sched::REC_CODE_FINE;
     }
+    const uint32_t str = ANY_STRIDE ? st.str : (uint32_t)(D * 2);
     if (rag) {
       static_for<G::RPL>([&](auto n) __attribute__((always_inline)) {
         constexpr int N = decltype(n)::value, OFF = decltype(lds_byte)::value + N * F_ISTR;
         const int row = psa_sched::rec_src(w) + lane_row + N;
-        psa_tiles::lds_copy16_row<OFF>(st.base, (uint32_t)(row < P_L - 1 ? row : P_L - 1), (uint32_t)(D * 2), f_chunk, wave_lds);
+        psa_tiles::lds_copy16_row<OFF>(st.base, (uint32_t)(row < P_L - 1 ? row : P_L - 1), str, f_chunk, wave_lds);
       });
-    } else {
-      const char* src = st.base + (uint64_t)((w & psa_sched::REC_SRC_MASK) * (uint32_t)(D * 2));
+    } else if (is_fine) {
+      // pooled rows, D elements apart: a run of rows per lane group
+      const uint32_t voff = fine_row(fids, lane, lane_row, P_bn_log2 - (int)(code & 3u)) * (uint32_t)(D * 2) + f_chunk;
       static_for<G::RPL>([&](auto n) __attribute__((always_inline)) {
         constexpr int N = decltype(n)::value;
-        psa_tiles::lds_copy16_imm<decltype(lds_byte)::value + N * F_ISTR, N * D * 2>(src, voff_s, wave_lds);
+        psa_tiles::lds_copy16_imm<decltype(lds_byte)::value + N * F_ISTR, N * D * 2>(st.base, voff, wave_lds);
+      });
+    } else {
+      const char* src = st.base + (uint64_t)((w & psa_sched::REC_SRC_MASK) * str);
+      static_for<G::RPL>([&](auto n) __attribute__((always_inline)) {
+        constexpr int N = decltype(n)::value, OFF = decltype(lds_byte)::value + N * F_ISTR;
+        if constexpr (ANY_STRIDE) psa_tiles::lds_copy16_imm<OFF, 0>(src + (uint64_t)(N * str), st.voff, wave_lds);
+        else psa_tiles::lds_copy16_imm<OFF, N * D * 2>(src, voff_s, wave_lds);
       });
     }
   };
@@ -385,14 +457,29 @@ __global__ __launch_bounds__(NW * 64, 2) void psa_fwd_lds_kernel(FwdParams p) {
     uint32_t pk[2][8];
     w_ptr wp = nullptr;
     uint32_t w_next = 0, w_next2 = 0;  // GS: words of tiles t+1 and t+2 (records T .. T+2 repeat record T-1)
+    uint64_t f_next = 0;               // WALK_REC_ANY: block ids of this wave's quarter of tile t+1, where that is a fine tile
+    auto dense_at = [&](int t) __attribute__((always_inline)) { return dense_word(t, T, wave, P_L, P_causal != 0, I * BM); };
+    auto fetch_fine = [&](uint32_t w, uint64_t& f) __attribute__((always_inline)) {
+      if constexpr (WALK == WALK_REC_ANY)
+        if (psa_sched::rec_code(w) >= psa_sched::REC_CODE_FINE) f = fine[psa_sched::rec_src(w) * 4 + wave];
+    };
     if constexpr (GS) {
-      wp = (w_ptr)(uintptr_t)((const uint32_t*)(p.sched_rec + (int64_t)logical * p.rec_stride) + wave);
-      w_cur = wp[0];
-      w_next = wp[4];
-      w_next2 = wp[8];
-      wp += 12;
-      issue_tile(st_k, true, w_cur, IC<0>{});
-      issue_tile(st_v, false, w_cur, IC<2 * F_TILE>{});
+      if constexpr (WALK == WALK_DENSE) {
+        w_cur = dense_at(0);
+        w_next = dense_at(1);
+        w_next2 = dense_at(2);
+      } else {
+        wp = (w_ptr)(uintptr_t)((const uint32_t*)(p.sched_rec + (int64_t)logical * p.rec_stride) + wave);
+        w_cur = wp[0];
+        w_next = wp[4];
+        w_next2 = wp[8];
+        wp += 12;
+      }
+      uint64_t f0 = 0;
+      fetch_fine(w_cur, f0);
+      issue_tile(st_k, true, w_cur, f0, IC<0>{});
+      issue_tile(st_v, false, w_cur, f0, IC<2 * F_TILE>{});
+      fetch_fine(w_next, f_next);
     } else {
       tile_src(0, ts);
       issue_rows(ts.kbase, ts.kstr, ts.lim, ts.src0, 0);
@@ -403,8 +490,8 @@ __global__ __launch_bounds__(NW * 64, 2) void psa_fwd_lds_kernel(FwdParams p) {
       constexpr int CUR = decltype(cur_c)::value;
       if (t + 1 < T) {
         if constexpr (GS) {
-          issue_tile(st_k, true, w_next, IC<(CUR ^ 1) * F_TILE>{});
-          issue_tile(st_v, false, w_next, IC<(2 + (CUR ^ 1)) * F_TILE>{});
+          issue_tile(st_k, true, w_next, f_next, IC<(CUR ^ 1) * F_TILE>{});
+          issue_tile(st_v, false, w_next, f_next, IC<(2 + (CUR ^ 1)) * F_TILE>{});
         } else {
           tile_src(t + 1, ts);
           issue_rows(ts.kbase, ts.kstr, ts.lim, ts.src0, (CUR ^ 1) * F_TILE);
@@ -423,8 +510,13 @@ __global__ __launch_bounds__(NW * 64, 2) void psa_fwd_lds_kernel(FwdParams p) {
       if constexpr (GS) {
         w_cur = w_next;
         w_next = w_next2;
-        w_next2 = *wp;  // the word of tile t+3 (one scalar load; the records are padded, so no bounds test)
-        wp += 4;
+        fetch_fine(w_next, f_next);
+        if constexpr (WALK == WALK_DENSE) {
+          w_next2 = dense_at(t + 3);
+        } else {
+          w_next2 = *wp;  // the word of tile t+3 (one scalar load; the records are padded, so no bounds test)
+          wp += 4;
+        }
       }
       TILE_SYNC();
     };
@@ -484,15 +576,17 @@ __global__ __launch_bounds__(NW * 64, 2) void psa_fwd_lds_kernel(FwdParams p) {
 // exponentials.
 #define PP_BARRIER() asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory")
 
-// GS: the rows' tiles come from a prebuilt schedule in device memory (psa_schedule.h; 128-key blocks, K / V rows D
-// elements apart) instead of being compacted from the map row here.  A wave fetches ONE word per tile (a scalar load,
+// GS: the rows' tiles come from a prebuilt schedule in device memory (psa_schedule.h) instead of being compacted from the
+// map row here.  A wave fetches ONE word per tile (a scalar load,
 // three tiles ahead): level, fill and the first source row of the 16-row quarter it copies.  A wave issues at most one
 // instruction per 4 cycles whatever its kind, so what bounds the vector phase is its instruction COUNT: a copy here is
 // two instructions (M0, then the load with the row step n * 256 as its immediate offset - which the hardware also adds
 // on the LDS side, so M0 carries the difference), the base pointer of a tile's level is kept while the level stays the
 // same (tiles of a row are sorted by level), and nothing is looked up per lane.
-template <int D, int NW, bool GS, class ET>
+template <int D, int NW, int WALK, class ET>
 __global__ __launch_bounds__(2 * NW * 64, 1) void psa_fwd_pp_kernel(FwdParams p) {
+  constexpr bool GS = WALK != WALK_MAP, ANY_STRIDE = WALK == WALK_REC_ANY;
+  static_assert(WALK != WALK_DENSE, "dense rows: one-row kernel or the list of the map walk");
   using x8 = typename ET::x8;
   using G = psa_tiles::LtGeom<D>;
   constexpr int F_TILE = G::TILE;
@@ -552,9 +646,11 @@ __global__ __launch_bounds__(2 * NW * 64, 1) void psa_fwd_pp_kernel(FwdParams p)
   using w_ptr = const __attribute__((address_space(4))) uint32_t*;
   using rec_ptr = const __attribute__((address_space(4))) u32x4*;
   rec_ptr recs = nullptr;
+  fine_ptr fine = nullptr;  // WALK_REC_ANY: block ids of the row's fine tiles
   int T;
   if constexpr (GS) {
     recs = (rec_ptr)(uintptr_t)(p.sched_rec + (int64_t)logical * p.rec_stride);
+    if constexpr (WALK == WALK_REC_ANY) fine = (fine_ptr)(uintptr_t)(p.sched_fine + (int64_t)logical * p.fine_stride * psa_sched::FINE_RUNS);
     T = active ? __builtin_amdgcn_readfirstlane(p.sched_tiles[logical]) : 0;
   } else {
     // both groups run the builder's barriers together
@@ -601,27 +697,6 @@ __global__ __launch_bounds__(2 * NW * 64, 1) void psa_fwd_pp_kernel(FwdParams p)
   // reference update, small enough to ride along with one MFMA of PV(t-1).  prob16: the exponentials.
   uint32_t d_cur = 0;  // descriptor word 0 of the tile whose logits are in s: level | masked << 2 | ...
   uint32_t w_cur = 0;  // GS: this wave's word of its record
-  auto mask_tile_rec = [&](int t, f32x16 (&s_cur)[2]) __attribute__((always_inline)) {
-    const int lv = psa_sched::rec_level(w_cur);
-    const int nvalid = psa_sched::rec_nvalid(w_cur);
-    const int qlim = (q_idx + 1) >> lv;
-    u32x4 r4 = {0u, 0u, 0u, 0u};
-    if (P_causal) r4 = recs[t];  // the source rows of all four quarters (rare path: fetched on demand)
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int r0 = c * 32 + g * 8 + hh * 4;
-        int keep = nvalid - r0;
-        if (P_causal) {
-          // slots r0 .. r0+3 lie in quarter 2c + g/2 of the tile, whose source rows are consecutive
-          const int src0 = psa_sched::rec_src(r4[c * 2 + (g >> 1)]) + (g & 1) * 8 + hh * 4;
-          keep = keep < qlim - src0 ? keep : qlim - src0;
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) s_cur[c][g * 4 + e] = e < keep ? s_cur[c][g * 4 + e] : -INFINITY;
-      }
-  };
   auto mask_tile = [&](int t, f32x16 (&s_cur)[2]) __attribute__((always_inline)) {
     const uint32_t d = d_cur;
     const int lv = d & 3;
@@ -802,45 +877,78 @@ __global__ __launch_bounds__(2 * NW * 64, 1) void psa_fwd_pp_kernel(FwdParams p)
   struct Stream {  // where one tensor's tiles currently come from: a level's rows (the level changes 3 times per row)
     const char* base;
     uint32_t code;
+    uint32_t str, voff;  // ANY_STRIDE: bytes between rows, this lane's offset
   };
-  Stream st_k = {kb0, 0u}, st_v = {vb0, 0u};
-  // first source row of this wave's quarter of the tile with word w; rag: the tile is ragged (rows are clamped per lane)
-  auto quarter_src = [&](Stream& st, bool is_k, uint32_t w, bool& rag) __attribute__((always_inline)) {
+  Stream st_k = {kb0, 0u, P_k_strb, (uint32_t)lane_row * P_k_strb + f_chunk}, st_v = {vb0, 0u, P_v_strb, (uint32_t)lane_row * P_v_strb + f_chunk};
+  // What the copies of this wave's quarter of a tile need: the (uniform) source of lane offset 0, the lane's offset, the
+  // bytes between rows.
+  struct Quarter {
+    const char* src;
+    uint32_t voff, str;
+  };
+  // rag: the tile is ragged (rows are clamped per lane); fids: the quarter's block ids where the tile is a fine one
+  auto quarter_src = [&](Stream& st, bool is_k, uint32_t w, uint64_t fids, bool& rag) __attribute__((always_inline)) {
     const uint32_t code = psa_sched::rec_code(w);
+    Quarter qs;
+    bool is_fine = false;
     if (code != st.code) {
-      st.code = code & 3u;  // (a ragged tile comes back here for every tile)
+      st.code = code & 3u;  // (a ragged or fine tile comes back here for every tile)
       st.base = is_k ? by_level((int)(code & 3u), kb0, kb1, kb2, kb3) : by_level((int)(code & 3u), vb0, vb1, vb2, vb3);
+      if constexpr (WALK == WALK_REC_ANY) {
+        st.str = (code & 3u) == 0 ? (is_k ? P_k_strb : P_v_strb) : (uint32_t)(D * 2);
+        st.voff = (uint32_t)lane_row * st.str + f_chunk;
+        is_fine = code >= psa_sched::REC_CODE_FINE;
+      }
       rag = rag || code == psa_sched::REC_CODE_RAGGED;
     }
-    return st.base + (uint64_t)((w & psa_sched::REC_SRC_MASK) * (uint32_t)(D * 2));
+    qs.str = ANY_STRIDE ? st.str : (uint32_t)(D * 2);
+    qs.voff = ANY_STRIDE ? st.voff : voff_s;
+    qs.src = st.base + (uint64_t)((w & psa_sched::REC_SRC_MASK) * qs.str);
+    if constexpr (WALK == WALK_REC_ANY)
+      if (is_fine) {
+        qs.src = st.base;
+        qs.voff = fine_row(fids, lane, lane_row, P_bn_log2 - (int)(code & 3u)) * (uint32_t)(D * 2) + f_chunk;
+      }
+    return qs;
   };
   // copy instruction N of the wave's quarter (tile rows 4i + N of the quarter) into the tile buffer at LDS_BYTE
-  auto issue_s = [&](const char* src, auto lds_byte, auto n) __attribute__((always_inline)) {
-    constexpr int N = decltype(n)::value;
-    psa_tiles::lds_copy16_imm<decltype(lds_byte)::value + N * F_ISTR, N * D * 2>(src, voff_s, wave_lds);
+  auto issue_s = [&](const Quarter& qs, auto lds_byte, auto n) __attribute__((always_inline)) {
+    constexpr int N = decltype(n)::value, OFF = decltype(lds_byte)::value + N * F_ISTR;
+    if constexpr (ANY_STRIDE) psa_tiles::lds_copy16_imm<OFF, 0>(qs.src + (uint64_t)(N * qs.str), qs.voff, wave_lds);
+    else psa_tiles::lds_copy16_imm<OFF, N * D * 2>(qs.src, qs.voff, wave_lds);
   };
   // the same with the first multiply-add of the exponentials that follow in the wait state between the write of M0 and
   // the copy (returns scale * x + y)
-  auto issue_s_fma = [&](const char* src, auto lds_byte, auto n, float x, float y) __attribute__((always_inline)) {
-    constexpr int N = decltype(n)::value;
-    return psa_tiles::lds_copy16_imm_fma<decltype(lds_byte)::value + N * F_ISTR, N * D * 2>(src, voff_s, wave_lds, P_scale_log2, x, y);
+  auto issue_s_fma = [&](const Quarter& qs, auto lds_byte, auto n, float x, float y) __attribute__((always_inline)) {
+    constexpr int N = decltype(n)::value, OFF = decltype(lds_byte)::value + N * F_ISTR;
+    if constexpr (ANY_STRIDE) return psa_tiles::lds_copy16_imm_fma<OFF, 0>(qs.src + (uint64_t)(N * qs.str), qs.voff, wave_lds, P_scale_log2, x, y);
+    else return psa_tiles::lds_copy16_imm_fma<OFF, N * D * 2>(qs.src, qs.voff, wave_lds, P_scale_log2, x, y);
   };
   // the same with a row index per lane, clamped to the last token (ragged tiles: the walk takes this form only in
   // phases that copy such a tile, so that the usual phase has no branch between its copies)
-  auto issue_clamped = [&](const char* base0, uint32_t w, auto lds_byte, auto n) __attribute__((always_inline)) {
+  auto issue_clamped = [&](const Stream& st, uint32_t w, uint64_t fids, auto lds_byte, auto n) __attribute__((always_inline)) {
     constexpr int N = decltype(n)::value, OFF = decltype(lds_byte)::value + N * F_ISTR;
-    const int lim = psa_sched::rec_code(w) == psa_sched::REC_CODE_RAGGED ? P_L - 1 : 0x7fffffff;
-    const int row = psa_sched::rec_src(w) + lane_row + N;
-    psa_tiles::lds_copy16_row<OFF>(base0, (uint32_t)(row < lim ? row : lim), (uint32_t)(D * 2), f_chunk, wave_lds);
+    const uint32_t code = psa_sched::rec_code(w);
+    const int lim = code == psa_sched::REC_CODE_RAGGED ? P_L - 1 : 0x7fffffff;
+    int row = psa_sched::rec_src(w) + lane_row;
+    if constexpr (WALK == WALK_REC_ANY)
+      if (code >= psa_sched::REC_CODE_FINE) row = (int)fine_row(fids, lane, lane_row, P_bn_log2 - (int)(code & 3u));
+    row += N;
+    psa_tiles::lds_copy16_row<OFF>(st.base, (uint32_t)(row < lim ? row : lim), ANY_STRIDE ? st.str : (uint32_t)(D * 2), f_chunk, wave_lds);
   };
-  auto issue_tile = [&](Stream& st, bool is_k, uint32_t w, auto lds_byte) __attribute__((always_inline)) {
+  auto issue_tile = [&](Stream& st, bool is_k, uint32_t w, uint64_t fids, auto lds_byte) __attribute__((always_inline)) {
     bool rag = false;
-    const char* src = quarter_src(st, is_k, w, rag);
-    if (rag) static_for<G::RPL>([&](auto n) __attribute__((always_inline)) { issue_clamped(st.base, w, lds_byte, n); });
-    else static_for<G::RPL>([&](auto n) __attribute__((always_inline)) { issue_s(src, lds_byte, n); });
+    const Quarter qs = quarter_src(st, is_k, w, fids, rag);
+    if (rag) static_for<G::RPL>([&](auto n) __attribute__((always_inline)) { issue_clamped(st, w, fids, lds_byte, n); });
+    else static_for<G::RPL>([&](auto n) __attribute__((always_inline)) { issue_s(qs, lds_byte, n); });
+  };
+  auto fetch_fine = [&](uint32_t w, uint64_t& f) __attribute__((always_inline)) {
+    if constexpr (WALK == WALK_REC_ANY)
+      if (psa_sched::rec_code(w) >= psa_sched::REC_CODE_FINE) f = fine[psa_sched::rec_src(w) * 4 + wave];
   };
   w_ptr wp = nullptr;                    // this wave's word of the record fetched next
   uint32_t w_v = 0, w_k = 0, w_next = 0;  // words of tiles t+1 (its V goes out next), t+2 (its K), of the next M phase
+  uint64_t f_v = 0, f_k = 0;  // WALK_REC_ANY: block ids of this wave's quarter of tiles t+1 and t+2, where those are fine tiles
   const int T_last = T > 0 ? T - 1 : 0;
   // first copies: K(0), V(0), K(1); ts is left describing tile min(1, T-1) for the copy of V(1)
   if constexpr (GS) {
@@ -850,9 +958,12 @@ __global__ __launch_bounds__(2 * NW * 64, 1) void psa_fwd_pp_kernel(FwdParams p)
       w_v = wp[4];
       w_k = wp[8];
       wp += 12;
-      issue_tile(st_k, true, w_next, IC<0>{});
-      issue_tile(st_v, false, w_next, IC<2 * F_TILE>{});
-      if (T > 1) issue_tile(st_k, true, w_v, IC<F_TILE>{});
+      uint64_t f0 = 0;
+      fetch_fine(w_next, f0);
+      fetch_fine(w_v, f_k);
+      issue_tile(st_k, true, w_next, f0, IC<0>{});
+      issue_tile(st_v, false, w_next, f0, IC<2 * F_TILE>{});
+      if (T > 1) issue_tile(st_k, true, w_v, f_k, IC<F_TILE>{});
     }
   } else if (T > 0) {
     TileSrc a;
@@ -903,7 +1014,7 @@ __global__ __launch_bounds__(2 * NW * 64, 1) void psa_fwd_pp_kernel(FwdParams p)
           cur_c, s, pk, alpha,
           [&]() __attribute__((always_inline)) {
             if (d_cur & 4) {
-              if constexpr (GS) mask_tile_rec(t, s);
+              if constexpr (GS) mask_words<WALK>(s, w_cur, t, recs, fine, P_bn_log2, P_causal != 0, q_idx, hh);
               else mask_tile(t, s);
             }
           },
@@ -966,25 +1077,32 @@ __global__ __launch_bounds__(2 * NW * 64, 1) void psa_fwd_pp_kernel(FwdParams p)
     if (t < T) {
       const uint32_t w3 = *wp;
       wp += 4;
+      // (the block ids of a fine K tile arrive during the copies of the V tile)
+      f_v = f_k;
+      fetch_fine(w_k, f_k);
       bool rag = false;
-      const char* src_v = quarter_src(st_v, false, w_v, rag);
-      const char* src_k = quarter_src(st_k, true, w_k, rag);
+      Quarter src_v = quarter_src(st_v, false, w_v, f_v, rag);
+      Quarter src_k;
+      if constexpr (WALK != WALK_REC_ANY) src_k = quarter_src(st_k, true, w_k, f_k, rag);
+      else rag = rag || psa_sched::rec_code(w_k) == psa_sched::REC_CODE_RAGGED;
       __builtin_amdgcn_s_waitcnt(0x0f70);  // K(t+1), V(t) of this wave have landed (visible to the group after the next barrier)
       float lsum = 0.f;
       if (!rag) {
         static_for<8>([&](auto cc) __attribute__((always_inline)) {
           constexpr int c = decltype(cc)::value;
           float x0;
+          if constexpr (WALK == WALK_REC_ANY && c == 4) src_k = quarter_src(st_k, true, w_k, f_k, rag);
           if constexpr (c < 4) x0 = issue_s_fma(src_v, IC<(2 + (CUR ^ 1)) * F_TILE>{}, IC<c>{}, s[c >> 2][(c & 3) * 4], nb);
           else x0 = issue_s_fma(src_k, IC<CUR * F_TILE>{}, IC<c - 4>{}, s[c >> 2][(c & 3) * 4], nb);
           prob4x(s[c >> 2], (c & 3) * 4, nb, pk[c >> 2] + (c & 3) * 2, lsum, x0);
           __builtin_amdgcn_sched_barrier(0);
         });
       } else {
+        if constexpr (WALK == WALK_REC_ANY) src_k = quarter_src(st_k, true, w_k, f_k, rag);  // (for the stream's state)
         static_for<8>([&](auto cc) __attribute__((always_inline)) {
           constexpr int c = decltype(cc)::value;
-          if constexpr (c < 4) issue_clamped(st_v.base, w_v, IC<(2 + (CUR ^ 1)) * F_TILE>{}, IC<c>{});
-          else issue_clamped(st_k.base, w_k, IC<CUR * F_TILE>{}, IC<c - 4>{});
+          if constexpr (c < 4) issue_clamped(st_v, w_v, f_v, IC<(2 + (CUR ^ 1)) * F_TILE>{}, IC<c>{});
+          else issue_clamped(st_k, w_k, f_k, IC<CUR * F_TILE>{}, IC<c - 4>{});
           prob4(s[c >> 2], (c & 3) * 4, nb, pk[c >> 2] + (c & 3) * 2, lsum);
           __builtin_amdgcn_sched_barrier(0);
         });
@@ -1050,37 +1168,37 @@ __global__ __launch_bounds__(2 * NW * 64, 1) void psa_fwd_pp_kernel(FwdParams p)
 }
 
 
-template <int D, int NW, bool GS = false>
+template <int D, int NW, int WALK = WALK_MAP>
 int launch_fwd(const FwdParams& p, int Nk, hipStream_t stream) {
-  // with a prebuilt schedule the workgroup keeps nothing but its tile buffers in LDS
-  size_t shmem = (size_t)4 * psa_tiles::LtGeom<D>::TILE + (GS ? 0 : (size_t)p.max_tiles * 8 + (size_t)Nk * 2);
+  // only the walk of the map itself keeps more than its tile buffers in LDS
+  size_t shmem = (size_t)4 * psa_tiles::LtGeom<D>::TILE + (WALK != WALK_MAP ? 0 : (size_t)p.max_tiles * 8 + (size_t)Nk * 2);
   if (shmem > 160 * 1024) return PSA_ERR_UNSUPPORTED;
   int rc = PSA_OK;
   psa_dispatch16(p.dtype, [&](auto et) {
     using ET = decltype(et);
-    if (hipFuncSetAttribute((const void*)psa_fwd_lds_kernel<D, NW, GS, ET>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem) != hipSuccess) {
+    if (hipFuncSetAttribute((const void*)psa_fwd_lds_kernel<D, NW, WALK, ET>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem) != hipSuccess) {
       rc = PSA_ERR_LAUNCH;
       return;
     }
-    hipLaunchKernelGGL((psa_fwd_lds_kernel<D, NW, GS, ET>), dim3((unsigned)(p.wg_chunk * p.wg_groups)), dim3(NW * 64), shmem, stream, p);
+    hipLaunchKernelGGL((psa_fwd_lds_kernel<D, NW, WALK, ET>), dim3((unsigned)(p.wg_chunk * p.wg_groups)), dim3(NW * 64), shmem, stream, p);
   });
   return rc;
 }
 
-template <int D, int NW, bool GS>
+template <int D, int NW, int WALK>
 int launch_fwd_pp(FwdParams& p, int Nk, hipStream_t stream) {
-  // with a prebuilt schedule the groups keep nothing but their tile buffers in LDS
-  const size_t sched = GS ? 0 : ((((size_t)p.max_tiles * 8 + (size_t)Nk * 2) + 15) & ~(size_t)15);
+  // only the walk of the map itself keeps more than its tile buffers in LDS
+  const size_t sched = WALK != WALK_MAP ? 0 : ((((size_t)p.max_tiles * 8 + (size_t)Nk * 2) + 15) & ~(size_t)15);
   p.grp_bytes = (int)(4 * psa_tiles::LtGeom<D>::TILE + sched);
   const size_t shmem = 2 * (size_t)p.grp_bytes;
   int rc = PSA_OK;
   psa_dispatch16(p.dtype, [&](auto et) {
     using ET = decltype(et);
-    if (hipFuncSetAttribute((const void*)psa_fwd_pp_kernel<D, NW, GS, ET>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem) != hipSuccess) {
+    if (hipFuncSetAttribute((const void*)psa_fwd_pp_kernel<D, NW, WALK, ET>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem) != hipSuccess) {
       rc = PSA_ERR_LAUNCH;
       return;
     }
-    hipLaunchKernelGGL((psa_fwd_pp_kernel<D, NW, GS, ET>), dim3((unsigned)((p.wg_chunk / 2) * p.wg_groups)), dim3(2 * NW * 64), shmem, stream, p);
+    hipLaunchKernelGGL((psa_fwd_pp_kernel<D, NW, WALK, ET>), dim3((unsigned)((p.wg_chunk / 2) * p.wg_groups)), dim3(2 * NW * 64), shmem, stream, p);
   });
   return rc;
 }
@@ -1156,7 +1274,10 @@ static int fwd_impl(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const void* k_p
   if (two_group) p.wg_chunk = (p.wg_chunk + 1) & ~1;  // pairs never straddle two groups of rows
   p.order = nullptr;
   p.q_index = q_index;
-  p.sched_rec = nullptr; p.sched_tiles = nullptr; p.rec_stride = 0;
+  p.sched_rec = nullptr; p.sched_tiles = nullptr; p.rec_stride = 0; p.sched_fine = nullptr; p.fine_stride = 0;
+  // the record walks form the copy offsets of ragged tiles with 24-bit multiplies
+  const bool rec_walk = psa_walk_shape_ok(D, block_m, block_n, L) && k.stride_l * 2 < (1 << 24) && v.stride_l * 2 < (1 << 24) &&
+                        k.stride_l > 0 && v.stride_l > 0;
   if (schedule != nullptr) {
     // prebuilt schedule (psa_build_schedule with the same shape arguments): issue order, tiles per row, tile records
     psa_sched::Geometry g;
@@ -1165,16 +1286,20 @@ static int fwd_impl(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const void* k_p
     const char* base = (const char*)schedule;
     p.wg_chunk = g.wg_chunk; p.wg_groups = g.wg_groups;
     p.order = (const int32_t*)(base + g.lay.order_off);
-    // the record walk assumes K / V rows D elements apart (the usual layout); other layouts walk the map in the
-    // schedule's issue order
+    // (rows too far apart for the record walk: the map is walked in the schedule's issue order)
     int rc;
-    if (k.stride_l == D && v.stride_l == D) {
+    if (rec_walk) {
       p.sched_rec = (const u32x4*)(base + g.lay.rec_off);
       p.sched_tiles = (const int32_t*)(base + g.lay.tiles_off);
       p.rec_stride = g.lay.rec_stride;
-      rc = D == 128 ? launch_fwd_pp<128, 4, true>(p, Nk, (hipStream_t)stream) : launch_fwd<64, 4, true>(p, Nk, (hipStream_t)stream);
+      p.sched_fine = (const uint16_t*)(base + g.lay.fine_off);
+      p.fine_stride = g.lay.fine_stride;
+      if (block_n == 128 && k.stride_l == D && v.stride_l == D)
+        rc = D == 128 ? launch_fwd_pp<128, 4, WALK_REC>(p, Nk, (hipStream_t)stream) : launch_fwd<64, 4, WALK_REC>(p, Nk, (hipStream_t)stream);
+      else
+        rc = D == 128 ? launch_fwd_pp<128, 4, WALK_REC_ANY>(p, Nk, (hipStream_t)stream) : launch_fwd<64, 4, WALK_REC_ANY>(p, Nk, (hipStream_t)stream);
     } else if (two_group) {
-      rc = launch_fwd_pp<128, 4, false>(p, Nk, (hipStream_t)stream);
+      rc = launch_fwd_pp<128, 4, WALK_MAP>(p, Nk, (hipStream_t)stream);
     } else {
       rc = D == 128 ? launch_fwd<128, 4>(p, Nk, (hipStream_t)stream) : launch_fwd<64, 4>(p, Nk, (hipStream_t)stream);
     }
@@ -1193,7 +1318,11 @@ static int fwd_impl(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const void* k_p
     p.order = order;
   }
   int rc;
-  if (two_group) rc = launch_fwd_pp<128, 4, false>(p, Nk, (hipStream_t)stream);
+  // Dense rows at head dim 64 (bound by vector instructions): computed records, 4393 -> 4115 us at 48 heads of 17776 tokens,
+  // 21.1 -> 17.7 us at 8 of 1000.  Head dim 128 is bound by power: the same walk in the two-group kernel took 0.8 % longer
+  // (12 heads of 32760 tokens), so it keeps the in-kernel list.
+  if (map == nullptr && rec_walk && D == 64) rc = launch_fwd<64, 4, WALK_DENSE>(p, Nk, (hipStream_t)stream);
+  else if (two_group) rc = launch_fwd_pp<128, 4, WALK_MAP>(p, Nk, (hipStream_t)stream);
   else if (D == 128 && block_m == 128) rc = launch_fwd<128, 4>(p, Nk, (hipStream_t)stream);
   else if (D == 128) rc = launch_fwd<128, 2>(p, Nk, (hipStream_t)stream);
   else if (block_m == 128) rc = launch_fwd<64, 4>(p, Nk, (hipStream_t)stream);
@@ -1224,8 +1353,20 @@ extern "C" int psa_fwd_scheduled(psa_tensor4 q, const int32_t* q_index, psa_tens
                                  int causal, psa_stream_t stream) {
   PSA_REQUIRE(schedule != nullptr && map != nullptr, PSA_ERR_ARG, "psa_fwd_scheduled: null schedule or map");
   PSA_REQUIRE((uintptr_t)schedule % 16 == 0, PSA_ERR_ARG, "psa_fwd_scheduled: schedule must be 16-byte aligned");
+  PSA_REQUIRE(q.dtype == PSA_DTYPE_F32 || psa_schedule_shape_ok(D, block_m, block_n, L), PSA_ERR_UNSUPPORTED,
+              "psa_fwd: no scheduled kernel for this shape");
   return fwd_impl(q, k, v, k_pool, v_pool, map, map_elem_bytes, out, lse, B, Hq, Hkv, L, D, block_m, block_n, sm_scale, causal,
                   nullptr, stream, q_index, schedule);
+}
+
+extern "C" int psa_fwd_walk(psa_tensor4 q, const int32_t* q_index, psa_tensor4 k, psa_tensor4 v, const void* k_pool,
+                            const void* v_pool, const void* map, int map_elem_bytes, const void* walk, psa_tensor4 out, float* lse,
+                            int B, int Hq, int Hkv, int L, int D, int block_m, int block_n, float sm_scale, int causal,
+                            psa_stream_t stream) {
+  PSA_REQUIRE(walk != nullptr && map != nullptr, PSA_ERR_ARG, "psa_fwd_walk: null walk or map");
+  PSA_REQUIRE((uintptr_t)walk % 16 == 0, PSA_ERR_ARG, "psa_fwd_walk: walk must be 16-byte aligned");
+  return fwd_impl(q, k, v, k_pool, v_pool, map, map_elem_bytes, out, lse, B, Hq, Hkv, L, D, block_m, block_n, sm_scale, causal,
+                  nullptr, stream, q_index, walk);
 }
 
 // ---- the variant that allocates nothing ------------------------------------------------------------------

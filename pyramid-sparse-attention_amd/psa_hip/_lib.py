@@ -102,6 +102,13 @@ SIGNATURES = {
         [Tensor4, c_void_p, Tensor4, Tensor4, c_void_p, c_void_p, c_void_p, c_int, c_void_p, Tensor4, c_void_p, c_int, c_int, c_int,
          c_int, c_int, c_int, c_int, c_float, c_int, c_void_p],
     ),
+    "psa_walk_bytes": (c_int64, [c_int, c_int, c_int, c_int, c_int, c_int, c_int]),
+    "psa_build_walk": (c_int, [c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_void_p]),
+    "psa_fwd_walk": (
+        c_int,
+        [Tensor4, c_void_p, Tensor4, Tensor4, c_void_p, c_void_p, c_void_p, c_int, c_void_p, Tensor4, c_void_p, c_int, c_int, c_int,
+         c_int, c_int, c_int, c_int, c_float, c_int, c_void_p],
+    ),
     "psa_fwd_noalloc": (
         c_int,
         [Tensor4, Tensor4, Tensor4, c_void_p, c_void_p, c_void_p, c_int, Tensor4, c_void_p, c_int, c_int, c_int, c_int,

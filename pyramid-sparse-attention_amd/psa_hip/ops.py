@@ -498,6 +498,13 @@ def build_schedule(level_map_: torch.Tensor, Hkv: int, L: int, D: int, block_m: 
     return out
 
 
+# Rows of the map above which a map of 64- / 32-key blocks is listed before it is walked.  The listing takes two launches
+# (about 5 us); the walk saves the look-ups, which bound the kernel at head dim 64.  Both sides in us, listed against in-kernel:
+# 520 rows head dim 64 51.4 / 48.6, 2080 rows 121.6 / 123.3; 16944 rows (45106 tokens, 48 heads) 4.5 ms / 4.9 ms.
+# At head dim 128, which is bound by power, 568 rows 94.1 / 95.9, 2080 rows 233 / 231 (in the layer 377 / 385).
+_WALK_MIN_ROWS = 1024
+
+
 def sparse_attention_fwd(
     q: torch.Tensor,
     k: torch.Tensor,
@@ -549,23 +556,28 @@ def sparse_attention_fwd(
     lse = torch.empty(B, Hq, L, dtype=torch.float32, device=q.device) if return_lse else None
     if q_index is not None:
         q_index = _check_index(q_index, L)
-    n_sched = 0
+    shape = (B, Hq, Hkv, L, D, block_m, block_n)
+    n_walk = 0
     if level_map_ is not None and balance and schedule is not False and qb.dtype in _T16:
-        n_sched = lib.psa_schedule_bytes(B, Hq, Hkv, L, D, block_m, block_n)
-    if n_sched > 0:
-        # the map's tile schedule is built once (one pass over the map) and walked by the kernel
-        if not isinstance(schedule, torch.Tensor):
-            schedule = build_schedule(level_map_, Hkv, L, D, block_m, block_n, causal)
+        if block_n == 128 or B * Hq * Mq > _WALK_MIN_ROWS:
+            n_walk = lib.psa_walk_bytes(*shape)
+    if n_walk > 0:
+        # the map's tiles are listed once (one pass over the map) and walked by the kernel
+        walk = schedule
+        if not isinstance(schedule, torch.Tensor) or block_n != 128:  # (build_schedule serves 128-key blocks)
+            walk = torch.empty(n_walk, dtype=torch.uint8, device=q.device)
+            with torch.cuda.device(q.device):
+                check(lib.psa_build_walk(_ptr(level_map_), level_map_.element_size(), _ptr(walk), *shape, int(causal), _stream(q)), "psa_build_walk")
         with torch.cuda.device(q.device):
-            check(lib.psa_fwd_scheduled(_t4(qb), _ptr(q_index), _t4(kb), _t4(vb), _ptr(kp), _ptr(vp), _ptr(level_map_),
-                                        level_map_.element_size(), _ptr(schedule), _t4(o), _ptr(lse), B, Hq, Hkv, L, D, block_m, block_n,
-                                        sm_scale, int(causal), _stream(q)), "psa_fwd_scheduled")
+            check(lib.psa_fwd_walk(_t4(qb), _ptr(q_index), _t4(kb), _t4(vb), _ptr(kp), _ptr(vp), _ptr(level_map_),
+                                   level_map_.element_size(), _ptr(walk), _t4(o), _ptr(lse), *shape, sm_scale, int(causal),
+                                   _stream(q)), "psa_fwd_walk")
     else:
         ws = None
         if level_map_ is not None and balance:
             ws = torch.empty(lib.psa_fwd_workspace_bytes(B, Hq, L, block_m) // 4, dtype=torch.int32, device=q.device)
         tail = (_t4(kb), _t4(vb), _ptr(kp), _ptr(vp), _ptr(level_map_), 1 if level_map_ is None else level_map_.element_size(), _t4(o),
-                _ptr(lse), B, Hq, Hkv, L, D, block_m, block_n, sm_scale, int(causal), _ptr(ws), _stream(q))
+                _ptr(lse), *shape, sm_scale, int(causal), _ptr(ws), _stream(q))
         with torch.cuda.device(q.device):
             if q_index is None:
                 check(lib.psa_fwd(_t4(qb), *tail), "psa_fwd")
