@@ -248,90 +248,128 @@ __global__ __launch_bounds__(256, 2) void psa_est_gemm_lds_kernel(EstParams p) {
   }
 }
 
+// The contraction for fp32 tensors: fp32 operands on the matrix cores' fp32 instruction (v_mfma_f32_16x16x4_f32), the same
+// workspace contents as the 16-bit kernel (group maxima R^T [key group][query row] in log2 units, row maxima per key
+// share).  One workgroup = 32 sampled query rows (two B-operand sets share every K operand) x one share of the keys; its 4
+// waves take 32-key steps in turn.  K rows go from global memory straight into the operand registers (a lane reads 16
+// consecutive bytes of a row per four k-steps; the next step's rows are requested before the current step's products), so
+// the waves run free of barriers.  Shares (grid z, up to 4) are cut until there are two workgroups per CU.
+// 2 heads x 1024 sampled rows x 1024 keys x 64: 72 us on the vector units (two LDS operands per 4 FMAs), 9 us here.
+template <int D, int GPC>
+__global__ __launch_bounds__(256) void psa_est_gemm_f32_kernel(EstParams p) {
+  constexpr int SQ = D / 16, RS = 2, NV = 1 << GPC;  // NV key groups per 32 keys
+  constexpr int kn_log2 = 5 - GPC, keep_n = 1 << kn_log2;
+  __shared__ float s_m[4][RS * 16];
+  const float* qg = (const float*)p.q;
+  const float* kg = (const float*)p.k;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, g4 = lane >> 4;
+  const int bh = blockIdx.y, h = bh % p.Hq, b = bh / p.Hq, hk = h / (p.Hq / p.Hkv);
+  const int row0 = blockIdx.x * (RS * 16);
+  const int32_t* oq = p.off_q ? p.off_q + (int64_t)bh * (1 << p.keep_m_log2) : nullptr;
+  const int32_t* ok = p.off_k ? p.off_k + ((int64_t)b * p.Hkv + hk) * keep_n : nullptr;
+  // operands: step 4 c + j takes channel 16 c + 4 g + j
+  f32x4 qf[RS][SQ];
+#pragma unroll
+  for (int rs = 0; rs < RS; ++rs) {
+    int src = sampled_src(row0 + rs * 16 + l16, p.Ms, p.keep_m_log2, p.bm, oq, p.Lq);
+    if (p.q_index != nullptr) src = clamp_row(p.q_index[src], p.Lq);
+    const float* qp = qg + b * p.q_sb + h * p.q_sh + (int64_t)src * p.q_sl + 4 * g4;
+#pragma unroll
+    for (int c = 0; c < SQ; ++c) qf[rs][c] = *(const f32x4*)(qp + 16 * c);
+  }
+  const float* kb = kg + b * p.k_sb + hk * p.k_sh + 4 * g4;
+  // (the sampled offset of a lane's key is the same in every step: steps span whole key groups)
+  const int off0 = ok ? ok[l16 & (keep_n - 1)] : l16 & (keep_n - 1);
+  const int off1 = ok ? ok[(16 + l16) & (keep_n - 1)] : (16 + l16) & (keep_n - 1);
+  const int last_off = ok ? ok[keep_n - 1] : keep_n - 1;
+  auto key_row = [&](int r, int off) __attribute__((always_inline)) {
+    // padding keys replicate the last sampled one (Ns is a multiple of keep_n)
+    const int src = r < p.Ns ? (r >> kn_log2) * p.bn + off : ((p.Ns - 1) >> kn_log2) * p.bn + last_off;
+    return kb + (int64_t)(src < p.Lk ? src : p.Lk - 1) * p.k_sl;
+  };
+  const int steps = p.Ns_pad / 32, ks = blockIdx.z;
+  const int s_begin = (int)((int64_t)steps * ks / p.ksplit), s_end = (int)((int64_t)steps * (ks + 1) / p.ksplit);
+  f32x4 ka[2][SQ];
+  auto load = [&](int st) __attribute__((always_inline)) {
+    const float* r0 = key_row(st * 32 + l16, off0);
+    const float* r1 = key_row(st * 32 + 16 + l16, off1);
+#pragma unroll
+    for (int c = 0; c < SQ; ++c) {
+      ka[0][c] = *(const f32x4*)(r0 + 16 * c);
+      ka[1][c] = *(const f32x4*)(r1 + 16 * c);
+    }
+  };
+  float m_run[RS];
+#pragma unroll
+  for (int rs = 0; rs < RS; ++rs) m_run[rs] = -INFINITY;
+  float* const rt = p.rt + (int64_t)bh * p.n_d * p.Ms_pad + row0 + l16;
+  int st = s_begin + wave;
+  if (st < s_end) load(st);
+  for (; st < s_end; st += 4) {
+    f32x4 s[RS][2];
+#pragma unroll
+    for (int rs = 0; rs < RS; ++rs)
+#pragma unroll
+      for (int x = 0; x < 2; ++x) s[rs][x] = f32x4{0.f, 0.f, 0.f, 0.f};
+    f32x4 a[2][SQ];
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+      for (int c = 0; c < SQ; ++c) a[x][c] = ka[x][c];
+    if (st + 4 < s_end) load(st + 4);
+#pragma unroll
+    for (int c = 0; c < SQ; ++c)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+          for (int rs = 0; rs < RS; ++rs) s[rs][x] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[x][c][j], qf[rs][c][j], s[rs][x], 0, 0, 0);
+    // accumulator: keys 4 g .. 4 g + 3 of block x of the row l16 of set rs
+#pragma unroll
+    for (int rs = 0; rs < RS; ++rs) {
+      float v[2];
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        v[x] = s[rs][x][0] * p.qk_scale;
+#pragma unroll
+        for (int i = 1; i < 4; ++i) v[x] = fmaxf(v[x], s[rs][x][i] * p.qk_scale);
+        v[x] = fmaxf(v[x], __shfl_xor(v[x], 16, 64));  // 8 keys
+        if constexpr (GPC < 2) v[x] = fmaxf(v[x], __shfl_xor(v[x], 32, 64));  // 16 keys
+      }
+      if constexpr (GPC == 0) v[0] = v[1] = fmaxf(v[0], v[1]);
+      m_run[rs] = fmaxf(m_run[rs], fmaxf(v[0], v[1]));
+      float* const o = rt + (int64_t)st * NV * p.Ms_pad + rs * 16;
+      if constexpr (GPC == 0) {
+        if (g4 == 0) o[0] = v[0];
+      } else if constexpr (GPC == 1) {
+        if (g4 < 2) o[(int64_t)g4 * p.Ms_pad] = g4 == 0 ? v[0] : v[1];
+      } else {
+        // groups of block x: 2 x (lanes of g = 0, 1) and 2 x + 1 (g = 2, 3)
+        if ((g4 & 1) == 0) {
+          o[(int64_t)(g4 >> 1) * p.Ms_pad] = v[0];
+          o[(int64_t)(2 + (g4 >> 1)) * p.Ms_pad] = v[1];
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int rs = 0; rs < RS; ++rs) {
+    float m = m_run[rs];
+    if constexpr (GPC == 2) m = fmaxf(m, __shfl_xor(m, 32, 64));
+    if (g4 == 0) s_m[wave][rs * 16 + l16] = m;
+  }
+  __syncthreads();
+  if (tid < RS * 16)
+    p.mrow[((int64_t)bh * p.ksplit + ks) * p.Ms_pad + row0 + tid] = fmaxf(fmaxf(s_m[0][tid], s_m[1][tid]), fmaxf(s_m[2][tid], s_m[3][tid]));
+}
+
 // one workgroup per (b, h, query group): Po[i, :] from R^T and m.
 // A lane reads 4 consecutive rows (16 bytes) of one key group, keep_m/4 neighbouring lanes cover the group's
 // rows (one contiguous run of the workspace), a wave 256/keep_m key groups per load; the maximum over the
 // group's rows is an in-lane maximum plus a butterfly over those lanes.
 // Leaves the un-normalised row in s_e[0 .. n_d) and returns its sum (fixed summation order); 256 threads.
-// The contraction for fp32 tensors: fp32 operands and arithmetic (vector FMAs), the same workspace contents as the
-// MFMA kernel (group maxima R^T [key group][query row] in log2 units, row maxima; one share of the keys).  One
-// workgroup per 64 sampled query rows; key tiles of 64 sampled keys go to LDS channel-major; thread (t / 16, t % 16)
-// owns rows ty + 16 i and keys tx + 16 j of a tile, the tile's logits pass through LDS for the group maxima.
-template <int D, int RI>
-__global__ __launch_bounds__(256) void psa_est_gemm_f32_kernel(EstParams p) {
-  constexpr int QR = 16 * RI;  // sampled query rows per workgroup
-  constexpr int DP = D + 1, KP = TK + 1;
-  extern __shared__ __align__(16) unsigned char smem_f32[];
-  float* Qs = (float*)smem_f32;  // [QR][DP]
-  float* Kt = Qs + QR * DP;      // [D][KP]
-  float* Ss = Kt + D * KP;       // [QR][KP]
-  const float* qg = (const float*)p.q;
-  const float* kg = (const float*)p.k;
-  const int tid = threadIdx.x, ty = tid >> 4, tx = tid & 15;
-  const int bh = blockIdx.y, h = bh % p.Hq, b = bh / p.Hq, hk = h / (p.Hq / p.Hkv);
-  const int row0 = blockIdx.x * QR;
-  const int32_t* oq = p.off_q ? p.off_q + (int64_t)bh * (1 << p.keep_m_log2) : nullptr;
-  const int32_t* ok = p.off_k ? p.off_k + ((int64_t)b * p.Hkv + hk) * (1 << p.keep_n_log2) : nullptr;
-  for (int u = tid; u < QR * (D / 4); u += 256) {
-    const int r = u / (D / 4), c4 = u % (D / 4);
-    int src = sampled_src(row0 + r, p.Ms, p.keep_m_log2, p.bm, oq, p.Lq);
-    if (p.q_index != nullptr) src = clamp_row(p.q_index[src], p.Lq);
-    const f32x4 x = *(const f32x4*)(qg + b * p.q_sb + h * p.q_sh + (int64_t)src * p.q_sl + c4 * 4);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) Qs[r * DP + c4 * 4 + e] = x[e];
-  }
-  const int keep_n = 1 << p.keep_n_log2, gpt = TK >> p.keep_n_log2;  // key groups per tile
-  float m_run = -INFINITY;  // of row (tid / 4) for the threads that write group maxima, see below
-  float* rt = p.rt + (int64_t)bh * p.n_d * p.Ms_pad + row0;
-  const float* kb = kg + b * p.k_sb + hk * p.k_sh;
-  for (int t0 = 0; t0 < p.Ns_pad; t0 += TK) {
-    __syncthreads();
-    for (int u = tid; u < TK * (D / 4); u += 256) {
-      const int r = u / (D / 4), c4 = u % (D / 4);
-      const int src = sampled_src(t0 + r, p.Ns, p.keep_n_log2, p.bn, ok, p.Lk);
-      const f32x4 x = *(const f32x4*)(kb + (int64_t)src * p.k_sl + c4 * 4);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) Kt[(c4 * 4 + e) * KP + r] = x[e];
-    }
-    __syncthreads();
-    float s[RI][4];
-#pragma unroll
-    for (int i = 0; i < RI; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) s[i][j] = 0.f;
-    for (int d = 0; d < D; ++d) {
-      float qv[RI], kv[4];
-#pragma unroll
-      for (int i = 0; i < RI; ++i) qv[i] = Qs[(ty + 16 * i) * DP + d];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) kv[j] = Kt[d * KP + tx + 16 * j];
-#pragma unroll
-      for (int i = 0; i < RI; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) s[i][j] = __builtin_fmaf(qv[i], kv[j], s[i][j]);
-    }
-#pragma unroll
-    for (int i = 0; i < RI; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) Ss[(ty + 16 * i) * KP + tx + 16 * j] = s[i][j] * p.qk_scale;
-    __syncthreads();
-    // group maxima: (row, group) pairs, row fastest so that the stores are coalesced
-    for (int u = tid; u < QR * gpt; u += 256) {
-      const int r = u % QR, g = u / QR;
-      float mx = -INFINITY;
-      for (int c = 0; c < keep_n; ++c) mx = fmaxf(mx, Ss[r * KP + g * keep_n + c]);
-      rt[(int64_t)((t0 >> p.keep_n_log2) + g) * p.Ms_pad + r] = mx;
-    }
-    // row maxima: thread t < QR keeps the maximum of row t
-    if (tid < QR) {
-      float mx = m_run;
-      for (int c = 0; c < TK; ++c) mx = fmaxf(mx, Ss[tid * KP + c]);
-      m_run = mx;
-    }
-  }
-  if (tid < QR) p.mrow[(int64_t)bh * p.Ms_pad + row0 + tid] = m_run;
-}
-
 __device__ __forceinline__ float est_reduce_row(const EstParams& p, float* s_e, float* s_part, int i, int bh) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int lpg_log2 = p.keep_m_log2 - 2;            // lanes per key group
@@ -417,20 +455,16 @@ int launch_est(EstParams& p, int B, hipStream_t stream, const LevelMapParams* lp
   while (p.ksplit < EST_MAX_KSPLIT && wgs * p.ksplit < 3 * 256 && tiles / (p.ksplit * 2) >= 8) p.ksplit *= 2;
   grid.z = (unsigned)p.ksplit;
   if (p.dtype == PSA_DTYPE_F32) {
+    // 32 rows per workgroup, 32 keys per step: shares of at least 4 steps (one per wave)
+    const int64_t wgs32 = (int64_t)(p.Ms_pad / 32) * B * p.Hq;
     p.ksplit = 1;
-    // 64 sampled rows per workgroup, or 32 / 16 while the launch would have fewer than two workgroups per CU
-    auto go = [&](auto ri_c) -> int {
-      constexpr int RI = decltype(ri_c)::value, QR = 16 * RI;
-      const size_t shmem = (size_t)(QR * (D + 1) + D * (TK + 1) + QR * (TK + 1)) * sizeof(float);
-      if (hipFuncSetAttribute((const void*)psa_est_gemm_f32_kernel<D, RI>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem) != hipSuccess)
-        return PSA_ERR_LAUNCH;
-      hipLaunchKernelGGL((psa_est_gemm_f32_kernel<D, RI>), dim3((unsigned)(p.Ms_pad / QR), (unsigned)(B * p.Hq)), dim3(256), shmem, stream, p);
-      return PSA_OK;
-    };
-    int ri = 4;
-    while (ri > 1 && (int64_t)(p.Ms_pad / (16 * ri)) * B * p.Hq < 512) ri >>= 1;
-    const int rc32 = ri == 4 ? go(std::integral_constant<int, 4>{}) : ri == 2 ? go(std::integral_constant<int, 2>{}) : go(std::integral_constant<int, 1>{});
-    if (rc32 != PSA_OK) return rc32;
+    while (p.ksplit < EST_MAX_KSPLIT && wgs32 * p.ksplit < 512 && p.Ns_pad / 32 / (p.ksplit * 2) >= 4) p.ksplit *= 2;
+    const dim3 g32((unsigned)(p.Ms_pad / 32), (unsigned)(B * p.Hq), (unsigned)p.ksplit);
+    switch (p.keep_n_log2) {
+      case 5: hipLaunchKernelGGL((psa_est_gemm_f32_kernel<D, 0>), g32, dim3(256), 0, stream, p); break;
+      case 4: hipLaunchKernelGGL((psa_est_gemm_f32_kernel<D, 1>), g32, dim3(256), 0, stream, p); break;
+      default: hipLaunchKernelGGL((psa_est_gemm_f32_kernel<D, 2>), g32, dim3(256), 0, stream, p); break;
+    }
   }
   psa_dispatch16(p.dtype, [&](auto et) {
     using ET = decltype(et);
