@@ -246,26 +246,33 @@ extern "C" int psa_list_from_map(const void* map, int map_elem_bytes, int32_t* l
 // ---------------------------------------------------------------------------------------
 // map = min(map, cap[bh, col])
 // ---------------------------------------------------------------------------------------
-__global__ void psa_map_min_cap_kernel(void* map, int map_elem, const int32_t* cap, int Mq, int Nk) {
+__global__ void psa_map_min_cap_kernel(void* map, int map_elem, const int32_t* cap, int Hq, int n_rep, int Mq, int Nk) {
   const int64_t bh = blockIdx.y;
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= (int64_t)Mq * Nk) return;
   const int col = (int)(i % Nk);
   const int64_t idx = bh * Mq * Nk + i;
   const int m = load_map(map, idx, map_elem);
-  const int c = cap[bh * Nk + col];
+  const int c = cap[((bh / Hq) * (Hq / n_rep) + (bh % Hq) / n_rep) * Nk + col];
   if (c < m) store_map(map, idx, map_elem, c);
+}
+
+// (cap per kv head: query head h of a batch takes the cap of kv head h / (Hq / Hkv))
+int psa_map_min_cap_heads(void* map, int map_elem_bytes, const int32_t* cap, int B, int Hq, int Hkv, int Mq, int Nk, psa_stream_t stream) {
+  const int64_t bh = (int64_t)B * Hq;
+  PSA_REQUIRE(map && cap, PSA_ERR_ARG, "psa_map_min_cap: null pointer");
+  PSA_REQUIRE(map_elem_bytes == 1 || map_elem_bytes == 4, PSA_ERR_ARG, "psa_map_min_cap: map_elem_bytes must be 1 or 4");
+  PSA_REQUIRE(bh > 0 && bh <= 65535 && Mq > 0 && Nk > 0 && Hkv > 0 && Hq % Hkv == 0, PSA_ERR_ARG, "psa_map_min_cap: bad sizes");
+  int64_t n = (int64_t)Mq * Nk;
+  hipLaunchKernelGGL(psa_map_min_cap_kernel, dim3((unsigned)((n + 255) / 256), (unsigned)bh), dim3(256), 0,
+                     (hipStream_t)stream, map, map_elem_bytes, cap, Hq, Hq / Hkv, Mq, Nk);
+  return psa_check_launch("psa_map_min_cap");
 }
 
 extern "C" int psa_map_min_cap(void* map, int map_elem_bytes, const int32_t* cap, int64_t bh, int Mq, int Nk,
                                psa_stream_t stream) {
-  PSA_REQUIRE(map && cap, PSA_ERR_ARG, "psa_map_min_cap: null pointer");
-  PSA_REQUIRE(map_elem_bytes == 1 || map_elem_bytes == 4, PSA_ERR_ARG, "psa_map_min_cap: map_elem_bytes must be 1 or 4");
-  PSA_REQUIRE(bh > 0 && bh <= 65535 && Mq > 0 && Nk > 0, PSA_ERR_ARG, "psa_map_min_cap: bad sizes");
-  int64_t n = (int64_t)Mq * Nk;
-  hipLaunchKernelGGL(psa_map_min_cap_kernel, dim3((unsigned)((n + 255) / 256), (unsigned)bh), dim3(256), 0,
-                     (hipStream_t)stream, map, map_elem_bytes, cap, Mq, Nk);
-  return psa_check_launch("psa_map_min_cap");
+  PSA_REQUIRE(bh > 0 && bh <= 65535, PSA_ERR_ARG, "psa_map_min_cap: bad sizes");
+  return psa_map_min_cap_heads(map, map_elem_bytes, cap, 1, (int)bh, (int)bh, Mq, Nk, stream);
 }
 
 // ---------------------------------------------------------------------------------------

@@ -15,6 +15,7 @@ from typing import Dict, Optional, Tuple
 
 import torch
 import torch.nn as nn
+from torch.autograd import forward_ad
 
 from .. import ops
 from ..kernels.psa_kernel_legacy import _sparse_attention
@@ -55,6 +56,8 @@ def sparse_attention_factory(BLOCK_M=128, BLOCK_N=32, POOLING_BLOCK_N=128, causa
     def _fn(q, k, v, block_sparse_dense, sm_scale=None):
         return _sparse_attention.apply(q, k, v, block_sparse_dense, sm_scale, BLOCK_M, POOLING_BLOCK_N, causal)
 
+    # (the layer on this function is also one library call: ops.causal_layer_fwd)
+    _fn.one_call_causal = bool(causal) if BLOCK_M == POOLING_BLOCK_N == 128 else None
     return _fn
 
 
@@ -82,6 +85,16 @@ def calc_density(mask: torch.Tensor, causal: bool):
 
 def adaptive_block_sparse_attn(q, k, v, config: AttentionConfig, sparse_attention_fn, compute_stats: bool = True):
     block = config.query_block
+    needs_grad = torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad)
+    # (dual tensors of forward-mode differentiation go to the autograd function, which has no such rule and says so)
+    plain = not needs_grad and forward_ad._current_level < 0
+    if (plain and not compute_stats and block == 128 and config.importance_method == "xattn"
+            and getattr(sparse_attention_fn, "one_call_causal", None) is bool(config.causal_main)):
+        out = ops.causal_layer_fwd(q, k, v, config.mask_ratios, config.mask_mode, config.text_length, block, config.xattn_stride,
+                                   config.xattn_chunk_size, config.causal_main,
+                                   (config.sim_2x_threshold, config.sim_4x_threshold, config.sim_8x_threshold))
+        if out is not None:
+            return out, 0.0, []
     with torch.no_grad():
         if config.importance_method != "xattn":
             raise ValueError(f"Unknown importance_method: {config.importance_method}")

@@ -11,8 +11,27 @@ from ._lib import Tensor4, check, lib
 LEVELS = (1, 2, 4, 8)
 
 
-def _stream(t: torch.Tensor):
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+def _stream(t: torch.Tensor) -> int:
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
+
+
+class _Here:
+    """The current device is the right one already."""
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *exc):
+        return False
+
+
+_HERE = _Here()
+
+
+def _on(device: torch.device):
+    """Context in which `device` is current (torch.cuda.device, whose bookkeeping costs more than a launch, only where the
+    device has to be switched)."""
+    return _HERE if device.index is None or device.index == torch.cuda.current_device() else torch.cuda.device(device)
 
 
 def _require_gpu(*ts):
@@ -32,8 +51,8 @@ def _kernel_view(x: torch.Tensor, types=(torch.bfloat16, torch.float16, torch.fl
         raise ValueError("expected a [B, H, L, D] tensor, got shape %s" % (tuple(x.shape),))
     if x.dtype not in types:
         x = x.to(torch.bfloat16)
-    per16 = 16 // x.element_size()
-    ok = x.stride(3) == 1 and all(s % per16 == 0 for s in x.stride()[:3]) and x.data_ptr() % 16 == 0
+    sb, sh, sl, sd = x.stride()
+    ok = sd == 1 and (sb | sh | sl) % (16 // x.element_size()) == 0 and x.data_ptr() % 16 == 0
     return x if ok else x.contiguous()
 
 
@@ -52,11 +71,12 @@ def _same_type(*ts):
 
 
 def _t4(x: torch.Tensor) -> Tensor4:
-    return Tensor4(x.data_ptr(), x.stride(0), x.stride(1), x.stride(2), _DTYPE_ID[x.dtype], 0)
+    sb, sh, sl, _ = x.stride()
+    return Tensor4(x.data_ptr(), sb, sh, sl, _DTYPE_ID[x.dtype], 0)
 
 
 def _ptr(t: Optional[torch.Tensor]):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 # ----------------------------------------------------------------------------- pooling
@@ -78,7 +98,7 @@ def pool_kv(k: torch.Tensor, v: torch.Tensor, block_n: int, out: Optional[Tuple[
         for t in (kp, vp):
             if t.dtype != k.dtype or t.numel() != n or not t.is_contiguous() or t.device != k.device:
                 raise ValueError("pool_kv: out must be two contiguous %s buffers of %d elements on %s" % (k.dtype, n, k.device))
-    with torch.cuda.device(k.device):
+    with _on(k.device):
         check(lib.psa_pool_kv(_t4(k), _t4(v), _ptr(kp), _ptr(vp), B, H, L, D, block_n, _stream(k)), "psa_pool_kv")
     return kp, vp
 
@@ -134,7 +154,7 @@ def pool_kv_indexed(k: torch.Tensor, v: torch.Tensor, index: torch.Tensor, block
     kp = torch.empty(n, dtype=k.dtype, device=k.device)
     vp = torch.empty(n, dtype=k.dtype, device=k.device)
     ko, vo = torch.empty_like(k, memory_format=torch.contiguous_format), torch.empty_like(v, memory_format=torch.contiguous_format)
-    with torch.cuda.device(k.device):
+    with _on(k.device):
         check(lib.psa_pool_kv_indexed(_t4(k), _t4(v), _ptr(index), _t4(ko), _t4(vo), _ptr(kp), _ptr(vp), B, H, L, D, block_n,
                                       _stream(k)), "psa_pool_kv_indexed")
     return kp, vp, ko, vo
@@ -168,7 +188,7 @@ def draw_sample_offsets(B: int, Hq: int, Hkv: int, block_m: int, keep_m: int, bl
         seed = (torch.initial_seed() * 0x9E3779B97F4A7C15 + _DRAWS[0]) & 0xFFFFFFFFFFFFFFFF
     off_q = torch.empty(B, Hq, keep_m, dtype=torch.int32, device=device)
     off_k = torch.empty(B, Hkv, keep_n, dtype=torch.int32, device=device)
-    with torch.cuda.device(device):
+    with _on(device):
         check(lib.psa_draw_sample_offsets(_ptr(off_q), _ptr(off_k), B * Hq, B * Hkv, block_m, keep_m, block_n, keep_n,
                                           int(seed) & 0xFFFFFFFFFFFFFFFF, _stream(off_q)), "psa_draw_sample_offsets")
     return off_q, off_k
@@ -206,7 +226,7 @@ def estimate_sampled(
     ws = torch.empty(lib.psa_estimate_workspace_bytes(B, Hq, Lq, Lk, block_m, block_n, keep_m, keep_n), dtype=torch.uint8, device=q.device)
     tail = (_ptr(off_q), _ptr(off_k), _ptr(scores), _ptr(ws), B, Hq, Hkv, Lq, Lk, D, block_m, block_n, keep_m, keep_n, float(sm_scale),
             out_rows, out_cols, _stream(q))
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         if q_index is None:
             check(lib.psa_estimate_sampled(_t4(q), _t4(k), *tail), "psa_estimate_sampled")
         else:
@@ -255,8 +275,7 @@ def estimate_sampled_map(
     if div < 1:
         raise ValueError("compute_tile must not exceed blocksize")
     n = len(items)
-    lv = (ctypes.c_int32 * n)(*[int(i[0]) for i in items])
-    hi = (ctypes.c_double * n)(*[float(i[1][1]) for i in items])
+    lv, hi = _level_items(items)
     tb = (text_length + block_n - 1) // block_n if text_length > 0 else 0
     # (maps wider than about 5000 columns do not fit the fused kernel's LDS: the library then needs the scores buffer)
     scores = torch.empty(B, Hq, Mq, Nk, dtype=torch.float32, device=q.device) if (return_scores or Nk > 4096) else None
@@ -264,7 +283,7 @@ def estimate_sampled_map(
     ws = torch.empty(lib.psa_estimate_workspace_bytes(B, Hq, Lq, Lk, block_m, block_n, keep_m, keep_n), dtype=torch.uint8, device=q.device)
     tail = (_ptr(off_q), _ptr(off_k), _ptr(scores), _ptr(ws), B, Hq, Hkv, Lq, Lk, D, block_m, block_n, keep_m, keep_n, float(sm_scale),
             Mq, Nk, _ptr(out), out.element_size(), m, n, lv, hi, div, tb, float(min_full_attn_ratio), _stream(q))
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         if q_index is None:
             check(lib.psa_estimate_sampled_map(_t4(q), _t4(k), *tail), "psa_estimate_sampled_map")
         else:
@@ -292,6 +311,11 @@ def _items(mask_ratios, mode: str):
     return items, m, newtype
 
 
+def _level_items(items):
+    n = len(items)
+    return (ctypes.c_int32 * n)(*[int(i[0]) for i in items]), (ctypes.c_double * n)(*[float(i[1][1]) for i in items])
+
+
 def level_map(
     scores: torch.Tensor,
     mask_ratios,
@@ -311,13 +335,12 @@ def level_map(
     s = scores.to(torch.float32).contiguous()
     B, H, Mq, Nk = s.shape
     n = len(items)
-    lv = (ctypes.c_int32 * n)(*[int(i[0]) for i in items])
-    hi = (ctypes.c_double * n)(*[float(i[1][1]) for i in items])
+    lv, hi = _level_items(items)
     rows = B * H * Mq
     div = blocksize // compute_tile
     if div < 1:
         raise ValueError("compute_tile must not exceed blocksize")
-    with torch.cuda.device(s.device):
+    with _on(s.device):
         if newtype:
             out = torch.empty(B, H, Mq, Nk + n, dtype=torch.int32, device=s.device)
             rc = lib.psa_level_map(_ptr(s), None, 4, _ptr(out), rows, Nk, m, n, lv, hi, div, 0, float(min_full_attn_ratio), _stream(s))
@@ -352,7 +375,7 @@ def level_map_qwen(scores: torch.Tensor, mask_ratios, text_length: int, mode: st
     special = min(-(-text_length // block_size) if text_length > 0 else 0, S)
     out = torch.empty(B, H, S, S, dtype=map_dtype, device=s.device)
     m = _lib.PSA_MODE_TOPK if mode == "topk" else _lib.PSA_MODE_THRESHOLDBOUND
-    with torch.cuda.device(s.device):
+    with _on(s.device):
         check(lib.psa_level_map_qwen(_ptr(s), _ptr(out), out.element_size(), B * H, S, m, n, lv, lo, hi, special, int(causal), _stream(s)),
               "psa_level_map_qwen")
     return out
@@ -367,7 +390,7 @@ def estimate_xattn(q: torch.Tensor, k: torch.Tensor, block_size: int = 128, stri
     Hkv, Lk = kb.shape[1], kb.shape[2]
     est = torch.empty(B, Hq, -(-Lq // block_size), -(-Lk // block_size), dtype=torch.float32, device=q.device)
     ws = torch.empty(lib.psa_estimate_xattn_workspace_bytes(B, Hq, Lq, Lk, block_size, stride, chunk_size), dtype=torch.uint8, device=q.device)
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         check(lib.psa_estimate_xattn(_t4(qb), _t4(kb), _ptr(est), _ptr(ws), B, Hq, Hkv, Lq, Lk, D, block_size, stride, chunk_size,
                                      int(causal), _stream(q)), "psa_estimate_xattn")
     return est
@@ -395,7 +418,7 @@ def gather_rows(tensors: Sequence[torch.Tensor], index: torch.Tensor) -> Tuple[t
     a_src = (Tensor4 * 3)(*[_t4(t) for t in srcs], *[_t4(srcs[0])] * (3 - n))
     a_dst = (Tensor4 * 3)(*[_t4(t) for t in outs], *[_t4(outs[0])] * (3 - n))
     heads = (ctypes.c_int * 3)(*[t.shape[1] for t in srcs], *[srcs[0].shape[1]] * (3 - n))
-    with torch.cuda.device(t0.device):
+    with _on(t0.device):
         check(lib.psa_gather_rows(a_src, a_dst, heads, n, _ptr(index), B, L_dst, L_src, D, t0.element_size(), _stream(t0)),
               "psa_gather_rows")
     return tuple(outs)
@@ -408,7 +431,7 @@ def map_from_list(list_mask: torch.Tensor, Nk: int, map_dtype: torch.dtype = tor
     lead, W = lm.shape[:-1], lm.shape[-1]
     rows = lm.numel() // W
     out = torch.empty(*lead, Nk, dtype=map_dtype, device=lm.device)
-    with torch.cuda.device(lm.device):
+    with _on(lm.device):
         check(lib.psa_map_from_list(_ptr(lm), _ptr(out), out.element_size(), rows, W, Nk, _stream(lm)), "psa_map_from_list")
     return out
 
@@ -422,7 +445,7 @@ def list_from_map(level_map_: torch.Tensor, blocksize: int = 32, compute_tile: i
     lead, Nk = m.shape[:-1], m.shape[-1]
     div = max(1, blocksize // compute_tile)
     out = torch.empty(*lead, Nk + 5, dtype=torch.int32, device=m.device)
-    with torch.cuda.device(m.device):
+    with _on(m.device):
         check(lib.psa_list_from_map(_ptr(m), m.element_size(), _ptr(out), m.numel() // Nk, Nk, div, _stream(m)), "psa_list_from_map")
     return out
 
@@ -434,7 +457,7 @@ def k_similarity(k: torch.Tensor, block_n: int, thr2: float, thr4: float, thr8: 
     B, H, L, D = kb.shape
     Nk = -(-L // block_n)
     out = torch.empty(B, H, Nk, dtype=torch.int32, device=k.device)
-    with torch.cuda.device(k.device):
+    with _on(k.device):
         check(lib.psa_ksim(_t4(kb), _ptr(out), B, H, L, D, block_n, float(thr2), float(thr4), float(thr8), _stream(k)), "psa_ksim")
     return out
 
@@ -448,7 +471,7 @@ def map_min_cap(level_map_: torch.Tensor, cap: torch.Tensor) -> torch.Tensor:
     cap = cap.to(torch.int32).contiguous()
     if tuple(cap.shape) != (B, H, Nk):
         raise ValueError("cap must be [B, H, Nk]")
-    with torch.cuda.device(level_map_.device):
+    with _on(level_map_.device):
         check(lib.psa_map_min_cap(_ptr(level_map_), level_map_.element_size(), _ptr(cap), B * H, Mq, Nk, _stream(cap)), "psa_map_min_cap")
     return level_map_
 
@@ -462,7 +485,7 @@ def density_stats(level_map_: torch.Tensor, causal: bool = False) -> Tuple[torch
     n_ws = lib.psa_density_stats_workspace_bytes(m.element_size(), B, H, Mq, Nk) // 4
     BH = B * H
     out = torch.empty(BH + 2 + H + n_ws, dtype=torch.float32, device=m.device)
-    with torch.cuda.device(m.device):
+    with _on(m.device):
         check(lib.psa_density_stats(_ptr(m), m.element_size(), B, H, Mq, Nk, int(causal), ctypes.c_void_p(out.data_ptr() + 4 * (BH + 2 + H)),
                                     _ptr(out), _stream(m)), "psa_density_stats")
     return out[:BH + 1], out[BH + 1], out[BH + 2:BH + 2 + H]
@@ -492,7 +515,7 @@ def build_schedule(level_map_: torch.Tensor, Hkv: int, L: int, D: int, block_m: 
         out = torch.empty(n, dtype=torch.uint8, device=level_map_.device)
     elif out.dtype != torch.uint8 or out.numel() < n or not out.is_contiguous() or out.device != level_map_.device:
         raise ValueError("schedule buffer must be a contiguous uint8 tensor of at least %d bytes" % n)
-    with torch.cuda.device(level_map_.device):
+    with _on(level_map_.device):
         check(lib.psa_build_schedule(_ptr(level_map_), level_map_.element_size(), _ptr(out), B, Hq, Hkv, L, D, block_m, block_n,
                                      int(causal), _stream(level_map_)), "psa_build_schedule")
     return out
@@ -503,6 +526,10 @@ def build_schedule(level_map_: torch.Tensor, Hkv: int, L: int, D: int, block_m: 
 # 520 rows head dim 64 51.4 / 48.6, 2080 rows 121.6 / 123.3; 16944 rows (45106 tokens, 48 heads) 4.5 ms / 4.9 ms.
 # At head dim 128, which is bound by power, 568 rows 94.1 / 95.9, 2080 rows 233 / 231 (in the layer 377 / 385).
 _WALK_MIN_ROWS = 1024
+
+
+def _lists_tiles(dtype: torch.dtype, block_n: int, rows: int) -> bool:
+    return dtype in _T16 and (block_n == 128 or rows > _WALK_MIN_ROWS)
 
 
 def sparse_attention_fwd(
@@ -558,17 +585,16 @@ def sparse_attention_fwd(
         q_index = _check_index(q_index, L)
     shape = (B, Hq, Hkv, L, D, block_m, block_n)
     n_walk = 0
-    if level_map_ is not None and balance and schedule is not False and qb.dtype in _T16:
-        if block_n == 128 or B * Hq * Mq > _WALK_MIN_ROWS:
-            n_walk = lib.psa_walk_bytes(*shape)
+    if level_map_ is not None and balance and schedule is not False and _lists_tiles(qb.dtype, block_n, B * Hq * Mq):
+        n_walk = lib.psa_walk_bytes(*shape)
     if n_walk > 0:
         # the map's tiles are listed once (one pass over the map) and walked by the kernel
         walk = schedule
         if not isinstance(schedule, torch.Tensor) or block_n != 128:  # (build_schedule serves 128-key blocks)
             walk = torch.empty(n_walk, dtype=torch.uint8, device=q.device)
-            with torch.cuda.device(q.device):
+            with _on(q.device):
                 check(lib.psa_build_walk(_ptr(level_map_), level_map_.element_size(), _ptr(walk), *shape, int(causal), _stream(q)), "psa_build_walk")
-        with torch.cuda.device(q.device):
+        with _on(q.device):
             check(lib.psa_fwd_walk(_t4(qb), _ptr(q_index), _t4(kb), _t4(vb), _ptr(kp), _ptr(vp), _ptr(level_map_),
                                    level_map_.element_size(), _ptr(walk), _t4(o), _ptr(lse), *shape, sm_scale, int(causal),
                                    _stream(q)), "psa_fwd_walk")
@@ -578,7 +604,7 @@ def sparse_attention_fwd(
             ws = torch.empty(lib.psa_fwd_workspace_bytes(B, Hq, L, block_m) // 4, dtype=torch.int32, device=q.device)
         tail = (_t4(kb), _t4(vb), _ptr(kp), _ptr(vp), _ptr(level_map_), 1 if level_map_ is None else level_map_.element_size(), _t4(o),
                 _ptr(lse), *shape, sm_scale, int(causal), _ptr(ws), _stream(q))
-        with torch.cuda.device(q.device):
+        with _on(q.device):
             if q_index is None:
                 check(lib.psa_fwd(_t4(qb), *tail), "psa_fwd")
             else:
@@ -604,6 +630,78 @@ def _side_stream(device: torch.device) -> "torch.cuda.Stream":
 
 
 # ----------------------------------------------------------------------------- whole layer, forward only
+def _layer_one_call(qb, kb, vb, off_q, off_k, mask_ratios, mode, block_m, block_n, tile_n, sm_scale, text_length, token_index=None,
+                    sim_thresholds=None):
+    """(out, map, cap) of psa_layer_fwd's sequence as one library call on one stream, or None where the arguments are not the
+    plain ones (the separate operators then run, or say what is wrong)."""
+    B, Hq, L, D = qb.shape
+    Hkv = kb.shape[1]
+    dev = qb.device
+    if kb.shape != (B, Hkv, L, D) or vb.shape != kb.shape or kb.device != dev or vb.device != dev:
+        return None
+    if mode not in ("topk", "thresholdbound") or mask_ratios is None or not sm_scale > 0 or tile_n > block_n:
+        return None
+    for o, H, keep in ((off_q, Hq, block_m // 4), (off_k, Hkv, block_n // 4)):
+        if o is None or o.dtype != torch.int32 or o.shape != (B, H, keep) or not o.is_contiguous() or o.device != dev:
+            return None
+    if sim_thresholds is not None and (Hq != Hkv or qb.dtype not in _T16):
+        return None
+    if token_index is not None:
+        if token_index.device != dev:
+            return None
+        token_index = _check_index(token_index, L)
+    items, m, _ = _items(mask_ratios, mode)
+    Mq, Nk = -(-L // block_m), -(-L // block_n)
+    walk = int(_lists_tiles(qb.dtype, block_n, B * Hq * Mq))
+    n_ws = lib.psa_layer_workspace_bytes(qb.element_size(), B, Hq, Hkv, L, D, block_m, block_n, int(token_index is not None), walk)
+    if n_ws <= 0:
+        return None
+    lv, hi = _level_items(items)
+    ws = torch.empty(n_ws, dtype=torch.uint8, device=dev)
+    mp = torch.empty(B, Hq, Mq, Nk, dtype=torch.int8, device=dev)
+    out = torch.empty(B, Hq, L, D, dtype=qb.dtype, device=dev)
+    cap = thr = None
+    if sim_thresholds is not None:
+        cap = torch.empty(B, Hkv, Nk, dtype=torch.int32, device=dev)
+        thr = (ctypes.c_float * 3)(*sim_thresholds)
+    tb = (text_length + block_n - 1) // block_n if text_length > 0 else 0
+    with _on(dev):
+        check(lib.psa_layer_fwd(_t4(qb), _t4(kb), _t4(vb), _ptr(token_index), off_q.data_ptr(), off_k.data_ptr(), thr, _ptr(cap),
+                                ws.data_ptr(), mp.data_ptr(), _t4(out), B, Hq, Hkv, L, D, block_m, block_n, sm_scale, m, len(items), lv, hi,
+                                block_n // tile_n, tb, 0.06, walk, _stream(qb)), "psa_layer_fwd")
+    return out, mp, cap
+
+
+def causal_layer_fwd(q, k, v, mask_ratios, mode, text_length, block, stride, chunk_size, causal, sim_thresholds):
+    """The causal layer (antidiagonal estimate -> level map -> similarity cap -> pooling -> attention) of bf16 tensors as one
+    library call, no gradient; None where the arguments are not the plain ones (the separate operators then run)."""
+    if not (q.is_cuda and k.device == q.device and v.device == q.device and q.dtype == k.dtype == v.dtype == torch.bfloat16):
+        return None
+    if q.dim() != 4 or k.dim() != 4 or k.shape != v.shape or not mask_ratios or mode not in ("topk", "energybound"):
+        return None
+    B, Hq, L, D = q.shape
+    Hkv = k.shape[1]
+    if k.shape != (B, Hkv, L, D) or Hkv == 0 or Hq % Hkv or len(mask_ratios) > _lib.PSA_MAX_LEVEL_ITEMS:
+        return None
+    n_ws = lib.psa_causal_layer_workspace_bytes(B, Hq, Hkv, L, D, block, stride, chunk_size)
+    if n_ws <= 0:
+        return None
+    q, k, v = _kernel_view(q), _kernel_view(k), _kernel_view(v)
+    items = list(mask_ratios.items())
+    lv, hi = _level_items(items)
+    lo = (ctypes.c_double * len(items))(*[float(i[1][0]) for i in items])
+    S = -(-L // block)
+    special = min(-(-text_length // block) if text_length > 0 else 0, S)
+    m = _lib.PSA_MODE_TOPK if mode == "topk" else _lib.PSA_MODE_THRESHOLDBOUND
+    ws = torch.empty(n_ws, dtype=torch.uint8, device=q.device)
+    out = torch.empty(B, Hq, L, D, dtype=q.dtype, device=q.device)
+    with _on(q.device):
+        check(lib.psa_causal_layer_fwd(_t4(q), _t4(k), _t4(v), (ctypes.c_float * 3)(*sim_thresholds), ws.data_ptr(), _t4(out), B, Hq, Hkv, L, D,
+                                       block, stride, chunk_size, D ** -0.5, m, len(items), lv, lo, hi, special, int(causal), _stream(q)),
+              "psa_causal_layer_fwd")
+    return out
+
+
 def psa_layer_fwd(
     q: torch.Tensor,
     k: torch.Tensor,
@@ -634,13 +732,25 @@ def psa_layer_fwd(
     qb, kb, vb = _same_type(_kernel_view(q), _kernel_view(k), _kernel_view(v))
     keep_m, keep_n = block_m // 4, block_n // 4
     sm_scale = qb.shape[-1] ** -0.5 if sm_scale is None else float(sm_scale)
+    small = kb.numel() * 2 < _SIDE_STREAM_MIN_BYTES
+    if level_cap is None and (small or token_index is not None):
+        # (a layer with the pooling pass on a stream of its own goes through the separate operators)
+        res = _layer_one_call(qb, kb, vb, off_q, off_k, mask_ratios, mode, block_m, block_n, tile_n, sm_scale, text_length, token_index,
+                              sim_thresholds)
+        if res is not None:
+            out, mp, cap = res
+            if out.dtype != q.dtype:
+                out = out.to(q.dtype)
+            if not (return_map or return_cap):
+                return out
+            return (out,) + ((mp,) if return_map else ()) + ((cap,) if return_cap else ())
     if token_index is not None:
         # token re-ordering (int32 permutation: position i = source row token_index[i]) without gather passes: the pooling
         # pass reads K, V through the index and leaves the re-ordered rows behind, the estimator and the attention kernel
         # read Q through it, and the attention kernel writes its rows back to their original places
         kp, vp, kb, vb = pool_kv_indexed(kb, vb, token_index, block_n)
     side = None
-    if token_index is None and kb.numel() * 2 >= _SIDE_STREAM_MIN_BYTES:
+    if token_index is None and not small:
         # the buffers come from the current stream's allocator; the side stream only runs the kernel
         main = torch.cuda.current_stream(qb.device)
         side = _side_stream(qb.device)
@@ -763,7 +873,7 @@ def sparse_attention_bwd(
     dk = torch.empty(B, Hkv, L, D, dtype=qb.dtype, device=q.device)
     dv = torch.empty(B, Hkv, L, D, dtype=qb.dtype, device=q.device)
     ws = torch.empty(lib.psa_bwd_workspace_bytes(B, Hq, Hkv, L, D, block_n), dtype=torch.uint8, device=q.device)
-    with torch.cuda.device(q.device):
+    with _on(q.device):
         check(
             lib.psa_bwd(_t4(qb), _t4(kb), _t4(vb), _ptr(kp), _ptr(vp), _ptr(level_map_),
                         1 if level_map_ is None else level_map_.element_size(), _t4(ob), _t4(dob), _ptr(lse), _t4(dq), _t4(dk), _t4(dv),

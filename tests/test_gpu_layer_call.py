@@ -1,0 +1,85 @@
+"""The layers as one library call (ops.psa_layer_fwd, ops.causal_layer_fwd) against the separate operators: same bits, on either
+side of the sizes where the tiles are listed, with and without token index and similarity cap, and on a stream of the caller's."""
+import pytest
+import torch
+
+from gpu_util import dev, rnd
+
+pytestmark = pytest.mark.gpu
+RATIOS = {1: (0.0, 0.1), 2: (0.1, 0.15), 4: (0.15, 0.15), 8: (0.15, 0.35), 0: (0.35, 1.0)}
+
+
+@pytest.mark.parametrize(
+    "B,Hq,Hkv,L,D,bm,bn,mode,dtype",
+    [
+        (1, 8, 8, 1000, 64, 128, 64, "topk", torch.bfloat16),
+        (2, 4, 2, 513, 128, 128, 128, "thresholdbound", torch.float16),   # GQA, 128-key blocks: listed tiles
+        (1, 38, 38, 3400, 64, 128, 32, "topk", torch.bfloat16),           # more rows than _WALK_MIN_ROWS
+        (1, 2, 2, 1024, 64, 64, 64, "thresholdbound", torch.float32),
+        (1, 1, 1, 1, 128, 128, 64, "topk", torch.bfloat16),
+    ],
+)
+@pytest.mark.parametrize("strided,indexed,capped", [(False, False, False), (True, False, True), (True, True, False), (False, True, True)])
+def test_one_call_equals_separate_operators(monkeypatch, B, Hq, Hkv, L, D, bm, bn, mode, dtype, strided, indexed, capped):
+    from psa_hip import ops
+
+    if capped and (Hq != Hkv or dtype == torch.float32):
+        pytest.skip("takes the separate operators")
+
+    q, k, v = (rnd(B, h, L, D, seed=L + i).to(dtype).to(dev()) for i, h in enumerate((Hq, Hkv, Hkv)))
+    if strided:
+        q, k, v = (x.transpose(1, 2).contiguous().transpose(1, 2) for x in (q, k, v))
+    off_q, off_k = ops.draw_sample_offsets(B, Hq, Hkv, bm, bm // 4, bn, bn // 4, dev(), seed=L)
+
+    index = torch.randperm(L, generator=torch.Generator().manual_seed(L)).to(torch.int32).to(dev()) if indexed else None
+
+    def layer():
+        return ops.psa_layer_fwd(q, k, v, off_q, off_k, RATIOS, mode, bm, bn, 16, return_map=True, return_cap=True, text_length=70,
+                                 token_index=index, sim_thresholds=(-0.1, 0.0, 0.1) if capped else None)
+
+    calls = []
+    real = ops._layer_one_call
+    monkeypatch.setattr(ops, "_layer_one_call", lambda *a: calls.append(real(*a)) or calls[-1])
+    out, mp, cap = layer()
+    assert calls and calls[0] is not None and (cap is not None) == capped
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        on_stream = layer()
+    s.synchronize()
+    monkeypatch.setattr(ops, "_layer_one_call", lambda *a: None)
+    ref = layer()
+    torch.cuda.synchronize()
+    for a, b in ((out, ref[0]), (mp, ref[1]), (on_stream[0], ref[0])):
+        assert torch.equal(a, b)
+    assert not capped or torch.equal(cap, ref[2])
+
+
+@pytest.mark.parametrize("Hq,Hkv,L,D,stride,mode,text", [(28, 4, 2345, 128, 8, "energybound", 512), (2, 2, 129, 64, 16, "topk", 0), (6, 3, 4200, 64, 4, "topk", 30)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_causal_one_call_equals_separate_operators(Hq, Hkv, L, D, stride, mode, text, causal):
+    from psa_hip.PSA_casual import AttentionConfig, PyramidAdaptiveBlockSparseAttnTrain
+
+    q, k, v = (rnd(2, h, L, D, seed=L + i).to(dev()) for i, h in enumerate((Hq, Hkv, Hkv)))
+    cfg = AttentionConfig(text_length=text, mask_mode=mode, xattn_stride=stride, causal_main=causal, sim_2x_threshold=-0.1, sim_4x_threshold=0.0,
+                          sim_8x_threshold=0.05)
+    m = PyramidAdaptiveBlockSparseAttnTrain(cfg, layer_idx=0)
+    a = m(q, k, v, layer_idx=0)
+    plain = m.sparse_attention_fn
+    m.sparse_attention_fn = lambda *x: plain(*x)  # a function of the caller's own: the separate operators
+    b = m(q, k, v, layer_idx=0)
+    torch.cuda.synchronize()
+    assert torch.equal(a, b)
+
+
+def test_one_call_refuses_what_the_operators_refuse():
+    from psa_hip import ops
+
+    q, k, v = (rnd(1, 2, 256, 64, seed=i).to(dev()) for i in range(3))
+    off_q, off_k = ops.draw_sample_offsets(1, 2, 2, 128, 32, 64, 16, dev(), seed=1)
+    go = lambda **kw: ops.psa_layer_fwd(*[kw.get(n, x) for n, x in (("q", q), ("k", k), ("v", v), ("off_q", off_q), ("off_k", off_k))],
+                                        kw.get("ratios", RATIOS), kw.get("mode", "topk"), 128, 64, kw.get("tile_n", 32))
+    for kw in (dict(mode="topk_newtype"), dict(mode="other"), dict(ratios=None), dict(off_q=off_q[:, :1]), dict(off_k=off_k.long()),
+               dict(k=k[:, :, :128]), dict(v=v[:, :1]), dict(tile_n=128), dict(q=q[0])):
+        with pytest.raises((ValueError, RuntimeError)):
+            go(**kw)
