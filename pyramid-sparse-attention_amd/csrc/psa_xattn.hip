@@ -7,7 +7,7 @@
 //
 // A is a plain NT GEMM of Q' [Mr, S*D] (the S rows of a group concatenated in reverse order) with
 // K' [Nr, S*D] (K viewed with S rows per line), i.e. MFMA-bound: 2*Mr*Nr*S*D flops (half under causality).
-// Kernel 1: 256 (m) x 256 (n) output tiles, 8 waves of 64 (m) x 128 (n); both operands go from global memory
+// Kernel 1: 256 (m) x 256 (n) output tiles, 8 waves of 64 (m) x 128 (n) (small launches: 128 x 128, see xattn_small); both operands go from global memory
 // straight into double-buffered LDS (global_load_lds_dwordx4, the padded + swizzled 64-row tile layout of
 // psa_tiles.h) in stages of 64 contraction elements, i.e. half a head-dim row of one of the S interleaved
 // tokens; the transposed product (rows = n, lanes = m) makes the per-row reductions over n in-lane.  The tile
@@ -18,21 +18,29 @@
 // reach HBM.  Kernel 2 (HBM-bound): per row the global max and denominator from the pairs, then the
 // block sums.  Rows / keys past the real length are zero vectors (zero padding to `chunk` tokens); padded
 // keys are not masked (logit 0), padded query rows contribute 0.
+#include <type_traits>
+
 #include "psa_common.h"
 #include "psa_tiles.h"
 
 namespace {
 
-constexpr int TM = 256, TN = 256, KC = 64;  // output tile and contraction chunk
+constexpr int KC = 64;                       // contraction chunk
 using XG = psa_tiles::LtGeom<KC>;            // LDS tiles: 64 rows of KC values
 constexpr int X_TILE = XG::TILE, X_ISTR = psa_tiles::LT_ISTR;
-constexpr int X_QT = TM / 64, X_KT = TN / 64;             // Q and K tiles per stage
-constexpr int X_STAGE = (X_QT + X_KT) * X_TILE;           // bytes per stage
-constexpr int X_GROUPS = (X_QT + X_KT) * 4;               // 16-row groups per stage
-constexpr int X_WAVES = 8, X_GPW = X_GROUPS / X_WAVES;    // groups copied per wave
-static_assert(X_GROUPS % X_WAVES == 0, "groups divide over the waves");
-constexpr int X_BUFS = 2;                                 // stages in LDS
-constexpr int X_NA = TN / 2 / 32, X_NC = TM / 4 / 32;     // 32 x 32 accumulators per wave: X_NA along n, X_NC along m
+// A workgroup's output tile: 64 * WM rows by 2 * 32 * NA keys, 2 * WM waves of 64 rows x 32 * NA keys.
+template <int WM_, int NA_>
+struct XTile {
+  static constexpr int WM = WM_, NA = NA_, NC = 2;                 // 32 x 32 accumulators per wave: NA along n, NC along m
+  static constexpr int TM = 64 * WM, TN = 64 * NA;
+  static constexpr int QT = TM / 64, KT = TN / 64;                 // Q and K tiles per stage
+  static constexpr int STAGE = (QT + KT) * X_TILE;                 // bytes per stage
+  static constexpr int WAVES = 2 * WM, GPW = (QT + KT) * 4 / WAVES;  // 16-row groups copied per wave
+  static_assert((QT + KT) * 4 % WAVES == 0 && NA % 2 == 0, "groups divide over the waves");
+};
+using XLarge = XTile<4, 4>;  // 256 x 256
+using XSmall = XTile<2, 2>;  // 128 x 128, two workgroups per CU
+constexpr int X_BUFS = 2;    // stages in LDS
 
 // rows past the end of Q / K are zero vectors: their copies read this page
 __device__ __align__(256) const unsigned char x_zero_page[256] = {};
@@ -53,15 +61,17 @@ struct XParams {
 };
 
 // output tiles of tile row tm that contain visible keys
+template <class X>
 __host__ __device__ inline int tiles_in_row(int tm, int tiles_n, int causal, int off) {
   if (!causal) return tiles_n;
-  const int last_n = (tm + 1) * TM - 1 + off;  // last visible strided key of the row's last query
-  const int n = last_n / TN + 1;
+  const int last_n = (tm + 1) * X::TM - 1 + off;  // last visible strided key of the row's last query
+  const int n = last_n / X::TN + 1;
   return n < tiles_n ? n : tiles_n;
 }
 
-template <int RBL>  // log2 of the strided keys per block
-__global__ __launch_bounds__(X_WAVES * 64, 1) void psa_xattn_gemm_kernel(XParams p) {
+template <int RBL, class X>  // log2 of the strided keys per block
+__global__ __launch_bounds__(X::WAVES * 64, X::WAVES == 8 ? 1 : 2) void psa_xattn_gemm_kernel(XParams p) {
+  constexpr int TM = X::TM, TN = X::TN, X_QT = X::QT, X_STAGE = X::STAGE, X_GPW = X::GPW, X_NA = X::NA, X_NC = X::NC;
   extern __shared__ __align__(16) unsigned char smem[];  // X_BUFS stages of [Q tiles | K tiles]
   // Workgroup ids go round-robin over the 8 XCDs and every XCD runs its ids in order.  The output tiles with
   // visible keys are listed (batch-head, tile row, tile column) and the list is cut into 8 contiguous shares, one
@@ -73,7 +83,7 @@ __global__ __launch_bounds__(X_WAVES * 64, 1) void psa_xattn_gemm_kernel(XParams
   const int bh = idx / p.act_per_bh;
   int tn = idx % p.act_per_bh, tm = 0;
   for (;; ++tm) {
-    const int row_n = tiles_in_row(tm, p.tiles_n, p.causal, p.off);
+    const int row_n = tiles_in_row<X>(tm, p.tiles_n, p.causal, p.off);
     if (tn < row_n) break;
     tn -= row_n;
   }
@@ -82,7 +92,7 @@ __global__ __launch_bounds__(X_WAVES * 64, 1) void psa_xattn_gemm_kernel(XParams
   const int hk = h / (p.Hq / p.Hkv);
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hh = lane >> 5;
-  const int wn = wave & 1, wm = wave >> 1;  // wave tile: rows m0 + 64 * wm .., keys n0 + 128 * wn ..
+  const int wn = wave & 1, wm = wave >> 1;  // wave tile: rows m0 + 64 * wm .., keys n0 + 32 * NA * wn ..
   const int S = 1 << p.S_log2;
 
   const char* qb = (const char*)(p.q + b * p.q_sb + h * p.q_sh);
@@ -108,29 +118,32 @@ __global__ __launch_bounds__(X_WAVES * 64, 1) void psa_xattn_gemm_kernel(XParams
     g_off[j] = ((uint32_t)idx << p.S_log2) * (is_q ? q_strb : k_strb) + f_chunk;
   }
   edge = ((int64_t)(m0 + TM) << p.S_log2) > p.Lq || ((int64_t)(n0 + TN) << p.S_log2) > p.Lk;  // (covers tiles that stick out of Mr / Nr)
-  // copy instruction `piece` (0 .. X_GPW * RPL - 1) of stage st
-  auto issue_piece = [&](int st, int piece) __attribute__((always_inline)) {
-    const int j = piece / RPL, n = piece % RPL;
+  // copies of stage st; EDGE: rows past the real length read the page of zeros (decided once per workgroup: a test per copy
+  // is a branch per copy)
+  auto issue_stage = [&](int st, auto edge_c) __attribute__((always_inline)) {
+    constexpr bool EDGE = decltype(edge_c)::value;
     const int i = st >> dc_log2, dc = st & ((1 << dc_log2) - 1);  // (shifts: a division here would run on the vector unit and take the base pointers with it)
     unsigned char* dst = smem + (st & 1) * X_STAGE;
-    const int g = wave * X_GPW + j, tile = g >> 2;
-    const bool is_q = tile < X_QT;
-    // token S-1-i of every query group, token i of every key group
-    const char* base = is_q ? qb + (uint64_t)(S - 1 - i) * q_strb + dc * (KC * 2) : kb + (uint64_t)i * k_strb + dc * (KC * 2);
-    const uint32_t rstr = (is_q ? q_strb : k_strb) << p.S_log2;
-    const uint32_t lds = psa_tiles::lds_addr_of(dst + tile * X_TILE + ((g & 3) * RPL + n) * X_ISTR);
-    if (!edge) {
-      psa_tiles::lds_copy16(base, g_off[j] + n * rstr, lds);
-    } else {
-      const int64_t tok = ((int64_t)(g_idx[j] + n) << p.S_log2) + (is_q ? S - 1 - i : i);
-      const bool real = tok < (is_q ? p.Lq : p.Lk);
-      const char* src = real ? base + (g_off[j] + n * rstr) : (const char*)x_zero_page + f_chunk;
-      psa_tiles::lds_copy16_addr(src, lds);
-    }
-  };
-  auto issue_stage = [&](int st) __attribute__((always_inline)) {
 #pragma unroll
-    for (int piece = 0; piece < X_GPW * RPL; ++piece) issue_piece(st, piece);
+    for (int j = 0; j < X_GPW; ++j) {
+      const int g = wave * X_GPW + j, tile = g >> 2;
+      const bool is_q = tile < X_QT;
+      // token S-1-i of every query group, token i of every key group
+      const char* base = is_q ? qb + (uint64_t)(S - 1 - i) * q_strb + dc * (KC * 2) : kb + (uint64_t)i * k_strb + dc * (KC * 2);
+      const uint32_t rstr = (is_q ? q_strb : k_strb) << p.S_log2;
+#pragma unroll
+      for (int n = 0; n < RPL; ++n) {
+        const uint32_t lds = psa_tiles::lds_addr_of(dst + tile * X_TILE + ((g & 3) * RPL + n) * X_ISTR);
+        if constexpr (!EDGE) {
+          psa_tiles::lds_copy16(base, g_off[j] + n * rstr, lds);
+        } else {
+          const int64_t tok = ((int64_t)(g_idx[j] + n) << p.S_log2) + (is_q ? S - 1 - i : i);
+          const bool real = tok < (is_q ? p.Lq : p.Lk);
+          const char* src = real ? base + (g_off[j] + n * rstr) : (const char*)x_zero_page + f_chunk;
+          psa_tiles::lds_copy16_addr(src, lds);
+        }
+      }
+    }
   };
   // operands: K rows (A) of tile wn, Q rows (B) of tile wm; rows l32 and l32 + 32; k-step ks: off[ks & 1] + 64 * (ks >> 1)
   uint32_t r_off[2];
@@ -144,30 +157,34 @@ __global__ __launch_bounds__(X_WAVES * 64, 1) void psa_xattn_gemm_kernel(XParams
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[a][c][i] = 0.f;
 
-  issue_stage(0);
-  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
-  __syncthreads();
-  for (int st = 0; st < stages; ++st) {
-    // invariant: buffer st&1 holds stage st and every wave is done with the other buffer
-    if (st + 1 < stages) issue_stage(st + 1);
-    PSA_LDS(const unsigned char) Qs = (PSA_LDS(const unsigned char))(smem) + (st & 1) * X_STAGE + wm * X_TILE;
-    PSA_LDS(const unsigned char) Ks = (PSA_LDS(const unsigned char))(smem) + (st & 1) * X_STAGE + (X_QT + wn * (X_NA / 2)) * X_TILE;
-#pragma unroll
-    for (int ks = 0; ks < KC / 16; ++ks) {
-      bf16x8 af[X_NA], bf[X_NC];
-      const uint32_t o = r_off[ks & 1] + (ks >> 1) * 64;
-#pragma unroll
-      for (int a = 0; a < X_NA; ++a) af[a] = *(PSA_LDS(const bf16x8))(Ks + o + (a >> 1) * X_TILE + (a & 1) * XG::HALF);
-#pragma unroll
-      for (int c = 0; c < X_NC; ++c) bf[c] = *(PSA_LDS(const bf16x8))(Qs + o + c * XG::HALF);
-#pragma unroll
-      for (int a = 0; a < X_NA; ++a)
-#pragma unroll
-        for (int c = 0; c < X_NC; ++c) acc[a][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[a], bf[c], acc[a][c], 0, 0, 0);
-    }
-    __builtin_amdgcn_s_waitcnt(0x0f70);  // the copies of stage st+1 were issued a stage ago
+  auto contract = [&](auto edge_c) __attribute__((always_inline)) {
+    issue_stage(0, edge_c);
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
     __syncthreads();
-  }
+    for (int st = 0; st < stages; ++st) {
+      // invariant: buffer st&1 holds stage st and every wave is done with the other buffer
+      if (st + 1 < stages) issue_stage(st + 1, edge_c);
+      PSA_LDS(const unsigned char) Qs = (PSA_LDS(const unsigned char))(smem) + (st & 1) * X_STAGE + wm * X_TILE;
+      PSA_LDS(const unsigned char) Ks = (PSA_LDS(const unsigned char))(smem) + (st & 1) * X_STAGE + (X_QT + wn * (X_NA / 2)) * X_TILE;
+#pragma unroll
+      for (int ks = 0; ks < KC / 16; ++ks) {
+        bf16x8 af[X_NA], bf[X_NC];
+        const uint32_t o = r_off[ks & 1] + (ks >> 1) * 64;
+#pragma unroll
+        for (int a = 0; a < X_NA; ++a) af[a] = *(PSA_LDS(const bf16x8))(Ks + o + (a >> 1) * X_TILE + (a & 1) * XG::HALF);
+#pragma unroll
+        for (int c = 0; c < X_NC; ++c) bf[c] = *(PSA_LDS(const bf16x8))(Qs + o + c * XG::HALF);
+#pragma unroll
+        for (int a = 0; a < X_NA; ++a)
+#pragma unroll
+          for (int c = 0; c < X_NC; ++c) acc[a][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[a], bf[c], acc[a][c], 0, 0, 0);
+      }
+      __builtin_amdgcn_s_waitcnt(0x0f70);  // the copies of stage st+1 were issued a stage ago
+      __syncthreads();
+    }
+  };
+  if (edge) contract(std::true_type{});
+  else contract(std::false_type{});
 
   // epilogue: accumulator (a, c): rows n = n0 + wn*128 + a*32 + (i/4)*8 + hh*4 + i%4, column m = m0 + wm*64 + c*32 + l32
   constexpr int OPB = 1 << (RBL - 3);  // 8-key octets per block: 1, 2 or 4
@@ -284,6 +301,23 @@ __global__ __launch_bounds__(256) void psa_xattn_reduce_kernel(XParams p, int ca
   }
 }
 
+// output tiles of one (batch, head) that hold visible keys of rows below rows_used; sets the tile counts of p
+template <class X>
+int active_tiles(XParams& p, int rows_used) {
+  p.tiles_m = (rows_used + X::TM - 1) / X::TM;
+  p.tiles_n = (p.Nr + X::TN - 1) / X::TN;
+  int n = 0;
+  for (int tm = 0; tm < p.tiles_m; ++tm) n += tiles_in_row<X>(tm, p.tiles_n, p.causal, p.off);
+  return n;
+}
+// Output tile of the launch.  A 128 x 128 tile is a quarter of the products at three quarters of the rate of a 256 x 256 one
+// (copies and LDS operands per product): it pays where the large tiles leave CUs idle, i.e. by rounds of the chip (256 large
+// tiles, 512 small ones; a round of small ones takes 0.65 of a round of large ones).  Contraction + reduction, 28 heads, stride 8,
+// large / small in us: 2345 tokens 37 / 22, 6000 40 / 42, 8192 69 / 50, 16384 154 / 168, 32768 599 / 702.
+bool xattn_small(int64_t n_large, int64_t n_small) {
+  return (n_small + 511) / 512 * 13 < (n_large + 255) / 256 * 20;
+}
+
 struct XGeom {
   int Lq_pad, Lk_pad, Mr, Nr, NB, MB;
 };
@@ -343,22 +377,25 @@ extern "C" int psa_estimate_xattn(psa_tensor4 q, psa_tensor4 k, float* est, void
   p.out_cols = (Lk + block_size - 1) / block_size;
   p.scale2 = 1.4426950408889634f / sqrtf((float)D) / (float)stride;
   hipStream_t st = (hipStream_t)stream;
-  p.tiles_m = (g.Mr + TM - 1) / TM;
-  p.tiles_n = (g.Nr + TN - 1) / TN;
-  p.act_per_bh = 0;
-  for (int tm = 0; tm < p.tiles_m; ++tm) p.act_per_bh += tiles_in_row(tm, p.tiles_n, p.causal, p.off);
-  const int64_t n_active = (int64_t)B * Hq * p.act_per_bh;
+  const int64_t heads = (int64_t)B * Hq;
+  // (every pair that the reduction reads is written: the tile rows end with the last q-block's, the rest is padding)
+  const int rows_used = p.out_rows * rb < g.Mr ? p.out_rows * rb : g.Mr;
+  const int64_t n_large = heads * active_tiles<XLarge>(p, rows_used), n_small = heads * active_tiles<XSmall>(p, rows_used);
+  const bool small = xattn_small(n_large, n_small);
+  const int64_t n_active = small ? n_small : n_large;
   PSA_REQUIRE(n_active < (1ll << 28), PSA_ERR_UNSUPPORTED, "psa_estimate_xattn: too many output tiles");
   p.n_active = (int)n_active;
   p.per_xcd = (int)((n_active + 7) / 8);
-  dim3 grid((unsigned)(p.per_xcd * 8));
-  const size_t shmem = X_BUFS * (size_t)X_STAGE;
-  auto launch = [&](auto kern) -> int {
+  auto launch = [&](auto x) -> int {
+    using X = decltype(x);
+    p.act_per_bh = active_tiles<X>(p, rows_used);
+    const size_t shmem = X_BUFS * (size_t)X::STAGE;
+    auto kern = rb == 8 ? psa_xattn_gemm_kernel<3, X> : rb == 16 ? psa_xattn_gemm_kernel<4, X> : psa_xattn_gemm_kernel<5, X>;
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem) != hipSuccess) return PSA_ERR_LAUNCH;
-    hipLaunchKernelGGL(kern, grid, dim3(X_WAVES * 64), shmem, st, p);
+    hipLaunchKernelGGL(kern, dim3((unsigned)(p.per_xcd * 8)), dim3(X::WAVES * 64), shmem, st, p);
     return PSA_OK;
   };
-  int rc = rb == 8 ? launch(psa_xattn_gemm_kernel<3>) : rb == 16 ? launch(psa_xattn_gemm_kernel<4>) : launch(psa_xattn_gemm_kernel<5>);
+  int rc = small ? launch(XSmall{}) : launch(XLarge{});
   PSA_REQUIRE(rc == PSA_OK, rc, "psa_estimate_xattn: cannot reserve LDS");
   rc = psa_check_launch("psa_estimate_xattn (contraction)");
   if (rc != PSA_OK) return rc;
