@@ -861,7 +861,7 @@ extern "C" int psa_bwd(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const void* 
       hipLaunchKernelGGL(psa_order::psa_row_cost_kernel, dim3((unsigned)((total + 3) / 4)), dim3(256), 0, st, map, map_elem_bytes, (int)total,
                          Mq, Nk, p.bn_log2, block_m, p.causal, cost);
       if (int e = psa_check_launch("psa_bwd (row cost)")) return e;
-      hipLaunchKernelGGL(psa_order::psa_chunk_sort_kernel, dim3((unsigned)groups), dim3(256), 0, st, cost, (int)total, chunk, ord);
+      hipLaunchKernelGGL(psa_order::psa_chunk_sort_kernel, dim3((unsigned)groups), dim3(psa_order::SORT_THREADS), 0, st, cost, (int)total, chunk, ord);
       if (int e = psa_check_launch("psa_bwd (row order)")) return e;
       order = ord;
     }
@@ -907,10 +907,10 @@ extern "C" int psa_bwd(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const void* 
       hipLaunchKernelGGL(psa_bwd_colcost_kernel, dim3((unsigned)Nk, (unsigned)(B * Hkv)), dim3(256), 0, st, p, wide0 ? 1 : 0, cost);
       if (int e = psa_check_launch("psa_bwd (column cost)")) return e;
       if (wide0) {
-        hipLaunchKernelGGL(psa_order::psa_chunk_sort_kernel, dim3((unsigned)groups_w), dim3(256), 0, st, cost, (int)n_wide, chunk_w, ord_w);
+        hipLaunchKernelGGL(psa_order::psa_chunk_sort_kernel, dim3((unsigned)groups_w), dim3(psa_order::SORT_THREADS), 0, st, cost, (int)n_wide, chunk_w, ord_w);
         order_wide = ord_w;
       }
-      hipLaunchKernelGGL(psa_order::psa_chunk_sort_kernel, dim3((unsigned)groups_r), dim3(256), 0, st, cost + n_wide, (int)n_rest, chunk_r,
+      hipLaunchKernelGGL(psa_order::psa_chunk_sort_kernel, dim3((unsigned)groups_r), dim3(psa_order::SORT_THREADS), 0, st, cost + n_wide, (int)n_rest, chunk_r,
                          ord_r);
       order_rest = ord_r;
       if (int e = psa_check_launch("psa_bwd (column order)")) return e;

@@ -14,7 +14,10 @@ namespace {  // one private copy per translation unit that launches them
 
 constexpr int COST_BINS = 2048, COST_BITS = 11;
 static_assert(COST_BINS == 1 << COST_BITS, "cost bins");
-constexpr int RADIX_IPT = 16, RADIX_CHUNK = 256 * RADIX_IPT;  // shares up to this many items are radix-sorted in LDS
+// One workgroup sorts a share, and only 8 or a few dozen shares exist: the sort is a chain of LDS round trips, so it runs 16
+// waves.  256 threads -> 1024: 448-row shares ranked 9.6 -> 6.8 us, shares of 896 rows (radix) 20.4 -> 13.5 us.
+constexpr int SORT_THREADS = 1024;
+constexpr int RADIX_IPT = 4, RADIX_CHUNK = SORT_THREADS * RADIX_IPT;  // shares up to this many items are radix-sorted in LDS
 constexpr int SMALL_CHUNK = 512;  // shares up to this many items are ordered by rank counting in one pass
 constexpr int MAX_PHASES = 64;
 constexpr int64_t PHASE_BYTES = 128ll << 20;  // operand bytes (K/V + pooled levels, or Q/dO) in use at one time
@@ -60,7 +63,7 @@ __global__ __launch_bounds__(256) void psa_row_cost_kernel(const void* map, int 
 }
 
 // one workgroup per share: stable counting sort of its items by decreasing cost (order[] holds item ids, -1 past the last item)
-__global__ __launch_bounds__(256) void psa_chunk_sort_kernel(const int32_t* cost, int total, int chunk, int32_t* order) {
+__global__ __launch_bounds__(SORT_THREADS) void psa_chunk_sort_kernel(const int32_t* cost, int total, int chunk, int32_t* order) {
   __shared__ int hist[COST_BINS];
   const int x = blockIdx.x, tid = threadIdx.x;
   const int r0 = x * chunk;
@@ -68,32 +71,35 @@ __global__ __launch_bounds__(256) void psa_chunk_sort_kernel(const int32_t* cost
     // short shares (the usual case): the slot of an item is its rank among the keys (decreasing cost, then index) -
     // the same stable order as the counting sort below, without histogram, scan and their barriers
     __shared__ __attribute__((aligned(16))) uint32_t keys[SMALL_CHUNK];
-    for (int i = tid; i < SMALL_CHUNK; i += 256)
+    if (const int i = tid; i < SMALL_CHUNK)
       keys[i] = i < chunk && r0 + i < total ? ((uint32_t)(COST_BINS - 1 - cost[r0 + i]) << 16) | (uint32_t)i : 0xffffffffu;
     __syncthreads();
-    const int n4 = (chunk + 3) >> 2;
-    for (int i = tid; i < chunk; i += 256) {
+    // two threads per item, each ranks it among half of the keys
+    static_assert(SORT_THREADS == 2 * SMALL_CHUNK, "two threads per item");
+    const int n4 = (chunk + 3) >> 2, i = tid >> 1;
+    {
       const uint32_t mine = keys[i];
       int rank = 0;
-      for (int j = 0; j < n4; ++j) {
+      for (int j = tid & 1; j < n4; j += 2) {
         const u32x4 k4 = ((const u32x4*)keys)[j];
         rank += (k4[0] < mine) + (k4[1] < mine) + (k4[2] < mine) + (k4[3] < mine);
       }
-      if (mine != 0xffffffffu) order[r0 + rank] = r0 + i;
+      rank += __shfl_xor(rank, 1, 64);
+      if ((tid & 1) == 0 && mine != 0xffffffffu) order[r0 + rank] = r0 + i;
     }
     const int valid = total - r0 < chunk ? (total - r0 > 0 ? total - r0 : 0) : chunk;
-    for (int i = valid + tid; i < chunk; i += 256) order[r0 + i] = -1;
+    for (int i = valid + tid; i < chunk; i += SORT_THREADS) order[r0 + i] = -1;
     return;
   }
   if (chunk <= RADIX_CHUNK) {
     // medium shares: stable binary radix sort (least significant bit first) on the inverted cost, one bit per pass; a
     // thread owns a run of consecutive items, so "earlier" is (earlier thread, then earlier in the run)
     __shared__ uint32_t kbuf[2][RADIX_CHUNK];
-    __shared__ int wave_tot[4];
-    const int ipt = (chunk + 255) >> 8;  // items per thread (<= RADIX_IPT)
+    __shared__ int wave_tot[SORT_THREADS / 64];
+    const int ipt = (chunk + SORT_THREADS - 1) / SORT_THREADS;  // items per thread (<= RADIX_IPT)
     const int i0 = tid * ipt;
     const int lane = tid & 63, wave = tid >> 6;
-    for (int i = tid; i < chunk; i += 256)
+    for (int i = tid; i < chunk; i += SORT_THREADS)
       kbuf[0][i] = r0 + i < total ? ((uint32_t)(COST_BINS - 1 - cost[r0 + i]) << 16) | (uint32_t)i : 0xffffffffu;
     __syncthreads();
     int src = 0;
@@ -105,7 +111,7 @@ __global__ __launch_bounds__(256) void psa_chunk_sort_kernel(const int32_t* cost
         k[e] = (e < ipt && i0 + e < chunk) ? kbuf[src][i0 + e] : 0xffffffffu;
         zeros += (e < ipt && i0 + e < chunk && !((k[e] >> bit) & 1u)) ? 1 : 0;
       }
-      // exclusive scan of the zero counts over the 256 threads
+      // exclusive scan of the zero counts over the threads
       int incl = zeros;
 #pragma unroll
       for (int d = 1; d < 64; d <<= 1) {
@@ -116,7 +122,7 @@ __global__ __launch_bounds__(256) void psa_chunk_sort_kernel(const int32_t* cost
       __syncthreads();
       int before = incl - zeros, all_zeros = 0;
 #pragma unroll
-      for (int w = 0; w < 4; ++w) {
+      for (int w = 0; w < SORT_THREADS / 64; ++w) {
         before += w < wave ? wave_tot[w] : 0;
         all_zeros += wave_tot[w];
       }
@@ -132,20 +138,20 @@ __global__ __launch_bounds__(256) void psa_chunk_sort_kernel(const int32_t* cost
       __syncthreads();
       src ^= 1;
     }
-    for (int i = tid; i < chunk; i += 256) {
+    for (int i = tid; i < chunk; i += SORT_THREADS) {
       const uint32_t key = kbuf[src][i];
       order[r0 + i] = key != 0xffffffffu ? r0 + (int)(key & 0xffffu) : -1;
     }
     return;
   }
-  for (int i = tid; i < COST_BINS; i += 256) hist[i] = 0;
+  for (int i = tid; i < COST_BINS; i += SORT_THREADS) hist[i] = 0;
   __syncthreads();
-  for (int i = tid; i < chunk; i += 256)
+  for (int i = tid; i < chunk; i += SORT_THREADS)
     if (r0 + i < total) atomicAdd(&hist[cost[r0 + i]], 1);
   __syncthreads();
-  {  // start offset of every bin, highest cost first: thread i owns the 8 bins COST_BINS-1-8i .. COST_BINS-8-8i
-    __shared__ int part[256];
-    constexpr int PER = COST_BINS / 256;
+  {  // start offset of every bin, highest cost first: thread i owns PER consecutive bins
+    __shared__ int part[SORT_THREADS];
+    constexpr int PER = COST_BINS / SORT_THREADS;
     int c[PER], sum = 0;
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
@@ -154,7 +160,7 @@ __global__ __launch_bounds__(256) void psa_chunk_sort_kernel(const int32_t* cost
     }
     part[tid] = sum;
     __syncthreads();
-    for (int d = 1; d < 256; d <<= 1) {  // inclusive scan over the threads
+    for (int d = 1; d < SORT_THREADS; d <<= 1) {  // inclusive scan over the threads
       const int add = tid >= d ? part[tid - d] : 0;
       __syncthreads();
       part[tid] += add;
@@ -168,10 +174,10 @@ __global__ __launch_bounds__(256) void psa_chunk_sort_kernel(const int32_t* cost
     }
   }
   __syncthreads();
-  // stable fill (items of equal cost keep their index order, so the issue order is the same in every run): 256 items at
+  // stable fill (items of equal cost keep their index order, so the issue order is the same in every run): SORT_THREADS items at
   // a time, an item's slot = start of its bin + the number of earlier items of the same cost
-  __shared__ int blk_cost[256];
-  for (int i0 = 0; i0 < chunk; i0 += 256) {
+  __shared__ int blk_cost[SORT_THREADS];
+  for (int i0 = 0; i0 < chunk; i0 += SORT_THREADS) {
     const int i = i0 + tid;
     const bool ok = i < chunk && r0 + i < total;
     const int c = ok ? cost[r0 + i] : -1;
@@ -179,7 +185,7 @@ __global__ __launch_bounds__(256) void psa_chunk_sort_kernel(const int32_t* cost
     __syncthreads();
     int before = 0, after = 0;
     if (ok) {
-      for (int j = 0; j < 256; ++j) {
+      for (int j = 0; j < SORT_THREADS; ++j) {
         const bool same = blk_cost[j] == c;
         before += (same && j < tid) ? 1 : 0;
         after += (same && j > tid) ? 1 : 0;
@@ -195,7 +201,7 @@ __global__ __launch_bounds__(256) void psa_chunk_sort_kernel(const int32_t* cost
   }
   // ids past the last row of the last share
   const int valid = total - r0 < chunk ? (total - r0 > 0 ? total - r0 : 0) : chunk;
-  for (int i = valid + tid; i < chunk; i += 256) order[r0 + i] = -1;
+  for (int i = valid + tid; i < chunk; i += SORT_THREADS) order[r0 + i] = -1;
 }
 
 }  // namespace
