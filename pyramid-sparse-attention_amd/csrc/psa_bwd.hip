@@ -283,12 +283,23 @@ constexpr int DKDV_SLOTS = 4;
 // ------------------------------------------------------------------------------------------------------
 constexpr int COL_BINS = psa_order::COST_BINS;
 
-// one workgroup per (kv head, kv-block): per-level counts over the column -> cost of each of its slots.  The costs of
-// the slots slot_lo .. of all blocks form one list per dK/dV launch: with a 128-key slot 0 that slot's list comes first
+// Costs of every walk in one launch, their sorts in another: both are latency-bound (a sort is one workgroup per share, 8 to 16
+// per list) and two cost launches and three sorts one after the other left the chip nearly idle.  Measured now 9 + 12.5 us;
+// training step of 48 heads x 8776 x 64 1208 -> 1198 us, of 12 heads x 32760 x 128 4549 -> 4543 us.  The first row_wgs workgroups: four rows each, costs of the dQ walk.  The others, one per
+// (kv head, kv-block): per-level counts over the column -> cost of each of its slots.  The
+// costs of the slots slot_lo .. of all blocks form one list per dK/dV launch: with a 128-key slot 0 that slot's list comes first
 // (n_blocks entries), then the list of the slots 1 .. 3.
-__global__ __launch_bounds__(256) void psa_bwd_colcost_kernel(BwdParams p, int wide0, int32_t* cost) {
+__global__ __launch_bounds__(256) void psa_bwd_cost_kernel(BwdParams p, int row_wgs, int32_t* cost_row, int wide0, int32_t* cost) {
   __shared__ int s_n[4];
-  const int J = blockIdx.x, bhk = blockIdx.y, b = bhk / p.Hkv, hk = bhk % p.Hkv;
+  if ((int)blockIdx.x < row_wgs) {
+    const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (row >= p.B * p.Hq * p.Mq) return;
+    const int c = psa_order::row_cost(p.map, p.map_elem, row, p.Mq, p.Nk, p.bn_log2, p.bm, p.causal);
+    if ((threadIdx.x & 63) == 0) cost_row[row] = c;
+    return;
+  }
+  const int64_t blk = (int)blockIdx.x - row_wgs;
+  const int J = (int)(blk % p.Nk), bhk = (int)(blk / p.Nk), b = bhk / p.Hkv, hk = bhk % p.Hkv;
   const int n_rep = p.Hq / p.Hkv, Mq = p.Mq, bn_log2 = p.bn_log2;
   if (threadIdx.x < 4) s_n[threadIdx.x] = 0;
   __syncthreads();
@@ -311,7 +322,7 @@ __global__ __launch_bounds__(256) void psa_bwd_colcost_kernel(BwdParams p, int w
   if ((int)threadIdx.x < DKDV_SLOTS) {
     const int lv = (int)threadIdx.x;
     const int c = s_n[lv] < COL_BINS - 1 ? s_n[lv] : COL_BINS - 1;
-    const int64_t blk = (int64_t)bhk * p.Nk + J, n_blocks = (int64_t)gridDim.y * p.Nk;
+    const int64_t n_blocks = (int64_t)p.B * p.Hkv * p.Nk;
     if (!wide0) cost[blk * DKDV_SLOTS + lv] = c;
     else if (lv == 0) cost[blk] = c;
     else cost[n_blocks + blk * (DKDV_SLOTS - 1) + (lv - 1)] = c;
@@ -845,27 +856,44 @@ extern "C" int psa_bwd(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const void* 
     const int rc = psa_check_launch("psa_bwd (delta)");
     if (rc != PSA_OK) return rc;
   }
-  // issue orders (costs and orders live behind lse2 in the workspace; every list is padded to whole shares)
-  int32_t* ws_int = (int32_t*)(p.lse2 + (int64_t)B * Hq * L);
-  // 2. dQ
-  {
-    const int64_t total = (int64_t)B * Hq * Mq;
-    PSA_REQUIRE(total < (1ll << 28), PSA_ERR_UNSUPPORTED, "psa_bwd: too many workgroups");
-    int chunk, groups;
-    const double kv_bytes = 2.0 * B * Hkv * (double)p.npad * D * 2.0 * (map != nullptr ? 1.875 : 1.0);
-    psa_order::deal(total, kv_bytes, B * Hkv, chunk, groups);
-    const int32_t* order = nullptr;
-    if (map != nullptr && total > 8 * 32) {
-      int32_t* cost = ws_int;
-      int32_t* ord = cost + total;
-      hipLaunchKernelGGL(psa_order::psa_row_cost_kernel, dim3((unsigned)((total + 3) / 4)), dim3(256), 0, st, map, map_elem_bytes, (int)total,
-                         Mq, Nk, p.bn_log2, block_m, p.causal, cost);
-      if (int e = psa_check_launch("psa_bwd (row cost)")) return e;
-      hipLaunchKernelGGL(psa_order::psa_chunk_sort_kernel, dim3((unsigned)groups), dim3(psa_order::SORT_THREADS), 0, st, cost, (int)total, chunk, ord);
-      if (int e = psa_check_launch("psa_bwd (row order)")) return e;
-      order = ord;
+  // 2. issue orders of the dQ rows and of the two lists of dK/dV slots: one launch for the costs, one for the sorts.  (Costs and
+  // orders live behind lse2 in the workspace; every list is padded to whole shares.)  The dK/dV slots are the 128-key level-0 slots
+  // (if block_n = 128) and the other slots.
+  const int64_t total = (int64_t)B * Hq * Mq, n_blocks = (int64_t)B * Hkv * Nk;
+  const bool wide0 = block_n > 64;
+  const int64_t n_wide = wide0 ? n_blocks : 0, n_rest = n_blocks * (wide0 ? DKDV_SLOTS - 1 : DKDV_SLOTS);
+  PSA_REQUIRE(total < (1ll << 28) && n_wide + n_rest < (1ll << 28), PSA_ERR_UNSUPPORTED, "psa_bwd: too many workgroups");
+  // shares by the K/V rows (dQ) and the Q/dO rows (dK/dV) that the walks stream
+  const double kv_bytes = 2.0 * B * Hkv * (double)p.npad * D * 2.0 * (map != nullptr ? 1.875 : 1.0);
+  const double qdo_bytes = 2.0 * B * Hq * (double)L * D * 2.0;
+  int chunk, groups, chunk_w = 1, groups_w = 8, chunk_r, groups_r;
+  psa_order::deal(total, kv_bytes, B * Hkv, chunk, groups);
+  if (wide0) psa_order::deal(n_wide, qdo_bytes, B * Hkv, chunk_w, groups_w);
+  psa_order::deal(n_rest, qdo_bytes, B * Hkv, chunk_r, groups_r);
+  const int32_t *order = nullptr, *order_wide = nullptr, *order_rest = nullptr;
+  const bool rows_ordered = map != nullptr && total > 8 * 32, cols_ordered = map != nullptr && n_blocks > 8;
+  if (rows_ordered || cols_ordered) {
+    int32_t* cost = (int32_t*)(p.lse2 + (int64_t)B * Hq * L);
+    int32_t* ord = cost + total;
+    int32_t* cost_c = cost + 2 * total + 16 * psa_order::MAX_PHASES;
+    int32_t* ord_w = cost_c + (n_wide + n_rest);
+    int32_t* ord_r = ord_w + (wide0 ? (int64_t)chunk_w * groups_w : 0);
+    const int row_wgs = rows_ordered ? (int)((total + 3) / 4) : 0;
+    hipLaunchKernelGGL(psa_bwd_cost_kernel, dim3((unsigned)(row_wgs + (cols_ordered ? n_blocks : 0))), dim3(256), 0, st, p, row_wgs, cost,
+                       wide0 ? 1 : 0, cost_c);
+    if (int e = psa_check_launch("psa_bwd (cost)")) return e;
+    psa_order::sort_lists<3>({{{cost, ord, (int)total, chunk, rows_ordered ? groups : 0},
+                               {cost_c, ord_w, (int)n_wide, chunk_w, cols_ordered && wide0 ? groups_w : 0},
+                               {cost_c + n_wide, ord_r, (int)n_rest, chunk_r, cols_ordered ? groups_r : 0}}}, st);
+    if (int e = psa_check_launch("psa_bwd (order)")) return e;
+    if (rows_ordered) order = ord;
+    if (cols_ordered) {
+      if (wide0) order_wide = ord_w;
+      order_rest = ord_r;
     }
-    ws_int += 2 * total + 16 * psa_order::MAX_PHASES;
+  }
+  // 3. dQ
+  {
     auto launch = [&](auto kern, size_t tile_bytes, int nw) -> int {
       const size_t shmem = tile_bytes + (size_t)p.max_tiles * 8 + (size_t)Nk * 2;
       if (shmem > 160 * 1024) return PSA_ERR_UNSUPPORTED;
@@ -883,38 +911,13 @@ extern "C" int psa_bwd(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const void* 
     rc = psa_check_launch("psa_bwd (dQ)");
     if (rc != PSA_OK) return rc;
   }
-  // 3. dK, dV per level: the 128-key level-0 slots (if block_n = 128) in one launch, the other slots in a second one
+  // 4. dK, dV per level: the 128-key level-0 slots (if block_n = 128) in one launch, the other slots in a second one
   {
     const int n_rep = Hq / Hkv;
-    const bool wide0 = block_n > 64;
-    const int64_t n_blocks = (int64_t)B * Hkv * Nk;
-    const int64_t n_wide = wide0 ? n_blocks : 0, n_rest = n_blocks * (wide0 ? DKDV_SLOTS - 1 : DKDV_SLOTS);
-    PSA_REQUIRE(n_wide + n_rest < (1ll << 28), PSA_ERR_UNSUPPORTED, "psa_bwd: too many workgroups");
     size_t shmem = (size_t)4 * (D == 128 ? LtGeom<128>::TILE : LtGeom<64>::TILE) + 256 * sizeof(float) + (size_t)n_rep * Mq * 4;
     const size_t red = (size_t)2 * 2 * (D / 32) * 16 * 64 * sizeof(float);
     if (shmem < red) shmem = red;
     PSA_REQUIRE(shmem <= 160 * 1024, PSA_ERR_UNSUPPORTED, "psa_bwd: too many q-blocks for the on-chip lists (LDS)");
-    // shares by the Q / dO rows the walk streams
-    const double qdo_bytes = 2.0 * B * Hq * (double)L * D * 2.0;
-    int chunk_w = 1, groups_w = 8, chunk_r, groups_r;
-    if (wide0) psa_order::deal(n_wide, qdo_bytes, B * Hkv, chunk_w, groups_w);
-    psa_order::deal(n_rest, qdo_bytes, B * Hkv, chunk_r, groups_r);
-    const int32_t *order_wide = nullptr, *order_rest = nullptr;
-    if (map != nullptr && n_blocks > 8) {
-      int32_t* cost = ws_int;
-      int32_t* ord_w = cost + (n_wide + n_rest);
-      int32_t* ord_r = ord_w + (wide0 ? (int64_t)chunk_w * groups_w : 0);
-      hipLaunchKernelGGL(psa_bwd_colcost_kernel, dim3((unsigned)Nk, (unsigned)(B * Hkv)), dim3(256), 0, st, p, wide0 ? 1 : 0, cost);
-      if (int e = psa_check_launch("psa_bwd (column cost)")) return e;
-      if (wide0) {
-        hipLaunchKernelGGL(psa_order::psa_chunk_sort_kernel, dim3((unsigned)groups_w), dim3(psa_order::SORT_THREADS), 0, st, cost, (int)n_wide, chunk_w, ord_w);
-        order_wide = ord_w;
-      }
-      hipLaunchKernelGGL(psa_order::psa_chunk_sort_kernel, dim3((unsigned)groups_r), dim3(psa_order::SORT_THREADS), 0, st, cost + n_wide, (int)n_rest, chunk_r,
-                         ord_r);
-      order_rest = ord_r;
-      if (int e = psa_check_launch("psa_bwd (column order)")) return e;
-    }
     auto launch = [&](auto kern, int64_t n_wg, int chunk, int groups, int slot_lo, int slot_cnt, const int32_t* order) -> int {
       if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem) != hipSuccess) return PSA_ERR_LAUNCH;
       hipLaunchKernelGGL(kern, dim3((unsigned)(chunk * groups)), dim3(256), shmem, st, p, slot_lo, slot_cnt, (int)n_wg, chunk, order);
@@ -942,7 +945,7 @@ extern "C" int psa_bwd(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const void* 
       return psa_check_launch("psa_bwd (dK/dV, 128-key slots)");
     }
   }
-  // 4. un-pool (blocks of 64 or 32 keys: every level went to the fp32 buffers)
+  // 5. un-pool (blocks of 64 or 32 keys: every level went to the fp32 buffers)
   {
     const int64_t units = (int64_t)L * (D / 4);
     dim3 grid((unsigned)((units + 255) / 256), (unsigned)(B * Hkv), 2);

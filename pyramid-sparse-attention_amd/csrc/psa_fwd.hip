@@ -1313,7 +1313,7 @@ static int fwd_impl(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const void* k_p
     hipLaunchKernelGGL(psa_order::psa_row_cost_kernel, dim3((unsigned)((total + 3) / 4)), dim3(256), 0, (hipStream_t)stream, map, map_elem_bytes,
                        (int)total, Mq, Nk, p.bn_log2, block_m, p.causal, cost);
     if (int e = psa_check_launch("psa_fwd (row cost)")) return e;
-    hipLaunchKernelGGL(psa_order::psa_chunk_sort_kernel, dim3(p.wg_groups), dim3(psa_order::SORT_THREADS), 0, (hipStream_t)stream, cost, (int)total, p.wg_chunk, order);
+    psa_order::sort_lists<1>({{{cost, order, (int)total, p.wg_chunk, p.wg_groups}}}, (hipStream_t)stream);
     if (int e = psa_check_launch("psa_fwd (row order)")) return e;
     p.order = order;
   }

@@ -36,12 +36,9 @@ static inline void deal(int64_t total, double operand_bytes, int n_heads, int& c
   chunk = (int)((total + groups - 1) / groups);
 }
 
-// tiles of 64 (pooled) keys that each row of the level map retains: the cost of a row walk
-__global__ __launch_bounds__(256) void psa_row_cost_kernel(const void* map, int map_elem, int total, int Mq, int Nk, int bn_log2,
-                                                         int bm, int causal, int32_t* cost) {
-  const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (row >= total) return;
-  const int I = row % Mq;
+// tiles of 64 (pooled) keys that a row of the level map retains, capped at the last bin: the cost of its row walk (one wave)
+__device__ __forceinline__ int row_cost(const void* map, int map_elem, int row, int Mq, int Nk, int bn_log2, int bm, int causal) {
+  const int I = row % Mq, lane = threadIdx.x & 63;
   int jmax = Nk;
   if (causal) {
     const int ce = (int)((((int64_t)(I + 1) * bm) + (1 << bn_log2) - 1) >> bn_log2);
@@ -54,18 +51,24 @@ __global__ __launch_bounds__(256) void psa_row_cost_kernel(const void* map, int 
 #pragma unroll
     for (int lv = 0; lv < 4; ++lv) cnt[lv] += __popcll(__ballot(lvl == (1 << lv)));
   }
-  if (lane == 0) {
-    int tiles = 0;
+  int tiles = 0;
 #pragma unroll
-    for (int lv = 0; lv < 4; ++lv) tiles += ((cnt[lv] << (bn_log2 - lv)) + 63) >> 6;
-    cost[row] = tiles < COST_BINS - 1 ? tiles : COST_BINS - 1;
-  }
+  for (int lv = 0; lv < 4; ++lv) tiles += ((cnt[lv] << (bn_log2 - lv)) + 63) >> 6;
+  return tiles < COST_BINS - 1 ? tiles : COST_BINS - 1;
 }
 
-// one workgroup per share: stable counting sort of its items by decreasing cost (order[] holds item ids, -1 past the last item)
-__global__ __launch_bounds__(SORT_THREADS) void psa_chunk_sort_kernel(const int32_t* cost, int total, int chunk, int32_t* order) {
+__global__ __launch_bounds__(256) void psa_row_cost_kernel(const void* map, int map_elem, int total, int Mq, int Nk, int bn_log2,
+                                                         int bm, int causal, int32_t* cost) {
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= total) return;
+  const int c = row_cost(map, map_elem, row, Mq, Nk, bn_log2, bm, causal);
+  if ((threadIdx.x & 63) == 0) cost[row] = c;
+}
+
+// one workgroup per share x: stable counting sort of its items by decreasing cost (order[] holds item ids, -1 past the last item)
+__device__ __forceinline__ void sort_share(const int32_t* cost, int total, int chunk, int32_t* order, int x) {
   __shared__ int hist[COST_BINS];
-  const int x = blockIdx.x, tid = threadIdx.x;
+  const int tid = threadIdx.x;
   const int r0 = x * chunk;
   if (chunk <= SMALL_CHUNK) {
     // short shares (the usual case): the slot of an item is its rank among the keys (decreasing cost, then index) -
@@ -202,6 +205,36 @@ __global__ __launch_bounds__(SORT_THREADS) void psa_chunk_sort_kernel(const int3
   // ids past the last row of the last share
   const int valid = total - r0 < chunk ? (total - r0 > 0 ? total - r0 : 0) : chunk;
   for (int i = valid + tid; i < chunk; i += SORT_THREADS) order[r0 + i] = -1;
+}
+
+// a list of items and its shares; groups = 0: no list
+struct SortList {
+  const int32_t* cost;
+  int32_t* order;
+  int total, chunk, groups;
+};
+// the shares of N lists in one launch: a share is one workgroup, so further lists run on CUs that would stand idle
+template <int N>
+struct SortLists {
+  SortList l[N];
+};
+template <int N>
+__global__ __launch_bounds__(SORT_THREADS) void psa_chunk_sort_kernel(SortLists<N> lists) {
+  int x = blockIdx.x;
+  SortList l = lists.l[0];
+#pragma unroll
+  for (int i = 1; i < N; ++i)
+    if (x >= l.groups) {
+      x -= l.groups;
+      l = lists.l[i];
+    }
+  if (x < l.groups) sort_share(l.cost, l.total, l.chunk, l.order, x);
+}
+template <int N>
+static inline void sort_lists(const SortLists<N>& lists, hipStream_t s) {
+  int groups = 0;
+  for (const SortList& l : lists.l) groups += l.groups;
+  if (groups) hipLaunchKernelGGL(psa_chunk_sort_kernel<N>, dim3((unsigned)groups), dim3(SORT_THREADS), 0, s, lists);
 }
 
 }  // namespace

@@ -180,7 +180,7 @@ static int build_schedule(const void* map, int map_elem_bytes, void* schedule, i
                      (size_t)ROWS_PER_WG * g.Nk * 2, s, map, map_elem_bytes, (int)g.rows, g.Mq, g.Nk, psa_ilog2(block_n), block_m, L,
                      causal ? 1 : 0, cost, tiles, recs, g.lay.rec_stride, (u32x4*)(base + g.lay.fine_off), g.lay.fine_stride);
   if (int e = psa_check_launch("psa_build_schedule (tiles)")) return e;
-  hipLaunchKernelGGL(psa_order::psa_chunk_sort_kernel, dim3(g.wg_groups), dim3(psa_order::SORT_THREADS), 0, s, cost, (int)g.rows, g.wg_chunk, order);
+  psa_order::sort_lists<1>({{{cost, order, (int)g.rows, g.wg_chunk, g.wg_groups}}}, s);
   return psa_check_launch("psa_build_schedule (order)");
 }
 
