@@ -288,8 +288,8 @@ constexpr int COL_BINS = psa_order::COST_BINS;
 // training step of 48 heads x 8776 x 64 1208 -> 1198 us, of 12 heads x 32760 x 128 4549 -> 4543 us.  The first row_wgs workgroups: four rows each, costs of the dQ walk.  The others, one per
 // (kv head, kv-block): per-level counts over the column -> cost of each of its slots.  The
 // costs of the slots slot_lo .. of all blocks form one list per dK/dV launch: with a 128-key slot 0 that slot's list comes first
-// (n_blocks entries), then the list of the slots 1 .. 3.
-__global__ __launch_bounds__(256) void psa_bwd_cost_kernel(BwdParams p, int row_wgs, int32_t* cost_row, int wide0, int32_t* cost) {
+// (n_blocks entries), then the list of the slots 1 .. 3.  The 128-key slots' costs are in units of wide_div q-blocks.
+__global__ __launch_bounds__(256) void psa_bwd_cost_kernel(BwdParams p, int row_wgs, int32_t* cost_row, int wide0, int wide_div, int32_t* cost) {
   __shared__ int s_n[4];
   if ((int)blockIdx.x < row_wgs) {
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -324,7 +324,7 @@ __global__ __launch_bounds__(256) void psa_bwd_cost_kernel(BwdParams p, int row_
     const int c = s_n[lv] < COL_BINS - 1 ? s_n[lv] : COL_BINS - 1;
     const int64_t n_blocks = (int64_t)p.B * p.Hkv * p.Nk;
     if (!wide0) cost[blk * DKDV_SLOTS + lv] = c;
-    else if (lv == 0) cost[blk] = c;
+    else if (lv == 0) cost[blk] = s_n[0] / wide_div < COL_BINS - 1 ? s_n[0] / wide_div : COL_BINS - 1;
     else cost[n_blocks + blk * (DKDV_SLOTS - 1) + (lv - 1)] = c;
   }
 }
@@ -879,8 +879,19 @@ extern "C" int psa_bwd(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const void* 
     int32_t* ord_w = cost_c + (n_wide + n_rest);
     int32_t* ord_r = ord_w + (wide0 ? (int64_t)chunk_w * groups_w : 0);
     const int row_wgs = rows_ordered ? (int)((total + 3) / 4) : 0;
+    // Where the Q / dO rows of a head group are about the size of an XCD's L2 (4 MiB), the 128-key slots of a share are issued in
+    // classes of a quarter of the longest possible list, head by head inside a class (the sort is stable): an XCD then works on one
+    // or two heads at a time and finds their rows in L2, where the exact longest-first order mixes all heads of the share, and the
+    // few long columns still go first.  Training steps in exact order / in classes: 48 heads x 8776 x 64 1195 / 1160 us,
+    // 24 x 12001 x 64 1028 / 999, 24 x 9000 x 128 1640 / 1601 (4.4 MiB), 12 x 10700 x 128 1013 / 983 (5.2 MiB).  Past the line the
+    // rows do not fit: 24 x 30000 x 64 (7.3 MiB) 4390 / 4442, 16 x 16000 x 128 (7.8 MiB) 1900 / 1936.  With fewer slots than the
+    // chip holds at once (512 or 768) only the tail counts: 12 x 4000 x 64 311 / 319; columns of fewer than 32
+    // q-blocks leave classes of a few: 48 x 3000 x 128 727 / 740.
+    // (shares of about one round, which also keep an XCD on one head, lose 3-5 % at 24 x 12001 x 64 and 32 x 6000 x 128)
+    const bool by_head = wide0 && qdo_bytes / (B * Hkv) <= 5.5 * 1024 * 1024 && n_wide > 768 && Hq / Hkv * Mq >= 32;
+    const int wide_div = by_head ? (Hq / Hkv * Mq + 3) / 4 : 1;
     hipLaunchKernelGGL(psa_bwd_cost_kernel, dim3((unsigned)(row_wgs + (cols_ordered ? n_blocks : 0))), dim3(256), 0, st, p, row_wgs, cost,
-                       wide0 ? 1 : 0, cost_c);
+                       wide0 ? 1 : 0, wide_div, cost_c);
     if (int e = psa_check_launch("psa_bwd (cost)")) return e;
     psa_order::sort_lists<3>({{{cost, ord, (int)total, chunk, rows_ordered ? groups : 0},
                                {cost_c, ord_w, (int)n_wide, chunk_w, cols_ordered && wide0 ? groups_w : 0},
