@@ -19,6 +19,9 @@ namespace {
 
 constexpr int TK32 = 64;
 
+// V rows of slots that hold no key: their probabilities are 0, which only a finite value leaves 0
+__device__ __align__(16) const float f32_zero_chunk[4] = {};
+
 struct F32Params {
   const float *q, *k, *v, *kp, *vp;
   float* o;
@@ -82,7 +85,8 @@ __global__ __launch_bounds__(256, 2) void psa_fwd_f32_kernel(F32Params p) {
   const int64_t BHkv = (int64_t)p.B * p.Hkv, bhk = (int64_t)b * p.Hkv + hk;
 
   // Copies: this wave brings tile rows 16 wave .. 16 wave + 15 of K and V.  LDS position c of a row holds chunk c ^ (row % 16).
-  // Slots past the last key replicate a retained row (their logits are masked).
+  // Slots past the last key: K replicates a retained row (their logits are masked), V is zero - a replicated row with an infinite
+  // value would turn the infinity that it rightly gives its channel into 0 * inf.
   const uint32_t lds0 = psa_tiles::lds_addr_of(smem);
   auto issue_tile = [&](int t, int stage) __attribute__((always_inline)) {
     const psa_tiles::TileRef tr = psa_tiles::tile_ref(tdesc, ids, t, p.bn_log2);
@@ -100,7 +104,8 @@ __global__ __launch_bounds__(256, 2) void psa_fwd_f32_kernel(F32Params p) {
       const int chunk = (lane % G::CH) ^ row16;
       const uint32_t at = lds0 + (uint32_t)(stage * 2 * G::TILE + (wave * 16 + n * G::RPB) * G::ROW);
       psa_tiles::lds_copy16_addr((const char*)(kbase + (int64_t)src * kstr + chunk * 4), at);
-      psa_tiles::lds_copy16_addr((const char*)(vbase + (int64_t)src * vstr + chunk * 4), at + G::TILE);
+      const float* vsrc = wave * 16 + row16 < tr.nvalid ? vbase + (int64_t)src * vstr + chunk * 4 : f32_zero_chunk;
+      psa_tiles::lds_copy16_addr((const char*)vsrc, at + G::TILE);
     }
   };
   // operand addresses: K row l16 of a 16-key block, chunk 4 s + g; V rows 4 g + i, chunk l16 (+ 16 for the upper channels)

@@ -76,3 +76,19 @@ def test_contraction_shares(H, L, block_n, D):
     p = torch.exp(r - r.amax(-1, keepdim=True)).view(1, H, Mq, 16, -1).amax(3)
     ref = (p / p.sum(-1, keepdim=True))[..., :Nk]
     assert float((got.double() - ref).abs().max()) <= 2e-6
+
+
+@pytest.mark.parametrize("L,bn", [(131, 64), (4099, 32), (192, 128)])  # partly filled tiles (192: an empty one); 16 and 32 rows per workgroup
+@pytest.mark.parametrize("lv", [1, 2, 8])
+@pytest.mark.parametrize("D", [64, 128])
+def test_infinite_value_stays_infinite(L, bn, lv, D):
+    """Every query sees the last key, whose value is +inf in one channel: that channel is +inf for every query (weights of
+    order 1 / L times inf; the empty slots of the last tile add nothing) and the others are finite."""
+    from psa_hip import ops
+
+    q, k, v = _rand(4, L, D, seed=L)
+    v[:, :, L - 1, 5] = float("inf")
+    m = torch.full((1, 4, -(-L // 64), -(-L // bn)), lv, dtype=torch.int8, device=dev())
+    o = ops.sparse_attention_fwd(q, k, v, m, 64, bn)
+    assert bool((o[..., 5] == float("inf")).all())
+    assert bool(torch.isfinite(o[..., [c for c in range(D) if c != 5]]).all())
