@@ -305,8 +305,10 @@ __device__ __forceinline__ int density_eighths1(int lv) {
   return lv == 1 ? 8 : lv == 2 ? 4 : lv == 4 ? 2 : lv == 8 ? 1 : 0;
 }
 
-__global__ __launch_bounds__(256) void psa_density_kernel(const void* map, int map_elem, int Mq, int Nk, int causal, int32_t* part) {
-  __shared__ int s_part[4];
+// part == nullptr (one share per map, whose count may need more than 32 bits): the density itself goes to out
+__global__ __launch_bounds__(256) void psa_density_kernel(const void* map, int map_elem, int Mq, int Nk, int causal, int32_t* part, double cells,
+                                                          float* out) {
+  __shared__ int64_t s_part[4];
   const int64_t bh = blockIdx.x;
   const int64_t n = (int64_t)Mq * Nk;
   const int tid = threadIdx.x, shares = gridDim.y;
@@ -346,15 +348,19 @@ __global__ __launch_bounds__(256) void psa_density_kernel(const void* map, int m
     const int64_t r = idx / Nk;
     if (!causal || idx - r * Nk <= r) acc += density_eighths1(load_map(map, bh * n + idx, map_elem));
   }
+  int64_t sum = acc;
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
-  if ((tid & 63) == 0) s_part[tid >> 6] = acc;
+  for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+  if ((tid & 63) == 0) s_part[tid >> 6] = sum;
   __syncthreads();
-  if (tid == 0) part[bh * shares + blockIdx.y] = s_part[0] + s_part[1] + s_part[2] + s_part[3];
+  if (tid != 0) return;
+  sum = s_part[0] + s_part[1] + s_part[2] + s_part[3];
+  if (part != nullptr) part[bh * shares + blockIdx.y] = (int32_t)sum;
+  else out[bh] = (float)((double)sum * 0.125 / cells);
 }
 
-// out: the BH densities, then their mean (summed in index order); with H > 0 also 1 - mean and the H per-head means over the
-// BH / H batches.  One workgroup.  (With one share per map the counts may lie in out[] itself.)
+// out: the BH densities (of part's counts; part == nullptr: there already), then their mean (summed in index order); with H > 0
+// also 1 - mean and the H per-head means over the BH / H batches.  One workgroup.
 __global__ __launch_bounds__(256) void psa_density_mean_kernel(const int32_t* part, int shares, int BH, int H, double cells, float* out) {
   __shared__ float s_d[256];
   const int tid = threadIdx.x;
@@ -362,9 +368,15 @@ __global__ __launch_bounds__(256) void psa_density_mean_kernel(const int32_t* pa
   for (int i0 = 0; i0 < BH; i0 += 256) {
     const int i = i0 + tid;
     if (i < BH) {
-      int64_t t = 0;
-      for (int s = 0; s < shares; ++s) t += part[(int64_t)i * shares + s];
-      s_d[tid] = out[i] = (float)((double)t * 0.125 / cells);
+      float d;
+      if (part != nullptr) {
+        int64_t t = 0;
+        for (int s = 0; s < shares; ++s) t += part[(int64_t)i * shares + s];
+        out[i] = d = (float)((double)t * 0.125 / cells);
+      } else {
+        d = out[i];
+      }
+      s_d[tid] = d;
     }
     __syncthreads();
     if (tid == 0)
@@ -385,13 +397,13 @@ __global__ __launch_bounds__(256) void psa_density_mean_kernel(const int32_t* pa
 
 static int density_run(const void* map, int map_elem_bytes, int64_t bh, int H, int Mq, int Nk, int causal, int shares, int32_t* part,
                        float* out, psa_stream_t stream) {
-  PSA_REQUIRE(map && out && part, PSA_ERR_ARG, "psa_density: null pointer");
+  PSA_REQUIRE(map && out, PSA_ERR_ARG, "psa_density: null pointer");
   PSA_REQUIRE(map_elem_bytes == 1 || map_elem_bytes == 4, PSA_ERR_ARG, "psa_density: map_elem_bytes must be 1 or 4");
   PSA_REQUIRE(bh > 0 && bh < (1 << 30) && Mq > 0 && Nk > 0, PSA_ERR_ARG, "psa_density: bad sizes");
   const int sq = Mq < Nk ? Mq : Nk;
   const double cells = causal ? (double)sq * (sq + 1) / 2.0 + (Mq > Nk ? (double)(Mq - Nk) * Nk : 0.0) : (double)Mq * Nk;
   hipLaunchKernelGGL(psa_density_kernel, dim3((unsigned)bh, (unsigned)shares), dim3(256), 0, (hipStream_t)stream, map, map_elem_bytes, Mq,
-                     Nk, causal, part);
+                     Nk, causal, part, cells, out);
   hipLaunchKernelGGL(psa_density_mean_kernel, dim3(1), dim3(256), 0, (hipStream_t)stream, part, shares, (int)bh, H, cells, out);
   return psa_check_launch("psa_density");
 }
@@ -399,7 +411,7 @@ static int density_run(const void* map, int map_elem_bytes, int64_t bh, int H, i
 // (no workspace: one share per map)
 extern "C" int psa_density(const void* map, int map_elem_bytes, int64_t bh, int Mq, int Nk, int causal, float* density_out,
                            psa_stream_t stream) {
-  return density_run(map, map_elem_bytes, bh, 0, Mq, Nk, causal, 1, (int32_t*)density_out, density_out, stream);
+  return density_run(map, map_elem_bytes, bh, 0, Mq, Nk, causal, 1, nullptr, density_out, stream);
 }
 
 static int density_shares(int map_elem_bytes, int64_t bh, int Mq, int Nk) {
@@ -407,7 +419,9 @@ static int density_shares(int map_elem_bytes, int64_t bh, int Mq, int Nk) {
   int64_t s = (units + DENS_UNITS - 1) / DENS_UNITS;
   // at least about two workgroups per CU, down to one 16-byte unit per thread
   while (s * bh < 512 && s * 256 < units) s *= 2;
-  return (int)(s < 1 ? 1 : (s > DENS_MAX_SHARES ? DENS_MAX_SHARES : s));
+  // (a share's count has 32 bits: at most 2^27 map entries per share)
+  const int64_t least = ((int64_t)Mq * Nk) >> 27, most = least > DENS_MAX_SHARES ? least : DENS_MAX_SHARES;
+  return (int)(s < 1 ? 1 : (s > most ? most : s));
 }
 extern "C" int64_t psa_density_stats_workspace_bytes(int map_elem_bytes, int B, int H, int Mq, int Nk) {
   if (B <= 0 || H <= 0 || Mq <= 0 || Nk <= 0) return 0;
@@ -417,6 +431,7 @@ extern "C" int psa_density_stats(const void* map, int map_elem_bytes, int B, int
                                  float* stats_out, psa_stream_t stream) {
   PSA_REQUIRE(B > 0 && H > 0, PSA_ERR_ARG, "psa_density_stats: B and H must be positive");
   PSA_REQUIRE(Mq > 0 && Nk > 0, PSA_ERR_ARG, "psa_density_stats: bad sizes");
+  PSA_REQUIRE(workspace, PSA_ERR_ARG, "psa_density_stats: null pointer");
   return density_run(map, map_elem_bytes, (int64_t)B * H, H, Mq, Nk, causal, density_shares(map_elem_bytes, (int64_t)B * H, Mq, Nk),
                      (int32_t*)workspace, stats_out, stream);
 }
