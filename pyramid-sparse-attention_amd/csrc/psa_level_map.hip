@@ -305,10 +305,14 @@ __device__ __forceinline__ int density_eighths1(int lv) {
   return lv == 1 ? 8 : lv == 2 ? 4 : lv == 4 ? 2 : lv == 8 ? 1 : 0;
 }
 
-// part == nullptr (one share per map, whose count may need more than 32 bits): the density itself goes to out
-__global__ __launch_bounds__(256) void psa_density_kernel(const void* map, int map_elem, int Mq, int Nk, int causal, int32_t* part, double cells,
+// part == nullptr (one share per map, whose count may need more than 32 bits): the density itself goes to out.
+// NT threads: 256 for shares, 1024 where one workgroup counts a map and only its own loads in flight hide their latency (int8 maps,
+// us with 256 / 1024 threads: 12 of 256 x 1024 30 / 18, causal 173 / 71; 48 of 353 x 1410 56 / 30, causal 315 / 125; 1000 of
+// 256 x 256 61 / 61, causal 114 / 104; 12 of 64 x 64 9.8 / 8.8).
+template <int NT>
+__global__ __launch_bounds__(NT) void psa_density_kernel(const void* map, int map_elem, int Mq, int Nk, int causal, int32_t* part, double cells,
                                                           float* out) {
-  __shared__ int64_t s_part[4];
+  __shared__ int64_t s_part[NT / 64];
   const int64_t bh = blockIdx.x;
   const int64_t n = (int64_t)Mq * Nk;
   const int tid = threadIdx.x, shares = gridDim.y;
@@ -320,7 +324,7 @@ __global__ __launch_bounds__(256) void psa_density_kernel(const void* map, int m
   const int64_t units = (n - head) / epu;
   const unsigned char* body = base + head * map_elem;
   int acc = 0;
-  for (int64_t u = (int64_t)blockIdx.y * 256 + tid; u < units; u += (int64_t)shares * 256) {
+  for (int64_t u = (int64_t)blockIdx.y * NT + tid; u < units; u += (int64_t)shares * NT) {
     const u32x4 w = *(const u32x4*)(body + u * 16);
     if (causal) {
       const int64_t i0 = head + u * epu;
@@ -343,7 +347,7 @@ __global__ __launch_bounds__(256) void psa_density_kernel(const void* map, int m
     }
   }
   const int64_t singles = n - units * epu;
-  for (int64_t i = (int64_t)blockIdx.y * 256 + tid; i < singles; i += (int64_t)shares * 256) {
+  for (int64_t i = (int64_t)blockIdx.y * NT + tid; i < singles; i += (int64_t)shares * NT) {
     const int64_t idx = i < head ? i : i + units * epu;
     const int64_t r = idx / Nk;
     if (!causal || idx - r * Nk <= r) acc += density_eighths1(load_map(map, bh * n + idx, map_elem));
@@ -354,7 +358,9 @@ __global__ __launch_bounds__(256) void psa_density_kernel(const void* map, int m
   if ((tid & 63) == 0) s_part[tid >> 6] = sum;
   __syncthreads();
   if (tid != 0) return;
-  sum = s_part[0] + s_part[1] + s_part[2] + s_part[3];
+  sum = 0;
+#pragma unroll
+  for (int w = 0; w < NT / 64; ++w) sum += s_part[w];
   if (part != nullptr) part[bh * shares + blockIdx.y] = (int32_t)sum;
   else out[bh] = (float)((double)sum * 0.125 / cells);
 }
@@ -402,8 +408,10 @@ static int density_run(const void* map, int map_elem_bytes, int64_t bh, int H, i
   PSA_REQUIRE(bh > 0 && bh < (1 << 30) && Mq > 0 && Nk > 0, PSA_ERR_ARG, "psa_density: bad sizes");
   const int sq = Mq < Nk ? Mq : Nk;
   const double cells = causal ? (double)sq * (sq + 1) / 2.0 + (Mq > Nk ? (double)(Mq - Nk) * Nk : 0.0) : (double)Mq * Nk;
-  hipLaunchKernelGGL(psa_density_kernel, dim3((unsigned)bh, (unsigned)shares), dim3(256), 0, (hipStream_t)stream, map, map_elem_bytes, Mq,
-                     Nk, causal, part, cells, out);
+  const bool wide = part == nullptr;
+  auto kern = wide ? psa_density_kernel<1024> : psa_density_kernel<256>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)bh, (unsigned)shares), dim3(wide ? 1024 : 256), 0, (hipStream_t)stream, map, map_elem_bytes, Mq, Nk,
+                     causal, part, cells, out);
   hipLaunchKernelGGL(psa_density_mean_kernel, dim3(1), dim3(256), 0, (hipStream_t)stream, part, shares, (int)bh, H, cells, out);
   return psa_check_launch("psa_density");
 }
