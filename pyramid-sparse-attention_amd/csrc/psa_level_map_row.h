@@ -117,13 +117,18 @@ __device__ __forceinline__ void row_prefix_sums(double* wide, const float* sw, f
 // Levels by fixed quotas need no sorted row: the level of a column follows from how many of the `n_cuts` keys of rank
 // cut[0], cut[1], .. its own key reaches.  A histogram of the keys (SEL_BINS bins, 16 per octave below the row's best
 // score) finds the bin of every cut, the few keys in that bin are ranked by counting, and one pass compares each key
-// with the cut keys.  A bin that holds more than SEL_CAP keys (ties, scores more than 64 octaves below the best) is
-// resolved by building the cut key bit by bit instead.  Measured with the reduction of the estimator's workspace, which the
-// launch also does and which now bounds it: 3072 rows of 1024 scores 157 -> 105 us (403 MB read), 16944 rows of 1410 scores
-// 1480 -> 585 us (3.05 GB read, 5.2 TB/s), against the bitonic network.  Below RANK_SORT_MAX ranking by counting is as fast
-// and also serves the other modes.
+// with the cut keys.  A cut whose bin holds more than SEL_CAP keys descends into it: a histogram of the bin's (key, column)
+// range in SEL_BINS finer bins, until the cut's bin fits.  One descent is enough for flat rows (logits of standard deviation 0.25
+// to 1 put one to three cuts of a row of 512 to 2048 scores there), equal scores take up to three more, down to the column.
+// Bound by latency (a dozen barriers, six more per descent).  3072 rows of 1024 scores in us, logits of deviation 3 / 1 / 0.5 /
+// 0.25: 21 / 26 / 34 / 41, bitonic network 65 to 71 whatever the scores; 3072 rows of 512: 17 / 18 / 20 / 28 against 34; of
+// 2048: 31 / 46 / 58 / 60 against 200.  (Building the cut key bit by bit over the whole row instead of descending: 21 / 58 / 138 /
+// 266 at 1024 scores.)  With the reduction of the estimator's workspace, which the launch also does and which bounds it: 16944
+// rows of 1410 scores 1480 -> 585 us (3.05 GB read, 5.2 TB/s).  Below RANK_SORT_MAX ranking by counting is as fast and also
+// serves the other modes.
 // LDS: (SEL_BINS + 2 * SEL_MAX_CUTS * SEL_CAP + 8 * SEL_MAX_CUTS) 4-byte words.  256 threads.
 constexpr int SEL_BINS = 1024, SEL_SHIFT = 19, SEL_CAP = 64, SEL_MAX_CUTS = 8;
+constexpr int SEL_COL_BITS = 13;  // columns of a row: at most 6144
 constexpr size_t SEL_LDS_BYTES = (SEL_BINS + 2 * SEL_MAX_CUTS * SEL_CAP + 8 * SEL_MAX_CUTS) * 4;
 __host__ __device__ inline bool level_map_selects(int mode, int n_cuts, int Nk) {
   return mode == PSA_MODE_TOPK && n_cuts <= SEL_MAX_CUTS && Nk > RANK_SORT_MAX;
@@ -138,6 +143,7 @@ __device__ __forceinline__ void level_map_row_select(const LevelMapParams& p, co
   int* n_in = before + SEL_MAX_CUTS;                      // [cut] keys in that bin
   int* fill = n_in + SEL_MAX_CUTS;                        // [cut] keys collected so far
   int* wsum = fill + SEL_MAX_CUTS;                        // [8] partial results of the waves
+  int* found = wsum + 8;                                  // [3] bin of a cut inside a crowded bin, keys before it, keys in it
   const int N = p.Nk, lane = tid & 63, wave = tid >> 6, C = p.n_cuts;
 
   for (int i = tid; i < SEL_BINS; i += NT) hist[i] = 0;
@@ -165,7 +171,8 @@ __device__ __forceinline__ void level_map_row_select(const LevelMapParams& p, co
   };
   for (int j = tid; j < N; j += NT) atomicAdd(&hist[bin_at(desc_key(src[j]))], 1);
   __syncthreads();
-  {
+  // hit(bin, keys before it, keys in it) for every bin that holds keys (one barrier inside)
+  auto scan_hist = [&](auto hit) __attribute__((always_inline)) {
     int c[PER], sum = 0;
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
@@ -185,16 +192,18 @@ __device__ __forceinline__ void level_map_row_select(const LevelMapParams& p, co
     for (int w = 0; w < NT / 64; ++w) run += w < wave ? wsum[4 + w] : 0;
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
-      if (c[e] > 0)
-        for (int t = 0; t < C; ++t)
-          if (p.cut[t] >= run && p.cut[t] < run + c[e]) {
-            bin_of[t] = tid * PER + e;
-            before[t] = run;
-            n_in[t] = c[e];
-          }
+      if (c[e] > 0) hit(tid * PER + e, run, c[e]);
       run += c[e];
     }
-  }
+  };
+  scan_hist([&](int bin, int first, int n) __attribute__((always_inline)) {
+    for (int t = 0; t < C; ++t)
+      if (p.cut[t] >= first && p.cut[t] < first + n) {
+        bin_of[t] = bin;
+        before[t] = first;
+        n_in[t] = n;
+      }
+  });
   __syncthreads();
   int cut_bin[SEL_MAX_CUTS];
 #pragma unroll
@@ -210,6 +219,13 @@ __device__ __forceinline__ void level_map_row_select(const LevelMapParams& p, co
       }
   }
   __syncthreads();
+  // the key of rank `rank` among the n candidates of cut t (one wave)
+  auto rank_cand = [&](int t, int n, int rank) __attribute__((always_inline)) {
+    const uint64_t mine = lane < n ? cand[t * SEL_CAP + lane] : ~0ull;
+    int below = 0;
+    for (int i = 0; i < n; ++i) below += cand[t * SEL_CAP + i] < mine ? 1 : 0;
+    if (lane < n && below == rank) cut_key[t] = mine;
+  };
   bool crowded = false;
 #pragma unroll
   for (int t = 0; t < SEL_MAX_CUTS; ++t)
@@ -218,30 +234,45 @@ __device__ __forceinline__ void level_map_row_select(const LevelMapParams& p, co
       if (n > SEL_CAP) {
         crowded = true;
       } else if ((t & 3) == wave) {
-        const uint64_t mine = lane < n ? cand[t * SEL_CAP + lane] : ~0ull;
-        int rank = 0;
-        for (int i = 0; i < n; ++i) rank += cand[t * SEL_CAP + i] < mine ? 1 : 0;
-        if (lane < n && rank == p.cut[t] - before[t]) cut_key[t] = mine;
+        rank_cand(t, n, p.cut[t] - before[t]);
       }
     }
   if (crowded) {  // uniform: the counts are the same for every thread
     for (int t = 0; t < C; ++t) {
-      if (n_in[t] <= SEL_CAP) continue;
-      uint64_t k0 = 0;
-      for (int bit = 63; bit >= 0; --bit) {
-        if (bit == 31) bit = 15;  // columns have 16 bits
-        const uint64_t probe = k0 | (1ull << bit);
-        int below = 0;
-        for (int j0 = 0; j0 < N; j0 += NT) {
-          const int j = j0 + tid;
-          below += __popcll(__ballot(j < N && (((uint64_t)desc_key(src[j < N ? j : 0]) << 32) | (uint32_t)j) < probe));
+      int n = n_in[t], rank = p.cut[t] - before[t];
+      if (n <= SEL_CAP) continue;
+      // the cut's bin as a range of (score key, column), 2^bits wide from lo (the last bin: everything past its start)
+      int bits = bin_of[t] < SEL_BINS - 1 ? SEL_SHIFT + SEL_COL_BITS : 32 + SEL_COL_BITS;
+      uint64_t lo = (uint64_t)(kmin + ((uint32_t)bin_of[t] << SEL_SHIFT)) << SEL_COL_BITS;
+      auto offset = [&](int j) __attribute__((always_inline)) { return (((uint64_t)desc_key(src[j]) << SEL_COL_BITS) | (uint32_t)j) - lo; };
+      while (n > SEL_CAP) {  // (keys are unique: 64 of them span more than 5 bits)
+        const int shift = bits - 10;
+        for (int i = tid; i < SEL_BINS; i += NT) hist[i] = 0;
+        __syncthreads();
+        for (int j = tid; j < N; j += NT) {
+          const uint64_t d = offset(j);
+          if (d >> bits == 0) atomicAdd(&hist[(int)(d >> shift)], 1);
         }
         __syncthreads();
-        if (lane == 0) wsum[wave] = below;
+        scan_hist([&](int bin, int first, int cnt) __attribute__((always_inline)) {
+          if (rank >= first && rank < first + cnt) {
+            found[0] = bin;
+            found[1] = first;
+            found[2] = cnt;
+          }
+        });
         __syncthreads();
-        if (wsum[0] + wsum[1] + wsum[2] + wsum[3] <= p.cut[t]) k0 = probe;
+        lo += (uint64_t)(uint32_t)found[0] << shift;
+        rank -= found[1];
+        n = found[2];
+        bits = shift;
       }
-      if (tid == 0) cut_key[t] = k0;
+      if (tid == 0) fill[t] = 0;
+      __syncthreads();
+      for (int j = tid; j < N; j += NT)
+        if (offset(j) >> bits == 0) cand[t * SEL_CAP + atomicAdd(&fill[t], 1)] = ((uint64_t)desc_key(src[j]) << 32) | (uint32_t)j;
+      __syncthreads();
+      if ((t & 3) == wave) rank_cand(t, n, rank);
     }
   }
   __syncthreads();

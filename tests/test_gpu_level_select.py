@@ -49,3 +49,53 @@ def test_density_stats(B, H, Mq, Nk, causal):
         np.testing.assert_allclose(float(d[-1]), ref.mean(), rtol=1e-6, atol=1e-9)
         np.testing.assert_allclose(float(sparsity), 1 - ref.mean(), rtol=1e-6)
         np.testing.assert_allclose(per_head.cpu().numpy(), ref.mean(0), rtol=1e-6, atol=1e-9)
+
+
+def _normal_scores(rows, Nk, deviation, seed):
+    """What the block estimate gives for independent normal logits: per key group the best of 8, per q-block the best of 32 rows."""
+    g = torch.Generator(device=dev()).manual_seed(seed)
+    z = torch.randn(rows, 32, Nk, generator=g, device=dev())
+    for _ in range(7):
+        z = torch.maximum(z, torch.randn(z.shape, generator=g, device=dev()))
+    z = z * deviation
+    s = torch.exp(z - z.amax(-1, keepdim=True)).amax(1)
+    return (s / s.sum(-1, keepdim=True)).view(1, 1, rows, Nk).contiguous()
+
+
+@pytest.mark.parametrize("Nk", [257, 1024, 2048, 6144])
+@pytest.mark.parametrize("deviation", [0.01, 0.25, 0.5, 1.0])
+def test_quota_levels_of_flat_rows(Nk, deviation):
+    """Hundreds of keys in the histogram bin of a cut."""
+    from psa_hip import ops
+
+    s = _normal_scores(6, Nk, deviation, Nk)
+    s[0, 0, 1] = torch.where(torch.arange(Nk, device=dev()) % 3 == 0, s[0, 0, 1, 0], s[0, 0, 1])  # a third of the row ties
+    s[0, 0, 2, : Nk // 2] = 0.0
+    ref = O.level_map(s.cpu().numpy(), QUOTAS, 0, "topk", blocksize=32, compute_tile=32)
+    got = ops.level_map(s, QUOTAS, 0, "topk", blocksize=32, compute_tile=32, map_dtype=torch.int32)
+    assert np.array_equal(got.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("Nk", [512, 1024, 2048])
+def test_flat_rows_cost_about_what_peaked_rows_cost(Nk):
+    """Time of flat rows against rows whose bins hold a few keys each, of one kernel on one card.  Each of the three cuts adds a
+    descent of about six barriers to a kernel of a dozen: a factor of up to two, measured 1.7 to 2.0.  A search through all bits
+    of the key took 8 to 16 times as long, a full sort of the row 2 to 7 times."""
+    from psa_hip import ops
+
+    def us(s):
+        go = lambda: ops.level_map(s, QUOTAS, 0, "topk", blocksize=32, compute_tile=32, map_dtype=torch.int8)
+        go()
+        times = []
+        for _ in range(5):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(5):
+                go()
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times)
+
+    flat, peaked = (_normal_scores(64, Nk, d, 1).expand(1, 48, 64, Nk).contiguous() for d in (0.25, 3.0))
+    assert us(flat) < 5.0 * us(peaked)
