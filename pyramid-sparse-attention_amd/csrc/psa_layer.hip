@@ -9,14 +9,17 @@ int psa_map_min_cap_heads(void* map, int map_elem_bytes, const int32_t* cap, int
 
 namespace {
 
-// consecutive parts of a workspace, 256-byte aligned
+// Consecutive parts of a workspace, 256-byte aligned.  What the estimate needs (gigabytes for long sequences of short blocks) is
+// dead once the map exists: the parts of the stages behind it start where the estimate's do (reuse), in stream order.
 struct Parts {
-  int64_t at = 0;
+  int64_t at = 0, top = 0;
   int64_t take(int64_t bytes) {
     const int64_t off = at;
     at = (at + bytes + 255) & ~(int64_t)255;
+    top = at > top ? at : top;
     return off;
   }
+  void reuse(int64_t from) { at = from; }
 };
 
 // pools, walk (or row order) and attention of either layer
@@ -24,10 +27,12 @@ struct AttnParts {
   int64_t kp, vp, walk, order;
   bool has_walk;
 };
-void attn_parts(Parts& w, int elem, int B, int Hq, int Hkv, int L, int D, int block_m, int block_n, int walk, AttnParts& a) {
+void pool_parts(Parts& w, int elem, int B, int Hkv, int L, int D, int block_n, AttnParts& a) {
   const int64_t pool = psa_pool_elems(B, Hkv, L, D, block_n) * elem;
   a.kp = w.take(pool);
   a.vp = w.take(pool);
+}
+void walk_parts(Parts& w, int elem, int B, int Hq, int Hkv, int L, int D, int block_m, int block_n, int walk, AttnParts& a) {
   const int64_t walk_bytes = walk && elem == 2 ? psa_walk_bytes(B, Hq, Hkv, L, D, block_m, block_n) : 0;
   a.has_walk = walk_bytes > 0;
   a.walk = a.has_walk ? w.take(walk_bytes) : -1;
@@ -55,13 +60,17 @@ bool layer_parts(int elem, int B, int Hq, int Hkv, int L, int D, int block_m, in
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || L <= 0 || D <= 0 || block_m < 4 || block_n < 4 || (elem != 2 && elem != 4)) return false;
   const int64_t Mq = (L + block_m - 1) / block_m, Nk = (L + block_n - 1) / block_n;
   Parts w;
-  p.est = w.take(psa_estimate_workspace_bytes(B, Hq, L, L, block_m, block_n, block_m / 4, block_n / 4));
-  p.scores = Nk > 4096 ? w.take((int64_t)B * Hq * Mq * Nk * 4) : -1;  // (maps too wide for the fused kernel's LDS)
   const int64_t rows = indexed ? (int64_t)B * Hkv * L * D * elem : 0;
   p.k_ord = w.take(rows);
   p.v_ord = w.take(rows);
-  attn_parts(w, elem, B, Hq, Hkv, L, D, block_m, block_n, walk, p.attn);
-  p.bytes = w.at;
+  if (indexed) pool_parts(w, elem, B, Hkv, L, D, block_n, p.attn);  // (filled with the ordered rows, before the estimate)
+  const int64_t from = w.at;
+  p.est = w.take(psa_estimate_workspace_bytes(B, Hq, L, L, block_m, block_n, block_m / 4, block_n / 4));
+  p.scores = Nk > 4096 ? w.take((int64_t)B * Hq * Mq * Nk * 4) : -1;  // (maps too wide for the fused kernel's LDS)
+  w.reuse(from);
+  if (!indexed) pool_parts(w, elem, B, Hkv, L, D, block_n, p.attn);
+  walk_parts(w, elem, B, Hq, Hkv, L, D, block_m, block_n, walk, p.attn);
+  p.bytes = w.top;
   return true;
 }
 
@@ -73,12 +82,15 @@ bool causal_parts(int B, int Hq, int Hkv, int L, int D, int block, int stride, i
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || L <= 0 || D <= 0 || block <= 0 || stride <= 0 || chunk <= 0) return false;
   const int64_t S = (L + block - 1) / block;
   Parts w;
-  p.est = w.take(psa_estimate_xattn_workspace_bytes(B, Hq, L, L, block, stride, chunk));
-  p.scores = w.take((int64_t)B * Hq * S * S * 4);
   p.map = w.take((int64_t)B * Hq * S * S);
   p.cap = w.take((int64_t)B * Hkv * S * 4);
-  attn_parts(w, 2, B, Hq, Hkv, L, D, block, block, 1, p.attn);
-  p.bytes = w.at;
+  const int64_t from = w.at;
+  p.est = w.take(psa_estimate_xattn_workspace_bytes(B, Hq, L, L, block, stride, chunk));
+  p.scores = w.take((int64_t)B * Hq * S * S * 4);
+  w.reuse(from);
+  pool_parts(w, 2, B, Hkv, L, D, block, p.attn);
+  walk_parts(w, 2, B, Hq, Hkv, L, D, block, block, 1, p.attn);
+  p.bytes = w.top;
   return true;
 }
 

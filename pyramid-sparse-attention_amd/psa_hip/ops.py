@@ -630,6 +630,12 @@ def _side_stream(device: torch.device) -> "torch.cuda.Stream":
 
 
 # ----------------------------------------------------------------------------- whole layer, forward only
+# Workspace above which a layer goes through the separate operators: they hand the estimate's scratch back before the output is
+# taken (48 heads x 45106 tokens with 32-key blocks: 4.0 GiB at most against 4.3), and the host's share, which one call saves, is
+# long hidden behind milliseconds of kernels.
+_ONE_CALL_MAX_BYTES = 1 << 30
+
+
 def _layer_one_call(qb, kb, vb, off_q, off_k, mask_ratios, mode, block_m, block_n, tile_n, sm_scale, text_length, token_index=None,
                     sim_thresholds=None):
     """(out, map, cap) of psa_layer_fwd's sequence as one library call on one stream, or None where the arguments are not the
@@ -654,7 +660,7 @@ def _layer_one_call(qb, kb, vb, off_q, off_k, mask_ratios, mode, block_m, block_
     Mq, Nk = -(-L // block_m), -(-L // block_n)
     walk = int(_lists_tiles(qb.dtype, block_n, B * Hq * Mq))
     n_ws = lib.psa_layer_workspace_bytes(qb.element_size(), B, Hq, Hkv, L, D, block_m, block_n, int(token_index is not None), walk)
-    if n_ws <= 0:
+    if not 0 < n_ws <= _ONE_CALL_MAX_BYTES:
         return None
     lv, hi = _level_items(items)
     ws = torch.empty(n_ws, dtype=torch.uint8, device=dev)
@@ -684,7 +690,7 @@ def causal_layer_fwd(q, k, v, mask_ratios, mode, text_length, block, stride, chu
     if k.shape != (B, Hkv, L, D) or Hkv == 0 or Hq % Hkv or len(mask_ratios) > _lib.PSA_MAX_LEVEL_ITEMS:
         return None
     n_ws = lib.psa_causal_layer_workspace_bytes(B, Hq, Hkv, L, D, block, stride, chunk_size)
-    if n_ws <= 0:
+    if not 0 < n_ws <= _ONE_CALL_MAX_BYTES:
         return None
     q, k, v = _kernel_view(q), _kernel_view(k), _kernel_view(v)
     items = list(mask_ratios.items())

@@ -83,3 +83,36 @@ def test_one_call_refuses_what_the_operators_refuse():
                dict(k=k[:, :, :128]), dict(v=v[:, :1]), dict(tile_n=128), dict(q=q[0])):
         with pytest.raises((ValueError, RuntimeError)):
             go(**kw)
+
+
+@pytest.mark.parametrize("causal", [False, True])
+def test_large_layers_hand_their_scratch_back_first(monkeypatch, causal):
+    """Above the workspace limit the separate operators run: same bits, and the output is not taken beside the estimate's scratch."""
+    from psa_hip import _lib, ops
+    from psa_hip.PSA_casual import AttentionConfig, PyramidAdaptiveBlockSparseAttnTrain
+
+    H, L, D = 8, 16000, 64
+    q, k, v = (rnd(1, H, L, D, seed=i).to(dev()) for i in range(3))
+    if causal:
+        m = PyramidAdaptiveBlockSparseAttnTrain(AttentionConfig(text_length=70, xattn_stride=4), layer_idx=0)
+        layer = lambda: m(q, k, v, layer_idx=0)
+    else:
+        off_q, off_k = ops.draw_sample_offsets(1, H, H, 128, 32, 32, 8, dev(), seed=1)
+        layer = lambda: ops.psa_layer_fwd(q, k, v, off_q, off_k, RATIOS, "topk", 128, 32, 16)
+
+    def run(limit):
+        monkeypatch.setattr(ops, "_ONE_CALL_MAX_BYTES", limit)
+        layer()
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        before = torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        out = layer()
+        torch.cuda.synchronize()
+        return out, torch.cuda.max_memory_allocated() - before
+
+    (a, one), (b, separate) = run(1 << 30), run(1 << 20)
+    assert torch.equal(a, b)
+    if not causal:  # (K below _SIDE_STREAM_MIN_BYTES, a layer that is one call; the estimate's stage is the larger one)
+        est = _lib.lib.psa_estimate_workspace_bytes(1, H, L, L, 128, 32, 32, 8)
+        assert one >= est + q.numel() * 2 > separate
