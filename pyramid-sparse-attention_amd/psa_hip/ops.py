@@ -526,10 +526,18 @@ def build_schedule(level_map_: torch.Tensor, Hkv: int, L: int, D: int, block_m: 
 # 520 rows head dim 64 51.4 / 48.6, 2080 rows 121.6 / 123.3; 16944 rows (45106 tokens, 48 heads) 4.5 ms / 4.9 ms.
 # At head dim 128, which is bound by power, 568 rows 94.1 / 95.9, 2080 rows 233 / 231 (in the layer 377 / 385).
 _WALK_MIN_ROWS = 1024
+# Bytes of a list above which such a map is walked in the kernel: the list has room for the longest possible walk, 10 to 20 times the
+# int8 map (290 MB for 48 heads x 45106 tokens of 32-key blocks; 40 heads x 262144 tokens of 64-key blocks would take 6.7 GB), and
+# the kernel needs none of it.  (Maps of 128-key blocks have always been listed.)
+_WALK_MAX_BYTES = 1 << 30
 
 
-def _lists_tiles(dtype: torch.dtype, block_n: int, rows: int) -> bool:
-    return dtype in _T16 and (block_n == 128 or rows > _WALK_MIN_ROWS)
+def _walk_bytes(dtype: torch.dtype, B: int, Hq: int, Hkv: int, L: int, D: int, block_m: int, block_n: int) -> int:
+    """Bytes of the tile list that a call on a level map builds for itself, 0: the map is walked in the kernel."""
+    if dtype not in _T16 or (block_n != 128 and B * Hq * -(-L // block_m) <= _WALK_MIN_ROWS):
+        return 0
+    n = lib.psa_walk_bytes(B, Hq, Hkv, L, D, block_m, block_n)
+    return n if block_n == 128 or n <= _WALK_MAX_BYTES else 0
 
 
 def sparse_attention_fwd(
@@ -585,8 +593,8 @@ def sparse_attention_fwd(
         q_index = _check_index(q_index, L)
     shape = (B, Hq, Hkv, L, D, block_m, block_n)
     n_walk = 0
-    if level_map_ is not None and balance and schedule is not False and _lists_tiles(qb.dtype, block_n, B * Hq * Mq):
-        n_walk = lib.psa_walk_bytes(*shape)
+    if level_map_ is not None and balance and schedule is not False:
+        n_walk = _walk_bytes(qb.dtype, *shape)
     if n_walk > 0:
         # the map's tiles are listed once (one pass over the map) and walked by the kernel
         walk = schedule
@@ -658,7 +666,7 @@ def _layer_one_call(qb, kb, vb, off_q, off_k, mask_ratios, mode, block_m, block_
         token_index = _check_index(token_index, L)
     items, m, _ = _items(mask_ratios, mode)
     Mq, Nk = -(-L // block_m), -(-L // block_n)
-    walk = int(_lists_tiles(qb.dtype, block_n, B * Hq * Mq))
+    walk = int(_walk_bytes(qb.dtype, B, Hq, Hkv, L, D, block_m, block_n) > 0)
     n_ws = lib.psa_layer_workspace_bytes(qb.element_size(), B, Hq, Hkv, L, D, block_m, block_n, int(token_index is not None), walk)
     if not 0 < n_ws <= _ONE_CALL_MAX_BYTES:
         return None

@@ -64,3 +64,42 @@ def test_dense_walk_equals_map_of_ones(H, Hkv, L, causal, block_n, strided, D):
     b = ops.sparse_attention_fwd(q, k, v, None, BM, block_n, causal=causal, return_lse=True)
     torch.cuda.synchronize()
     _same(a, b)
+
+
+@pytest.mark.parametrize("block_n,listed", [(32, False), (64, False), (128, True)])
+def test_lists_have_a_byte_limit(monkeypatch, block_n, listed):
+    """Above the limit a map of 32- / 64-key blocks is walked in the kernel, by the operator and by the layer in one call: same bits,
+    and no memory for a list.  (128-key blocks: always listed.)"""
+    from psa_hip import ops
+
+    H, L, D = 80, 1800, 64
+    q, k, v = _inputs(1, H, H, L, D, L, False)
+    lmap = torch.from_numpy(random_map(1, H, -(-L // BM), -(-L // block_n), L)).to(torch.int8).to(dev())
+    ratios = {1: (0.0, 0.1), 2: (0.1, 0.15), 4: (0.15, 0.2), 8: (0.2, 0.35), 0: (0.35, 1.0)}
+    off_q, off_k = ops.draw_sample_offsets(1, H, H, BM, 32, block_n, block_n // 4, dev(), seed=1)
+    idx = torch.randperm(L, generator=torch.Generator().manual_seed(1)).to(torch.int32).to(dev())
+    shape = (1, H, H, L, D, BM, block_n)
+    calls = []
+    one_call = ops._layer_one_call
+    monkeypatch.setattr(ops, "_layer_one_call", lambda *a: calls.append(one_call(*a)) or calls[-1])
+
+    def run():
+        fwd = lambda: ops.sparse_attention_fwd(q, k, v, lmap, BM, block_n, return_lse=True)
+        fwd()
+        torch.cuda.synchronize()
+        before = torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        a = fwd()[:2]
+        torch.cuda.synchronize()
+        peak = torch.cuda.max_memory_allocated() - before
+        return a, ops.psa_layer_fwd(q, k, v, off_q, off_k, ratios, "topk", BM, block_n, 16, token_index=idx), peak
+
+    (a, la, peak_a), n = run(), ops._walk_bytes(q.dtype, *shape)
+    assert n > 0
+    monkeypatch.setattr(ops, "_WALK_MAX_BYTES", n - 1)
+    assert (ops._walk_bytes(q.dtype, *shape) == n) == listed
+    b, lb, peak_b = run()
+    _same(a, b)
+    assert torch.equal(la, lb)
+    assert all(c is not None for c in calls)
+    assert listed or peak_b < peak_a - n // 2

@@ -36,3 +36,22 @@ def test_causal_layer_stages_share_their_scratch(B, Hq, Hkv, L, D, block, stride
     need = B * Hq * S * S + 4 * B * Hkv * S + max(est, behind)
     got = lib.psa_causal_layer_workspace_bytes(B, Hq, Hkv, L, D, block, stride, 4096)
     assert need <= got <= need + SLACK
+
+
+@pytest.mark.parametrize("dtype,shape,listed", [
+    ("bfloat16", (1, 48, 48, 45106, 64, 128, 32), True),
+    ("bfloat16", (2, 48, 48, 45106, 64, 128, 64), True),
+    ("bfloat16", (1, 40, 40, 262144, 128, 128, 64), False),  # 6.7 GB of list
+    ("float16", (1, 40, 40, 262144, 128, 128, 128), True),   # 128-key blocks have always been listed
+    ("bfloat16", (1, 8, 8, 1000, 64, 128, 64), False),       # few rows
+    ("float32", (1, 48, 48, 45106, 64, 128, 32), False),
+    ("bfloat16", (1, 48, 48, 45106, 64, 64, 32), False),     # 64-row q-blocks
+])
+def test_tile_lists_are_bounded(dtype, shape, listed):
+    import torch
+    from psa_hip import ops
+    from psa_hip._lib import lib
+
+    n = ops._walk_bytes(getattr(torch, dtype), *shape)
+    assert n == (lib.psa_walk_bytes(*shape) if listed else 0)
+    assert (n > 0) == listed and (shape[-1] == 128 or n <= 1 << 30)
