@@ -87,9 +87,9 @@ def adaptive_block_sparse_attn(q, k, v, config: AttentionConfig, sparse_attentio
     block = config.query_block
     needs_grad = torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad)
     # (dual tensors of forward-mode differentiation go to the autograd function, which has no such rule and says so)
-    plain = not needs_grad and forward_ad._current_level < 0
-    if (plain and not compute_stats and block == 128 and config.importance_method == "xattn"
-            and getattr(sparse_attention_fn, "one_call_causal", None) is bool(config.causal_main)):
+    if (not needs_grad and not compute_stats and block == 128 and config.importance_method == "xattn"
+            and getattr(sparse_attention_fn, "one_call_causal", None) is bool(config.causal_main)
+            and all(forward_ad.unpack_dual(t).tangent is None for t in (q, k, v))):
         out = ops.causal_layer_fwd(q, k, v, config.mask_ratios, config.mask_mode, config.text_length, block, config.xattn_stride,
                                    config.xattn_chunk_size, config.causal_main,
                                    (config.sim_2x_threshold, config.sim_4x_threshold, config.sim_8x_threshold))

@@ -11,8 +11,14 @@ from ._lib import Tensor4, check, lib
 LEVELS = (1, 2, 4, 8)
 
 
+# (the raw handle without a Stream object around it, where this torch has that call: 0.2 us against 2.0, several times per layer)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(t: torch.Tensor) -> int:
-    return torch._C._cuda_getCurrentRawStream(t.device.index)
+    if _raw_stream is None:
+        return torch.cuda.current_stream(t.device).cuda_stream
+    return _raw_stream(t.device.index)
 
 
 class _Here:

@@ -116,3 +116,50 @@ def test_large_layers_hand_their_scratch_back_first(monkeypatch, causal):
     if not causal:  # (K below _SIDE_STREAM_MIN_BYTES, a layer that is one call; the estimate's stage is the larger one)
         est = _lib.lib.psa_estimate_workspace_bytes(1, H, L, L, 128, 32, 32, 8)
         assert one >= est + q.numel() * 2 > separate
+
+
+def test_causal_one_call_leaves_dual_tensors_to_the_autograd_function(monkeypatch):
+    """Forward-mode differentiation has no rule here: it is refused.  An open level alone changes nothing."""
+    from torch.autograd import forward_ad
+
+    from psa_hip import ops
+    from psa_hip.PSA_casual import AttentionConfig, PyramidAdaptiveBlockSparseAttnTrain
+
+    q, k, v = (rnd(1, 2, 300, 64, seed=i).to(dev()) for i in range(3))
+    m = PyramidAdaptiveBlockSparseAttnTrain(AttentionConfig(text_length=0), layer_idx=0)
+    with torch.no_grad():
+        a = m(q, k, v, layer_idx=0)
+        calls = []
+        one_call = ops.causal_layer_fwd
+        monkeypatch.setattr(ops, "causal_layer_fwd", lambda *x: calls.append(1) or one_call(*x))
+        with forward_ad.dual_level():
+            b = m(q, k, v, layer_idx=0)
+            assert calls
+            with pytest.raises(RuntimeError):
+                m(q, k, forward_ad.make_dual(v, torch.ones_like(v)), layer_idx=0)
+            assert len(calls) == 1
+    assert torch.equal(a, b)
+
+
+def test_layer_runs_on_the_current_stream_without_the_raw_handle(monkeypatch):
+    """The public way to the stream's handle, for a torch without the shorter call: the layer follows work that the caller's stream
+    still has to do, as with it."""
+    from psa_hip import ops
+
+    q, k, v = (rnd(1, 2, 1000, 64, seed=i).to(dev()) for i in range(3))
+    off_q, off_k = ops.draw_sample_offsets(1, 2, 2, 128, 32, 64, 16, dev(), seed=1)
+    outs = []
+    for raw in (ops._raw_stream, None):
+        monkeypatch.setattr(ops, "_raw_stream", raw)
+        s = torch.cuda.Stream()
+        assert ops._stream(q) == torch.cuda.current_stream().cuda_stream
+        s.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(s):
+            assert ops._stream(q) == s.cuda_stream
+            x = q
+            for _ in range(50):
+                x = x * 1.0
+            outs.append(ops.psa_layer_fwd(x, k, v, off_q, off_k, RATIOS, "topk", 128, 64, 16))
+        torch.cuda.current_stream().wait_stream(s)
+        torch.cuda.synchronize()
+    assert torch.equal(outs[0], outs[1])
