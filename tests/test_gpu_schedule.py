@@ -79,8 +79,8 @@ def test_schedule_is_reusable_and_deterministic():
     assert lib.psa_schedule_bytes(B, H, H, L, 32, BM, BN) == 0 and lib.psa_schedule_bytes(B, H, H, L, D, 64, BN) == 0
 
 
-def test_strided_rows_fall_back_to_the_map_walk():
-    """K / V rows that are not D elements apart ([B, L, H, D] storage) use the schedule's order with the map walk."""
+def test_strided_rows_walk_the_same_schedule():
+    """K / V rows that are not D elements apart ([B, L, H, D] storage): the same records walked with the rows' own stride."""
     from psa_hip import ops
 
     B, H, L = 1, 2, 1500
@@ -93,6 +93,31 @@ def test_strided_rows_fall_back_to_the_map_walk():
     o1 = ops.sparse_attention_fwd(q, kt, vt, lmap, BM, BN)
     torch.cuda.synchronize()
     assert kt.stride(2) != D and torch.equal(o0, o1)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_strided_rows_fall_back_to_the_map_walk(D):
+    """K / V rows 16 MiB apart, further than the record walk's 24-bit row strides reach: the map walk in the schedule's order.  Head
+    dim 64 is the same kernel, hence the same bits; head dim 128 goes from the two-group kernel to the one-row one, which rounds
+    its probabilities against another running maximum."""
+    from psa_hip import ops
+
+    H, L, step = 2, 126, 1 << 23
+    q, k, v = _inputs(1, 1, 1, L, seed=6, D=D)
+    q = q.expand(1, H, L, D).contiguous()
+    far = torch.empty(L * step, dtype=k.dtype, device=dev())  # (2.1 GB; rows of K and V side by side)
+    kf, vf = (far.as_strided((1, 1, L, D), (L * step, L * step, step, 1), at) for at in (0, D))
+    kf.copy_(k)
+    vf.copy_(v)
+    lmap = torch.tensor([1, 2], dtype=torch.int8, device=dev()).view(1, H, 1, 1)
+    pools = ops.pool_kv(k, v, BN)
+    for sched in (ops.build_schedule(lmap, 1, L, D, BM, BN), None):
+        a = ops.sparse_attention_fwd(q, k, v, lmap, BM, BN, pools=pools, schedule=sched)
+        b = ops.sparse_attention_fwd(q, kf, vf, lmap, BM, BN, pools=pools, schedule=sched)
+        torch.cuda.synchronize()
+        assert kf.stride(2) * 2 >= 1 << 24
+        mx, mean = attn_errors(b, a.cpu())
+        assert torch.equal(a, b) if D == 64 else mx <= MAX_ABS and mean <= MEAN_ABS, (mx, mean)
 
 
 @pytest.mark.parametrize("H,Hkv,L", [(3, 3, 128 * 40), (40, 1, 128 * 128), (64, 1, 128 * 300 + 5), (160, 1, 128 * 300)])
@@ -137,3 +162,36 @@ def test_issue_order_is_a_stable_sort_of_every_share(H, Hkv, L):
         share = share[share >= 0]
         want = sorted(share.tolist(), key=lambda r: (-min(int(tiles[r]), 2047), r))
         assert share.tolist() == want, s0
+
+
+@pytest.mark.parametrize("D", [128, 64])
+@pytest.mark.parametrize("strided,causal,indexed", [(False, False, False), (True, False, True), (False, True, False), (True, True, False)])
+def test_fwd_scheduled_entry_point(D, strided, causal, indexed):
+    """psa_fwd_scheduled itself (the operator calls psa_fwd_walk): the bits of psa_fwd / psa_fwd_indexed."""
+    from psa_hip import ops
+    from psa_hip._lib import check, lib
+
+    B, Hq, Hkv, L = 2, 4, 2, 1930
+    q, k, v = _inputs(B, Hq, Hkv, L, seed=9, D=D)
+    if strided:
+        k, v = (x.transpose(1, 2).contiguous().transpose(1, 2) for x in (k, v))
+    Mq, Nk = -(-L // BM), -(-L // BN)
+    lmap = torch.from_numpy(random_map(B, Hq, Mq, Nk, 4, ensure_row=False)).to(torch.int8).to(dev())
+    qi = torch.randperm(L, generator=torch.Generator().manual_seed(L)).to(torch.int32).to(dev()) if indexed else None
+    kp, vp = ops.pool_kv(k, v, BN)
+    sched = ops.build_schedule(lmap, Hkv, L, D, BM, BN, causal)
+    o = torch.full((B, Hq, L, D), float("nan"), dtype=q.dtype, device=q.device)
+    lse = torch.full((B, Hq, L), float("nan"), dtype=torch.float32, device=q.device)
+
+    def call(schedule, bn=BN):
+        check(lib.psa_fwd_scheduled(ops._t4(q), ops._ptr(qi), ops._t4(k), ops._t4(v), ops._ptr(kp), ops._ptr(vp), ops._ptr(lmap), 1, schedule,
+                                    ops._t4(o), ops._ptr(lse), B, Hq, Hkv, L, D, BM, bn, D ** -0.5, int(causal), ops._stream(q)))
+
+    call(sched.data_ptr())
+    ref, rl, _ = ops.sparse_attention_fwd(q, k, v, lmap, BM, BN, causal=causal, return_lse=True, q_index=qi, schedule=False)
+    torch.cuda.synchronize()
+    assert torch.equal(o, ref) and torch.equal(lse.nan_to_num(neginf=-1e30), rl.nan_to_num(neginf=-1e30))
+    # (refused on the host, nothing is launched)
+    for args in ((sched.data_ptr(), 64), (sched.data_ptr(), 32), (None, BN), (sched.data_ptr() + 4, BN)):
+        with pytest.raises(ValueError):
+            call(*args)
