@@ -666,16 +666,16 @@ def _layer_one_call(qb, kb, vb, off_q, off_k, mask_ratios, mode, block_m, block_
             return None
     if sim_thresholds is not None and (Hq != Hkv or qb.dtype not in _T16):
         return None
-    if token_index is not None:
-        if token_index.device != dev:
-            return None
-        token_index = _check_index(token_index, L)
+    if token_index is not None and token_index.device != dev:
+        return None
     items, m, _ = _items(mask_ratios, mode)
     Mq, Nk = -(-L // block_m), -(-L // block_n)
     walk = int(_walk_bytes(qb.dtype, B, Hq, Hkv, L, D, block_m, block_n) > 0)
     n_ws = lib.psa_layer_workspace_bytes(qb.element_size(), B, Hq, Hkv, L, D, block_m, block_n, int(token_index is not None), walk)
     if not 0 < n_ws <= _ONE_CALL_MAX_BYTES:
         return None
+    if token_index is not None:
+        token_index = _check_index(token_index, L)
     lv, hi = _level_items(items)
     ws = torch.empty(n_ws, dtype=torch.uint8, device=dev)
     mp = torch.empty(B, Hq, Mq, Nk, dtype=torch.int8, device=dev)
