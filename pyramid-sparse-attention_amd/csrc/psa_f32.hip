@@ -12,6 +12,8 @@
 // between the two products, and a row maximum is two lane exchanges.  Channels are dealt so that a lane's operands of four
 // steps are 16 consecutive bytes (one ds_read_b128); rows are XOR-swizzled by 16-byte chunks: conflict-free.
 // 2 heads of 4096 tokens x 64, 64-key blocks, 80 % sparse: 109 us on the vector units (two LDS operands per 4 FMAs), 36 us here.
+#include <type_traits>
+
 #include "psa_common.h"
 #include "psa_tiles.h"
 
@@ -88,8 +90,8 @@ __global__ __launch_bounds__(256, 2) void psa_fwd_f32_kernel(F32Params p) {
   // Slots past the last key: K replicates a retained row (their logits are masked), V is zero - a replicated row with an infinite
   // value would turn the infinity that it rightly gives its channel into 0 * inf.
   const uint32_t lds0 = psa_tiles::lds_addr_of(smem);
-  auto issue_tile = [&](int t, int stage) __attribute__((always_inline)) {
-    const psa_tiles::TileRef tr = psa_tiles::tile_ref(tdesc, ids, t, p.bn_log2);
+  auto issue_rows = [&](const psa_tiles::TileRef& tr, int stage, auto full_c) __attribute__((always_inline)) {
+    constexpr bool FULL = decltype(full_c)::value;  // every slot holds a key (a select per copy otherwise)
     const float* kbase = tr.lv == 0 ? kb0 : p.kp + psa_tiles::pool_row_offset(tr.lv, BHkv, bhk, p.npad) * D;
     const float* vbase = tr.lv == 0 ? vb0 : p.vp + psa_tiles::pool_row_offset(tr.lv, BHkv, bhk, p.npad) * D;
     const int64_t kstr = tr.lv == 0 ? p.k_sl : D, vstr = tr.lv == 0 ? p.v_sl : D;
@@ -98,15 +100,22 @@ __global__ __launch_bounds__(256, 2) void psa_fwd_f32_kernel(F32Params p) {
       const int row16 = n * G::RPB + lane / G::CH;
       const int pos = (tr.lt << 6) + wave * 16 + row16;
       int bi = pos >> tr.sbs_log2;
-      bi = bi < tr.cnt - 1 ? bi : tr.cnt - 1;
+      if constexpr (!FULL) bi = bi < tr.cnt - 1 ? bi : tr.cnt - 1;
       int src = ((int)tr.ids[bi] << tr.sbs_log2) + (pos & ((1 << tr.sbs_log2) - 1));
-      if (tr.lv == 0) src = src < p.L ? src : p.L - 1;
+      if constexpr (!FULL)
+        if (tr.lv == 0) src = src < p.L ? src : p.L - 1;
       const int chunk = (lane % G::CH) ^ row16;
       const uint32_t at = lds0 + (uint32_t)(stage * 2 * G::TILE + (wave * 16 + n * G::RPB) * G::ROW);
       psa_tiles::lds_copy16_addr((const char*)(kbase + (int64_t)src * kstr + chunk * 4), at);
-      const float* vsrc = wave * 16 + row16 < tr.nvalid ? vbase + (int64_t)src * vstr + chunk * 4 : f32_zero_chunk;
+      const float* vsrc = vbase + (int64_t)src * vstr + chunk * 4;
+      if constexpr (!FULL) vsrc = wave * 16 + row16 < tr.nvalid ? vsrc : f32_zero_chunk;
       psa_tiles::lds_copy16_addr((const char*)vsrc, at + G::TILE);
     }
+  };
+  auto issue_tile = [&](int t, int stage) __attribute__((always_inline)) {
+    const psa_tiles::TileRef tr = psa_tiles::tile_ref(tdesc, ids, t, p.bn_log2);
+    if (tr.nvalid == TK32) issue_rows(tr, stage, std::true_type{});
+    else issue_rows(tr, stage, std::false_type{});
   };
   // operand addresses: K row l16 of a 16-key block, chunk 4 s + g; V rows 4 g + i, chunk l16 (+ 16 for the upper channels)
   uint32_t k_off[4], v_off[4];
