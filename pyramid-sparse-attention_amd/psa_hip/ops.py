@@ -109,7 +109,9 @@ def pool_kv(k: torch.Tensor, v: torch.Tensor, block_n: int, out: Optional[Tuple[
     return kp, vp
 
 
-_VALID_INDEX: Dict[Tuple[int, int, int, int], bool] = {}
+# (address, version, length, device) -> the checked index itself: held, so that no other tensor can come to lie at that address
+_VALID_INDEX: Dict[Tuple[int, int, int, int], torch.Tensor] = {}
+_VALID_INDEX_MAX = 64
 
 
 def validate_token_index(index: torch.Tensor, L: int) -> None:
@@ -130,20 +132,20 @@ def validate_token_index(index: torch.Tensor, L: int) -> None:
 def _check_index(index: torch.Tensor, L: int) -> torch.Tensor:
     """A token index the kernels can use: int32, one entry per token, a permutation of 0 .. L-1.  A bad entry would make
     a kernel read or write another row (the kernels clamp reads and drop stores outside the tensor, so nothing faults,
-    but rows of the output would stay unwritten): the contents are checked once per index tensor (keyed on its storage
-    and version, so an index built once per model costs one check)."""
+    but rows of the output would stay unwritten): the contents are checked once per index tensor (keyed on its address
+    and version, so an index built once per model costs one check).  The last few checked ones are kept alive."""
     if index.dtype != torch.int32 or index.dim() != 1 or index.numel() != L:
         raise ValueError("index must be a 1-D int32 tensor with one entry per token (%d)" % L)
-    index = index.contiguous()
-    if index.is_inference():  # no version counter to key a cached verdict on: checked on every call
+    if index.is_inference() or not index.is_contiguous():  # no version counter to key a verdict on, or a copy per call: checked every time
+        index = index.contiguous()
         validate_token_index(index, L)
         return index
     key = (index.data_ptr(), index._version, L, index.device.index if index.device.index is not None else -1)
     if key not in _VALID_INDEX:
         validate_token_index(index, L)
-        if len(_VALID_INDEX) > 64:
+        if len(_VALID_INDEX) >= _VALID_INDEX_MAX:
             _VALID_INDEX.clear()
-        _VALID_INDEX[key] = True
+        _VALID_INDEX[key] = index
     return index
 
 

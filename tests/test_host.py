@@ -220,3 +220,33 @@ def test_token_index_validator_rejects_what_is_not_a_permutation():
         ops.validate_token_index(good.to(torch.int64), L)
     with pytest.raises(ValueError):
         ops.validate_token_index(good[:-1], L)
+
+
+def test_token_index_verdict_ends_with_its_index():
+    """The contents of an index are checked once; another index that comes to lie at the address of a freed one is checked again."""
+    import pytest
+    import torch
+
+    from psa_hip import ops
+
+    L = 9 << 20  # (a mapping of its own: the address of a freed one is handed out again)
+    good = torch.arange(L, dtype=torch.int32)
+    assert ops._check_index(good, L) is good
+    del good
+    others = []
+    for _ in range(5):
+        others.append(torch.zeros(L, dtype=torch.int32))
+        with pytest.raises(ValueError):
+            ops._check_index(others[-1], L)
+    L = 1000
+    # an index changed in place, and a strided one (a copy per call)
+    good = torch.arange(L, dtype=torch.int32)
+    ops._check_index(good, L)
+    good[0] = 1
+    with pytest.raises(ValueError):
+        ops._check_index(good, L)
+    twice = torch.arange(L, dtype=torch.int32).repeat_interleave(2)
+    assert torch.equal(ops._check_index(twice[::2], L), twice[::2])
+    with pytest.raises(ValueError):
+        ops._check_index(torch.zeros(2 * L, dtype=torch.int32)[::2], L)
+    assert len(ops._VALID_INDEX) <= ops._VALID_INDEX_MAX
