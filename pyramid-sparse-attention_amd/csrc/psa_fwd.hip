@@ -93,7 +93,7 @@ struct FwdParams {
 //   WALK_REC_ANY  prebuilt records, any block size and row stride
 //   WALK_DENSE    no map: every key at level 0, the records are computed; any row stride (one-row kernel)
 // Measured against WALK_MAP: head dim 64 5 - 7 % of the layer (48 heads of 17776 tokens x 2, 128-key blocks, and of 45106
-// tokens, 32-key blocks); head dim 128, bound by power, 0 - 2 %.
+// tokens, 32-key blocks); head dim 128 0 - 2 %.
 enum { WALK_MAP = 0, WALK_REC = 1, WALK_REC_ANY = 2, WALK_DENSE = 3 };
 
 // The word of tile t of a dense row (the form psa_schedule.h gives the records), for quarter g; scalar arithmetic only.

@@ -124,7 +124,7 @@ __device__ __forceinline__ void row_prefix_sums(double* wide, const float* sw, f
 // 0.25: 21 / 26 / 34 / 41, bitonic network 65 to 71 whatever the scores; 3072 rows of 512: 17 / 18 / 20 / 28 against 34; of
 // 2048: 31 / 46 / 58 / 60 against 200.  (Building the cut key bit by bit over the whole row instead of descending: 21 / 58 / 138 /
 // 266 at 1024 scores.)  With the reduction of the estimator's workspace, which the launch also does and which bounds it: 16944
-// rows of 1410 scores 1480 -> 585 us (3.05 GB read, 5.2 TB/s).  Below RANK_SORT_MAX ranking by counting is as fast and also
+// rows of 1410 scores 1480 -> 600 us (3.05 GB read, 5.1 TB/s).  Below RANK_SORT_MAX ranking by counting is as fast and also
 // serves the other modes.
 // LDS: (SEL_BINS + 2 * SEL_MAX_CUTS * SEL_CAP + 8 * SEL_MAX_CUTS) 4-byte words.  256 threads.
 constexpr int SEL_BINS = 1024, SEL_SHIFT = 19, SEL_CAP = 64, SEL_MAX_CUTS = 8;

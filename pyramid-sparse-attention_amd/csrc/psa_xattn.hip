@@ -186,7 +186,7 @@ __global__ __launch_bounds__(X::WAVES * 64, X::WAVES == 8 ? 1 : 2) void psa_xatt
   if (edge) contract(std::true_type{});
   else contract(std::false_type{});
 
-  // epilogue: accumulator (a, c): rows n = n0 + wn*128 + a*32 + (i/4)*8 + hh*4 + i%4, column m = m0 + wm*64 + c*32 + l32
+  // epilogue: accumulator (a, c): rows n = n0 + wn * TN / 2 + a*32 + (i/4)*8 + hh*4 + i%4, column m = m0 + wm*64 + c*32 + l32
   constexpr int OPB = 1 << (RBL - 3);  // 8-key octets per block: 1, 2 or 4
   float* ws = p.ws + (int64_t)bh * p.NB * p.Mr * 2;
 #pragma unroll

@@ -532,7 +532,7 @@ def build_schedule(level_map_: torch.Tensor, Hkv: int, L: int, D: int, block_m: 
 # Rows of the map above which a map of 64- / 32-key blocks is listed before it is walked.  The listing takes two launches
 # (about 5 us); the walk saves the look-ups, which bound the kernel at head dim 64.  Both sides in us, listed against in-kernel:
 # 520 rows head dim 64 51.4 / 48.6, 2080 rows 121.6 / 123.3; 16944 rows (45106 tokens, 48 heads) 4.5 ms / 4.9 ms.
-# At head dim 128, which is bound by power, 568 rows 94.1 / 95.9, 2080 rows 233 / 231 (in the layer 377 / 385).
+# At head dim 128 568 rows 94.1 / 95.9, 2080 rows 233 / 231 (in the layer 377 / 385).
 _WALK_MIN_ROWS = 1024
 # Bytes of a list above which such a map is walked in the kernel: the list has room for the longest possible walk, 10 to 20 times the
 # int8 map (290 MB for 48 heads x 45106 tokens of 32-key blocks; 40 heads x 262144 tokens of 64-key blocks would take 6.7 GB), and
