@@ -264,3 +264,28 @@ def test_fwd_reference_is_raised(D, bn, how, dtype, shape):
     assert mx <= MAX_ABS and mean <= MEAN_ABS, (mx, mean)
     # (logits of up to 500 in fp32 sums of 16-bit products: 1e-4 relative)
     assert float((res[1].cpu().double() - ref_lse).abs().max()) <= 2e-2 + 1e-4 * 500
+
+
+@pytest.mark.parametrize("D,bn,how", [(64, 128, "records"), (64, 64, "map"), (64, 128, "dense"), (128, 128, "records"), (128, 32, "records"),
+                                      (128, 64, "map64"), (128, 128, "dense")])
+@pytest.mark.parametrize("return_lse", [True, False])
+def test_fwd_range_of_v(D, bn, how, return_lse):
+    # Logits that rise by up to 50 (log2 units) behind the first tile, V of 2^100: what is accumulated is V weighted by at most 2^8 over
+    # 700 keys, 2^118 at most.  A power of two changes no rounding, so the bound is that of the other forward tests.
+    from psa_hip import ops
+
+    L = 700
+    bm = 64 if how == "map64" else 128
+    q, k, v = (rnd(1, 2, L, D, seed=41 + i) for i in range(3))
+    q[..., 0] = 1.0
+    k[..., 0] = ((torch.arange(L) // 64 % 5) * (12.5 * D ** 0.5 / 1.4427)).to(k.dtype)
+    Mq, Nk = -(-L // bm), -(-L // bn)
+    lmap = None if how == "dense" else random_map(1, 2, Mq, Nk, seed=6, p=(0.1, 0.5, 0.2, 0.1, 0.1))
+    m_dev = None if lmap is None else torch.from_numpy(lmap).to(dev())
+    big = torch.tensor(2.0 ** 100, dtype=v.dtype)
+    res = ops.sparse_attention_fwd(q.to(dev()), k.to(dev()), (v * big).to(dev()), m_dev, bm, bn, return_lse=return_lse,
+                                   schedule=None if how == "records" else False)
+    out = (res[0] if return_lse else res) / big.to(dev())
+    ref, _ = O.psa_attention_dense(q, k, v, np.ones((1, 2, Mq, Nk), np.int32) if lmap is None else lmap, bm, bn)
+    mx, mean = attn_errors(out, ref)
+    assert mx <= MAX_ABS and mean <= MEAN_ABS, (mx, mean)
