@@ -289,3 +289,29 @@ def test_fwd_range_of_v(D, bn, how, return_lse):
     ref, _ = O.psa_attention_dense(q, k, v, np.ones((1, 2, Mq, Nk), np.int32) if lmap is None else lmap, bm, bn)
     mx, mean = attn_errors(out, ref)
     assert mx <= MAX_ABS and mean <= MEAN_ABS, (mx, mean)
+
+
+@pytest.mark.parametrize("D,bm,bn,how", [(64, 128, 128, "records"), (64, 128, 32, "records"), (64, 128, 64, "map"), (64, 64, 64, "map"), (64, 128, 128, "dense"),
+                                         (128, 128, 128, "records"), (128, 128, 32, "records"), (128, 128, 128, "map"), (128, 64, 64, "map"), (128, 128, 128, "dense")])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("causal", [False, True])
+def test_fwd_lse_of_unrounded_probabilities(D, bm, bn, how, dtype, causal):
+    # The log-sum-exp is taken from fp32 probabilities.  Logits: sums of D products whose magnitudes add up to less than 30 (times
+    # the scale), in fp32: 30 * 2^-24 * sqrt(D) = 2e-5; the other terms (exponentials and the logarithm to 1 ulp, 1000 additions of
+    # positive numbers) stay below 1e-5.  Sums of the rounded probabilities are off by 2^-9 / sqrt(keys that carry the sum): 5e-4 rms.
+    from psa_hip import ops
+
+    if causal and bm != bn:
+        pytest.skip("causal maps are square in the reference")
+    L = 900
+    q, k, v = (rnd(1, 2, L, D, seed=51 + i, dtype=dtype, scale=s) for i, s in enumerate((3.0, 1.0, 1.0)))
+    Mq, Nk = -(-L // bm), -(-L // bn)
+    lmap = None if how == "dense" else random_map(1, 2, Mq, Nk, seed=7, p=(0.2, 0.5, 0.1, 0.1, 0.1))
+    m_dev = None if lmap is None else torch.from_numpy(lmap).to(dev())
+    lse = ops.sparse_attention_fwd(q.to(dev()), k.to(dev()), v.to(dev()), m_dev, bm, bn, causal=causal, return_lse=True,
+                                   schedule=None if how == "records" else False)[1].cpu().double()
+    _, ref = O.psa_attention_dense(q, k, v, np.ones((1, 2, Mq, Nk), np.int32) if lmap is None else lmap, bm, bn, causal=causal)
+    fin = torch.isfinite(ref)
+    assert torch.equal(torch.isfinite(lse), fin)
+    d = (lse[fin] - ref[fin]).abs()
+    assert float(d.max()) <= 3e-5, float(d.max())
