@@ -40,7 +40,7 @@ def _kernels(tmp_path):
 
 
 @pytest.mark.skipif(READELF is None, reason="llvm-readelf of the ROCm toolchain not found")
-@pytest.mark.parametrize("kernel,instances", [("psa_fwd_kernel", 20)])
+@pytest.mark.parametrize("kernel,instances", [("psa_fwd_kernel", 20), ("psa_fwd_lds_kernel", 20)])
 def test_forward_kernels_do_not_spill(kernel, instances, tmp_path):
     found = {n: m for n, m in _kernels(tmp_path).items() if re.search(r"\d%sI" % kernel, n)}
     assert len(found) == instances, sorted(found)
