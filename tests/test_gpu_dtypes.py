@@ -67,9 +67,9 @@ def test_estimator_in_the_input_type(dtype, B, Hq, Hkv, L, D, bm, bn):
 @pytest.mark.parametrize(
     "B,Hq,Hkv,L,D,bm,bn,causal",
     [
-        (1, 2, 2, 128 * 9 + 40, 128, 128, 128, False),   # fp16: the two-group kernel on a prebuilt schedule, ragged end
+        (1, 2, 2, 128 * 9 + 40, 128, 128, 128, False),   # fp16: a prebuilt schedule, ragged end
         (1, 4, 2, 128 * 6, 128, 128, 128, True),          # causal, grouped heads
-        (2, 2, 1, 700, 64, 128, 128, False),              # head dim 64: the one-row kernel
+        (2, 2, 1, 700, 64, 128, 128, False),              # head dim 64
         (1, 2, 2, 1000, 64, 64, 64, True),                # blocks of 64
         (1, 1, 1, 900, 128, 64, 128, False),              # block_m != block_n
     ],

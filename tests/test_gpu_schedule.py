@@ -32,7 +32,7 @@ def _inputs(B, Hq, Hkv, L, seed, D=D):
         (1, 1, 1, 4100, False, False, (0.9, 0.025, 0.025, 0.025, 0.025)),  # rows with very few tiles, empty rows
     ],
 )
-@pytest.mark.parametrize("D", [128, 64])  # the two-group kernel / the one-row kernel
+@pytest.mark.parametrize("D", [128, 64])
 def test_scheduled_walk_equals_map_walk(B, Hq, Hkv, L, causal, indexed, p, D):
     from psa_hip import ops
 
@@ -97,9 +97,8 @@ def test_strided_rows_walk_the_same_schedule():
 
 @pytest.mark.parametrize("D", [64, 128])
 def test_strided_rows_fall_back_to_the_map_walk(D):
-    """K / V rows 16 MiB apart, further than the record walk's 24-bit row strides reach: the map walk in the schedule's order.  Head
-    dim 64 is the same kernel, hence the same bits; head dim 128 goes from the two-group kernel to the one-row one, which rounds
-    its probabilities against another running maximum."""
+    """K / V rows 16 MiB apart, further than the record walk's 24-bit row strides reach: the map walk in the schedule's order, the
+    same arithmetic and so the same bits."""
     from psa_hip import ops
 
     H, L, step = 2, 126, 1 << 23
@@ -116,8 +115,7 @@ def test_strided_rows_fall_back_to_the_map_walk(D):
         b = ops.sparse_attention_fwd(q, kf, vf, lmap, BM, BN, pools=pools, schedule=sched)
         torch.cuda.synchronize()
         assert kf.stride(2) * 2 >= 1 << 24
-        mx, mean = attn_errors(b, a.cpu())
-        assert torch.equal(a, b) if D == 64 else mx <= MAX_ABS and mean <= MEAN_ABS, (mx, mean)
+        assert torch.equal(a, b)
 
 
 @pytest.mark.parametrize("H,Hkv,L", [(3, 3, 128 * 40), (40, 1, 128 * 128), (64, 1, 128 * 300 + 5), (160, 1, 128 * 300)])
