@@ -53,16 +53,16 @@ WORKLOADS.update({
 WAN13 = {1: (0.0, 0.5), 2: (0.5, 0.6), 4: (0.6, 0.7), 8: (0.7, 0.8), 0: (0.8, 1.0)}
 
 
-def fwd_traffic_bytes(workload):
-    """HBM-side bytes per launch of the forward kernel from the committed rocprofv3 counter summaries
-    (profiles/*.txt, line `roofline.traffic <workload> <kernel> <bytes>`), or None."""
+def fwd_traffic_bytes(workload, kernel):
+    """HBM-side bytes per launch of a forward kernel from the committed rocprofv3 counter summaries
+    (profiles/*.txt, line `roofline.traffic <workload> <kernel> <bytes>`), or None where they hold none of that kernel."""
     import glob
 
     for path in sorted(glob.glob(os.path.join(ROOT, "profiles", "*.txt"))):
         try:
             for line in open(path):
                 f = line.split()
-                if len(f) >= 4 and f[0] == "roofline.traffic" and f[1] == workload:
+                if len(f) >= 4 and f[:3] == ["roofline.traffic", workload, kernel]:
                     return float(f[3])
         except OSError:
             pass
@@ -280,6 +280,7 @@ def run_other(args, w, torch, ops, make_qkv, sample_offsets, dev):
     stages["step"] = round(ms_step, 4)
     if args.copy_calib:
         copy_calib(torch, dev)
+    fwd_kernel = "psa_fwd_kernel" if D == 128 else "psa_fwd_lds_kernel"
     return {
         "metric": METRIC, "value": round(dense_flops / (ms_step * 1e-3) / 1e12, 2),
         "unit": "effective TFLOP/s (dense-equivalent flops of the step / step time)",
@@ -290,9 +291,10 @@ def run_other(args, w, torch, ops, make_qkv, sample_offsets, dev):
         "config": {"workload": w["name"], "L": L, "block_m": bm, "block_n": bn, "density": round(density, 4),
                    "sparsity": round(1 - density, 4)},
         "stages_ms": stages,
-        "roofline": {"kernel": "psa_fwd_kernel" if D == 128 else "psa_fwd_lds_kernel", "bound": "mfma",
+        "roofline": {"kernel": fwd_kernel, "bound": "mfma",
                      "achieved": round(fwd_flops / (t_fwd_avg * 1e-3) / 1e12, 2), "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
-                     "frac": round(fwd_flops / (t_fwd_avg * 1e-3) / 1e12 / PEAK_BF16_TFLOPS, 4), "traffic": fwd_traffic_bytes(args.workload),
+                     "frac": round(fwd_flops / (t_fwd_avg * 1e-3) / 1e12 / PEAK_BF16_TFLOPS, 4),
+                     "traffic": fwd_traffic_bytes(args.workload, fwd_kernel),
                      "flops_per_launch": fwd_flops, "avg_launch_ms": round(t_fwd_avg, 4)},
         "cpu_baseline": cpu,
     }
@@ -489,17 +491,17 @@ def main():
     pool_bytes = 2.0 * B * H * (Nk * bn) * D * q.element_size() * (1 + 7 / 8)
     est_flops = 2.0 * (Mq * km) * (Nk * kn) * D * B * H
 
+    fwd_kernel = "psa_fwd_f32_kernel" if tdtype == torch.float32 else "psa_fwd_kernel" if D == 128 else "psa_fwd_lds_kernel"
     roofline = {
-        "kernel": ("psa_fwd_f32_kernel" if tdtype == torch.float32 else
-                   "psa_fwd_kernel" if D == 128 else "psa_fwd_lds_kernel"),
-        "bound": "mfma",  # (the fp32 kernel computes on the vector units; its peak is the fp32 figure)
+        "kernel": fwd_kernel,
+        "bound": "mfma",  # (fp32: the matrix cores' fp32 instructions and their peak)
         "achieved": round(exec_flops / (t_fwd_avg * 1e-3) / 1e12, 2),
         "peak": peak,
         "unit": "TFLOP/s",
         "frac": round(exec_flops / (t_fwd_avg * 1e-3) / 1e12 / peak, 4),
         # HBM-side bytes per launch from rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE runs of this command (scaled by the
-        # readings of --copy-calib's 1 GiB kernel); measured for the default workload only
-        "traffic": fwd_traffic_bytes(args.workload),
+        # readings of --copy-calib's 1 GiB kernel), where they were measured on this kernel
+        "traffic": fwd_traffic_bytes(args.workload, fwd_kernel),
         "flops_per_launch": exec_flops,
         "avg_launch_ms": round(t_fwd_avg, 4),
         # context, not the fraction that counts: the shader clock under this kernel (the board's power limit holds it under

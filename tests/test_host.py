@@ -250,3 +250,15 @@ def test_token_index_verdict_ends_with_its_index():
     with pytest.raises(ValueError):
         ops._check_index(torch.zeros(2 * L, dtype=torch.int32)[::2], L)
     assert len(ops._VALID_INDEX) <= ops._VALID_INDEX_MAX
+
+
+def test_bench_traffic_is_the_timed_kernels(tmp_path, monkeypatch):
+    """roofline.traffic comes from a counter line of the kernel that is timed; a line of another kernel is no substitute."""
+    import bench
+
+    (tmp_path / "profiles").mkdir()
+    (tmp_path / "profiles" / "a.txt").write_text("roofline.traffic c2 psa_old_kernel 1.0e+09\nroofline.traffic c3 psa_fwd_kernel 2.0e+09\n"
+                                                 "roofline.traffic c2 psa_fwd_kernel 3.0e+09\n")
+    monkeypatch.setattr(bench, "ROOT", str(tmp_path))
+    assert bench.fwd_traffic_bytes("c2", "psa_fwd_kernel") == 3.0e9
+    assert bench.fwd_traffic_bytes("c2", "psa_fwd_lds_kernel") is None
