@@ -305,16 +305,38 @@ struct TileSrc {
   int src0[G16];  // first of the lane's consecutive source rows, per group
 };
 
+// The wave's rows of a tile with descriptor (d0, d1): block id of the first of the lane's consecutive rows, per group, and, from
+// it, that row
+template <int D, int G16>
+__device__ __forceinline__ void lt_tile_ids(int bn_log2, uint32_t d0, uint32_t d1, const uint16_t* ids, int wave, int lane, int (&id)[G16]) {
+  const int nvalid = (d0 >> 3) & 127, cnt = d1 >> 16, sbs_log2 = bn_log2 - (int)(d0 & 3);
+  const uint16_t* lids = ids + (d1 & 0xffff);
+#pragma unroll
+  for (int gi = 0; gi < G16; ++gi) {
+    int bi = ((int)(d0 >> 10) * TK + (wave * G16 + gi) * 16 + lt_fetch_row<D>(lane)) >> sbs_log2;
+    if (nvalid < TK) bi = bi < cnt - 1 ? bi : cnt - 1;  // some slots are empty: clamp them onto real rows (their logits are masked)
+    id[gi] = lids[bi];
+  }
+}
+template <int D, int G16>
+__device__ __forceinline__ void lt_tile_rows(int bn_log2, uint32_t d0, const int (&id)[G16], int wave, int lane, int (&src0)[G16]) {
+  const int sbs_log2 = bn_log2 - (int)(d0 & 3);
+#pragma unroll
+  for (int gi = 0; gi < G16; ++gi) {
+    const int g = (int)(d0 >> 10) * TK + (wave * G16 + gi) * 16 + lt_fetch_row<D>(lane);
+    src0[gi] = (id[gi] << sbs_log2) + (g & ((1 << sbs_log2) - 1));
+  }
+}
+// last valid row when the tile may run past the sequence end, else INT_MAX
+__device__ __forceinline__ int lt_tile_lim(uint32_t d0, int L) { return ((d0 >> 3) & 127) < TK && (d0 & 3) == 0 ? L - 1 : 0x7fffffff; }
+
 template <int D, int G16>
 __device__ __forceinline__ void lt_tile_src(const KvSource& kv, const u32x2* tdesc, const uint16_t* ids, int t, int wave, int lane,
                                             TileSrc<G16>& a) {
   const u32x2 dd = tdesc[t];
   const uint32_t d0 = __builtin_amdgcn_readfirstlane(dd[0]);
   const uint32_t d1 = __builtin_amdgcn_readfirstlane(dd[1]);
-  const int lv = d0 & 3, nvalid = (d0 >> 3) & 127, lt = d0 >> 10;
-  const int cnt = d1 >> 16;
-  const uint16_t* lids = ids + (d1 & 0xffff);
-  const int sbs_log2 = kv.bn_log2 - lv;
+  const int lv = d0 & 3;
   // max(lv - 1, 0) from a table in a constant: a saturating subtraction would be a vector instruction and drag the
   // 64-bit offset arithmetic below (and the copy base pointers) from the scalar to the vector unit
   const int lm1 = (0x2100 >> (4 * lv)) & 3;
@@ -323,15 +345,10 @@ __device__ __forceinline__ void lt_tile_src(const KvSource& kv, const u32x2* tde
   a.vbase = lv == 0 ? kv.v0 : kv.vp + pool_off;
   a.kstr = lv == 0 ? kv.k_strb : (uint32_t)(D * 2);
   a.vstr = lv == 0 ? kv.v_strb : (uint32_t)(D * 2);
-  const bool ragged = nvalid < TK;  // some slots are empty: clamp them onto real rows (their logits are masked)
-  a.lim = (ragged && lv == 0) ? kv.L - 1 : 0x7fffffff;
-#pragma unroll
-  for (int gi = 0; gi < G16; ++gi) {
-    const int g = (lt << 6) + (wave * G16 + gi) * 16 + lt_fetch_row<D>(lane);
-    int bi = g >> sbs_log2;
-    if (ragged) bi = bi < cnt - 1 ? bi : cnt - 1;
-    a.src0[gi] = ((int)lids[bi] << sbs_log2) + (g & ((1 << sbs_log2) - 1));
-  }
+  a.lim = lt_tile_lim(d0, kv.L);
+  int id[G16];
+  lt_tile_ids<D, G16>(kv.bn_log2, d0, d1, ids, wave, lane, id);
+  lt_tile_rows<D, G16>(kv.bn_log2, d0, id, wave, lane, a.src0);
 }
 
 // One global -> LDS copy instruction: lane l's 16 bytes at sbase + voff(l) land at LDS address lds_addr + 16 * l.

@@ -1,5 +1,6 @@
 """The forward kernels keep their state in registers: a spilled one comes back through a wait for the vector-memory counter, which
-also waits for the tile copies in flight.  The compiler notes the spills of every kernel in the code object of the library."""
+also waits for the tile copies in flight, and a spilled scalar takes two instructions of the loop.  The compiler notes the spills of
+every kernel in the code object of the library."""
 import os
 import re
 import shutil
@@ -33,7 +34,7 @@ def _kernels(tmp_path):
                 notes = subprocess.run([READELF, "--notes", str(path)], check=True, capture_output=True, text=True).stdout
                 for block in re.split(r"\n\s+- \.a(?:gpr_count|rgs):", notes)[1:]:
                     # (the kernel's own name is the last one, behind those of its arguments)
-                    meta = dict(re.findall(r"\.(name|vgpr_spill_count|private_segment_fixed_size):\s+(\S+)\s*$", block, re.M))
+                    meta = dict(re.findall(r"\.(name|[sv]gpr_spill_count|private_segment_fixed_size):\s+(\S+)\s*$", block, re.M))
                     res[meta["name"]] = meta
         at = blob.find(magic, at + 1)
     return res
@@ -44,5 +45,5 @@ def _kernels(tmp_path):
 def test_forward_kernels_do_not_spill(kernel, instances, tmp_path):
     found = {n: m for n, m in _kernels(tmp_path).items() if re.search(r"\d%sI" % kernel, n)}
     assert len(found) == instances, sorted(found)
-    spilled = {n: m for n, m in found.items() if int(m["vgpr_spill_count"]) or int(m["private_segment_fixed_size"])}
+    spilled = {n: m for n, m in found.items() if any(int(m[c]) for c in ("vgpr_spill_count", "sgpr_spill_count", "private_segment_fixed_size"))}
     assert not spilled, spilled
