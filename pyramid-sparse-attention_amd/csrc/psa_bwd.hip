@@ -478,8 +478,8 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
   const int nq = s_nq;
 
   // ---- lane-invariant LDS addressing (tile layout: see the forward kernel) ---------------------------
-  // copy: wave w fills the 16-row group w of both tiles; lane (fq = lane/16, pos = lane%16) of block n writes
-  // row fq of that block, i.e. tile row 16w + 4fq + n, chunk pos ^ fq
+  // copy: wave w fills the 16-row group w of both tiles; lane (fq = lane / CH, pos = lane % CH) of block n writes
+  // row fq of that block, i.e. tile row 16w + RPL * fq + n, chunk pos ^ lt_key(fq)
   // (recomputed from the lane id at every use - see issue_step - instead of living in registers across the matrix work:
   // this kernel has no register to spare, and a spilled value comes back through a vmcnt wait that would also wait
   // for the tile copies in flight)

@@ -81,8 +81,6 @@ __device__ __forceinline__ int rec_src(uint32_t w) { return (int)(w & REC_SRC_MA
 }  // namespace psa_sched
 
 // host side (psa_schedule.hip)
-// dealing of the rows of the forward walk to the XCDs
-void psa_fwd_deal(int B, int Hq, int Hkv, int L, int D, int block_m, int block_n, bool has_map, int& chunk, int& groups);
 // shapes for which schedules exist (psa_schedule_*: 128-key blocks; psa_walk_*: every block_n)
 bool psa_schedule_shape_ok(int D, int block_m, int block_n, int L);
 bool psa_walk_shape_ok(int D, int block_m, int block_n, int L);

@@ -133,15 +133,6 @@ __global__ __launch_bounds__(64 * ROWS_PER_WG) void psa_sched_build_kernel(const
 
 }  // namespace
 
-// dealing of the rows of the forward walk: shared by psa_build_schedule and the forward launch
-void psa_fwd_deal(int B, int Hq, int Hkv, int L, int D, int block_m, int block_n, bool has_map, int& chunk, int& groups) {
-  const int Mq = (L + block_m - 1) / block_m, Nk = (L + block_n - 1) / block_n;
-  const int64_t total = (int64_t)B * Hq * Mq;
-  const double kv_bytes = 2.0 * B * Hkv * ((double)Nk * block_n) * D * 2.0 * (has_map ? 1.875 : 1.0);
-  psa_order::deal(total, kv_bytes, B * Hkv, chunk, groups);
-  chunk = (chunk + 1) & ~1;  // (shares of even length: the layout that schedule buffers are sized for)
-}
-
 // schedules of the public psa_schedule_* entry points
 bool psa_schedule_shape_ok(int D, int block_m, int block_n, int L) {
   return (D == 128 || D == 64) && block_m == 128 && block_n == 128 && (int64_t)((L + 127) / 128) * 128 <= (1 << psa_sched::REC_SRC_BITS);
@@ -159,7 +150,11 @@ bool psa_schedule_geometry(int B, int Hq, int Hkv, int L, int D, int block_m, in
   g.Nk = (L + block_n - 1) / block_n;
   g.rows = (int64_t)B * Hq * g.Mq;
   if (g.rows >= (1ll << 28)) return false;
-  psa_fwd_deal(B, Hq, Hkv, L, D, block_m, block_n, true, g.wg_chunk, g.wg_groups);
+  // dealing of the rows to the XCDs, by the bytes of K, V and their pooled levels
+  const double kv_bytes = 2.0 * B * Hkv * ((double)g.Nk * block_n) * D * 2.0 * 1.875;
+  psa_order::deal(g.rows, kv_bytes, B * Hkv, g.wg_chunk, g.wg_groups);
+  // Shares of even length: no walk needs them, but a caller may keep a schedule, and its layout follows from the share size.
+  g.wg_chunk = (g.wg_chunk + 1) & ~1;
   g.lay = psa_sched::layout(g.rows, g.Nk, block_n, (int64_t)g.wg_chunk * g.wg_groups);
   return true;
 }

@@ -180,9 +180,9 @@ __device__ __forceinline__ int64_t pool_row_offset(int lv, int64_t BHkv, int64_t
 //   * One copy instruction moves 1024 bytes (64 lanes x 16 bytes land at consecutive LDS addresses), i.e. a
 //     BLOCK of RPB = 512 / D rows (4 rows of 256 bytes for D = 128, 8 rows of 128 bytes for D = 64); the blocks
 //     of a tile are LT_ISTR = 1024 + 64 bytes apart.
-//   * Row r of a block stores its 16-byte chunks XOR-swizzled: chunk c sits at position c ^ (r * RPB / 16)...
-//     in short c ^ r for D = 128 and c ^ (r >> 1) for D = 64 (applied on the global side: a lane fetches the
-//     chunk that belongs at its LDS position).
+//   * Row r of a block stores its 16-byte chunks XOR-swizzled: chunk c sits at position c ^ lt_key(r), the key being
+//     0, 3, 2, 1 for r = 0 .. 3 (D = 128) or r >> 1 = 0 .. 3 (D = 64); applied on the global side: a lane fetches the
+//     chunk that belongs at its LDS position.
 //   * Inside each group of 16 tile rows the rows are stored transposed (block n, row r holds tile row
 //     RPL * r + n, RPL = 16 / RPB blocks per group), so the RPL rows a lane fetches are CONSECUTIVE tile rows.
 // Padding and swizzle make the 128-bit row reads and the transposing reads bank-conflict free, and both only
@@ -196,7 +196,7 @@ struct LtGeom {
   static constexpr int RPL = 16 / RPB;      // blocks per 16-row group = consecutive tile rows per lane
   static constexpr int BLOCKS = 64 / RPB;   // blocks per tile
   static constexpr int TILE = BLOCKS * LT_ISTR;
-  static constexpr int SW_SHIFT = RPB == 4 ? 0 : 1;  // swizzle key of block row r: r >> SW_SHIFT (0..3)
+  static constexpr int SW_SHIFT = RPB == 4 ? 0 : 1;  // block rows r with one r >> SW_SHIFT share a swizzle key (lt_key)
   static constexpr int HALF = (32 / RPB) * LT_ISTR;  // byte distance of tile rows r and r + 32
   static constexpr int GROUP = RPL * LT_ISTR;        // byte distance of consecutive 16-row groups
 };
@@ -398,21 +398,6 @@ __device__ __forceinline__ void lds_copy16_imm(const char* sbase, uint32_t voff,
                :
                : "v"(voff), "s"(lds_base), "s"(sbase), "n"(OFF - IMM), "n"(IMM)
                : "memory", "scc", "m0");
-}
-// the same with a multiply-add a * b + c (a uniform) in the wait state between the write of M0 and the copy, where the
-// hardware needs an instruction anyway: the caller passes one that it has to execute in any case
-template <int OFF, int IMM>
-__device__ __forceinline__ float lds_copy16_imm_fma(const char* sbase, uint32_t voff, uint32_t lds_base, float a, float b, float c) {
-  static_assert(IMM >= 0 && IMM < 4096 && OFF >= IMM, "immediate offset range");
-  sbase = uniform_ptr(sbase);
-  lds_base = __builtin_amdgcn_readfirstlane(lds_base);
-  a = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(uint32_t, a)));
-  float r;
-  asm volatile("s_add_u32 m0, %2, %4\n\tv_fma_f32 %0, %6, %7, %8\n\tglobal_load_lds_dwordx4 %1, %3 offset:%5"
-               : "=&v"(r)
-               : "v"(voff), "s"(lds_base), "s"(sbase), "n"(OFF - IMM), "n"(IMM), "s"(a), "v"(b), "v"(c)
-               : "memory", "scc", "m0");
-  return r;
 }
 // the same with a full per-lane address
 __device__ __forceinline__ void lds_copy16_addr(const char* vaddr, uint32_t lds_addr) {

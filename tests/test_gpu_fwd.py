@@ -125,10 +125,10 @@ def test_fwd_dense_equals_sdpa_and_all_ones_map():
     assert mx <= MAX_ABS and mean <= MEAN_ABS
 
 
-def test_fwd_long_sequence_takes_the_one_row_kernel():
-    # with 128-key blocks the schedules of two rows stop fitting into LDS above ~85k tokens: the launch falls back
-    # to one row per workgroup.  Dense attention on 88k tokens against torch SDPA on the GPU (bf16), plus a sparse
-    # map through the size-independent property that rows whose blocks are all level 1 equal the dense rows.
+def test_fwd_long_sequence():
+    # Dense attention on 88k tokens against torch SDPA on the GPU (bf16), plus a sparse map through the size-independent
+    # property that rows whose blocks are all level 1 equal the dense rows.  Walked in the kernel, the map row's lists take
+    # the workgroup past half of the LDS (above ~71k tokens of 128-key blocks): one workgroup per CU, the same bits.
     from psa_hip import ops
 
     B, H, L, D = 1, 1, 88000, 128
@@ -145,6 +145,7 @@ def test_fwd_long_sequence_takes_the_one_row_kernel():
     rows = torch.arange(L, device=dev()) // 128 % 7 == 0
     assert float((o2[..., rows, :].float() - ref[..., rows, :]).abs().max()) <= MAX_ABS
     assert torch.isfinite(o2.float()).all()
+    assert torch.equal(ops.sparse_attention_fwd(q, k, v, mp, 128, 128, schedule=False), o2)
 
 
 def test_fwd_lossless_pooling_invariant_full_size_heads():
