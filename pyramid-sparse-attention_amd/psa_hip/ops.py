@@ -530,9 +530,10 @@ def build_schedule(level_map_: torch.Tensor, Hkv: int, L: int, D: int, block_m: 
 
 
 # Rows of the map above which a map of 64- / 32-key blocks is listed before it is walked.  The listing takes two launches
-# (about 5 us); the walk saves the look-ups, which bound the kernel at head dim 64.  Both sides in us, listed against in-kernel:
-# 520 rows head dim 64 51.4 / 48.6, 2080 rows 121.6 / 123.3; 16944 rows (45106 tokens, 48 heads) 4.5 ms / 4.9 ms.
-# At head dim 128 568 rows 94.1 / 95.9, 2080 rows 233 / 231 (in the layer 377 / 385).
+# (about 5 us); the walk saves the look-ups, which bound the kernel at head dim 64.  Both sides in us, listed against in-kernel, on random
+# maps of 32-key blocks: head dim 64 128 rows 23.6 / 16.9, 520 rows 52.6 / 53.8, 1040 rows 82.8 / 83.0, 3072 rows 596 / 639; head dim 128
+# 128 rows 29.4 / 22.6, 520 rows 89.6 / 87.9, 1040 rows 137.6 / 137.1, 3072 rows 1121 / 1105 (there the in-kernel walk is level or
+# ahead by up to 2 % at every count; the order of issue is sorted either way).
 _WALK_MIN_ROWS = 1024
 # Bytes of a list above which such a map is walked in the kernel: the list has room for the longest possible walk, 10 to 20 times the
 # int8 map (290 MB for 48 heads x 45106 tokens of 32-key blocks; 40 heads x 262144 tokens of 64-key blocks would take 6.7 GB), and
