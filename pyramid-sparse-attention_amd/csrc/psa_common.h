@@ -19,6 +19,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef short short4v __attribute__((ext_vector_type(4)));
 typedef _Float16 f16_t;
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
@@ -91,10 +92,11 @@ struct EtBf16 {
   static __device__ __forceinline__ u32x2 read_tr(PSA_LDS_PTR(unsigned char) a) {
     return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4bf16((PSA_LDS_PTR(bf16x4))a));
   }
-  // acc + lo + hi of a packed pair (the rounded values)
-  static __device__ __forceinline__ float add_pair(uint32_t packed, float acc) {
-    const bf16x2 ones = {(bf16_t)1.0f, (bf16_t)1.0f};
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, packed), ones, acc, false);
+  // c + the lane's four values of two packed pairs, in all of c's registers: a 4 x 4 x 4 product with ones, whose B operand is one
+  // column per lane
+  static __device__ __forceinline__ f32x4 add_quad(uint32_t p01, uint32_t p23, f32x4 c) {
+    const short4v ones = {0x3f80, 0x3f80, 0x3f80, 0x3f80};
+    return __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(ones, __builtin_bit_cast(short4v, u32x2{p01, p23}), c, 0, 0, 0);
   }
 };
 struct EtF16 {
@@ -111,9 +113,9 @@ struct EtF16 {
   static __device__ __forceinline__ u32x2 read_tr(PSA_LDS_PTR(unsigned char) a) {
     return EtBf16::read_tr(a);  // (the transposing read moves 16-bit words whatever they hold)
   }
-  static __device__ __forceinline__ float add_pair(uint32_t packed, float acc) {
-    const f16x2 ones = {(f16_t)1.0f, (f16_t)1.0f};
-    return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, packed), ones, acc, false);
+  static __device__ __forceinline__ f32x4 add_quad(uint32_t p01, uint32_t p23, f32x4 c) {
+    const f16x4 ones = {(f16_t)1.0f, (f16_t)1.0f, (f16_t)1.0f, (f16_t)1.0f};
+    return __builtin_amdgcn_mfma_f32_4x4x4f16(ones, __builtin_bit_cast(f16x4, u32x2{p01, p23}), c, 0, 0, 0);
   }
 };
 // calls f(trait) for a 16-bit dtype id; false for any other id
