@@ -94,9 +94,16 @@ struct EtBf16 {
   }
   // c + the lane's four values of two packed pairs, in all of c's registers: a 4 x 4 x 4 product with ones, whose B operand is one
   // column per lane
-  static __device__ __forceinline__ f32x4 add_quad(uint32_t p01, uint32_t p23, f32x4 c) {
-    const short4v ones = {0x3f80, 0x3f80, 0x3f80, 0x3f80};
-    return __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(ones, __builtin_bit_cast(short4v, u32x2{p01, p23}), c, 0, 0, 0);
+  static __device__ __forceinline__ f32x4 add_quad(u32x2 ones, uint32_t p01, uint32_t p23, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_4x4x4bf16_1k(__builtin_bit_cast(short4v, ones), __builtin_bit_cast(short4v, u32x2{p01, p23}), c, 0, 0, 0);
+  }
+  // its operand of ones; ANEW: for kernels that have no registers to keep it over their loop
+  template <bool ANEW>
+  static __device__ __forceinline__ u32x2 quad_ones() {
+    uint32_t x = 0x3f803f80u, y = 0x3f803f80u;
+    if constexpr (!ANEW) return u32x2{x, y};
+    asm volatile("" : "+v"(x), "+v"(y));  // (the moves are the compiler's: it keeps the distance that an MFMA needs behind them)
+    return u32x2{x, y};
   }
 };
 struct EtF16 {
@@ -113,9 +120,15 @@ struct EtF16 {
   static __device__ __forceinline__ u32x2 read_tr(PSA_LDS_PTR(unsigned char) a) {
     return EtBf16::read_tr(a);  // (the transposing read moves 16-bit words whatever they hold)
   }
-  static __device__ __forceinline__ f32x4 add_quad(uint32_t p01, uint32_t p23, f32x4 c) {
-    const f16x4 ones = {(f16_t)1.0f, (f16_t)1.0f, (f16_t)1.0f, (f16_t)1.0f};
-    return __builtin_amdgcn_mfma_f32_4x4x4f16(ones, __builtin_bit_cast(f16x4, u32x2{p01, p23}), c, 0, 0, 0);
+  static __device__ __forceinline__ f32x4 add_quad(u32x2 ones, uint32_t p01, uint32_t p23, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_4x4x4f16(__builtin_bit_cast(f16x4, ones), __builtin_bit_cast(f16x4, u32x2{p01, p23}), c, 0, 0, 0);
+  }
+  template <bool ANEW>
+  static __device__ __forceinline__ u32x2 quad_ones() {
+    uint32_t x = 0x3c003c00u, y = 0x3c003c00u;
+    if constexpr (!ANEW) return u32x2{x, y};
+    asm volatile("" : "+v"(x), "+v"(y));  // (the moves are the compiler's: it keeps the distance that an MFMA needs behind them)
+    return u32x2{x, y};
   }
 };
 // calls f(trait) for a 16-bit dtype id; false for any other id
