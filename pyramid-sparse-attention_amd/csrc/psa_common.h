@@ -197,6 +197,17 @@ __device__ __forceinline__ int lane_id() {
   return l;
 }
 
+// Wave priority that falls by one from phase to phase, modulo 4: of the waves of a SIMD the one that is behind goes first, unless it is
+// three phases and more behind.
+__device__ __forceinline__ void falling_priority(int phase) {
+  switch (phase & 3) {
+    case 0: __builtin_amdgcn_s_setprio(3); break;
+    case 1: __builtin_amdgcn_s_setprio(2); break;
+    case 2: __builtin_amdgcn_s_setprio(1); break;
+    default: __builtin_amdgcn_s_setprio(0);
+  }
+}
+
 // Row of a token index (token re-ordering), never out of bounds: a value outside 0 .. L-1 - the caller's mistake, the
 // Python mirror rejects such an index - reads row 0 / L-1 instead of faulting.
 __device__ __forceinline__ int clamp_row(int v, int L) { return v < 0 ? 0 : (v < L ? v : L - 1); }
