@@ -292,6 +292,13 @@ int psa_fwd_walk(psa_tensor4 q, const int32_t* q_index, psa_tensor4 k, psa_tenso
                  const void* map, int map_elem_bytes, const void* walk, psa_tensor4 out, float* lse, int B, int Hq, int Hkv,
                  int L, int D, int block_m, int block_n, float sm_scale, int causal, psa_stream_t stream);
 
+/* psa_estimate_sampled_map (keep = block / 4; Lq == Lk), psa_map_min_cap with cap (int32 [B, Hq, Nk], may be NULL) and psa_build_walk of
+ * the int8 map: same results, and the map's kernel applies the cap and lists the tiles where the map is not too wide for it. */
+int psa_estimate_walk(psa_tensor4 q, psa_tensor4 k, const int32_t* off_q, const int32_t* off_k, const int32_t* token_index,
+                      const int32_t* cap, float* scores, void* workspace, void* map_out, void* walk, int B, int Hq, int Hkv,
+                      int L, int D, int block_m, int block_n, float sm_scale, int mode, int n_items, const int32_t* item_level,
+                      const double* item_hi, int align_div, int text_blocks, double min_full_attn_ratio, psa_stream_t stream);
+
 /* The sparse layer in one call, non-causal, on one stream: psa_pool_kv -> psa_estimate_sampled_map (keep = block / 4, int8 map)
  * -> psa_fwd (walk == 0) or psa_build_walk + psa_fwd_walk (walk != 0, where that shape has a walk).  Same launches and results as
  * the separate calls.  token_index (may be NULL): the layer works on the re-ordered tokens (psa_pool_kv_indexed, and the
@@ -304,6 +311,15 @@ int psa_layer_fwd(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const int32_t* to
                   psa_tensor4 out, int B, int Hq, int Hkv, int L, int D, int block_m, int block_n, float sm_scale, int mode,
                   int n_items, const int32_t* item_level, const double* item_hi, int align_div, int text_blocks,
                   double min_full_attn_ratio, int walk, psa_stream_t stream);
+/* The same with a second buffer (256-byte aligned; NULL: as above) of psa_layer_extra_bytes(...) bytes, whose parts are filled while the
+ * workspace still holds the estimate's scratch: the level map's kernel then applies the cap and lists the tiles, and the pooling pass
+ * forms the cap.  Same results in fewer launches. */
+int64_t psa_layer_extra_bytes(int elem_bytes, int B, int Hq, int Hkv, int L, int D, int block_m, int block_n, int indexed, int walk);
+int psa_layer_fwd_extra(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const int32_t* token_index, const int32_t* off_q,
+                        const int32_t* off_k, const float* sim_thresholds, int32_t* cap_out, void* workspace, void* extra,
+                        void* map_out, psa_tensor4 out, int B, int Hq, int Hkv, int L, int D, int block_m, int block_n,
+                        float sm_scale, int mode, int n_items, const int32_t* item_level, const double* item_hi, int align_div,
+                        int text_blocks, double min_full_attn_ratio, int walk, psa_stream_t stream);
 /* The causal layer in one call (bf16; block = block_m = block_n): psa_estimate_xattn -> psa_level_map_qwen (int8 map) -> psa_ksim
  * and the cap of each query head's kv head -> psa_pool_kv -> psa_build_walk + psa_fwd_walk (psa_fwd where the shape has no walk). */
 int64_t psa_causal_layer_workspace_bytes(int B, int Hq, int Hkv, int L, int D, int block, int stride, int chunk);
@@ -311,6 +327,12 @@ int psa_causal_layer_fwd(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const floa
                          int B, int Hq, int Hkv, int L, int D, int block, int stride, int chunk, float sm_scale, int mode,
                          int n_items, const int32_t* item_level, const double* item_lo, const double* item_hi,
                          int special_blocks, int causal, psa_stream_t stream);
+/* The same with a second buffer, as psa_layer_fwd_extra. */
+int64_t psa_causal_layer_extra_bytes(int B, int Hq, int Hkv, int L, int D, int block, int stride, int chunk);
+int psa_causal_layer_fwd_extra(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const float* sim_thresholds, void* workspace, void* extra,
+                               psa_tensor4 out, int B, int Hq, int Hkv, int L, int D, int block, int stride, int chunk,
+                               float sm_scale, int mode, int n_items, const int32_t* item_level, const double* item_lo,
+                               const double* item_hi, int special_blocks, int causal, psa_stream_t stream);
 
 /* psa_fwd without a workspace argument and without any allocation: the row-ordering scratch is a fixed array inside
  * the library (one copy per GPU, about 0.5 MiB, held until the process ends).  This entry point has no counterpart in

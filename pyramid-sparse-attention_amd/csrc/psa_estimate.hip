@@ -17,6 +17,7 @@
 // group's rows of R - m, exp2, row sum in a fixed order, normalisation.
 #include "psa_common.h"
 #include "psa_level_map_row.h"
+#include "psa_schedule.h"
 #include "psa_tiles.h"
 
 namespace {
@@ -424,14 +425,17 @@ __global__ __launch_bounds__(256) void psa_est_reduce_kernel(EstParams p) {
 
 // The same, followed by the level map of the row while its scores are still in LDS: the workspace pass (HBM) of
 // one workgroup overlaps the sorting (VALU / LDS) of the others, and a launch and a round trip of the scores
-// through memory go away.  LDS: [level-map scratch: lm_bytes][n_d floats].  p.scores may be null.
+// through memory go away.  The row's levels end in LDS too (psa_sched::end_map_row): similarity cap, map, tile records.
+// LDS: [level-map scratch: lm_bytes][n_d floats][Nk levels].  p.scores may be null.
 // (80 registers, six waves per SIMD: at 82, five, 3072 rows of 1024 scores take 109.5 us instead of 104.1)
-__global__ __launch_bounds__(256, 6) void psa_est_reduce_map_kernel(EstParams p, LevelMapParams lp, int lm_bytes) {
+__global__ __launch_bounds__(256, 6) void psa_est_reduce_map_kernel(EstParams p, LevelMapParams lp, psa_sched::MapEnd end, int lm_bytes) {
   extern __shared__ __align__(16) unsigned char smem_rm[];
   __shared__ float s_part[4];
   __shared__ int s_cnt[PSA_MAX_LEVEL_ITEMS];
   __shared__ int s_iv[PSA_MAX_LEVEL_ITEMS][2];
+  __shared__ int s_lists[16];
   float* s_e = (float*)(smem_rm + lm_bytes);
+  uint8_t* s_lv = (uint8_t*)(s_e + p.n_d);
   const int i = blockIdx.x, bh = blockIdx.y, tid = threadIdx.x;
   const float total = est_reduce_row(p, s_e, s_part, i, bh);
   const int64_t row = (int64_t)bh * p.out_rows + i;
@@ -441,11 +445,12 @@ __global__ __launch_bounds__(256, 6) void psa_est_reduce_map_kernel(EstParams p,
     if (p.scores) p.scores[row * p.out_cols + j] = v;
   }
   __syncthreads();
-  level_map_row(lp, s_e, row, smem_rm, s_cnt, s_iv, tid, 256);
+  level_map_row(lp, s_e, row, smem_rm, s_cnt, s_iv, tid, 256, s_lv);
+  psa_sched::end_map_row(end, s_lv, lp.Nk, row, bh, i, (uint16_t*)smem_rm, s_lists, tid);
 }
 
 template <int D>
-int launch_est(EstParams& p, int B, hipStream_t stream, const LevelMapParams* lp, bool* map_done) {
+int launch_est(EstParams& p, int B, hipStream_t stream, const LevelMapParams* lp, const psa_sched::MapEnd& end, bool* map_done) {
   const int rows_needed = p.out_rows << p.keep_m_log2;
   dim3 grid((unsigned)((rows_needed + 255) / 256), (unsigned)(B * p.Hq));
   // 256-row workgroups: cut the key range until about 3 workgroups per CU exist (the kernel's occupancy),
@@ -482,8 +487,10 @@ int launch_est(EstParams& p, int B, hipStream_t stream, const LevelMapParams* lp
     hipLaunchKernelGGL(psa_est_reduce_kernel, rgrid, dim3(256), (size_t)p.n_d * sizeof(float), stream, p);
     return psa_check_launch("psa_estimate_sampled (reduction)");
   }
-  const size_t lm_bytes = (level_map_lds_bytes(*lp) + 15) & ~(size_t)15;
-  const size_t shmem = lm_bytes + (size_t)p.n_d * sizeof(float);
+  size_t lm_bytes = level_map_lds_bytes(*lp);
+  lm_bytes = lm_bytes > (size_t)lp->Nk * 2 ? lm_bytes : (size_t)lp->Nk * 2;  // (later the ids of the row's lists)
+  lm_bytes = (lm_bytes + 15) & ~(size_t)15;
+  const size_t shmem = lm_bytes + (size_t)p.n_d * sizeof(float) + (size_t)lp->Nk;
   if (shmem > 150 * 1024) {
     // very wide maps: the row of scores and the level-map scratch do not fit into LDS together - two kernels
     PSA_REQUIRE(p.scores != nullptr, PSA_ERR_ARG, "psa_estimate_sampled_map: maps of %d columns need the scores buffer", lp->Nk);
@@ -495,7 +502,7 @@ int launch_est(EstParams& p, int B, hipStream_t stream, const LevelMapParams* lp
     hipError_t e = hipFuncSetAttribute((const void*)psa_est_reduce_map_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
     PSA_REQUIRE(e == hipSuccess, PSA_ERR_LAUNCH, "psa_estimate_sampled_map: cannot reserve %zu bytes of LDS", shmem);
   }
-  hipLaunchKernelGGL(psa_est_reduce_map_kernel, rgrid, dim3(256), shmem, stream, p, *lp, (int)lm_bytes);
+  hipLaunchKernelGGL(psa_est_reduce_map_kernel, rgrid, dim3(256), shmem, stream, p, *lp, end, (int)lm_bytes);
   *map_done = true;
   return psa_check_launch("psa_estimate_sampled_map (reduction + level map)");
 }
@@ -528,7 +535,7 @@ namespace {
 int est_run(psa_tensor4 q, psa_tensor4 k, const int32_t* off_q, const int32_t* off_k, const int32_t* q_index, float* scores,
             void* workspace, int B, int Hq,
             int Hkv, int Lq, int Lk, int D, int block_m, int block_n, int keep_m, int keep_n, float sm_scale, int out_rows,
-            int out_cols, LevelMapParams* lp, bool* map_done, psa_stream_t stream) {
+            int out_cols, LevelMapParams* lp, const psa_sched::MapEnd& end, bool* map_done, psa_stream_t stream) {
   PSA_REQUIRE(q.ptr && k.ptr && (scores || lp) && workspace, PSA_ERR_ARG, "psa_estimate_sampled: null pointer");
   PSA_REQUIRE(B > 0 && Hq > 0 && Hkv > 0 && Lq > 0 && Lk > 0, PSA_ERR_ARG, "psa_estimate_sampled: sizes must be positive");
   PSA_REQUIRE(Hq % Hkv == 0, PSA_ERR_ARG, "psa_estimate_sampled: Hq must be a multiple of Hkv");
@@ -564,7 +571,7 @@ int est_run(psa_tensor4 q, psa_tensor4 k, const int32_t* off_q, const int32_t* o
     PSA_REQUIRE(lp->Nk == out_cols, PSA_ERR_ARG, "psa_estimate_sampled_map: the map has %d columns, the scores %d", lp->Nk, out_cols);
     lp->scores = nullptr;
   }
-  return D == 128 ? launch_est<128>(p, B, (hipStream_t)stream, lp, map_done) : launch_est<64>(p, B, (hipStream_t)stream, lp, map_done);
+  return D == 128 ? launch_est<128>(p, B, (hipStream_t)stream, lp, end, map_done) : launch_est<64>(p, B, (hipStream_t)stream, lp, end, map_done);
 }
 }  // namespace
 
@@ -574,7 +581,7 @@ extern "C" int psa_estimate_sampled(psa_tensor4 q, psa_tensor4 k, const int32_t*
   PSA_REQUIRE(scores, PSA_ERR_ARG, "psa_estimate_sampled: null pointer");
   bool unused = false;
   return est_run(q, k, off_q, off_k, nullptr, scores, workspace, B, Hq, Hkv, Lq, Lk, D, block_m, block_n, keep_m, keep_n, sm_scale,
-                 out_rows, out_cols, nullptr, &unused, stream);
+                 out_rows, out_cols, nullptr, psa_sched::MapEnd{}, &unused, stream);
 }
 
 extern "C" int psa_estimate_sampled_indexed(psa_tensor4 q, const int32_t* q_index, psa_tensor4 k, const int32_t* off_q,
@@ -584,14 +591,16 @@ extern "C" int psa_estimate_sampled_indexed(psa_tensor4 q, const int32_t* q_inde
   PSA_REQUIRE(scores && q_index, PSA_ERR_ARG, "psa_estimate_sampled_indexed: null pointer");
   bool unused = false;
   return est_run(q, k, off_q, off_k, q_index, scores, workspace, B, Hq, Hkv, Lq, Lk, D, block_m, block_n, keep_m, keep_n, sm_scale,
-                 out_rows, out_cols, nullptr, &unused, stream);
+                 out_rows, out_cols, nullptr, psa_sched::MapEnd{}, &unused, stream);
 }
 
+// cap ([B * Hq][Nk], null: none) and walk (null: none) are served here only where the map comes out of the fused kernel (ended: it did)
 static int est_map_run(psa_tensor4 q, psa_tensor4 k, const int32_t* off_q, const int32_t* off_k, const int32_t* q_index, float* scores,
                        void* workspace, int B, int Hq, int Hkv, int Lq, int Lk, int D, int block_m, int block_n,
                        int keep_m, int keep_n, float sm_scale, int out_rows, int out_cols, void* map_out,
                        int map_elem_bytes, int mode, int n_items, const int32_t* item_level, const double* item_hi,
-                       int align_div, int text_blocks, double min_full_attn_ratio, psa_stream_t stream) {
+                       int align_div, int text_blocks, double min_full_attn_ratio, psa_stream_t stream, const int32_t* cap = nullptr,
+                       void* walk = nullptr, bool* ended = nullptr) {
   PSA_REQUIRE(map_out, PSA_ERR_ARG, "psa_estimate_sampled_map: null pointer");
   PSA_REQUIRE(map_elem_bytes == 1 || map_elem_bytes == 4, PSA_ERR_ARG, "psa_estimate_sampled_map: map_elem_bytes must be 1 or 4");
   PSA_REQUIRE(out_cols > 0, PSA_ERR_ARG, "psa_estimate_sampled_map: out_cols must be positive");
@@ -599,9 +608,18 @@ static int est_map_run(psa_tensor4 q, psa_tensor4 k, const int32_t* off_q, const
   const int rc = level_map_fill_params(lp, out_cols, mode, n_items, item_level, item_hi, align_div, text_blocks, min_full_attn_ratio);
   if (rc != PSA_OK) return rc;
   lp.map_out = map_out; lp.map_elem = map_elem_bytes;
+  psa_sched::MapEnd end = {};
+  end.map_out = map_out; end.map_elem = map_elem_bytes;
+  end.cap = cap; end.Hq = Hq; end.n_rep = 1;
+  if (walk != nullptr) {
+    psa_sched::Geometry g;
+    PSA_REQUIRE(psa_schedule_geometry(B, Hq, Hkv, Lq, D, block_m, block_n, g), PSA_ERR_UNSUPPORTED, "psa_build_schedule: shape out of range");
+    psa_walk_end(end, walk, g, block_m, block_n, Lq, 0);
+  }
   bool map_done = false;
   const int rc2 = est_run(q, k, off_q, off_k, q_index, scores, workspace, B, Hq, Hkv, Lq, Lk, D, block_m, block_n, keep_m, keep_n,
-                          sm_scale, out_rows, out_cols, &lp, &map_done, stream);
+                          sm_scale, out_rows, out_cols, &lp, end, &map_done, stream);
+  if (ended != nullptr) *ended = map_done;
   if (rc2 != PSA_OK || map_done) return rc2;
   return psa_level_map(scores, map_out, map_elem_bytes, nullptr, (int64_t)B * Hq * out_rows, out_cols, mode, n_items, item_level, item_hi,
                        align_div, text_blocks, min_full_attn_ratio, stream);
@@ -627,4 +645,15 @@ extern "C" int psa_estimate_sampled_map_indexed(psa_tensor4 q, const int32_t* q_
   return est_map_run(q, k, off_q, off_k, q_index, scores, workspace, B, Hq, Hkv, Lq, Lk, D, block_m, block_n, keep_m, keep_n, sm_scale,
                      out_rows, out_cols, map_out, map_elem_bytes, mode, n_items, item_level, item_hi, align_div, text_blocks,
                      min_full_attn_ratio, stream);
+}
+
+// Map, similarity cap and tile records of a layer (psa_layer.hip): where *ended, the cap is applied and the records of `walk` are written
+// (its issue order is not).
+int psa_estimate_layer_map(psa_tensor4 q, psa_tensor4 k, const int32_t* off_q, const int32_t* off_k, const int32_t* q_index, float* scores,
+                           void* workspace, int B, int Hq, int Hkv, int L, int D, int block_m, int block_n, float sm_scale, void* map_out, int mode,
+                           int n_items, const int32_t* item_level, const double* item_hi, int align_div, int text_blocks,
+                           double min_full_attn_ratio, const int32_t* cap, void* walk, bool* ended, psa_stream_t stream) {
+  return est_map_run(q, k, off_q, off_k, q_index, scores, workspace, B, Hq, Hkv, L, L, D, block_m, block_n, block_m / 4, block_n / 4, sm_scale,
+                     (L + block_m - 1) / block_m, (L + block_n - 1) / block_n, map_out, 1, mode, n_items, item_level, item_hi, align_div,
+                     text_blocks, min_full_attn_ratio, stream, cap, walk, ended);
 }

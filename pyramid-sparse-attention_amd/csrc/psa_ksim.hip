@@ -6,6 +6,7 @@
 // channels (16-byte loads, D/8 lanes per row), forms the partial dot products and squared norms of
 // its channels, and the D/8 lanes of a token group reduce them with butterflies.
 #include "psa_common.h"
+#include "psa_ksim_row.h"
 
 namespace {
 
@@ -36,53 +37,12 @@ __global__ __launch_bounds__(256) void psa_ksim_kernel(KsimParams p) {
       f[i][2 * j + 1] = ET::from_bits(w[j] >> 16);
     }
   }
-  // 8 squared norms, dots (0,1) (2,3) (4,5) (6,7) | (0,3) (4,7) | (0,7)
   float v[15];
-#pragma unroll
-  for (int i = 0; i < 15; ++i) v[i] = 0.f;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] += f[i][e] * f[i][e];
-    v[8] += f[0][e] * f[1][e];
-    v[9] += f[2][e] * f[3][e];
-    v[10] += f[4][e] * f[5][e];
-    v[11] += f[6][e] * f[7][e];
-    v[12] += f[0][e] * f[3][e];
-    v[13] += f[4][e] * f[7][e];
-    v[14] += f[0][e] * f[7][e];
-  }
-  for (int o = lpr >> 1; o > 0; o >>= 1) {
-#pragma unroll
-    for (int i = 0; i < 15; ++i) v[i] += __shfl_xor(v[i], o, 64);
-  }
-  if (c == 0) {
-    float n[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) n[i] = sqrtf(v[i] + 1e-12f);
-    s_part[0][g] = v[8] / (n[0] * n[1] + 1e-6f) + v[9] / (n[2] * n[3] + 1e-6f) + v[10] / (n[4] * n[5] + 1e-6f) +
-                   v[11] / (n[6] * n[7] + 1e-6f);
-    s_part[1][g] = v[12] / (n[0] * n[3] + 1e-6f) + v[13] / (n[4] * n[7] + 1e-6f);
-    s_part[2][g] = v[14] / (n[0] * n[7] + 1e-6f);
-  }
+  psa_ksim_row::pair_sums(f, v);
+  psa_ksim_row::group_sums(v, lpr);
+  if (c == 0) psa_ksim_row::group_cosines(v, s_part[0][g], s_part[1][g], s_part[2][g]);
   __syncthreads();
-  if (threadIdx.x == 0) {
-    const int ng = p.bn >> 3;
-    float s2 = 0.f, s4 = 0.f, s8 = 0.f;
-    for (int i = 0; i < ng; ++i) {
-      s2 += s_part[0][i];
-      s4 += s_part[1][i];
-      s8 += s_part[2][i];
-    }
-    s2 /= (float)(p.bn >> 1);
-    s4 /= (float)(p.bn >> 2);
-    s8 /= (float)(p.bn >> 3);
-    int lv = 1;
-    if (s2 > p.t2) lv = 2;
-    if (s4 > p.t4) lv = 4;
-    if (s8 > p.t8) lv = 8;
-    p.out[(int64_t)bh * p.Nk + J] = lv;
-  }
+  if (threadIdx.x == 0) p.out[(int64_t)bh * p.Nk + J] = psa_ksim_row::block_cap(s_part[0], s_part[1], s_part[2], p.bn, p.t2, p.t4, p.t8);
 }
 
 }  // namespace

@@ -133,7 +133,8 @@ constexpr size_t SEL_LDS_BYTES = (SEL_BINS + 2 * SEL_MAX_CUTS * SEL_CAP + 8 * SE
 __host__ __device__ inline bool level_map_selects(int mode, int n_cuts, int Nk) {
   return mode == PSA_MODE_TOPK && n_cuts <= SEL_MAX_CUTS && Nk > RANK_SORT_MAX;
 }
-__device__ __forceinline__ void level_map_row_select(const LevelMapParams& p, const float* src, int64_t row, unsigned char* smem, int tid) {
+__device__ __forceinline__ void level_map_row_select(const LevelMapParams& p, const float* src, int64_t row, unsigned char* smem, int tid,
+                                                     uint8_t* lds_out) {
   constexpr int NT = 256, PER = SEL_BINS / NT;
   uint64_t* cand = (uint64_t*)smem;                       // [cut][SEL_CAP] keys of the bin that holds the cut
   uint64_t* cut_key = cand + SEL_MAX_CUTS * SEL_CAP;      // [cut] key of rank cut[c]
@@ -285,17 +286,19 @@ __device__ __forceinline__ void level_map_row_select(const LevelMapParams& p, co
 #pragma unroll
     for (int t = 0; t < SEL_MAX_CUTS; ++t) lv = k >= ck[t] ? p.seg_level[t + 1] : lv;
     if (j >= N - p.text_blocks) lv = 1;
-    store_map(p.map_out, row * N + j, p.map_elem, lv);
+    if (lds_out != nullptr) lds_out[j] = (uint8_t)lv;
+    else store_map(p.map_out, row * N + j, p.map_elem, lv);
   }
 }
 
 // One row of the level map.  `src` = the row's N scores (global memory or LDS), `smem` = level_map_lds_bytes(p) bytes
 // of 16-byte aligned LDS, s_cnt / s_iv = PSA_MAX_LEVEL_ITEMS (x2) ints of LDS; called by all nt threads of the workgroup.
+// lds_out: the levels go there (a byte per column, LDS) instead of to p.map_out.
 __device__ __forceinline__ void level_map_row(const LevelMapParams& p, const float* src, int64_t row, unsigned char* smem,
-                                              int* s_cnt, int (*s_iv)[2], int tid, int nt) {
+                                              int* s_cnt, int (*s_iv)[2], int tid, int nt, uint8_t* lds_out = nullptr) {
   const int N = p.Nk;
   if (p.list_out == nullptr && level_map_selects(p.mode, p.n_cuts, N)) {
-    level_map_row_select(p, src, row, smem, tid);
+    level_map_row_select(p, src, row, smem, tid, lds_out);
     return;
   }
   uint64_t* key = (uint64_t*)smem;            // [sort_pad(N)]
@@ -373,7 +376,8 @@ __device__ __forceinline__ void level_map_row(const LevelMapParams& p, const flo
         if (i >= s_iv[t][0] && i < s_iv[t][1]) lv = p.level[t];
       const int col = sidx[i];
       if (col >= N - p.text_blocks) lv = 1;
-      store_map(p.map_out, row * N + col, p.map_elem, lv);
+      if (lds_out != nullptr) lds_out[col] = (uint8_t)lv;
+      else store_map(p.map_out, row * N + col, p.map_elem, lv);
     }
   }
   if (p.list_out) {
@@ -391,6 +395,89 @@ __device__ __forceinline__ void level_map_row(const LevelMapParams& p, const flo
       dst[cidx] = v;
     }
   }
+}
+
+
+// ---- the causal Qwen2.5-VL example: square map, per-row ratio windows, fix-ups (psa_level_map.hip) ----
+struct QwenMapParams {
+  const float* scores;
+  void* map_out;
+  int map_elem;
+  int S;       // blocks per side
+  int mode;    // PSA_MODE_TOPK: rank windows on the causal row length; PSA_MODE_THRESHOLDBOUND: cumulative-mass windows
+  int n_items;
+  int level[PSA_MAX_LEVEL_ITEMS];
+  float lo[PSA_MAX_LEVEL_ITEMS];  // energy mode: max(lo, previous hi); rank mode: lo
+  float hi[PSA_MAX_LEVEL_ITEMS];
+  int special;  // trailing blocks (rows and columns) forced to level 1
+  int causal;
+};
+// LDS of a row of n scores
+__host__ __device__ inline size_t qwen_row_lds_bytes(int n) { return (size_t)sort_pad(n) * 8 + (size_t)n * 12; }
+// Levels of row i_row from its scores `src`, handed to store(column, level).  Only the first n columns are ranked: n = S, or the
+// i_row + 1 columns of a causal row whose other scores are all 0 - those sort last whatever the rest (no score is negative), add
+// nothing to a prefix sum and are skipped above the diagonal anyway.
+template <class Store>
+__device__ __forceinline__ void qwen_map_row(const QwenMapParams& p, const float* src, int i_row, int n, unsigned char* smem, int tid, int nt,
+                                             Store store) {
+  uint64_t* key = (uint64_t*)smem;
+  float* sw = (float*)(key + sort_pad(n));
+  int* sidx = (int*)(sw + n);
+  float* c32 = (float*)(sidx + n);
+  sort_row_desc(key, sw, sidx, src, n, tid, nt);
+  if (p.mode == PSA_MODE_THRESHOLDBOUND) row_prefix_sums((double*)key, sw, c32, n, tid, nt);
+  const float total = p.mode == PSA_MODE_THRESHOLDBOUND ? fmaxf(c32[n - 1], 1e-10f) : 1.f;
+  const float valid_len = p.causal ? (float)(i_row + 1) : (float)p.S;
+  for (int pos = tid; pos < n; pos += nt) {
+    int lv = 0;
+    if (p.mode == PSA_MODE_THRESHOLDBOUND) {
+      const float r = c32[pos] / total;
+      for (int t = 0; t < p.n_items; ++t)
+        if (r > p.lo[t] && r <= p.hi[t]) lv = p.level[t];
+    } else {
+      for (int t = 0; t < p.n_items; ++t) {
+        int s0 = (int)(valid_len * p.lo[t]), e0 = (int)(valid_len * p.hi[t]);
+        s0 = s0 < p.S ? s0 : p.S;
+        e0 = e0 < p.S ? e0 : p.S;
+        if (pos >= s0 && pos < e0) lv = p.level[t];
+      }
+    }
+    const int col = sidx[pos];
+    if (col >= p.S - p.special || i_row >= p.S - p.special) lv = 1;
+    if (p.causal && col > i_row) lv = 0;
+    if (col == i_row || col == 0) lv = 1;
+    store(col, lv);
+  }
+  for (int col = n + tid; col < p.S; col += nt) store(col, 0);  // (n < S: above the diagonal)
+}
+
+static inline int qwen_map_fill_params(QwenMapParams& p, int S, int mode, int n_items, const int32_t* item_level, const double* item_lo,
+                                       const double* item_hi, int special_blocks, int causal) {
+  PSA_REQUIRE(item_level && item_lo && item_hi, PSA_ERR_ARG, "psa_level_map_qwen: null pointer");
+  PSA_REQUIRE(mode == PSA_MODE_TOPK || mode == PSA_MODE_THRESHOLDBOUND, PSA_ERR_ARG, "mode must be 'topk' or 'energybound'");
+  PSA_REQUIRE(n_items >= 1 && n_items <= PSA_MAX_LEVEL_ITEMS, PSA_ERR_ARG, "mask_ratios must not be empty (1..%d items)", PSA_MAX_LEVEL_ITEMS);
+  PSA_REQUIRE(S > 0 && S <= 6144, PSA_ERR_UNSUPPORTED, "psa_level_map_qwen: sizes out of range");
+  p.scores = nullptr; p.map_out = nullptr; p.map_elem = 1; p.S = S; p.mode = mode; p.n_items = n_items;
+  p.special = special_blocks < 0 ? 0 : (special_blocks > S ? S : special_blocks);
+  p.causal = causal ? 1 : 0;
+  double prev_hi = 0.0;
+  for (int t = 0; t < PSA_MAX_LEVEL_ITEMS; ++t) {
+    p.level[t] = 0; p.lo[t] = 0.f; p.hi[t] = 0.f;
+  }
+  for (int t = 0; t < n_items; ++t) {
+    const int lv = item_level[t];
+    PSA_REQUIRE(lv == 0 || lv == 1 || lv == 2 || lv == 4 || lv == 8, PSA_ERR_ARG, "psa_level_map_qwen: level %d not in {0,1,2,4,8}", lv);
+    p.level[t] = lv;
+    if (mode == PSA_MODE_THRESHOLDBOUND) {
+      const double lower = item_lo[t] > prev_hi ? item_lo[t] : prev_hi;
+      prev_hi = item_hi[t];
+      p.lo[t] = (float)lower;
+    } else {
+      p.lo[t] = (float)item_lo[t];
+    }
+    p.hi[t] = (float)item_hi[t];
+  }
+  return PSA_OK;
 }
 
 

@@ -6,6 +6,8 @@
 #include "psa_schedule.h"
 
 namespace {
+using namespace psa_sched;
+static_assert(COST_LIMIT == psa_order::COST_BINS - 1, "the last bin");
 
 constexpr int ROWS_PER_WG = 4;
 
@@ -19,33 +21,20 @@ __global__ __launch_bounds__(64 * ROWS_PER_WG) void psa_sched_build_kernel(const
   const bool live = row < rows;
   uint16_t* ids = s_ids + wave * Nk;
   const int I = live ? row % Mq : 0;
-  int jmax = live ? Nk : 0;
-  if (causal) {
-    const int ce = (int)((((int64_t)(I + 1) * bm) + (1 << bn_log2) - 1) >> bn_log2);
-    jmax = ce < jmax ? ce : jmax;
-  }
+  const int jmax = live ? reached_blocks(Nk, I, bm, bn_log2, causal != 0) : 0;
   const int64_t mrow = (int64_t)row * Nk;
-  int cnt[4] = {0, 0, 0, 0};
+  RowLists rl;
+#pragma unroll
+  for (int lv = 0; lv < 4; ++lv) rl.cnt[lv] = 0;
   for (int j0 = 0; j0 < jmax; j0 += 64) {
     const int j = j0 + lane;
     const int lvl = j < jmax ? load_map(map, mrow + j, map_elem) : 0;
 #pragma unroll
-    for (int lv = 0; lv < 4; ++lv) cnt[lv] += __popcll(__ballot(lvl == (1 << lv)));
+    for (int lv = 0; lv < 4; ++lv) rl.cnt[lv] += __popcll(__ballot(lvl == (1 << lv)));
   }
-  int io[4], to[5];
+  row_offsets(rl, bn_log2);
   {
-    int i = 0, t = 0;
-#pragma unroll
-    for (int lv = 0; lv < 4; ++lv) {
-      io[lv] = i;
-      to[lv] = t;
-      i += cnt[lv];
-      t += ((cnt[lv] << (bn_log2 - lv)) + 63) >> 6;
-    }
-    to[4] = t;
-  }
-  {
-    int run[4] = {io[0], io[1], io[2], io[3]};
+    int run[4] = {rl.io[0], rl.io[1], rl.io[2], rl.io[3]};
     const uint64_t lt_mask = (1ull << lane) - 1ull;
     for (int j0 = 0; j0 < jmax; j0 += 64) {
       const int j = j0 + lane;
@@ -59,76 +48,14 @@ __global__ __launch_bounds__(64 * ROWS_PER_WG) void psa_sched_build_kernel(const
     }
   }
   __syncthreads();  // (a wave only reads its own ids; the barrier orders the writes before the reads)
-  const int T = to[4];
-  u32x4* out = recs + (int64_t)row * rec_stride;
+  const int T = rl.to[4];
   if (live && lane == 0) {
     tiles[row] = T;
-    cost[row] = T < psa_order::COST_BINS - 1 ? T : psa_order::COST_BINS - 1;
+    cost[row] = T < COST_LIMIT ? T : COST_LIMIT;
   }
-  const int64_t q_first_row = (int64_t)I * bm;
-  for (int t = lane; t < T; t += 64) {
-    const int lv = (t >= to[1]) + (t >= to[2]) + (t >= to[3]);
-    int lt = t, c_lv = cnt[0], io_lv = io[0];
-#pragma unroll
-    for (int l = 1; l < 4; ++l)
-      if (lv == l) {
-        lt = t - to[l];
-        c_lv = cnt[l];
-        io_lv = io[l];
-      }
-    const int sbs_log2 = bn_log2 - lv;
-    int nvalid = (c_lv << sbs_log2) - (lt << 6);
-    nvalid = nvalid < 64 ? nvalid : 64;
-    const int last_blk = ids[io_lv + (((lt << 6) + nvalid - 1) >> sbs_log2)];
-    if (lv == 0) {
-      const int over = (((lt << 6) + nvalid - 1) & ((1 << sbs_log2) - 1)) + 1 - (L - (last_blk << sbs_log2));
-      if (over > 0) nvalid = nvalid - over > 0 ? nvalid - over : 0;
-    }
-    const bool diag = causal && ((((int64_t)last_blk + 1) << bn_log2) - 1 > q_first_row);
-    u32x4 r;
-    bool ragged = false;
-    const bool is_fine = sbs_log2 < 4;
-    // fine tiles are the last ones of a row (the levels come in ascending order): their index counts from the first
-    const int fine_at = t - (bn_log2 - 2 < 4 ? to[2] : to[3]);
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      if (is_fine) {
-        r[g] = (uint32_t)fine_at;
-        continue;
-      }
-      const int gpos = (lt << 6) + 16 * g;
-      int bi = gpos >> sbs_log2;
-      bi = bi < c_lv - 1 ? bi : c_lv - 1;
-      const int src = ((int)ids[io_lv + bi] << sbs_log2) + (gpos & ((1 << sbs_log2) - 1));
-      ragged |= lv == 0 && src + 15 >= L;
-      r[g] = (uint32_t)src;
-    }
-    if (is_fine) {
-      u32x4* f = fine + ((int64_t)row * fine_stride + fine_at) * (psa_sched::FINE_RUNS * 2 / 16);
-#pragma unroll
-      for (int h8 = 0; h8 < psa_sched::FINE_RUNS / 8; ++h8) {
-        u32x4 w;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          int bi = ((lt << 6) + 4 * (8 * h8 + e)) >> sbs_log2;
-          bi = bi < c_lv - 1 ? bi : c_lv - 1;
-          const uint32_t id = ids[io_lv + bi];
-          w[e >> 1] = (e & 1) ? w[e >> 1] | (id << 16) : id;
-        }
-        f[h8] = w;
-      }
-    }
-    const uint32_t code = ragged ? psa_sched::REC_CODE_RAGGED : is_fine ? 4u + (uint32_t)lv : (uint32_t)lv;
-    const uint32_t hi = (code << psa_sched::REC_CODE_SHIFT) |
-                        ((uint32_t)(diag || nvalid < 64) << psa_sched::REC_MASKED_BIT) | ((uint32_t)nvalid << psa_sched::REC_NVALID_SHIFT);
-#pragma unroll
-    for (int g = 0; g < 4; ++g) r[g] |= hi;
-    out[t] = r;
-    if (t == T - 1) {
-#pragma unroll
-      for (int e = 1; e <= psa_sched::REC_PAD; ++e) out[t + e] = r;
-    }
-  }
+  if (live)
+    write_records(rl, ids, lane, 64, bn_log2, L, causal != 0, (int64_t)I * bm, recs + (int64_t)row * rec_stride,
+                  fine + (int64_t)row * fine_stride * (FINE_RUNS * 2 / 16));
 }
 
 }  // namespace
@@ -159,6 +86,28 @@ bool psa_schedule_geometry(int B, int Hq, int Hkv, int L, int D, int block_m, in
   return true;
 }
 
+int psa_walk_order(void* walk, const psa_sched::Geometry& g, psa_stream_t stream) {
+  char* base = (char*)walk;
+  psa_order::sort_lists<1>({{{(const int32_t*)(base + g.lay.cost_off), (int32_t*)(base + g.lay.order_off), (int)g.rows, g.wg_chunk, g.wg_groups}}},
+                           (hipStream_t)stream);
+  return psa_check_launch("psa_build_schedule (order)");
+}
+
+void psa_walk_end(psa_sched::MapEnd& e, void* walk, const psa_sched::Geometry& g, int block_m, int block_n, int L, int causal) {
+  char* base = (char*)walk;
+  e.recs = (u32x4*)(base + g.lay.rec_off);
+  e.fine = (u32x4*)(base + g.lay.fine_off);
+  e.tiles = (int32_t*)(base + g.lay.tiles_off);
+  e.cost = (int32_t*)(base + g.lay.cost_off);
+  e.rec_stride = g.lay.rec_stride;
+  e.fine_stride = g.lay.fine_stride;
+  e.bn_log2 = psa_ilog2(block_n);
+  e.bm = block_m;
+  e.L = L;
+  e.Mq = g.Mq;
+  e.causal = causal ? 1 : 0;
+}
+
 static int build_schedule(const void* map, int map_elem_bytes, void* schedule, int B, int Hq, int Hkv, int L, int D, int block_m,
                           int block_n, int causal, psa_stream_t stream) {
   PSA_REQUIRE((uintptr_t)schedule % 16 == 0, PSA_ERR_ARG, "psa_build_schedule: schedule must be 16-byte aligned");
@@ -167,7 +116,6 @@ static int build_schedule(const void* map, int map_elem_bytes, void* schedule, i
   PSA_REQUIRE((size_t)ROWS_PER_WG * g.Nk * 2 <= 64 * 1024, PSA_ERR_UNSUPPORTED, "psa_build_schedule: more than 8192 kv-blocks");
   char* base = (char*)schedule;
   hipStream_t s = (hipStream_t)stream;
-  int32_t* order = (int32_t*)(base + g.lay.order_off);
   int32_t* cost = (int32_t*)(base + g.lay.cost_off);
   int32_t* tiles = (int32_t*)(base + g.lay.tiles_off);
   u32x4* recs = (u32x4*)(base + g.lay.rec_off);
@@ -175,8 +123,7 @@ static int build_schedule(const void* map, int map_elem_bytes, void* schedule, i
                      (size_t)ROWS_PER_WG * g.Nk * 2, s, map, map_elem_bytes, (int)g.rows, g.Mq, g.Nk, psa_ilog2(block_n), block_m, L,
                      causal ? 1 : 0, cost, tiles, recs, g.lay.rec_stride, (u32x4*)(base + g.lay.fine_off), g.lay.fine_stride);
   if (int e = psa_check_launch("psa_build_schedule (tiles)")) return e;
-  psa_order::sort_lists<1>({{{cost, order, (int)g.rows, g.wg_chunk, g.wg_groups}}}, s);
-  return psa_check_launch("psa_build_schedule (order)");
+  return psa_walk_order(schedule, g, stream);
 }
 
 extern "C" int64_t psa_schedule_bytes(int B, int Hq, int Hkv, int L, int D, int block_m, int block_n) {

@@ -21,6 +21,9 @@
 #include <type_traits>
 
 #include "psa_common.h"
+#include "psa_level_map_row.h"
+#include "psa_pool_rows.h"
+#include "psa_schedule.h"
 #include "psa_tiles.h"
 
 namespace {
@@ -69,14 +72,29 @@ __host__ __device__ inline int tiles_in_row(int tm, int tiles_n, int causal, int
   return n < tiles_n ? n : tiles_n;
 }
 
-template <int RBL, class X>  // log2 of the strided keys per block
-__global__ __launch_bounds__(X::WAVES * 64, X::WAVES == 8 ? 1 : 2) void psa_xattn_gemm_kernel(XParams p) {
+// Pooling (and similarity cap) as further workgroups of a contraction with small tiles: both only read K, the contraction leaves CUs
+// idle there, and the launches of the two passes are as long as their work (28 heads x 2345 tokens: 18 + 4
+// + 5 -> 19 us).
+struct PoolPart {
+  PoolParams p;
+  int first, nx, heads;  // first workgroup; workgroups per (tensor, head); heads
+};
+
+template <int RBL, class X, bool POOL>  // RBL: log2 of the strided keys per block
+__global__ __launch_bounds__(X::WAVES * 64, X::WAVES == 8 ? 1 : 2) void psa_xattn_gemm_kernel(XParams p, PoolPart pool) {
   constexpr int TM = X::TM, TN = X::TN, X_QT = X::QT, X_STAGE = X::STAGE, X_GPW = X::GPW, X_NA = X::NA, X_NC = X::NC;
   extern __shared__ __align__(16) unsigned char smem[];  // X_BUFS stages of [Q tiles | K tiles]
   // Workgroup ids go round-robin over the 8 XCDs and every XCD runs its ids in order.  The output tiles with
   // visible keys are listed (batch-head, tile row, tile column) and the list is cut into 8 contiguous shares, one
   // per XCD: all tiles cost the same, so the XCDs finish together, and the ~32 tiles an XCD works on at a time
   // are neighbours that find each other's Q and K rows in its L2.
+  if constexpr (POOL) {
+    if ((int)blockIdx.x >= pool.first) {
+      const int u = (int)blockIdx.x - pool.first, w = u / pool.nx;
+      pool_rows<false, true, Pool16<EtBf16>>(pool.p, u % pool.nx, w % pool.heads, w / pool.heads, pool.heads);
+      return;
+    }
+  }
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
   const int idx = xcd * p.per_xcd + slot;
   if (idx >= p.n_active) return;
@@ -227,12 +245,10 @@ __global__ __launch_bounds__(X::WAVES * 64, X::WAVES == 8 ? 1 : 2) void psa_xatt
 // one workgroup per (b, h, q-block): 256 threads; thread t handles key blocks t, t+256, ...
 // cached != 0: the (maximum, sum) pairs of the workgroup's rows are read from the workspace once into dynamic LDS
 // ([key block][row], NB * rb pairs) and the three passes below run on that copy instead of on memory.
-__global__ __launch_bounds__(256) void psa_xattn_reduce_kernel(XParams p, int cached) {
-  extern __shared__ __align__(16) unsigned char s_cache[];
+// The row of block scores goes to dst.
+__device__ __forceinline__ void xattn_reduce_row(const XParams& p, int cached, unsigned char* s_cache, int I, int bh, int tid, float* dst) {
   __shared__ float s_M[32], s_inv[32];
   __shared__ float s_big[256];
-  const int I = blockIdx.x, bh = blockIdx.y;
-  const int tid = threadIdx.x;
   const int rb = 1 << p.rb_log2;
   const int m0 = I * rb;
   const float* ws = p.ws + (int64_t)bh * p.NB * p.Mr * 2;
@@ -243,9 +259,22 @@ __global__ __launch_bounds__(256) void psa_xattn_reduce_kernel(XParams p, int ca
     f32x2* c = (f32x2*)s_cache;
     const int jlim = p.causal ? (((m0 + rb - 1 + p.off) >> p.rb_log2) + 1) : p.NB;  // key blocks any row of the q-block sees
     const int jn = jlim < p.NB ? jlim : p.NB;
-    for (int u = tid; u < jn * rb; u += 256) {
-      const int J = u >> p.rb_log2, rr = u & (rb - 1);
-      c[u] = *(const f32x2*)(ws + ((int64_t)J * p.Mr + m0 + rr) * 2);
+    // two pairs per load, four loads in flight per thread: one load after the other is a round trip to memory each (the map's
+    // kernel, 28 heads x 32768 tokens, 150 -> 125 us)
+    const int n2 = jn * rb >> 1, half_log2 = p.rb_log2 - 1;
+    for (int u0 = tid; u0 < n2; u0 += 4 * 256) {
+      f32x4 x[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        int u = u0 + e * 256;
+        u = u < n2 ? u : n2 - 1;
+        x[e] = *(const f32x4*)(ws + ((int64_t)(u >> half_log2) * p.Mr + m0 + 2 * (u & (rb / 2 - 1))) * 2);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int u = u0 + e * 256;
+        if (u < n2) *(f32x4*)(c + 2 * u) = x[e];
+      }
     }
     __syncthreads();
     ws = (const float*)s_cache;
@@ -285,7 +314,6 @@ __global__ __launch_bounds__(256) void psa_xattn_reduce_kernel(XParams p, int ca
   }
   __syncthreads();
   // pass 2: Est[I, J] = sum_r sum[r, J] * exp2(max[r, J] - M_r) / l_r
-  float* dst = p.est + ((int64_t)bh * p.out_rows + I) * p.out_cols;
   for (int J = tid; J < p.out_cols; J += 256) {
     float e = 0.f;
     for (int rr = 0; rr < rb; ++rr) {
@@ -299,6 +327,35 @@ __global__ __launch_bounds__(256) void psa_xattn_reduce_kernel(XParams p, int ca
     }
     dst[J] = e;
   }
+}
+
+__global__ __launch_bounds__(256) void psa_xattn_reduce_kernel(XParams p, int cached) {
+  extern __shared__ __align__(16) unsigned char s_cache[];
+  const int I = blockIdx.x, bh = blockIdx.y;
+  xattn_reduce_row(p, cached, s_cache, I, bh, (int)threadIdx.x, p.est + ((int64_t)bh * p.out_rows + I) * p.out_cols);
+}
+
+// The same, followed by the causal layer's level map of the row while its scores are in LDS, and by what ends a map row (similarity cap,
+// map, tile records): one launch instead of reduction, map, cap and list, and a causal row ranks only the columns that it
+// sees (a third of the comparisons).  LDS: [pairs, then scratch of the map: scratch bytes][S scores][S levels].
+// 28 heads x 32768 tokens 69 + 65 + 8 + 18 -> 125 us, x 2345 tokens 5 + 5 + 4 + 4 -> 10.
+__global__ __launch_bounds__(256) void psa_xattn_map_kernel(XParams p, int cached, int scratch, QwenMapParams mp, psa_sched::MapEnd end) {
+  extern __shared__ __align__(16) unsigned char s_cache[];
+  __shared__ int s_lists[16];
+  const int I = blockIdx.x, bh = blockIdx.y, tid = threadIdx.x, S = mp.S;
+  float* s_e = (float*)(s_cache + scratch);
+  uint8_t* s_lv = (uint8_t*)(s_e + S);
+  xattn_reduce_row(p, cached, s_cache, I, bh, tid, s_e);
+  __syncthreads();
+  int n = S;
+  if (mp.causal && p.off == 0) {
+    // (scores above the diagonal are 0; NaNs, whose place in the order depends on their sign, are ranked among all columns)
+    bool nan = false;
+    for (int j = tid; j <= I; j += 256) nan |= s_e[j] != s_e[j];
+    if (!__syncthreads_or(nan)) n = I + 1;
+  }
+  qwen_map_row(mp, s_e, I, n, s_cache, tid, 256, [&](int col, int lv) __attribute__((always_inline)) { s_lv[col] = (uint8_t)lv; });
+  psa_sched::end_map_row(end, s_lv, S, (int64_t)bh * S + I, bh, I, (uint16_t*)s_cache, s_lists, tid);
 }
 
 // output tiles of one (batch, head) that hold visible keys of rows below rows_used; sets the tile counts of p
@@ -340,9 +397,17 @@ extern "C" int64_t psa_estimate_xattn_workspace_bytes(int B, int Hq, int Lq, int
   return (int64_t)B * Hq * g.NB * g.Mr * 2 * (int64_t)sizeof(float);
 }
 
-extern "C" int psa_estimate_xattn(psa_tensor4 q, psa_tensor4 k, float* est, void* workspace, int B, int Hq, int Hkv, int Lq,
-                                  int Lk, int D, int block_size, int stride, int chunk_size, int causal, psa_stream_t stream) {
-  PSA_REQUIRE(q.ptr && k.ptr && est && workspace, PSA_ERR_ARG, "psa_estimate_xattn: null pointer");
+// What psa_xattn_layer_map adds to an estimate: the level map of the layer in place of the scores
+struct XattnMap {
+  QwenMapParams mp;
+  psa_sched::MapEnd end;
+  PoolParams* pool;  // pooling and cap of the layer, run beside the contraction (pool_blocks, pool_heads) or before it by the caller
+  int pool_nx, pool_heads;
+};
+
+static int xattn_run(psa_tensor4 q, psa_tensor4 k, float* est, void* workspace, int B, int Hq, int Hkv, int Lq,
+                     int Lk, int D, int block_size, int stride, int chunk_size, int causal, psa_stream_t stream, XattnMap* xm) {
+  PSA_REQUIRE(q.ptr && k.ptr && (est || xm) && workspace, PSA_ERR_ARG, "psa_estimate_xattn: null pointer");
   PSA_REQUIRE(B > 0 && Hq > 0 && Hkv > 0 && Lq > 0 && Lk > 0, PSA_ERR_ARG, "psa_estimate_xattn: sizes must be positive");
   PSA_REQUIRE(Hq % Hkv == 0, PSA_ERR_ARG, "psa_estimate_xattn: Hq must be a multiple of Hkv");
   PSA_REQUIRE(D == 64 || D == 128, PSA_ERR_UNSUPPORTED, "psa_estimate_xattn: head dim %d not in {64, 128}", D);
@@ -386,15 +451,29 @@ extern "C" int psa_estimate_xattn(psa_tensor4 q, psa_tensor4 k, float* est, void
   PSA_REQUIRE(n_active < (1ll << 28), PSA_ERR_UNSUPPORTED, "psa_estimate_xattn: too many output tiles");
   p.n_active = (int)n_active;
   p.per_xcd = (int)((n_active + 7) / 8);
+  PoolPart pool = {};
   auto launch = [&](auto x) -> int {
     using X = decltype(x);
+    constexpr bool CAN_POOL = X::WAVES * 64 == 256;  // (the pooling pass is written for 256 threads)
     p.act_per_bh = active_tiles<X>(p, rows_used);
     const size_t shmem = X_BUFS * (size_t)X::STAGE;
-    auto kern = rb == 8 ? psa_xattn_gemm_kernel<3, X> : rb == 16 ? psa_xattn_gemm_kernel<4, X> : psa_xattn_gemm_kernel<5, X>;
+    auto kern = rb == 8 ? psa_xattn_gemm_kernel<3, X, false> : rb == 16 ? psa_xattn_gemm_kernel<4, X, false> : psa_xattn_gemm_kernel<5, X, false>;
+    int64_t blocks = (int64_t)p.per_xcd * 8;
+    if constexpr (CAN_POOL) {
+      if (xm != nullptr && xm->pool != nullptr) {
+        kern = rb == 8 ? psa_xattn_gemm_kernel<3, X, true> : rb == 16 ? psa_xattn_gemm_kernel<4, X, true> : psa_xattn_gemm_kernel<5, X, true>;
+        pool.p = *xm->pool;
+        pool.first = (int)blocks;
+        pool.nx = xm->pool_nx;
+        pool.heads = xm->pool_heads;
+        blocks += (int64_t)xm->pool_nx * xm->pool_heads * 2;
+      }
+    }
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem) != hipSuccess) return PSA_ERR_LAUNCH;
-    hipLaunchKernelGGL(kern, dim3((unsigned)(p.per_xcd * 8)), dim3(X::WAVES * 64), shmem, st, p);
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(X::WAVES * 64), shmem, st, p, pool);
     return PSA_OK;
   };
+  if (!small && xm != nullptr && xm->pool != nullptr) psa_pool_launch_cap(*xm->pool, xm->pool_nx, xm->pool_heads, st);
   int rc = small ? launch(XSmall{}) : launch(XLarge{});
   PSA_REQUIRE(rc == PSA_OK, rc, "psa_estimate_xattn: cannot reserve LDS");
   rc = psa_check_launch("psa_estimate_xattn (contraction)");
@@ -402,6 +481,50 @@ extern "C" int psa_estimate_xattn(psa_tensor4 q, psa_tensor4 k, float* est, void
   // the pairs of one q-block: NB * rb * 8 bytes; cached in LDS when that leaves room for several workgroups per CU
   const size_t cache_bytes = (size_t)p.NB * ((size_t)1 << p.rb_log2) * 8;
   const int cached = cache_bytes <= 48 * 1024 ? 1 : 0;
+  if (xm != nullptr) {
+    const size_t map_bytes = qwen_row_lds_bytes(p.out_cols);  // (more than the 2 bytes per column of the lists' ids)
+    size_t scratch = cached && cache_bytes > map_bytes ? cache_bytes : map_bytes;
+    scratch = (scratch + 15) & ~(size_t)15;
+    const size_t shmem = scratch + (size_t)p.out_cols * 5;
+    if (shmem > 48 * 1024) {
+      hipError_t e = hipFuncSetAttribute((const void*)psa_xattn_map_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
+      PSA_REQUIRE(e == hipSuccess, PSA_ERR_LAUNCH, "psa_level_map_qwen: cannot reserve %zu bytes of LDS", shmem);
+    }
+    hipLaunchKernelGGL(psa_xattn_map_kernel, dim3((unsigned)p.out_rows, (unsigned)(B * Hq)), dim3(256), shmem, st, p, cached, (int)scratch, xm->mp,
+                       xm->end);
+    return psa_check_launch("psa_estimate_xattn (reduction + level map)");
+  }
   hipLaunchKernelGGL(psa_xattn_reduce_kernel, dim3((unsigned)p.out_rows, (unsigned)(B * Hq)), dim3(256), cached ? cache_bytes : 0, st, p, cached);
   return psa_check_launch("psa_estimate_xattn (reduction)");
+}
+
+extern "C" int psa_estimate_xattn(psa_tensor4 q, psa_tensor4 k, float* est, void* workspace, int B, int Hq, int Hkv, int Lq,
+                                  int Lk, int D, int block_size, int stride, int chunk_size, int causal, psa_stream_t stream) {
+  PSA_REQUIRE(est, PSA_ERR_ARG, "psa_estimate_xattn: null pointer");
+  return xattn_run(q, k, est, workspace, B, Hq, Hkv, Lq, Lk, D, block_size, stride, chunk_size, causal, stream, nullptr);
+}
+
+// Pooling, similarity cap, estimate, level map, cap on the map and tile records (walk, null: none) of the causal layer (psa_layer.hip).
+int psa_xattn_layer_map(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, void* workspace, void* k_pool, void* v_pool, int32_t* cap,
+                        const float* thresholds, void* map, void* walk, int B, int Hq, int Hkv, int L, int D,
+                        int block, int stride, int chunk, int mode, int n_items, const int32_t* item_level, const double* item_lo,
+                        const double* item_hi, int special_blocks, int causal, psa_stream_t stream) {
+  const int S = (L + block - 1) / block;
+  XattnMap xm = {};
+  int rc = qwen_map_fill_params(xm.mp, S, mode, n_items, item_level, item_lo, item_hi, special_blocks, causal);
+  if (rc != PSA_OK) return rc;
+  PoolParams pool;
+  rc = psa_pool_params(pool, k, v, nullptr, nullptr, nullptr, k_pool, v_pool, B, Hkv, L, D, block, cap, thresholds);
+  if (rc != PSA_OK) return rc;
+  xm.end.map_out = map; xm.end.map_elem = 1;
+  xm.end.cap = cap; xm.end.Hq = Hq; xm.end.n_rep = Hkv > 0 ? Hq / Hkv : 1;
+  if (walk != nullptr) {
+    psa_sched::Geometry g;
+    PSA_REQUIRE(psa_schedule_geometry(B, Hq, Hkv, L, D, block, block, g), PSA_ERR_UNSUPPORTED, "psa_build_schedule: shape out of range");
+    psa_walk_end(xm.end, walk, g, block, block, L, causal);
+  }
+  xm.pool = &pool;
+  xm.pool_nx = (int)((pool.npad / 8 * (D / 8) + 255) / 256);
+  xm.pool_heads = B * Hkv;
+  return xattn_run(q, k, nullptr, workspace, B, Hq, Hkv, L, L, D, block, stride, chunk, causal, stream, &xm);
 }

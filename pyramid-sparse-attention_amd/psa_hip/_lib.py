@@ -122,6 +122,24 @@ SIGNATURES = {
         [Tensor4, Tensor4, Tensor4, POINTER(c_float), c_void_p, Tensor4, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float,
          c_int, c_int, POINTER(c_int32), POINTER(c_double), POINTER(c_double), c_int, c_int, c_void_p],
     ),
+    "psa_estimate_walk": (
+        c_int,
+        [Tensor4, Tensor4, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int,
+         c_int, c_int, c_float, c_int, c_int, POINTER(c_int32), POINTER(c_double), c_int, c_int, c_double, c_void_p],
+    ),
+    "psa_layer_extra_bytes": (c_int64, [c_int] * 10),
+    "psa_layer_fwd_extra": (
+        c_int,
+        [Tensor4, Tensor4, Tensor4, c_void_p, c_void_p, c_void_p, POINTER(c_float), c_void_p, c_void_p, c_void_p, c_void_p, Tensor4, c_int,
+         c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int, POINTER(c_int32), POINTER(c_double), c_int, c_int, c_double,
+         c_int, c_void_p],
+    ),
+    "psa_causal_layer_extra_bytes": (c_int64, [c_int] * 8),
+    "psa_causal_layer_fwd_extra": (
+        c_int,
+        [Tensor4, Tensor4, Tensor4, POINTER(c_float), c_void_p, c_void_p, Tensor4, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
+         c_float, c_int, c_int, POINTER(c_int32), POINTER(c_double), POINTER(c_double), c_int, c_int, c_void_p],
+    ),
     "psa_fwd_noalloc": (
         c_int,
         [Tensor4, Tensor4, Tensor4, c_void_p, c_void_p, c_void_p, c_int, Tensor4, c_void_p, c_int, c_int, c_int, c_int,

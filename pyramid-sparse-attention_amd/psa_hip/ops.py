@@ -564,6 +564,7 @@ def sparse_attention_fwd(
     balance: bool = True,
     q_index: Optional[torch.Tensor] = None,
     schedule=None,
+    _walk: Optional[torch.Tensor] = None,
 ):
     """Pyramid sparse attention forward.  level_map_ None = dense attention.  Returns out (dtype and
     shape of q) or (out, lse fp32 [B,H,L], (k_pool, v_pool)).  balance=True issues the rows of the map
@@ -606,8 +607,8 @@ def sparse_attention_fwd(
         n_walk = _walk_bytes(qb.dtype, *shape)
     if n_walk > 0:
         # the map's tiles are listed once (one pass over the map) and walked by the kernel
-        walk = schedule
-        if not isinstance(schedule, torch.Tensor) or block_n != 128:  # (build_schedule serves 128-key blocks)
+        walk = schedule if _walk is None else _walk  # (_walk: the layer's, listed by the kernel that formed the map)
+        if _walk is None and (not isinstance(schedule, torch.Tensor) or block_n != 128):  # (build_schedule serves 128-key blocks)
             walk = torch.empty(n_walk, dtype=torch.uint8, device=q.device)
             with _on(q.device):
                 check(lib.psa_build_walk(_ptr(level_map_), level_map_.element_size(), _ptr(walk), *shape, int(causal), _stream(q)), "psa_build_walk")
@@ -674,13 +675,18 @@ def _layer_one_call(qb, kb, vb, off_q, off_k, mask_ratios, mode, block_m, block_
     items, m, _ = _items(mask_ratios, mode)
     Mq, Nk = -(-L // block_m), -(-L // block_n)
     walk = int(_walk_bytes(qb.dtype, B, Hq, Hkv, L, D, block_m, block_n) > 0)
-    n_ws = lib.psa_layer_workspace_bytes(qb.element_size(), B, Hq, Hkv, L, D, block_m, block_n, int(token_index is not None), walk)
+    sizes = (qb.element_size(), B, Hq, Hkv, L, D, block_m, block_n, int(token_index is not None), walk)
+    n_ws = lib.psa_layer_workspace_bytes(*sizes)
     if not 0 < n_ws <= _ONE_CALL_MAX_BYTES:
         return None
+    n_extra = lib.psa_layer_extra_bytes(*sizes)  # (multiples of 256 bytes, both)
+    if n_ws + n_extra > _ONE_CALL_MAX_BYTES:
+        n_extra = 0
     if token_index is not None:
         token_index = _check_index(token_index, L)
     lv, hi = _level_items(items)
-    ws = torch.empty(n_ws, dtype=torch.uint8, device=dev)
+    ws = torch.empty(n_ws + n_extra, dtype=torch.uint8, device=dev)
+    at = ws.data_ptr()
     mp = torch.empty(B, Hq, Mq, Nk, dtype=torch.int8, device=dev)
     out = torch.empty(B, Hq, L, D, dtype=qb.dtype, device=dev)
     cap = thr = None
@@ -689,10 +695,47 @@ def _layer_one_call(qb, kb, vb, off_q, off_k, mask_ratios, mode, block_m, block_
         thr = (ctypes.c_float * 3)(*sim_thresholds)
     tb = (text_length + block_n - 1) // block_n if text_length > 0 else 0
     with _on(dev):
-        check(lib.psa_layer_fwd(_t4(qb), _t4(kb), _t4(vb), _ptr(token_index), off_q.data_ptr(), off_k.data_ptr(), thr, _ptr(cap),
-                                ws.data_ptr(), mp.data_ptr(), _t4(out), B, Hq, Hkv, L, D, block_m, block_n, sm_scale, m, len(items), lv, hi,
-                                block_n // tile_n, tb, 0.06, walk, _stream(qb)), "psa_layer_fwd")
+        check(lib.psa_layer_fwd_extra(_t4(qb), _t4(kb), _t4(vb), _ptr(token_index), off_q.data_ptr(), off_k.data_ptr(), thr, _ptr(cap),
+                                      at, at + n_ws if n_extra else None, mp.data_ptr(), _t4(out), B, Hq, Hkv, L, D, block_m, block_n, sm_scale, m,
+                                      len(items), lv, hi, block_n // tile_n, tb, 0.06, walk, _stream(qb)), "psa_layer_fwd")
     return out, mp, cap
+
+
+def _map_and_walk(qb, kb, off_q, off_k, mask_ratios, mode, block_m, block_n, tile_n, sm_scale, text_length, token_index, cap):
+    """(map, tile list) of estimate_sampled_map, map_min_cap and psa_build_walk in one library call, or None where the layer has no
+    list or the arguments are not the plain ones (the separate operators then run, or say what is wrong)."""
+    B, Hq, L, D = qb.shape
+    Hkv = kb.shape[1]
+    dev = qb.device
+    if kb.shape != (B, Hkv, L, D) or kb.device != dev or Hkv == 0 or Hq % Hkv or tile_n > block_n or not sm_scale > 0:
+        return None
+    if mode not in ("topk", "thresholdbound") or mask_ratios is None:
+        return None
+    for o, H, keep in ((off_q, Hq, block_m // 4), (off_k, Hkv, block_n // 4)):
+        if o is None or o.dtype != torch.int32 or o.shape != (B, H, keep) or not o.is_contiguous() or o.device != dev:
+            return None
+    Mq, Nk = -(-L // block_m), -(-L // block_n)
+    if cap is not None and (cap.dtype != torch.int32 or cap.shape != (B, Hq, Nk) or not cap.is_contiguous() or cap.device != dev):
+        return None
+    if token_index is not None and token_index.device != dev:
+        return None
+    n_walk = _walk_bytes(qb.dtype, B, Hq, Hkv, L, D, block_m, block_n)
+    if n_walk <= 0:
+        return None
+    items, m, _ = _items(mask_ratios, mode)
+    if token_index is not None:
+        token_index = _check_index(token_index, L)
+    lv, hi = _level_items(items)
+    tb = (text_length + block_n - 1) // block_n if text_length > 0 else 0
+    mp = torch.empty(B, Hq, Mq, Nk, dtype=torch.int8, device=dev)
+    walk = torch.empty(n_walk, dtype=torch.uint8, device=dev)
+    scores = torch.empty(B, Hq, Mq, Nk, dtype=torch.float32, device=dev) if Nk > 4096 else None
+    ws = torch.empty(lib.psa_estimate_workspace_bytes(B, Hq, L, L, block_m, block_n, block_m // 4, block_n // 4), dtype=torch.uint8, device=dev)
+    with _on(dev):
+        check(lib.psa_estimate_walk(_t4(qb), _t4(kb), off_q.data_ptr(), off_k.data_ptr(), _ptr(token_index), _ptr(cap), _ptr(scores), ws.data_ptr(),
+                                    mp.data_ptr(), walk.data_ptr(), B, Hq, Hkv, L, D, block_m, block_n, sm_scale, m, len(items), lv, hi,
+                                    block_n // tile_n, tb, 0.06, _stream(qb)), "psa_estimate_walk")
+    return mp, walk
 
 
 def causal_layer_fwd(q, k, v, mask_ratios, mode, text_length, block, stride, chunk_size, causal, sim_thresholds):
@@ -709,6 +752,9 @@ def causal_layer_fwd(q, k, v, mask_ratios, mode, text_length, block, stride, chu
     n_ws = lib.psa_causal_layer_workspace_bytes(B, Hq, Hkv, L, D, block, stride, chunk_size)
     if not 0 < n_ws <= _ONE_CALL_MAX_BYTES:
         return None
+    n_extra = lib.psa_causal_layer_extra_bytes(B, Hq, Hkv, L, D, block, stride, chunk_size)
+    if n_ws + n_extra > _ONE_CALL_MAX_BYTES:
+        n_extra = 0
     q, k, v = _kernel_view(q), _kernel_view(k), _kernel_view(v)
     items = list(mask_ratios.items())
     lv, hi = _level_items(items)
@@ -716,11 +762,13 @@ def causal_layer_fwd(q, k, v, mask_ratios, mode, text_length, block, stride, chu
     S = -(-L // block)
     special = min(-(-text_length // block) if text_length > 0 else 0, S)
     m = _lib.PSA_MODE_TOPK if mode == "topk" else _lib.PSA_MODE_THRESHOLDBOUND
-    ws = torch.empty(n_ws, dtype=torch.uint8, device=q.device)
+    ws = torch.empty(n_ws + n_extra, dtype=torch.uint8, device=q.device)
+    at = ws.data_ptr()
     out = torch.empty(B, Hq, L, D, dtype=q.dtype, device=q.device)
     with _on(q.device):
-        check(lib.psa_causal_layer_fwd(_t4(q), _t4(k), _t4(v), (ctypes.c_float * 3)(*sim_thresholds), ws.data_ptr(), _t4(out), B, Hq, Hkv, L, D,
-                                       block, stride, chunk_size, D ** -0.5, m, len(items), lv, lo, hi, special, int(causal), _stream(q)),
+        check(lib.psa_causal_layer_fwd_extra(_t4(q), _t4(k), _t4(v), (ctypes.c_float * 3)(*sim_thresholds), at, at + n_ws if n_extra else None,
+                                             _t4(out), B, Hq, Hkv, L, D, block, stride, chunk_size, D ** -0.5, m, len(items), lv, lo, hi,
+                                             special, int(causal), _stream(q)),
               "psa_causal_layer_fwd")
     return out
 
@@ -787,15 +835,20 @@ def psa_layer_fwd(
         if level_cap is not None:
             raise ValueError("pass either level_cap or sim_thresholds")
         level_cap = k_similarity(kb, block_n, *sim_thresholds)
-    mp = estimate_sampled_map(qb, kb, off_q, off_k, block_m, block_n, keep_m, keep_n, mask_ratios, text_length, mode,
-                              compute_tile=tile_n, map_dtype=torch.int8, sm_scale=sm_scale, q_index=token_index)
-    if level_cap is not None:
-        mp = map_min_cap(mp, level_cap)
+    walk = None
+    both = _map_and_walk(qb, kb, off_q, off_k, mask_ratios, mode, block_m, block_n, tile_n, sm_scale, text_length, token_index, level_cap)
+    if both is not None:
+        mp, walk = both
+    else:
+        mp = estimate_sampled_map(qb, kb, off_q, off_k, block_m, block_n, keep_m, keep_n, mask_ratios, text_length, mode,
+                                  compute_tile=tile_n, map_dtype=torch.int8, sm_scale=sm_scale, q_index=token_index)
+        if level_cap is not None:
+            mp = map_min_cap(mp, level_cap)
     if side is not None:
         main.wait_stream(side)
     elif token_index is None:
         kp, vp = pool_kv(kb, vb, block_n)
-    out = sparse_attention_fwd(qb, kb, vb, mp, block_m, block_n, sm_scale, pools=(kp, vp), q_index=token_index)
+    out = sparse_attention_fwd(qb, kb, vb, mp, block_m, block_n, sm_scale, pools=(kp, vp), q_index=token_index, _walk=walk)
     if out.dtype != q.dtype:
         out = out.to(q.dtype)
     if not (return_map or return_cap):
