@@ -285,7 +285,8 @@ extern "C" int psa_causal_layer_fwd_extra(psa_tensor4 q, psa_tensor4 k, psa_tens
   int32_t* cap = (int32_t*)(ws + p.cap);
   void* const map = ws + p.map;
   int rc;
-  if (extra != nullptr) {
+  // (wider maps: a row's scores, levels and sorting scratch, 17 to 25 bytes per column, do not fit LDS together)
+  if (extra != nullptr && S <= 4096) {
     const CausalExtra e = causal_extra(B, Hq, Hkv, L, D, block);
     char* ex = (char*)extra;
     void *kp = ex + e.kp, *vp = ex + e.vp, *walk = e.walk >= 0 ? ex + e.walk : nullptr;

@@ -86,3 +86,30 @@ def test_causal_map_in_one_launch(Hq, Hkv, L, D, stride, mode, nan):
     m.sparse_attention_fn = lambda *x: plain(*x)  # a function of the caller's own: the separate operators
     b = m(q, k, v, layer_idx=0)
     assert torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(torch.nan_to_num(a), torch.nan_to_num(b))
+
+
+def test_causal_rows_too_wide_for_one_launch():
+    """5800 blocks per row: scores, levels and sorting scratch of a row do not fit LDS together; the layer's second buffer changes nothing."""
+    import ctypes
+
+    from psa_hip import _lib, ops
+    from psa_hip._lib import check, lib
+
+    B, H, D, block, stride = 1, 1, 64, 64, 8
+    L = 5800 * block - 3
+    chunk = 128 * stride
+    q, k, v = (rnd(B, H, L, D, seed=i).to(dev()) for i in range(3))
+    items = list(RATIOS.items())
+    lv, hi = ops._level_items(items)
+    lo = (ctypes.c_double * len(items))(*[float(i[1][0]) for i in items])
+    shape = (B, H, H, L, D, block, stride, chunk)
+    ws = torch.empty(lib.psa_causal_layer_workspace_bytes(*shape), dtype=torch.uint8, device=dev())
+    extra = torch.empty(lib.psa_causal_layer_extra_bytes(*shape), dtype=torch.uint8, device=dev())
+    outs = []
+    for second in (None, extra.data_ptr()):
+        out = torch.empty_like(q)
+        check(lib.psa_causal_layer_fwd_extra(ops._t4(q), ops._t4(k), ops._t4(v), (ctypes.c_float * 3)(0.9, 0.9, 0.9), ws.data_ptr(), second,
+                                             ops._t4(out), *shape, D ** -0.5, _lib.PSA_MODE_TOPK, len(items), lv, lo, hi, 0, 1, ops._stream(q)),
+              "psa_causal_layer_fwd")
+        outs.append(out)
+    assert torch.equal(*outs)
