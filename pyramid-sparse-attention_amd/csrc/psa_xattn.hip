@@ -7,12 +7,16 @@
 //
 // A is a plain NT GEMM of Q' [Mr, S*D] (the S rows of a group concatenated in reverse order) with
 // K' [Nr, S*D] (K viewed with S rows per line), i.e. MFMA-bound: 2*Mr*Nr*S*D flops (half under causality).
-// Kernel 1: 256 (m) x 256 (n) output tiles, 8 waves of 64 (m) x 128 (n) (small launches: 128 x 128, see xattn_small); both operands go from global memory
-// straight into double-buffered LDS (global_load_lds_dwordx4, the padded + swizzled 64-row tile layout of
+// Kernel 1: 256 (m) x 256 (n) output tiles, 4 waves of 128 x 128 (small launches: 128 x 128 tiles, see xattn_small); both operands go
+// from global memory straight into double-buffered LDS (buffer_load_dwordx4 .. lds, the padded + swizzled 64-row tile layout of
 // psa_tiles.h) in stages of 64 contraction elements, i.e. half a head-dim row of one of the S interleaved
-// tokens; the transposed product (rows = n, lanes = m) makes the per-row reductions over n in-lane.  The tile
-// size is set by the copy path and LDS: a 256 x 256 tile needs 32 bytes of copies per CU cycle at the full MFMA
-// rate (the path delivers 64; a 128 x 128 tile would need all of it) and 0.75 LDS operand reads per MFMA.
+// tokens; the transposed product (rows = n, lanes = m) makes part of the reductions over n in-lane.  A 256 x 256 tile needs 32 bytes of
+// copies per CU cycle at the full MFMA rate (the path delivers 64; a 128 x 128 tile would need all of it).
+// What bounds it: MFMAs (0.57 of the cycles at 28 heads x 32768 tokens, stride 8) at the clock that the board's power leaves (1.85 GHz),
+// and the epilogue, 256 exponentials and about 1500 other vector instructions per lane and tile.  Before, 8 waves of 64 x 128 on 32 x 32 x 16
+// MFMAs read LDS as fast as it goes (0.375 operand reads per 16 x 16 x 32 MFMA, now 0.25), met at a barrier with nothing in registers, and a
+// tile began with its first copies: contraction 512 -> 435 us there (1.17 PFLOP/s with the tiles' padding); with the reduction
+// 12001 tokens 107 -> 85, 8192 48 -> 43, 2345 21.8 -> 16.6, 16 heads x 12000 67 -> 53, 12 x 1500, stride 16, 32 -> 21.5.
 // The epilogue reduces each (row m, key block J) to a pair
 // (local max, sum of exp2(z - local max)) in an fp32 workspace laid out [J][m] - the logits never
 // reach HBM.  Kernel 2 (HBM-bound): per row the global max and denominator from the pairs, then the
@@ -31,22 +35,20 @@ namespace {
 constexpr int KC = 64;                       // contraction chunk
 using XG = psa_tiles::LtGeom<KC>;            // LDS tiles: 64 rows of KC values
 constexpr int X_TILE = XG::TILE, X_ISTR = psa_tiles::LT_ISTR;
-// A workgroup's output tile: 64 * WM rows by 2 * 32 * NA keys, 2 * WM waves of 64 rows x 32 * NA keys.
-template <int WM_, int NA_>
+// A workgroup's output tile: 2 x 2 waves, each 16 * NC rows (m) x 16 * NA keys (n) in accumulators of 16 x 16.
+template <int NA_, int NC_, int PER_CU_>
 struct XTile {
-  static constexpr int WM = WM_, NA = NA_, NC = 2;                 // 32 x 32 accumulators per wave: NA along n, NC along m
-  static constexpr int TM = 64 * WM, TN = 64 * NA;
+  static constexpr int NA = NA_, NC = NC_, PER_CU = PER_CU_;       // PER_CU: workgroups per CU
+  static constexpr int TM = 32 * NC, TN = 32 * NA;
   static constexpr int QT = TM / 64, KT = TN / 64;                 // Q and K tiles per stage
   static constexpr int STAGE = (QT + KT) * X_TILE;                 // bytes per stage
-  static constexpr int WAVES = 2 * WM, GPW = (QT + KT) * 4 / WAVES;  // 16-row groups copied per wave
-  static_assert((QT + KT) * 4 % WAVES == 0 && NA % 2 == 0, "groups divide over the waves");
+  static constexpr int GPW = QT + KT;                              // 16-row groups copied per wave
+  static_assert(QT == KT && NA % 4 == 0 && NC % 4 == 0, "two waves copy Q, two K");
 };
-using XLarge = XTile<4, 4>;  // 256 x 256
-using XSmall = XTile<2, 2>;  // 128 x 128, two workgroups per CU
+using XLarge = XTile<8, 8, 1>;  // 256 x 256, 256 accumulator registers per lane, one wave per SIMD
+using XSmall = XTile<4, 4, 2>;  // 128 x 128
 constexpr int X_BUFS = 2;    // stages in LDS
-
-// rows past the end of Q / K are zero vectors: their copies read this page
-__device__ __align__(256) const unsigned char x_zero_page[256] = {};
+constexpr int X_CUS_PER_XCD = 32;
 
 struct XParams {
   const bf16_t *q, *k;
@@ -61,6 +63,7 @@ struct XParams {
   int out_rows, out_cols;
   float scale2;
   int tiles_m, tiles_n, act_per_bh, n_active, per_xcd;  // output tiles; those with visible keys per (batch, head) / in all / per XCD
+  int slots;  // workgroups per XCD
 };
 
 // output tiles of tile row tm that contain visible keys
@@ -80,14 +83,165 @@ struct PoolPart {
   int first, nx, heads;  // first workgroup; workgroups per (tensor, head); heads
 };
 
-template <int RBL, class X, bool POOL>  // RBL: log2 of the strided keys per block
-__global__ __launch_bounds__(X::WAVES * 64, X::WAVES == 8 ? 1 : 2) void psa_xattn_gemm_kernel(XParams p, PoolPart pool) {
-  constexpr int TM = X::TM, TN = X::TN, X_QT = X::QT, X_STAGE = X::STAGE, X_GPW = X::GPW, X_NA = X::NA, X_NC = X::NC;
+// 16 bytes per lane of the buffer `desc` at byte offset voff + soff into LDS at lds + off + 16 * lane (bytes past its records: zeros).
+__device__ __forceinline__ void lds_copy16_buffer(u32x4 desc, uint32_t voff, uint32_t soff, uint32_t lds, int off) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) desc[i] = __builtin_amdgcn_readfirstlane(desc[i]);
+  lds = __builtin_amdgcn_readfirstlane(lds);
+  soff = __builtin_amdgcn_readfirstlane(soff);
+  uint32_t at;
+  // (the offset in one vector register: the range check leaves a scalar one out)
+  asm volatile("s_add_u32 m0, %1, %5\n\tv_add_u32 %0, %2, %3\n\tbuffer_load_dwordx4 %0, %4, 0 offen lds"
+               : "=&v"(at)
+               : "s"(lds), "s"(soff), "v"(voff), "s"(desc), "i"(off)
+               : "memory", "scc", "m0");
+}
+// v_max3_f32 as such: of fmaxf the compiler makes the NaNs of an MFMA's results canonical first, an instruction per value
+__device__ __forceinline__ float max3_raw(float a, float b, float c) {
+  float r;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+
+// a of the lanes' own and of the neighbouring 16 lanes, b likewise: the even 16-lane rows return max / sum for a, the odd ones for b
+template <bool SUM>
+__device__ __forceinline__ float pair16(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
+  const uint32_t r0 = r[0], r1 = r[1];  // r0 = rows (a0, b0, a2, b2), r1 = (a1, b1, a3, b3)
+  const float x = __builtin_bit_cast(float, r0), y = __builtin_bit_cast(float, r1);
+  return SUM ? x + y : fmaxf(x, y);
+}
+// ... between the half-waves: lanes 0 - 31 return it for a, lanes 32 - 63 for b
+template <bool SUM>
+__device__ __forceinline__ float pair32(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
+  const uint32_t r0 = r[0], r1 = r[1];
+  const float x = __builtin_bit_cast(float, r0), y = __builtin_bit_cast(float, r1);
+  return SUM ? x + y : fmaxf(x, y);
+}
+// even: the even 16-lane row of each half-wave in both of its rows; odd: the odd one
+__device__ __forceinline__ void spread16(float v, float& even, float& odd) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, v);
+  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  const uint32_t r0 = r[0], r1 = r[1];
+  even = __builtin_bit_cast(float, r0);
+  odd = __builtin_bit_cast(float, r1);
+}
+
+// Pairs (maximum, sum of exp2(z - maximum)) of a wave's rows m0w .. and key blocks n0w .., from its accumulators:
+// acc[a][c][i] = logit of key n0w + 16 a + 4 lg + i and row m0w + 16 c + l16.  Four pairs at a time, so that after the exchanges every
+// 16-lane row holds a pair of its own to store.  MASK: some key is not visible.  Both variants and both tiles give the same bits.
+template <int RBL, class X, bool MASK>
+__device__ __forceinline__ void xattn_pairs(f32x4 (&acc)[X::NA][X::NC], float* ws, int Mr, int m0w, int n0w, int off, float scale2, int lane) {
+  const int l16 = lane & 15, lg = lane >> 4;
+  constexpr int KP = RBL == 3 ? X::NA : (16 * X::NA) >> (RBL + 1);  // groups of four pairs per two row blocks
+#pragma unroll
+  for (int cp = 0; cp < X::NC / 2; ++cp) {
+#pragma unroll
+    for (int kp = 0; kp < KP; ++kp) {
+      // the four lists of logits that are reduced together: RBL 3: key blocks of accumulators (a, a + 1) of one row block, two per
+      // accumulator; else key blocks (2 kp, 2 kp + 1) of two row blocks
+      constexpr int GB = RBL == 3 ? 1 : 1 << (RBL - 4), NE = RBL == 3 ? 2 : 4;  // accumulators per list, lists
+      float z[NE][4 * GB], mx[NE];
+#pragma unroll
+      for (int e = 0; e < NE; ++e) {
+        const int c = RBL == 3 ? 2 * cp + (kp & 1) : 2 * cp + (e >> 1);
+        const int m = m0w + 16 * c + l16;
+#pragma unroll
+        for (int g = 0; g < GB; ++g) {
+          const int a = RBL == 3 ? 2 * (kp >> 1) + e : (2 * kp + (e & 1)) * GB + g;
+          if constexpr (X::PER_CU == 1) asm volatile("" : "+a"(acc[a][c]));  // (read here: ahead of the branch between the variants all of them would not fit)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            z[e][4 * g + i] = !MASK || n0w + 16 * a + 4 * lg + i <= m + off ? acc[a][c][i] : -INFINITY;
+          }
+        }
+        mx[e] = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < 4 * GB; i += 2) mx[e] = max3_raw(z[e][i], z[e][i + 1], mx[e]);
+      }
+      float top, ref[NE];
+      if constexpr (RBL == 3) {
+        top = pair16<false>(mx[0], mx[1]);
+      } else {
+        top = pair32<false>(pair16<false>(mx[0], mx[1]), pair16<false>(mx[2], mx[3]));
+      }
+      top *= scale2;
+      const float r = top == -INFINITY ? 0.f : -top;
+      if constexpr (RBL == 3) {
+        spread16(r, ref[0], ref[1]);
+      } else {
+        float lo, hi;
+        half_wave_swap(r, lo, hi);
+        spread16(lo, ref[0], ref[1]);
+        spread16(hi, ref[2], ref[3]);
+      }
+      float sm[NE];
+#pragma unroll
+      for (int e = 0; e < NE; ++e) {
+        sm[e] = fast_exp2(__builtin_fmaf(z[e][0], scale2, ref[e]));
+#pragma unroll
+        for (int i = 1; i < 4 * GB; ++i) sm[e] += fast_exp2(__builtin_fmaf(z[e][i], scale2, ref[e]));  // (fused in words: the same bits whatever the variant)
+      }
+      f32x2 pr;
+      pr[0] = top;
+      int J, c;
+      if constexpr (RBL == 3) {
+        pr[1] = pair16<true>(sm[0], sm[1]);
+        J = (n0w >> 3) + 2 * (2 * (kp >> 1) + (lg & 1)) + (lg >> 1);
+        c = 2 * cp + (kp & 1);
+      } else {
+        pr[1] = pair32<true>(pair16<true>(sm[0], sm[1]), pair16<true>(sm[2], sm[3]));
+        J = (n0w >> RBL) + 2 * kp + (lg & 1);
+        c = 2 * cp + (lg >> 1);
+      }
+      *(f32x2*)(ws + ((int64_t)J * Mr + m0w + 16 * c + l16) * 2) = pr;
+      if (X::PER_CU == 1 && (kp & 1)) __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+}
+
+// acc += a * b.  With 256 accumulator registers per lane the compiler has no spare one, and moves accumulators about between
+// the MFMAs (about every second one, with the waits that go with it): there the instruction is written with its accumulator in place.
+// What the compiler does not know then: nothing but these MFMAs may touch an accumulator between xattn_mfma_begin and _end.
+template <class X>
+__device__ __forceinline__ void xattn_mfma(f32x4& acc, const bf16x8& a, const bf16x8& b) {
+  if constexpr (X::PER_CU > 1) acc = EtBf16::mfma16(a, b, acc);
+  else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
+}
+// Zeroes the accumulators; the MFMAs may read them behind this.  (A first k-step of its own, without the zeros, spills.)
+template <class X>
+__device__ __forceinline__ void xattn_mfma_begin(f32x4 (&acc)[X::NA][X::NC]) {
+#pragma unroll
+  for (int a = 0; a < X::NA; ++a)
+#pragma unroll
+    for (int c = 0; c < X::NC; ++c) {
+      acc[a][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if constexpr (X::PER_CU == 1) asm volatile("" : "+a"(acc[a][c]));
+    }
+  if constexpr (X::PER_CU == 1) asm volatile("s_nop 7");
+}
+// The results may be read behind this: the last MFMA (4 passes) has been over for long.
+template <class X>
+__device__ __forceinline__ void xattn_mfma_end(f32x4 (&acc)[X::NA][X::NC]) {
+  asm volatile("s_nop 15\n\ts_nop 15");
+#pragma unroll
+  for (int a = 0; a < X::NA; ++a)
+#pragma unroll
+    for (int c = 0; c < X::NC; ++c) {
+      if constexpr (X::PER_CU == 1) asm volatile("" : "+a"(acc[a][c]));
+      else asm volatile("" : "+v"(acc[a][c]));
+    }
+}
+// RBL: log2 of the strided keys per block; ROWS: rows of Q or K overlap in memory (strides below the head dim)
+template <int RBL, class X, bool POOL, bool ROWS>
+__global__ __launch_bounds__(256, X::PER_CU) void psa_xattn_gemm_kernel(XParams p, PoolPart pool) {
+  constexpr int TM = X::TM, TN = X::TN, X_QT = X::QT, X_STAGE = X::STAGE, GPW = X::GPW, NA = X::NA, NC = X::NC;
   extern __shared__ __align__(16) unsigned char smem[];  // X_BUFS stages of [Q tiles | K tiles]
   // Workgroup ids go round-robin over the 8 XCDs and every XCD runs its ids in order.  The output tiles with
   // visible keys are listed (batch-head, tile row, tile column) and the list is cut into 8 contiguous shares, one
   // per XCD: all tiles cost the same, so the XCDs finish together, and the ~32 tiles an XCD works on at a time
-  // are neighbours that find each other's Q and K rows in its L2.
+  // are neighbours that find each other's Q and K rows in its L2.  Workgroup `slot` of an XCD takes tiles slot, slot + slots, ..
   if constexpr (POOL) {
     if ((int)blockIdx.x >= pool.first) {
       const int u = (int)blockIdx.x - pool.first, w = u / pool.nx;
@@ -95,151 +249,177 @@ __global__ __launch_bounds__(X::WAVES * 64, X::WAVES == 8 ? 1 : 2) void psa_xatt
       return;
     }
   }
-  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-  const int idx = xcd * p.per_xcd + slot;
-  if (idx >= p.n_active) return;
-  const int bh = idx / p.act_per_bh;
-  int tn = idx % p.act_per_bh, tm = 0;
-  for (;; ++tm) {
-    const int row_n = tiles_in_row<X>(tm, p.tiles_n, p.causal, p.off);
-    if (tn < row_n) break;
-    tn -= row_n;
-  }
-  const int m0 = tm * TM, n0 = tn * TN;
-  const int h = bh % p.Hq, b = bh / p.Hq;
-  const int hk = h / (p.Hq / p.Hkv);
+  const int xcd = blockIdx.x & 7, share0 = xcd * p.per_xcd;
+  int share1 = share0 + p.per_xcd;
+  share1 = share1 < p.n_active ? share1 : p.n_active;
+  int idx = share0 + (int)(blockIdx.x >> 3);
+  if (idx >= share1) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int l32 = lane & 31, hh = lane >> 5;
-  const int wn = wave & 1, wm = wave >> 1;  // wave tile: rows m0 + 64 * wm .., keys n0 + 32 * NA * wn ..
+  const int l16 = lane & 15, lg = lane >> 4;
+  const int wn = wave & 1, wm = wave >> 1;  // wave tile: rows m0 + 16 * NC * wm .., keys n0 + 16 * NA * wn ..
   const int S = 1 << p.S_log2;
-
-  const char* qb = (const char*)(p.q + b * p.q_sb + h * p.q_sh);
-  const char* kb = (const char*)(p.k + b * p.k_sb + hk * p.k_sh);
-  const uint32_t q_strb = (uint32_t)p.q_sl * 2u, k_strb = (uint32_t)p.k_sl * 2u;
   const int dc_log2 = p.D == 2 * KC ? 1 : 0;  // 64-channel chunks per row: 1 (D = 64) or 2 (D = 128)
-  const int stages = S << dc_log2;
+  const int real_stages = S << dc_log2, stages = real_stages < 2 ? 2 : real_stages;  // (a second one of zeros: a tile spans both buffers)
 
-  // copies: wave w moves the 16-row groups w*X_GPW .. of a stage (group g: tile g/4, rows 16*(g%4)..), a lane
-  // the RPL consecutive rows frow.. of each group; a row is one strided index (S tokens apart in memory)
+  // copies: waves 0, 1 move the Q rows of a stage, waves 2, 3 the K rows: GPW groups of 16 rows, of which a lane fetches the RPL
+  // consecutive ones from frow on; a row is one strided index (S tokens apart in memory).  They go through a buffer descriptor of the
+  // (batch, head) slice, whose range check answers rows past the real length with zeros: every tile takes the same path, and a copy is a
+  // scalar and a vector instruction beside the load.
   constexpr int RPL = XG::RPL;
+  const bool is_q = wave < 2;
   const uint32_t f_chunk = psa_tiles::lt_fetch_chunk<KC>(lane);
   const int frow = psa_tiles::lt_fetch_row<KC>(lane);
-  int g_idx[X_GPW];       // strided index (m or n) of the lane's first row of each group
-  uint32_t g_off[X_GPW];  // its byte offset inside the (batch, head) slice, token 0 of the S, contraction chunk 0
-  bool edge = false;      // some row of this tile reaches past the real length: take the checked path
-#pragma unroll
-  for (int j = 0; j < X_GPW; ++j) {
-    const int g = wave * X_GPW + j, tile = g >> 2;
-    const bool is_q = tile < X_QT;
-    const int idx = (is_q ? m0 + tile * 64 : n0 + (tile - X_QT) * 64) + (g & 3) * 16 + frow;
-    g_idx[j] = idx;
-    g_off[j] = ((uint32_t)idx << p.S_log2) * (is_q ? q_strb : k_strb) + f_chunk;
-  }
-  edge = ((int64_t)(m0 + TM) << p.S_log2) > p.Lq || ((int64_t)(n0 + TN) << p.S_log2) > p.Lk;  // (covers tiles that stick out of Mr / Nr)
-  // copies of stage st; EDGE: rows past the real length read the page of zeros (decided once per workgroup: a test per copy
-  // is a branch per copy)
-  auto issue_stage = [&](int st, auto edge_c) __attribute__((always_inline)) {
-    constexpr bool EDGE = decltype(edge_c)::value;
-    const int i = st >> dc_log2, dc = st & ((1 << dc_log2) - 1);  // (shifts: a division here would run on the vector unit and take the base pointers with it)
-    unsigned char* dst = smem + (st & 1) * X_STAGE;
-#pragma unroll
-    for (int j = 0; j < X_GPW; ++j) {
-      const int g = wave * X_GPW + j, tile = g >> 2;
-      const bool is_q = tile < X_QT;
-      // token S-1-i of every query group, token i of every key group
-      const char* base = is_q ? qb + (uint64_t)(S - 1 - i) * q_strb + dc * (KC * 2) : kb + (uint64_t)i * k_strb + dc * (KC * 2);
-      const uint32_t rstr = (is_q ? q_strb : k_strb) << p.S_log2;
-#pragma unroll
-      for (int n = 0; n < RPL; ++n) {
-        const uint32_t lds = psa_tiles::lds_addr_of(dst + tile * X_TILE + ((g & 3) * RPL + n) * X_ISTR);
-        if constexpr (!EDGE) {
-          psa_tiles::lds_copy16(base, g_off[j] + n * rstr, lds);
-        } else {
-          const int64_t tok = ((int64_t)(g_idx[j] + n) << p.S_log2) + (is_q ? S - 1 - i : i);
-          const bool real = tok < (is_q ? p.Lq : p.Lk);
-          const char* src = real ? base + (g_off[j] + n * rstr) : (const char*)x_zero_page + f_chunk;
-          psa_tiles::lds_copy16_addr(src, lds);
-        }
-      }
+  const uint32_t strb = (uint32_t)(is_q ? p.q_sl : p.k_sl) * 2u, rstr = strb << p.S_log2;
+  const int limit = is_q ? p.Lq : p.Lk;
+  const uint32_t slice_bytes = (uint32_t)(limit - 1) * strb + (uint32_t)p.D * 2u;
+  const uint32_t dst0 = psa_tiles::lds_addr_of(smem) + wave * GPW * XG::GROUP;  // (the tiles of a stage follow each other without a gap)
+
+  // a tile, and what this wave's copies of it need
+  struct Tile {
+    int bh, m0, n0;
+    u32x4 desc;     // the slice of Q or K; no records: nothing to copy
+    uint32_t voff;  // byte offset of the lane's first row, token 0 of the S, contraction chunk 0
+    int row0;       // its strided index (ROWS)
+  };
+  auto locate = [&](int at) __attribute__((always_inline)) {
+    Tile t;
+    t.bh = at / p.act_per_bh;
+    int tn = at % p.act_per_bh, tm = 0;
+    for (;; ++tm) {
+      const int row_n = tiles_in_row<X>(tm, p.tiles_n, p.causal, p.off);
+      if (tn < row_n) break;
+      tn -= row_n;
+    }
+    t.m0 = tm * TM;
+    t.n0 = tn * TN;
+    const int h = t.bh % p.Hq, b = t.bh / p.Hq;
+    const char* slice = is_q ? (const char*)(p.q + b * p.q_sb + h * p.q_sh) : (const char*)(p.k + b * p.k_sb + (h / (p.Hq / p.Hkv)) * p.k_sh);
+    const uint64_t a = (uint64_t)(uintptr_t)psa_tiles::uniform_ptr(slice);
+    t.desc = u32x4{(uint32_t)a, (uint32_t)(a >> 32) & 0xffffu, slice_bytes, 0x00020000u};  // raw buffer, no stride, 32-bit data format
+    t.row0 = (is_q ? t.m0 : t.n0) + (wave & 1) * (GPW * 16) + frow;
+    t.voff = ((uint32_t)t.row0 << p.S_log2) * strb + f_chunk;
+    return t;
+  };
+  // what the copies of one stage need, in scalar registers but for the lane's part
+  struct Cursor {
+    u32x4 desc;
+    uint32_t voff, soff, lds;
+    int row0, tok0;
+  };
+  auto cursor = [&](const u32x4& desc, uint32_t voff, int row0, int st) __attribute__((always_inline)) {
+    st = __builtin_amdgcn_readfirstlane(st);
+    const int i = st >> dc_log2, dc = st & ((1 << dc_log2) - 1);
+    Cursor c;
+    c.tok0 = is_q ? S - 1 - i : i;  // token S-1-i of every query group, token i of every key group
+    c.soff = __builtin_amdgcn_readfirstlane((uint32_t)c.tok0 * strb + (uint32_t)(dc * (KC * 2)));
+    c.lds = __builtin_amdgcn_readfirstlane(dst0 + (st & 1) * X_STAGE);
+    c.voff = voff;
+    c.row0 = row0;
+    uint32_t d0 = __builtin_amdgcn_readfirstlane(desc[0]), d1 = __builtin_amdgcn_readfirstlane(desc[1]);
+    uint32_t d2 = __builtin_amdgcn_readfirstlane(st < real_stages ? desc[2] : 0u), d3 = desc[3];
+    // (a scalar register that the vector unit wrote may be read by a load five cycles later; the compiler does not see the loads)
+    asm volatile("s_nop 4" : "+s"(d0), "+s"(d1), "+s"(d2), "+s"(d3));
+    c.desc = u32x4{d0, d1, d2, d3};
+    return c;
+  };
+  const uint32_t rstep = __builtin_amdgcn_readfirstlane(rstr);
+  auto copy = [&](const Cursor& t, int u) __attribute__((always_inline)) {  // u of GPW * RPL
+    const int row = 16 * (u / RPL) + u % RPL;
+    if constexpr (!ROWS) {
+      lds_copy16_buffer(t.desc, t.voff, t.soff + (uint32_t)row * rstep, t.lds, u * X_ISTR);
+    } else {
+      // (token by token: the byte after a row may belong to the next)
+      const bool real = ((int64_t)(t.row0 + row) << p.S_log2) + t.tok0 < limit;
+      lds_copy16_buffer(t.desc, real ? t.voff + t.soff + (uint32_t)row * rstep : 0xfffffff0u, 0, t.lds, u * X_ISTR);
     }
   };
-  // operands: K rows (A) of tile wn, Q rows (B) of tile wm; rows l32 and l32 + 32; k-step ks: off[ks & 1] + 64 * (ks >> 1)
-  uint32_t r_off[2];
-  psa_tiles::lt_row_operand<KC>(l32, hh, r_off);
+  const uint32_t r_off = psa_tiles::lt_row_operand16<KC>(l16, lg);
+  PSA_LDS(const unsigned char) const Qs = (PSA_LDS(const unsigned char))(smem) + wm * NC * XG::GROUP + r_off;
+  PSA_LDS(const unsigned char) const Ks = (PSA_LDS(const unsigned char))(smem) + X_QT * X_TILE + wn * NA * XG::GROUP + r_off;
 
-  f32x16 acc[X_NA][X_NC];
+  // Operands of the k-step at hand and of the next one.  A k-step (32 channels) is NA * NC MFMAs; the next one's operands are read and,
+  // in the second k-step of a stage, the copies of the stage after the next issued between them.  The barrier lies between the k-steps of a
+  // stage: what the MFMAs behind it need is in registers, and the buffer whose last operands were read before it can be filled.
+  // The next k-step's operands are read into registers of their own, but for the first six K ones: theirs are free once the MFMAs
+  // of the operand are issued, and what is read last has to be there at the barrier.
+  constexpr int NA_IN = NA - 2;  // K operands that are replaced in place
+  f32x4 acc[NA][NC];
+  bf16x8 bq[2][NC], ak[NA_IN], al[2][2];
+  auto read_q = [&](int st, int kk, int c) __attribute__((always_inline)) {
+    bq[kk][c] = *(PSA_LDS(const bf16x8))(Qs + (st & 1) * X_STAGE + c * XG::GROUP + kk * 64);
+  };
+  auto read_k = [&](int st, int kk, int a) __attribute__((always_inline)) {
+    const bf16x8 v = *(PSA_LDS(const bf16x8))(Ks + (st & 1) * X_STAGE + a * XG::GROUP + kk * 64);
+    if (a < NA_IN) ak[a] = v;
+    else al[kk][a - NA_IN] = v;
+  };
+  // MFMAs of k-step kk, one K operand after the other, and between them, one at a time so that the matrix pipe does not run dry, the reads
+  // of the next k-step's operands (stage st_r) and the copies at t.  (One body for every stage: accumulators that several
+  // variants of a step hand on are moved from register to register, and spilled.)
+  auto step = [&](auto kk_c, int st_r, const Cursor& t) __attribute__((always_inline)) {
+    constexpr int KK = decltype(kk_c)::value, NX = NA * NC, NCP = GPW * RPL, NR = NC + 2;
+    constexpr int CPS = NX / NCP;  // MFMAs per copy
+    static_assert(CPS >= 2, "copies fit");
 #pragma unroll
-  for (int a = 0; a < X_NA; ++a)
-#pragma unroll
-    for (int c = 0; c < X_NC; ++c)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[a][c][i] = 0.f;
-
-  auto contract = [&](auto edge_c) __attribute__((always_inline)) {
-    issue_stage(0, edge_c);
-    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
-    __syncthreads();
-    for (int st = 0; st < stages; ++st) {
-      // invariant: buffer st&1 holds stage st and every wave is done with the other buffer
-      if (st + 1 < stages) issue_stage(st + 1, edge_c);
-      PSA_LDS(const unsigned char) Qs = (PSA_LDS(const unsigned char))(smem) + (st & 1) * X_STAGE + wm * X_TILE;
-      PSA_LDS(const unsigned char) Ks = (PSA_LDS(const unsigned char))(smem) + (st & 1) * X_STAGE + (X_QT + wn * (X_NA / 2)) * X_TILE;
-#pragma unroll
-      for (int ks = 0; ks < KC / 16; ++ks) {
-        bf16x8 af[X_NA], bf[X_NC];
-        const uint32_t o = r_off[ks & 1] + (ks >> 1) * 64;
-#pragma unroll
-        for (int a = 0; a < X_NA; ++a) af[a] = *(PSA_LDS(const bf16x8))(Ks + o + (a >> 1) * X_TILE + (a & 1) * XG::HALF);
-#pragma unroll
-        for (int c = 0; c < X_NC; ++c) bf[c] = *(PSA_LDS(const bf16x8))(Qs + o + c * XG::HALF);
-#pragma unroll
-        for (int a = 0; a < X_NA; ++a)
-#pragma unroll
-          for (int c = 0; c < X_NC; ++c) acc[a][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[a], bf[c], acc[a][c], 0, 0, 0);
+    for (int x = 0; x < NX; ++x) {
+      const int a = x / NC, c = x % NC;
+      xattn_mfma<X>(acc[a][c], a < NA_IN ? ak[a] : al[KK][a - NA_IN], bq[KK][c]);
+      // even MFMAs: Q operands and the last two K operands; the last MFMA of an operand: its successor
+      if (x % 2 == 0 && x / 2 < NR) {
+        if (x / 2 < NC) read_q(st_r, KK ^ 1, x / 2);
+        else read_k(st_r, KK ^ 1, NA_IN + x / 2 - NC);
       }
-      __builtin_amdgcn_s_waitcnt(0x0f70);  // the copies of stage st+1 were issued a stage ago
+      if (c == NC - 1 && a < NA_IN) read_k(st_r, KK ^ 1, a);
+      if (KK == 1 && x % CPS == 1) copy(t, x / CPS);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
+  Tile cur = locate(idx);
+#pragma unroll
+  for (int st = 0; st < 2; ++st) {
+    const Cursor c = cursor(cur.desc, cur.voff, cur.row0, st);
+#pragma unroll
+    for (int u = 0; u < GPW * RPL; ++u) copy(c, u);
+  }
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < NC; ++c) read_q(0, 0, c);
+#pragma unroll
+  for (int a = 0; a < NA; ++a) read_k(0, 0, a);
+  for (;;) {
+    // the first two stages of the next tile are copied in the last two of this one, and the operands of its first k-step read in the last
+    // k-step: it begins with all that it needs (behind the last tile: zeros, that nothing uses)
+    idx += p.slots;
+    const bool more = idx < share1;
+    Tile next = cur;
+    if (more) next = locate(idx);
+    else next.desc[2] = 0;
+    xattn_mfma_begin<X>(acc);
+    int st = 0;
+    do {
+      const bool here = st + 2 < stages;
+      u32x4 desc;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) desc[i] = here ? cur.desc[i] : next.desc[i];
+      const Cursor ahead = cursor(desc, here ? cur.voff : next.voff, here ? cur.row0 : next.row0, here ? st + 2 : st + 2 - stages);
+      step(std::integral_constant<int, 0>{}, st, ahead);
+      __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the copies of stage st+1 were issued a stage ago
       __syncthreads();
+      step(std::integral_constant<int, 1>{}, st + 1, ahead);
+    } while (++st < stages);
+    xattn_mfma_end<X>(acc);
+    const int m0w = cur.m0 + wm * (16 * NC), n0w = cur.n0 + wn * (16 * NA);
+    float* const ws = p.ws + (int64_t)cur.bh * p.NB * p.Mr * 2;
+    if (m0w < p.Mr && n0w < p.Nr) {  // (Mr and Nr are multiples of 128)
+      if (p.causal && n0w + 16 * NA - 1 > m0w + p.off) xattn_pairs<RBL, X, true>(acc, ws, p.Mr, m0w, n0w, p.off, p.scale2, lane);
+      else xattn_pairs<RBL, X, false>(acc, ws, p.Mr, m0w, n0w, p.off, p.scale2, lane);
     }
-  };
-  if (edge) contract(std::true_type{});
-  else contract(std::false_type{});
-
-  // epilogue: accumulator (a, c): rows n = n0 + wn * TN / 2 + a*32 + (i/4)*8 + hh*4 + i%4, column m = m0 + wm*64 + c*32 + l32
-  constexpr int OPB = 1 << (RBL - 3);  // 8-key octets per block: 1, 2 or 4
-  float* ws = p.ws + (int64_t)bh * p.NB * p.Mr * 2;
-#pragma unroll
-  for (int c = 0; c < X_NC; ++c) {
-    const int m = m0 + wm * 64 + c * 32 + l32;
-    const int nlim = p.causal ? m + p.off : 0x7fffffff;  // visible keys: n <= nlim
-#pragma unroll
-    for (int a = 0; a < X_NA; ++a) {
-      const int nb0 = n0 + wn * (TN / 2) + a * 32;
-      float z[16];
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int n = nb0 + (i >> 2) * 8 + hh * 4 + (i & 3);
-        z[i] = n <= nlim ? acc[a][c][i] * p.scale2 : -INFINITY;
-      }
-      // an octet of 8 consecutive keys = registers 4o..4o+3 of both half-waves; OPB octets form a block
-#pragma unroll
-      for (int blk = 0; blk < 4 / OPB; ++blk) {
-        float mx = -INFINITY;
-#pragma unroll
-        for (int i = 0; i < 4 * OPB; ++i) mx = fmaxf(mx, z[blk * 4 * OPB + i]);
-        mx = half_wave_max(mx);
-        const float ref = mx == -INFINITY ? 0.f : mx;
-        float sm = 0.f;
-#pragma unroll
-        for (int i = 0; i < 4 * OPB; ++i) sm += fast_exp2(z[blk * 4 * OPB + i] - ref);
-        sm = half_wave_sum(sm);
-        if (hh == 0 && m < p.Mr && nb0 < p.Nr) {
-          const int J = (nb0 + blk * 8 * OPB) >> RBL;
-          f32x2 pr = {mx, sm};
-          *(f32x2*)(ws + ((int64_t)J * p.Mr + m) * 2) = pr;
-        }
-      }
-    }
+    if (!more) break;
+    cur = next;
   }
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // no copy outlives the workgroup's LDS
 }
 
 // one workgroup per (b, h, q-block): 256 threads; thread t handles key blocks t, t+256, ...
@@ -367,12 +547,13 @@ int active_tiles(XParams& p, int rows_used) {
   for (int tm = 0; tm < p.tiles_m; ++tm) n += tiles_in_row<X>(tm, p.tiles_n, p.causal, p.off);
   return n;
 }
-// Output tile of the launch.  A 128 x 128 tile is a quarter of the products at three quarters of the rate of a 256 x 256 one
-// (copies and LDS operands per product): it pays where the large tiles leave CUs idle, i.e. by rounds of the chip (256 large
-// tiles, 512 small ones; a round of small ones takes 0.65 of a round of large ones).  Contraction + reduction, 28 heads, stride 8,
-// large / small in us: 2345 tokens 37 / 22, 6000 40 / 42, 8192 69 / 50, 16384 154 / 168, 32768 599 / 702.
+// Output tile of the launch.  A 128 x 128 tile is a quarter of the products at five sixths of the rate of a 256 x 256 one or less
+// (copies and LDS operands per product): it pays where the large tiles leave CUs idle.  Large tiles cost by rounds of the chip (256), small
+// ones, two workgroups per CU that end one by one, 0.6 of that per 512 and half a round for the end.  Contraction + reduction, 28 heads,
+// stride 8, large / small in us: 2345 tokens 32 / 16.5, 6000 35 / 35, 8192 62 / 42, 12001 92 / 85, 16384 126 / 137, 32768 490 / 611; 16 heads x 12000
+// 62 / 52.
 bool xattn_small(int64_t n_large, int64_t n_small) {
-  return (n_small + 511) / 512 * 13 < (n_large + 255) / 256 * 20;
+  return (n_small + 256) * 3 < (n_large + 255) / 256 * 2560;
 }
 
 struct XGeom {
@@ -430,6 +611,8 @@ static int xattn_run(psa_tensor4 q, psa_tensor4 k, float* est, void* workspace, 
   p.q = (const bf16_t*)q.ptr; p.k = (const bf16_t*)k.ptr;
   p.q_sb = q.stride_b; p.q_sh = q.stride_h; p.q_sl = q.stride_l;
   p.k_sb = k.stride_b; p.k_sh = k.stride_h; p.k_sl = k.stride_l;
+  if (Lq == 1) p.q_sl = D;  // (a single row's stride may be anything, and says where the padding begins)
+  if (Lk == 1) p.k_sl = D;
   p.ws = (float*)workspace; p.est = est;
   p.Hq = Hq; p.Hkv = Hkv; p.Lq = Lq; p.Lk = Lk; p.D = D;
   p.S_log2 = psa_ilog2(stride); p.rb_log2 = psa_ilog2(rb);
@@ -446,7 +629,9 @@ static int xattn_run(psa_tensor4 q, psa_tensor4 k, float* est, void* workspace, 
   // (every pair that the reduction reads is written: the tile rows end with the last q-block's, the rest is padding)
   const int rows_used = p.out_rows * rb < g.Mr ? p.out_rows * rb : g.Mr;
   const int64_t n_large = heads * active_tiles<XLarge>(p, rows_used), n_small = heads * active_tiles<XSmall>(p, rows_used);
-  const bool small = xattn_small(n_large, n_small);
+  // rows that overlap (expanded tensors) take the kernel that checks every row, which has small tiles only
+  const bool overlap = (Lq > 1 && q.stride_l < D) || (Lk > 1 && k.stride_l < D);
+  const bool small = overlap || xattn_small(n_large, n_small);
   const int64_t n_active = small ? n_small : n_large;
   PSA_REQUIRE(n_active < (1ll << 28), PSA_ERR_UNSUPPORTED, "psa_estimate_xattn: too many output tiles");
   p.n_active = (int)n_active;
@@ -454,23 +639,31 @@ static int xattn_run(psa_tensor4 q, psa_tensor4 k, float* est, void* workspace, 
   PoolPart pool = {};
   auto launch = [&](auto x) -> int {
     using X = decltype(x);
-    constexpr bool CAN_POOL = X::WAVES * 64 == 256;  // (the pooling pass is written for 256 threads)
+    constexpr bool SMALL = std::is_same_v<X, XSmall>;
     p.act_per_bh = active_tiles<X>(p, rows_used);
     const size_t shmem = X_BUFS * (size_t)X::STAGE;
-    auto kern = rb == 8 ? psa_xattn_gemm_kernel<3, X, false> : rb == 16 ? psa_xattn_gemm_kernel<4, X, false> : psa_xattn_gemm_kernel<5, X, false>;
-    int64_t blocks = (int64_t)p.per_xcd * 8;
-    if constexpr (CAN_POOL) {
+    auto pick = [&](auto pool_c, auto rows_c) {
+      constexpr bool P = decltype(pool_c)::value, R = decltype(rows_c)::value;
+      return rb == 8 ? psa_xattn_gemm_kernel<3, X, P, R> : rb == 16 ? psa_xattn_gemm_kernel<4, X, P, R> : psa_xattn_gemm_kernel<5, X, P, R>;
+    };
+    auto kern = pick(std::false_type{}, std::false_type{});
+    // large tiles: one workgroup per CU, which takes a tile after the other and copies ahead; small ones: one each
+    p.slots = SMALL || p.per_xcd < X_CUS_PER_XCD ? p.per_xcd : X_CUS_PER_XCD;
+    int64_t blocks = (int64_t)p.slots * 8;
+    if constexpr (SMALL) {
       if (xm != nullptr && xm->pool != nullptr) {
-        kern = rb == 8 ? psa_xattn_gemm_kernel<3, X, true> : rb == 16 ? psa_xattn_gemm_kernel<4, X, true> : psa_xattn_gemm_kernel<5, X, true>;
+        kern = overlap ? pick(std::true_type{}, std::true_type{}) : pick(std::true_type{}, std::false_type{});
         pool.p = *xm->pool;
         pool.first = (int)blocks;
         pool.nx = xm->pool_nx;
         pool.heads = xm->pool_heads;
         blocks += (int64_t)xm->pool_nx * xm->pool_heads * 2;
+      } else if (overlap) {
+        kern = pick(std::false_type{}, std::true_type{});
       }
     }
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem) != hipSuccess) return PSA_ERR_LAUNCH;
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(X::WAVES * 64), shmem, st, p, pool);
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), shmem, st, p, pool);
     return PSA_OK;
   };
   if (!small && xm != nullptr && xm->pool != nullptr) psa_pool_launch_cap(*xm->pool, xm->pool_nx, xm->pool_heads, st);

@@ -47,3 +47,12 @@ def test_forward_kernels_do_not_spill(kernel, instances, tmp_path):
     assert len(found) == instances, sorted(found)
     spilled = {n: m for n, m in found.items() if any(int(m[c]) for c in ("vgpr_spill_count", "sgpr_spill_count", "private_segment_fixed_size"))}
     assert not spilled, spilled
+
+
+@pytest.mark.skipif(READELF is None, reason="llvm-readelf of the ROCm toolchain not found")
+def test_the_contraction_keeps_its_accumulators(tmp_path):
+    """The MFMAs of its large tile are written with their accumulators in place: nothing else may move them in between."""
+    found = {n: m for n, m in _kernels(tmp_path).items() if "psa_xattn_gemm_kernel" in n}
+    assert len(found) == 15, sorted(found)
+    spilled = {n: m for n, m in found.items() if any(int(m[c]) for c in ("vgpr_spill_count", "sgpr_spill_count", "private_segment_fixed_size"))}
+    assert not spilled, spilled
