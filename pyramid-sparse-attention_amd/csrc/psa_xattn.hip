@@ -13,10 +13,13 @@
 // tokens; the transposed product (rows = n, lanes = m) makes part of the reductions over n in-lane.  A 256 x 256 tile needs 32 bytes of
 // copies per CU cycle at the full MFMA rate (the path delivers 64; a 128 x 128 tile would need all of it).
 // What bounds it: MFMAs (0.57 of the cycles at 28 heads x 32768 tokens, stride 8) at the clock that the board's power leaves (1.85 GHz),
-// and the epilogue, 256 exponentials and about 1500 other vector instructions per lane and tile.  Before, 8 waves of 64 x 128 on 32 x 32 x 16
-// MFMAs read LDS as fast as it goes (0.375 operand reads per 16 x 16 x 32 MFMA, now 0.25), met at a barrier with nothing in registers, and a
-// tile began with its first copies: contraction 512 -> 435 us there (1.17 PFLOP/s with the tiles' padding); with the reduction
+// the epilogue, 256 exponentials and about 1500 other vector instructions per lane and tile with nothing beside them (a fifth of a
+// tile), and copies that are still in flight at a stage's barrier (a seventh).  A wave of 128 x 128 reads 0.25 operands from LDS per MFMA; the 8
+// waves of 64 x 128 before it read 0.375, met at a barrier with no operand in registers (0.48 of the cycles), and each tile began
+// with its first copies: contraction 512 -> 435 us there (1.17 PFLOP/s with the tiles' padding); with the reduction
 // 12001 tokens 107 -> 85, 8192 48 -> 43, 2345 21.8 -> 16.6, 16 heads x 12000 67 -> 53, 12 x 1500, stride 16, 32 -> 21.5.
+// Taken back: the tiles of four tile rows column by column, so that an XCD works on a block of the output (32768 tokens 491 -> 484, 16384
+// 126 -> 132).
 // The epilogue reduces each (row m, key block J) to a pair
 // (local max, sum of exp2(z - local max)) in an fp32 workspace laid out [J][m] - the logits never
 // reach HBM.  Kernel 2 (HBM-bound): per row the global max and denominator from the pairs, then the
