@@ -425,8 +425,9 @@ __global__ __launch_bounds__(256) void psa_est_reduce_kernel(EstParams p) {
 
 // The same, followed by the level map of the row while its scores are still in LDS: the workspace pass (HBM) of
 // one workgroup overlaps the sorting (VALU / LDS) of the others, and a launch and a round trip of the scores
-// through memory go away.  The row's levels end in LDS too (psa_sched::end_map_row): similarity cap, map, tile records.
-// LDS: [level-map scratch: lm_bytes][n_d floats][Nk levels].  p.scores may be null.
+// through memory go away.  With a similarity cap or a list of tiles the row's levels end in LDS too (psa_sched::end_map_row; else
+// end.map_out is null and they go straight to the map: rows of few levels lose 1.5 of 40 us per layer by the way through LDS).
+// LDS: [level-map scratch: lm_bytes][n_d floats][Nk levels, if they end there].  p.scores may be null.
 // (80 registers, six waves per SIMD: at 82, five, 3072 rows of 1024 scores take 109.5 us instead of 104.1)
 __global__ __launch_bounds__(256, 6) void psa_est_reduce_map_kernel(EstParams p, LevelMapParams lp, psa_sched::MapEnd end, int lm_bytes) {
   extern __shared__ __align__(16) unsigned char smem_rm[];
@@ -445,12 +446,13 @@ __global__ __launch_bounds__(256, 6) void psa_est_reduce_map_kernel(EstParams p,
     if (p.scores) p.scores[row * p.out_cols + j] = v;
   }
   __syncthreads();
-  level_map_row(lp, s_e, row, smem_rm, s_cnt, s_iv, tid, 256, s_lv);
-  psa_sched::end_map_row(end, s_lv, lp.Nk, row, bh, i, (uint16_t*)smem_rm, s_lists, tid);
+  const bool ends = end.map_out != nullptr;
+  level_map_row(lp, s_e, row, smem_rm, s_cnt, s_iv, tid, 256, ends ? s_lv : nullptr);
+  if (ends) psa_sched::end_map_row(end, s_lv, lp.Nk, row, bh, i, (uint16_t*)smem_rm, s_lists, tid);
 }
 
 template <int D>
-int launch_est(EstParams& p, int B, hipStream_t stream, const LevelMapParams* lp, const psa_sched::MapEnd& end, bool* map_done) {
+int launch_est(EstParams& p, int B, hipStream_t stream, const LevelMapParams* lp, psa_sched::MapEnd& end, bool* map_done) {
   const int rows_needed = p.out_rows << p.keep_m_log2;
   dim3 grid((unsigned)((rows_needed + 255) / 256), (unsigned)(B * p.Hq));
   // 256-row workgroups: cut the key range until about 3 workgroups per CU exist (the kernel's occupancy),
@@ -487,11 +489,21 @@ int launch_est(EstParams& p, int B, hipStream_t stream, const LevelMapParams* lp
     hipLaunchKernelGGL(psa_est_reduce_kernel, rgrid, dim3(256), (size_t)p.n_d * sizeof(float), stream, p);
     return psa_check_launch("psa_estimate_sampled (reduction)");
   }
-  size_t lm_bytes = level_map_lds_bytes(*lp);
-  lm_bytes = lm_bytes > (size_t)lp->Nk * 2 ? lm_bytes : (size_t)lp->Nk * 2;  // (later the ids of the row's lists)
-  lm_bytes = (lm_bytes + 15) & ~(size_t)15;
-  const size_t shmem = lm_bytes + (size_t)p.n_d * sizeof(float) + (size_t)lp->Nk;
-  if (shmem > 150 * 1024) {
+  constexpr size_t MOST = 150 * 1024;
+  const size_t map_scratch = level_map_lds_bytes(*lp), row_bytes = (size_t)p.n_d * sizeof(float), ids = (size_t)lp->Nk * 2;
+  auto pad16 = [](size_t n) { return (n + 15) & ~(size_t)15; };
+  size_t lm_bytes = pad16(map_scratch), shmem = lm_bytes + row_bytes;
+  if (end.map_out != nullptr) {
+    const size_t lm_end = pad16(map_scratch > ids ? map_scratch : ids);  // (later the ids of the row's lists)
+    const size_t sh_end = lm_end + row_bytes + (size_t)lp->Nk;
+    if (sh_end > MOST) {
+      end.map_out = nullptr;  // wide rows: the map alone comes out of this kernel, or of the next
+    } else {
+      lm_bytes = lm_end;
+      shmem = sh_end;
+    }
+  }
+  if (shmem > MOST) {
     // very wide maps: the row of scores and the level-map scratch do not fit into LDS together - two kernels
     PSA_REQUIRE(p.scores != nullptr, PSA_ERR_ARG, "psa_estimate_sampled_map: maps of %d columns need the scores buffer", lp->Nk);
     hipLaunchKernelGGL(psa_est_reduce_kernel, rgrid, dim3(256), (size_t)p.n_d * sizeof(float), stream, p);
@@ -535,7 +547,7 @@ namespace {
 int est_run(psa_tensor4 q, psa_tensor4 k, const int32_t* off_q, const int32_t* off_k, const int32_t* q_index, float* scores,
             void* workspace, int B, int Hq,
             int Hkv, int Lq, int Lk, int D, int block_m, int block_n, int keep_m, int keep_n, float sm_scale, int out_rows,
-            int out_cols, LevelMapParams* lp, const psa_sched::MapEnd& end, bool* map_done, psa_stream_t stream) {
+            int out_cols, LevelMapParams* lp, psa_sched::MapEnd& end, bool* map_done, psa_stream_t stream) {
   PSA_REQUIRE(q.ptr && k.ptr && (scores || lp) && workspace, PSA_ERR_ARG, "psa_estimate_sampled: null pointer");
   PSA_REQUIRE(B > 0 && Hq > 0 && Hkv > 0 && Lq > 0 && Lk > 0, PSA_ERR_ARG, "psa_estimate_sampled: sizes must be positive");
   PSA_REQUIRE(Hq % Hkv == 0, PSA_ERR_ARG, "psa_estimate_sampled: Hq must be a multiple of Hkv");
@@ -580,8 +592,9 @@ extern "C" int psa_estimate_sampled(psa_tensor4 q, psa_tensor4 k, const int32_t*
                                     int keep_m, int keep_n, float sm_scale, int out_rows, int out_cols, psa_stream_t stream) {
   PSA_REQUIRE(scores, PSA_ERR_ARG, "psa_estimate_sampled: null pointer");
   bool unused = false;
+  psa_sched::MapEnd none = {};
   return est_run(q, k, off_q, off_k, nullptr, scores, workspace, B, Hq, Hkv, Lq, Lk, D, block_m, block_n, keep_m, keep_n, sm_scale,
-                 out_rows, out_cols, nullptr, psa_sched::MapEnd{}, &unused, stream);
+                 out_rows, out_cols, nullptr, none, &unused, stream);
 }
 
 extern "C" int psa_estimate_sampled_indexed(psa_tensor4 q, const int32_t* q_index, psa_tensor4 k, const int32_t* off_q,
@@ -590,11 +603,12 @@ extern "C" int psa_estimate_sampled_indexed(psa_tensor4 q, const int32_t* q_inde
                                             int out_rows, int out_cols, psa_stream_t stream) {
   PSA_REQUIRE(scores && q_index, PSA_ERR_ARG, "psa_estimate_sampled_indexed: null pointer");
   bool unused = false;
+  psa_sched::MapEnd none = {};
   return est_run(q, k, off_q, off_k, q_index, scores, workspace, B, Hq, Hkv, Lq, Lk, D, block_m, block_n, keep_m, keep_n, sm_scale,
-                 out_rows, out_cols, nullptr, psa_sched::MapEnd{}, &unused, stream);
+                 out_rows, out_cols, nullptr, none, &unused, stream);
 }
 
-// cap ([B * Hq][Nk], null: none) and walk (null: none) are served here only where the map comes out of the fused kernel (ended: it did)
+// cap ([B * Hq][Nk], null: none) and walk (null: none) are served here only where a row's levels fit the fused kernel's LDS (ended: they did)
 static int est_map_run(psa_tensor4 q, psa_tensor4 k, const int32_t* off_q, const int32_t* off_k, const int32_t* q_index, float* scores,
                        void* workspace, int B, int Hq, int Hkv, int Lq, int Lk, int D, int block_m, int block_n,
                        int keep_m, int keep_n, float sm_scale, int out_rows, int out_cols, void* map_out,
@@ -609,7 +623,8 @@ static int est_map_run(psa_tensor4 q, psa_tensor4 k, const int32_t* off_q, const
   if (rc != PSA_OK) return rc;
   lp.map_out = map_out; lp.map_elem = map_elem_bytes;
   psa_sched::MapEnd end = {};
-  end.map_out = map_out; end.map_elem = map_elem_bytes;
+  if (cap != nullptr || walk != nullptr) end.map_out = map_out;
+  end.map_elem = map_elem_bytes;
   end.cap = cap; end.Hq = Hq; end.n_rep = 1;
   if (walk != nullptr) {
     psa_sched::Geometry g;
@@ -619,7 +634,7 @@ static int est_map_run(psa_tensor4 q, psa_tensor4 k, const int32_t* off_q, const
   bool map_done = false;
   const int rc2 = est_run(q, k, off_q, off_k, q_index, scores, workspace, B, Hq, Hkv, Lq, Lk, D, block_m, block_n, keep_m, keep_n,
                           sm_scale, out_rows, out_cols, &lp, end, &map_done, stream);
-  if (ended != nullptr) *ended = map_done;
+  if (ended != nullptr) *ended = map_done && end.map_out != nullptr;
   if (rc2 != PSA_OK || map_done) return rc2;
   return psa_level_map(scores, map_out, map_elem_bytes, nullptr, (int64_t)B * Hq * out_rows, out_cols, mode, n_items, item_level, item_hi,
                        align_div, text_blocks, min_full_attn_ratio, stream);

@@ -113,3 +113,29 @@ def test_causal_rows_too_wide_for_one_launch():
               "psa_causal_layer_fwd")
         outs.append(out)
     assert torch.equal(*outs)
+
+
+@pytest.mark.parametrize("mode,Nk", [("thresholdbound", 5300), ("topk", 5300)])
+def test_wide_maps_need_no_scores(mode, Nk):
+    """A map that is only stored keeps its levels out of LDS: rows of 5300 sorted scores fit beside their sorting scratch
+    (8 * 8192 + 12 * 5300 + 4 * 5300 = 150336 bytes of 153600), without the buffer of scores."""
+    from psa_hip import ops
+    from psa_hip._lib import check, lib
+
+    B, H, D, bm, bn = 1, 1, 64, 128, 32
+    L = Nk * bn - 5
+    q, k = (rnd(B, H, L, D, seed=i).to(dev()) for i in range(2))
+    off_q, off_k = ops.draw_sample_offsets(B, H, H, bm, bm // 4, bn, bn // 4, dev(), seed=3)
+    items, m, div = ops._items(RATIOS, mode)
+    lv, hi = ops._level_items(items)
+    Mq = -(-L // bm)
+    ws = torch.empty(lib.psa_estimate_workspace_bytes(B, H, L, L, bm, bn, bm // 4, bn // 4), dtype=torch.uint8, device=dev())
+    maps = []
+    for scores in (None, torch.empty(B, H, Mq, Nk, dtype=torch.float32, device=dev())):
+        mp = torch.zeros(B, H, Mq, Nk, dtype=torch.int32, device=dev())
+        check(lib.psa_estimate_sampled_map(ops._t4(q), ops._t4(k), off_q.data_ptr(), off_k.data_ptr(), ops._ptr(scores), ws.data_ptr(), B, H, H, L, L, D,
+                                           bm, bn, bm // 4, bn // 4, D ** -0.5, Mq, Nk, mp.data_ptr(), 4, m, len(items), lv, hi, 1, 0, 0.06,
+                                           ops._stream(q)), "psa_estimate_sampled_map")
+        maps.append(mp)
+    ref = ops.level_map(scores, RATIOS, 0, mode, blocksize=bn, compute_tile=bn, map_dtype=torch.int32)
+    assert torch.equal(maps[0], ref) and torch.equal(maps[1], ref)
