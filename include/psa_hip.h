@@ -313,7 +313,8 @@ int psa_layer_fwd(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const int32_t* to
                   double min_full_attn_ratio, int walk, psa_stream_t stream);
 /* The same with a second buffer (256-byte aligned; NULL: as above) of psa_layer_extra_bytes(...) bytes, whose parts are filled while the
  * workspace still holds the estimate's scratch: the level map's kernel then applies the cap and lists the tiles, and the pooling pass
- * forms the cap.  Same results in fewer launches. */
+ * forms the cap.  Same results in fewer launches.  Without sim_thresholds only the first psa_walk_bytes(...) bytes of it are used (walk !=
+ * 0; none with walk == 0). */
 int64_t psa_layer_extra_bytes(int elem_bytes, int B, int Hq, int Hkv, int L, int D, int block_m, int block_n, int indexed, int walk);
 int psa_layer_fwd_extra(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const int32_t* token_index, const int32_t* off_q,
                         const int32_t* off_k, const float* sim_thresholds, int32_t* cap_out, void* workspace, void* extra,

@@ -116,20 +116,22 @@ extern "C" int64_t psa_layer_workspace_bytes(int elem_bytes, int B, int Hq, int 
 
 namespace {
 // What a layer may have beside its workspace, whose parts overlap in time: buffers that are filled while the estimate's scratch is
-// still in use.  They let the level map's kernel write the tile records and the pooling pass form the similarity cap.
+// still in use.  They let the level map's kernel write the tile records and the pooling pass form the similarity cap.  Pools that no
+// cap is formed beside (capped == 0; token re-ordering, whose pools come first anyway) stay in the workspace: a layer of 12 heads x 32760 tokens
+// takes 24 MiB here instead of 192.
 struct LayerExtra {
   int64_t kp, vp, walk, bytes;
 };
-LayerExtra layer_extra(int elem, int B, int Hq, int Hkv, int L, int D, int block_m, int block_n, int indexed, int walk) {
+LayerExtra layer_extra(int elem, int B, int Hq, int Hkv, int L, int D, int block_m, int block_n, int indexed, int walk, bool capped) {
   LayerExtra e = {-1, -1, -1, 0};
   Parts w;
-  if (!indexed) {
+  const int64_t walk_bytes = walk && elem == 2 ? psa_walk_bytes(B, Hq, Hkv, L, D, block_m, block_n) : 0;
+  if (walk_bytes > 0) e.walk = w.take(walk_bytes);
+  if (capped && !indexed) {
     const int64_t pool = psa_pool_elems(B, Hkv, L, D, block_n) * elem;
     e.kp = w.take(pool);
     e.vp = w.take(pool);
   }
-  const int64_t walk_bytes = walk && elem == 2 ? psa_walk_bytes(B, Hq, Hkv, L, D, block_m, block_n) : 0;
-  if (walk_bytes > 0) e.walk = w.take(walk_bytes);
   e.bytes = w.top;
   return e;
 }
@@ -138,7 +140,7 @@ LayerExtra layer_extra(int elem, int B, int Hq, int Hkv, int L, int D, int block
 extern "C" int64_t psa_layer_extra_bytes(int elem_bytes, int B, int Hq, int Hkv, int L, int D, int block_m, int block_n, int indexed, int walk) {
   LayerParts p;
   if (!layer_parts(elem_bytes, B, Hq, Hkv, L, D, block_m, block_n, indexed, walk, p)) return 0;
-  return layer_extra(elem_bytes, B, Hq, Hkv, L, D, block_m, block_n, indexed, walk).bytes;
+  return layer_extra(elem_bytes, B, Hq, Hkv, L, D, block_m, block_n, indexed, walk, true).bytes;
 }
 
 extern "C" int psa_layer_fwd(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const int32_t* token_index, const int32_t* off_q,
@@ -163,7 +165,7 @@ extern "C" int psa_layer_fwd_extra(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, 
   LayerParts p;
   PSA_REQUIRE(layer_parts(elem, B, Hq, Hkv, L, D, block_m, block_n, token_index != nullptr, walk, p), PSA_ERR_ARG, "psa_layer_fwd: bad shape");
   LayerExtra e = {-1, -1, -1, 0};
-  if (extra != nullptr) e = layer_extra(elem, B, Hq, Hkv, L, D, block_m, block_n, token_index != nullptr, walk);
+  if (extra != nullptr) e = layer_extra(elem, B, Hq, Hkv, L, D, block_m, block_n, token_index != nullptr, walk, sim_thresholds != nullptr);
   char *ws = (char*)workspace, *ex = (char*)extra;
   char* kp = e.kp >= 0 ? ex + e.kp : ws + p.attn.kp;
   char* vp = e.vp >= 0 ? ex + e.vp : ws + p.attn.vp;

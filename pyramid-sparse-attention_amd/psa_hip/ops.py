@@ -674,12 +674,14 @@ def _layer_one_call(qb, kb, vb, off_q, off_k, mask_ratios, mode, block_m, block_
         return None
     items, m, _ = _items(mask_ratios, mode)
     Mq, Nk = -(-L // block_m), -(-L // block_n)
-    walk = int(_walk_bytes(qb.dtype, B, Hq, Hkv, L, D, block_m, block_n) > 0)
+    n_walk = _walk_bytes(qb.dtype, B, Hq, Hkv, L, D, block_m, block_n)
+    walk = int(n_walk > 0)
     sizes = (qb.element_size(), B, Hq, Hkv, L, D, block_m, block_n, int(token_index is not None), walk)
-    n_ws = lib.psa_layer_workspace_bytes(*sizes)
+    n_ws = lib.psa_layer_workspace_bytes(*sizes)  # (a multiple of 256 bytes)
     if not 0 < n_ws <= _ONE_CALL_MAX_BYTES:
         return None
-    n_extra = lib.psa_layer_extra_bytes(*sizes)  # (multiples of 256 bytes, both)
+    # the second buffer: for the list alone, for pools too where the pooling pass forms the cap
+    n_extra = n_walk if sim_thresholds is None else lib.psa_layer_extra_bytes(*sizes)
     if n_ws + n_extra > _ONE_CALL_MAX_BYTES:
         n_extra = 0
     if token_index is not None:

@@ -163,3 +163,96 @@ def test_layer_runs_on_the_current_stream_without_the_raw_handle(monkeypatch):
         torch.cuda.current_stream().wait_stream(s)
         torch.cuda.synchronize()
     assert torch.equal(outs[0], outs[1])
+
+
+def _peak(layer):
+    """What a call holds at most beside what was there before it."""
+    layer()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    out = layer()
+    torch.cuda.synchronize()
+    return out, torch.cuda.max_memory_allocated() - before
+
+
+@pytest.mark.parametrize("L,bn,dtype,capped", [
+    (1000, 64, torch.bfloat16, False),    # few rows of 64-key blocks: neither cap nor list
+    (1000, 64, torch.float32, False),
+    (1000, 128, torch.float16, False),    # a list, no cap
+    (1000, 64, torch.bfloat16, True),     # a cap: pools beside the estimate's scratch
+])
+def test_layers_take_no_memory_that_serves_nothing(L, bn, dtype, capped):
+    from psa_hip import _lib, ops
+
+    H, D, up = 8, 64, lambda n: -(-n // 512) * 512  # (granularity of torch's allocations)
+    q, k, v = (rnd(1, H, L, D, seed=i).to(dtype).to(dev()) for i in range(3))
+    off_q, off_k = ops.draw_sample_offsets(1, H, H, 128, 32, bn, bn // 4, dev(), seed=1)
+    _, peak = _peak(lambda: ops.psa_layer_fwd(q, k, v, off_q, off_k, RATIOS, "topk", 128, bn, 16, sim_thresholds=(0.9, 0.9, 0.9) if capped else None))
+    shape, Mq, Nk = (1, H, H, L, D, 128, bn), -(-L // 128), -(-L // bn)
+    walk = ops._walk_bytes(dtype, *shape)
+    assert (walk > 0) == (bn == 128)
+    need = _lib.lib.psa_layer_workspace_bytes(q.element_size(), *shape, 0, int(walk > 0)) + -(-walk // 256) * 256
+    if capped:
+        need += 2 * (-(-2 * _lib.lib.psa_pool_elems(1, H, L, D, bn) // 256) * 256)
+    assert peak <= up(need) + up(H * Mq * Nk) + up(H * L * D * q.element_size()) + (up(H * Nk * 4) if capped else 0)
+
+
+@pytest.mark.parametrize("Hq,Hkv,L,D,bn,mode,indexed,capped", [
+    (8, 8, 1000, 64, 64, "topk", False, False),
+    (4, 2, 513, 128, 128, "thresholdbound", False, False),   # listed
+    (4, 4, 1537, 128, 128, "topk", False, True),             # ... with the cap, pooling behind the map
+    (4, 4, 1537, 128, 128, "topk", True, True),              # ... formed by the pooling pass of the ordered rows, applied by the map's kernel
+    (38, 38, 3400, 64, 32, "topk", True, False),             # listed 32-key blocks
+    (38, 38, 3400, 64, 32, "thresholdbound", False, True),
+])
+def test_one_call_without_its_second_buffer(monkeypatch, Hq, Hkv, L, D, bn, mode, indexed, capped):
+    """Between the limits for one buffer and for two the stages behind the map overlay the estimate's scratch, and list, cap and pooling
+    come from launches of their own where the map's kernel and the pooling pass have no place for them."""
+    from psa_hip import ops
+
+    q, k, v = (rnd(1, h, L, D, seed=L + i).to(dev()) for i, h in enumerate((Hq, Hkv, Hkv)))
+    off_q, off_k = ops.draw_sample_offsets(1, Hq, Hkv, 128, 32, bn, bn // 4, dev(), seed=L)
+    index = torch.randperm(L, generator=torch.Generator().manual_seed(L)).to(torch.int32).to(dev()) if indexed else None
+
+    def layer():
+        return ops.psa_layer_fwd(q, k, v, off_q, off_k, RATIOS, mode, 128, bn, 16, return_map=True, return_cap=True, text_length=70,
+                                 token_index=index, sim_thresholds=(0.3, 0.1, 0.0) if capped else None)
+
+    shape = (1, Hq, Hkv, L, D, 128, bn)
+    walk = int(ops._walk_bytes(q.dtype, *shape) > 0)
+    n_ws = ops.lib.psa_layer_workspace_bytes(2, *shape, int(indexed), walk)
+    seconds, call = [], ops.lib.psa_layer_fwd_extra
+    monkeypatch.setattr(ops.lib, "psa_layer_fwd_extra", lambda *a: seconds.append(a[9]) or call(*a))
+    with_it = layer()
+    monkeypatch.setattr(ops, "_ONE_CALL_MAX_BYTES", n_ws)
+    without = layer()
+    assert len(seconds) == 2 and (seconds[0] is not None) == bool(walk or (capped and not indexed)) and seconds[1] is None
+    monkeypatch.setattr(ops, "_layer_one_call", lambda *a: None)
+    ref = layer()
+    for got in (with_it, without):
+        for a, b in zip(got, ref):
+            assert (a is None and b is None) or torch.equal(a, b)
+
+
+@pytest.mark.parametrize("Hq,Hkv,L,D,stride,mode", [(28, 4, 2345, 128, 8, "energybound"), (8, 8, 12001, 128, 8, "topk"), (2, 2, 129, 64, 16, "topk")])
+def test_causal_one_call_without_its_second_buffer(monkeypatch, Hq, Hkv, L, D, stride, mode):
+    from psa_hip import ops
+    from psa_hip.PSA_casual import AttentionConfig, PyramidAdaptiveBlockSparseAttnTrain
+
+    q, k, v = (rnd(1, h, L, D, seed=L + i).to(dev()) for i, h in enumerate((Hq, Hkv, Hkv)))
+    m = PyramidAdaptiveBlockSparseAttnTrain(AttentionConfig(text_length=130, mask_mode=mode, xattn_stride=stride, sim_2x_threshold=-0.1,
+                                                            sim_4x_threshold=0.0, sim_8x_threshold=0.05), layer_idx=0)
+    sizes, size = [], ops.lib.psa_causal_layer_workspace_bytes
+    monkeypatch.setattr(ops.lib, "psa_causal_layer_workspace_bytes", lambda *a: sizes.append(size(*a)) or sizes[-1])
+    seconds, call = [], ops.lib.psa_causal_layer_fwd_extra
+    monkeypatch.setattr(ops.lib, "psa_causal_layer_fwd_extra", lambda *a: seconds.append(a[5]) or call(*a))
+    a = m(q, k, v, layer_idx=0)
+    monkeypatch.setattr(ops, "_ONE_CALL_MAX_BYTES", sizes[0])
+    b = m(q, k, v, layer_idx=0)
+    assert len(seconds) == 2 and seconds[0] is not None and seconds[1] is None
+    plain = m.sparse_attention_fn
+    m.sparse_attention_fn = lambda *x: plain(*x)  # a function of the caller's own: the separate operators
+    c = m(q, k, v, layer_idx=0)
+    assert torch.equal(a, c) and torch.equal(b, c)
