@@ -649,8 +649,8 @@ def _side_stream(device: torch.device) -> "torch.cuda.Stream":
 
 # ----------------------------------------------------------------------------- whole layer, forward only
 # Workspace above which a layer goes through the separate operators: they hand the estimate's scratch back before the output is
-# taken (48 heads x 45106 tokens with 32-key blocks: 4.0 GiB at most against 4.3), and the host's share, which one call saves, is
-# long hidden behind milliseconds of kernels.
+# taken (48 heads x 45106 tokens with 32-key blocks: 4011 MiB at most, as one call 4274, with the second buffer 4551), and the host's share,
+# which one call saves, is long hidden behind milliseconds of kernels.
 _ONE_CALL_MAX_BYTES = 1 << 30
 
 
@@ -837,8 +837,13 @@ def psa_layer_fwd(
         if level_cap is not None:
             raise ValueError("pass either level_cap or sim_thresholds")
         level_cap = k_similarity(kb, block_n, *sim_thresholds)
-    walk = None
-    both = _map_and_walk(qb, kb, off_q, off_k, mask_ratios, mode, block_m, block_n, tile_n, sm_scale, text_length, token_index, level_cap)
+    walk = both = None
+    # Map and list from one launch hold the list beside the estimate's scratch; later it lies beside the output.  Scratch above the
+    # output's size goes back first: the list would add to what the layer holds at most (48 heads x 45106 tokens with 32-key blocks: 2995
+    # MiB of scratch, 277 of list, 264 of output; 4288 MiB at most instead of 4011, for 5994 us instead of 6011).
+    B, Hq, L = qb.shape[:3]
+    if lib.psa_estimate_workspace_bytes(B, Hq, L, kb.shape[2], block_m, block_n, keep_m, keep_n) <= qb.numel() * qb.element_size():
+        both = _map_and_walk(qb, kb, off_q, off_k, mask_ratios, mode, block_m, block_n, tile_n, sm_scale, text_length, token_index, level_cap)
     if both is not None:
         mp, walk = both
     else:

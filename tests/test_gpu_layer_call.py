@@ -177,6 +177,33 @@ def _peak(layer):
     return out, torch.cuda.max_memory_allocated() - before
 
 
+@pytest.mark.parametrize("H,L,D,bn", [
+    (12, 20000, 64, 32),    # scratch of the estimate above the output: the list waits for it to go
+    (12, 20000, 128, 128),  # below: the map's kernel writes the list
+])
+@pytest.mark.parametrize("indexed", [False, True])
+def test_a_list_from_the_map_kernel_takes_no_more_memory(monkeypatch, H, L, D, bn, indexed):
+    """The separate operators with map and list from one launch hold no more at once than with a launch each; same bits."""
+    from psa_hip import _lib, ops
+
+    q, k, v = (rnd(1, H, L, D, seed=i).to(dev()) for i in range(3))
+    off_q, off_k = ops.draw_sample_offsets(1, H, H, 128, 32, bn, bn // 4, dev(), seed=1)
+    index = torch.randperm(L, generator=torch.Generator().manual_seed(L)).to(torch.int32).to(dev()) if indexed else None
+    monkeypatch.setattr(ops, "_layer_one_call", lambda *a: None)
+    real, calls = ops._map_and_walk, []
+
+    def run(fused):
+        monkeypatch.setattr(ops, "_map_and_walk", (lambda *a: calls.append(1) or real(*a)) if fused else lambda *a: None)
+        return _peak(lambda: ops.psa_layer_fwd(q, k, v, off_q, off_k, RATIOS, "topk", 128, bn, 16, token_index=index))
+
+    (a, one), (b, plain) = run(True), run(False)
+    slack = 4 << 20  # (torch leaves up to 1 MiB at the end of a large block)
+    assert ops._walk_bytes(q.dtype, 1, H, H, L, D, 128, bn) > 2 * slack
+    assert torch.equal(a, b) and one <= plain + slack
+    est = _lib.lib.psa_estimate_workspace_bytes(1, H, L, L, 128, bn, 32, bn // 4)
+    assert bool(calls) == (est <= q.numel() * 2) == (bn == 128)
+
+
 @pytest.mark.parametrize("L,bn,dtype,capped", [
     (1000, 64, torch.bfloat16, False),    # few rows of 64-key blocks: neither cap nor list
     (1000, 64, torch.float32, False),
