@@ -29,3 +29,20 @@ def attn_errors(out_gpu, ref):
 
 # tolerance of the task statement for bf16 attention outputs
 MAX_ABS, MEAN_ABS = 2e-2, 2e-3
+
+
+def xattn_tile(heads, Lq, Lk, block, stride, chunk, causal):
+    """Output tile of the antidiagonal contraction's launch (csrc/psa_xattn.hip, xattn_small; rows that do not overlap) and how many of
+    them the busiest workgroup takes: ("large" | "small", tiles)."""
+    up = lambda n, m: -(-n // m) * m
+    Mr, Nr = up(Lq, chunk) // stride, up(Lk, chunk) // stride
+    rows = min(-(-Lq // block) * (block // stride), Mr)
+
+    def tiles(edge):
+        per_row = lambda tm: min(-(-Nr // edge), ((tm + 1) * edge - 1 + Nr - Mr) // edge + 1) if causal else -(-Nr // edge)
+        return heads * sum(per_row(tm) for tm in range(-(-rows // edge)))
+
+    large, small = tiles(256), tiles(128)
+    if (small + 256) * 3 < -(-large // 256) * 2560:
+        return "small", 1
+    return "large", -(-(-(-large // 8)) // 32)  # 8 XCDs, 32 workgroups each

@@ -8,7 +8,7 @@ import pytest
 import torch
 
 import psa_oracle as O
-from gpu_util import dev, rnd
+from gpu_util import dev, rnd, xattn_tile
 
 pytestmark = pytest.mark.gpu
 
@@ -24,19 +24,24 @@ def _check(q, k, block, stride, chunk, causal, heads=None):
         np.testing.assert_allclose(got[:, h:h + 1].numpy(), ref.numpy(), rtol=1e-4, atol=1e-9)
 
 
-@pytest.mark.parametrize("Hq,Hkv,Lq,Lk,D,block,stride,chunk,causal", [
-    (64, 64, 4096, 4096, 64, 64, 8, 1024, True),      # large tiles, key blocks of 8 strided keys
-    (60, 30, 3999, 3999, 128, 128, 8, 1024, True),    # ... of 16, the last group of tokens partly past the sequence
-    (64, 64, 2050, 2050, 64, 128, 4, 512, False),     # ... of 32; half a tile past the padded rows
-    (64, 64, 1024, 4096, 64, 128, 4, 512, True),      # queries at the end of longer keys
-    (2, 1, 129, 129, 128, 128, 16, 2048, True),       # small tiles
-    (3, 3, 1025, 1025, 64, 64, 8, 1024, False),
-    (1, 1, 1, 1, 64, 128, 4, 512, True),
-    (2, 2, 500, 500, 64, 32, 1, 128, True),           # a single stage
-    (2, 2, 515, 515, 128, 32, 1, 128, False),         # two
-    (64, 64, 1100, 1100, 64, 32, 1, 128, True),       # a single stage, large tiles, one after the other
+@pytest.mark.parametrize("Hq,Hkv,Lq,Lk,D,block,stride,chunk,causal,tile", [
+    (64, 64, 4096, 4096, 64, 64, 8, 1024, True, ("large", 1)),     # key blocks of 8 strided keys
+    (60, 30, 3999, 3999, 128, 128, 8, 1024, True, ("large", 1)),   # ... of 16, the last group of tokens partly past the sequence
+    (28, 28, 2050, 2050, 64, 128, 4, 512, False, ("large", 1)),    # ... of 32; half a tile past the padded rows
+    (64, 64, 2050, 2050, 64, 128, 4, 512, False, ("small", 1)),
+    (64, 64, 1024, 4096, 64, 128, 4, 512, True, ("large", 1)),     # queries at the end of longer keys
+    (64, 32, 2050, 2050, 128, 128, 4, 2048, False, ("large", 3)),  # one tile after the other, whole chunks of padding
+    (170, 85, 3999, 3999, 64, 64, 8, 1024, True, ("large", 2)),    # ... masked and unmasked ones
+    (2, 1, 129, 129, 128, 128, 16, 2048, True, ("small", 1)),
+    (3, 3, 1025, 1025, 64, 64, 8, 1024, False, ("small", 1)),
+    (1, 1, 1, 1, 64, 128, 4, 512, True, ("small", 1)),
+    (2, 2, 500, 500, 64, 32, 1, 128, True, ("small", 1)),          # a single stage
+    (2, 2, 515, 515, 128, 32, 1, 128, False, ("small", 1)),        # two
+    (64, 64, 1100, 1100, 64, 32, 1, 128, True, ("small", 1)),
+    (34, 34, 1100, 1100, 64, 32, 1, 128, True, ("large", 2)),      # a single stage (a second one of zeros) per tile, one tile after the other
 ])
-def test_edges(Hq, Hkv, Lq, Lk, D, block, stride, chunk, causal):
+def test_edges(Hq, Hkv, Lq, Lk, D, block, stride, chunk, causal, tile):
+    assert xattn_tile(Hq, Lq, Lk, block, stride, chunk, causal) == tile
     q, k = rnd(1, Hq, Lq, D, seed=Lq).to(dev()), rnd(1, Hkv, Lk, D, seed=Lk + 1).to(dev())
     _check(q, k, block, stride, chunk, causal, heads=(0, Hq // 2, Hq - 1))
 

@@ -4,15 +4,9 @@ same bits.  (test_gpu_causal compares the estimate with the oracle.)"""
 import pytest
 import torch
 
-from gpu_util import dev, rnd
+from gpu_util import dev, rnd, xattn_tile
 
 pytestmark = pytest.mark.gpu
-
-
-def _tiles(edge, H, L, stride, chunk, causal):
-    rows, keys = -(-L // 128) * 128 // stride, -(-L // chunk) * chunk // stride
-    per_head = sum(min(-(-keys // edge), tm + 1 if causal else 1 << 30) for tm in range(-(-rows // edge)))
-    return per_head * H
 
 
 @pytest.mark.parametrize("H,L,stride,chunk,D,causal", [
@@ -24,14 +18,11 @@ def _tiles(edge, H, L, stride, chunk, causal):
 def test_tiles_give_the_same_bits(H, L, stride, chunk, D, causal):
     from psa_hip import ops
 
-    def small(n):
-        lo, sm = _tiles(256, n, L, stride, chunk, causal), _tiles(128, n, L, stride, chunk, causal)
-        return -(-sm // 512) * 13 < -(-lo // 256) * 20
-
+    kind = lambda heads: xattn_tile(heads, L, L, 128, stride, chunk, causal)[0]
     group = 2
-    assert small(group)
+    assert kind(group) == "small"
     if L > 129:
-        assert not small(H)
+        assert kind(H) == "large"
     q, k = (rnd(1, H, L, D, seed=L + i).to(dev()) for i in range(2))
     whole = ops.estimate_xattn(q, k, 128, stride, causal, chunk)
     for h in range(0, H, 14):
