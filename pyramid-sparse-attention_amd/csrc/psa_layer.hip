@@ -287,7 +287,8 @@ extern "C" int psa_causal_layer_fwd_extra(psa_tensor4 q, psa_tensor4 k, psa_tens
   int32_t* cap = (int32_t*)(ws + p.cap);
   void* const map = ws + p.map;
   int rc;
-  // (wider maps: a row's scores, levels and sorting scratch, 17 to 25 bytes per column, do not fit LDS together)
+  // (a row's scores, levels and sorting scratch take 25 to 33 bytes of LDS per column: 100 KiB at 4096 columns, 132 just above, and from 5800 on
+  // they do not fit together)
   if (extra != nullptr && S <= 4096) {
     const CausalExtra e = causal_extra(B, Hq, Hkv, L, D, block);
     char* ex = (char*)extra;
