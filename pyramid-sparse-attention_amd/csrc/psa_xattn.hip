@@ -12,12 +12,12 @@
 // psa_tiles.h) in stages of 64 contraction elements, i.e. half a head-dim row of one of the S interleaved
 // tokens; the transposed product (rows = n, lanes = m) makes part of the reductions over n in-lane.  A 256 x 256 tile needs 32 bytes of
 // copies per CU cycle at the full MFMA rate (the path delivers 64; a 128 x 128 tile would need all of it).
-// What bounds it: MFMAs (0.57 of the cycles at 28 heads x 32768 tokens, stride 8) at the clock that the board's power leaves (1.85 GHz),
+// What bounds it: MFMAs (0.57 of the cycles at 28 heads x 32768 tokens, stride 8) at the clock that the board's power leaves (1.63 - 1.86 GHz),
 // the epilogue, 256 exponentials and about 1500 other vector instructions per lane and tile with nothing beside them (a fifth of a
 // tile), and copies that are still in flight at a stage's barrier (a seventh).  A wave of 128 x 128 reads 0.25 operands from LDS per MFMA; the 8
 // waves of 64 x 128 before it read 0.375, met at a barrier with no operand in registers (0.48 of the cycles), and each tile began
-// with its first copies: contraction 512 -> 435 us there (1.17 PFLOP/s with the tiles' padding); with the reduction
-// 12001 tokens 107 -> 85, 8192 48 -> 43, 2345 21.8 -> 16.6, 16 heads x 12000 67 -> 53, 12 x 1500, stride 16, 32 -> 21.5.
+// with its first copies: contraction alone 512 -> 435, 561 -> 509 us by card (0.94 - 1.11 PFLOP/s of the products under the diagonal,
+// 0.06 more with the tiles' padding), with the reduction 581 -> 490, 567 -> 511; 12001 tokens 107 -> 85, 8192 48 -> 43, 2345 21.8 -> 16.6, 16 heads x 12000 67 -> 53, 12 x 1500, stride 16, 32 -> 21.5.
 // Taken back: the tiles of four tile rows column by column, so that an XCD works on a block of the output (32768 tokens 491 -> 484, 16384
 // 126 -> 132).
 // The epilogue reduces each (row m, key block J) to a pair
