@@ -190,6 +190,51 @@ __device__ __forceinline__ float quarter_wave_sum(float v) {
   return half_wave_sum(__builtin_bit_cast(float, r0) + __builtin_bit_cast(float, r1));
 }
 
+// Exchanges inside a wave without the LDS round trip of __shfl (ds_bpermute: about 100 cycles each and an address register): DPP
+// within rows of 16 lanes, row broadcasts and half-wave swaps beyond.  Lanes without a source get `old`.
+template <int CTRL, int ROW_MASK = 0xf>
+__device__ __forceinline__ uint32_t dpp_u32(uint32_t old, uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)v, CTRL, ROW_MASK, 0xf, false);
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp_f32(float v) {  // (every lane has a source)
+  return __builtin_bit_cast(float, dpp_u32<CTRL>(0u, __builtin_bit_cast(uint32_t, v)));
+}
+constexpr int DPP_XOR1 = 0xb1, DPP_XOR2 = 0x4e, DPP_ROW_SHR = 0x110, DPP_ROW_ROR = 0x120, DPP_HALF_MIRROR = 0x141, DPP_BCAST15 = 0x142,
+              DPP_BCAST31 = 0x143;
+// op over lanes 0 .. l in lane l; IDENTITY is what lanes without a source contribute
+template <uint32_t IDENTITY, class Op>
+__device__ __forceinline__ uint32_t wave_scan_u32(uint32_t v, Op op) {
+  v = op(v, dpp_u32<DPP_ROW_SHR + 1>(IDENTITY, v));
+  v = op(v, dpp_u32<DPP_ROW_SHR + 2>(IDENTITY, v));
+  v = op(v, dpp_u32<DPP_ROW_SHR + 4>(IDENTITY, v));
+  v = op(v, dpp_u32<DPP_ROW_SHR + 8>(IDENTITY, v));
+  v = op(v, dpp_u32<DPP_BCAST15, 0xa>(IDENTITY, v));
+  return op(v, dpp_u32<DPP_BCAST31, 0xc>(IDENTITY, v));
+}
+__device__ __forceinline__ int wave_scan_add(int v) {
+  return (int)wave_scan_u32<0u>((uint32_t)v, [](uint32_t a, uint32_t b) { return a + b; });
+}
+__device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)wave_scan_u32<0xffffffffu>(v, [](uint32_t a, uint32_t b) { return a < b ? a : b; }), 63);
+}
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)wave_scan_u32<0u>(v, [](uint32_t a, uint32_t b) { return a > b ? a : b; }), 63);
+}
+// Sum over the wave in every lane, in the order of a butterfly over lane ^ 32, 16, 8, 4, 2, 1.  (Lanes l and l ^ 8 agree once they are
+// added, so a rotation by 4 brings what l ^ 4 holds.)
+__device__ __forceinline__ float wave_sum_f32(float v) {
+  v = half_wave_sum(v);
+  const uint32_t u = __builtin_bit_cast(uint32_t, v);
+  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  const uint32_t r0 = r[0], r1 = r[1];
+  v = __builtin_bit_cast(float, r0) + __builtin_bit_cast(float, r1);
+  v += dpp_f32<DPP_ROW_ROR + 8>(v);
+  v += dpp_f32<DPP_ROW_ROR + 4>(v);
+  v += dpp_f32<DPP_XOR2>(v);
+  return v + dpp_f32<DPP_XOR1>(v);
+}
+
 // The lane's index, formed anew: for kernels that have no register to keep it in.
 __device__ __forceinline__ int lane_id() {
   int l;

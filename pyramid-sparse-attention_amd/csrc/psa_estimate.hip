@@ -386,7 +386,9 @@ __device__ __forceinline__ float est_reduce_row(const EstParams& p, float* s_e, 
   const float* rt = p.rt + (int64_t)bh * p.n_d * p.Ms_pad + r0;
   auto group = [&](int j, const f32x4& x) __attribute__((always_inline)) {
     float v = fmaxf(fmaxf(x[0] - m[0], x[1] - m[1]), fmaxf(x[2] - m[2], x[3] - m[3]));
-    for (int o = (1 << lpg_log2) >> 1; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+    if (lpg_log2 > 2) v = fmaxf(v, dpp_f32<DPP_HALF_MIRROR>(v));
+    if (lpg_log2 > 1) v = fmaxf(v, dpp_f32<DPP_XOR2>(v));  // (behind the mirror: the two halves of 8 lanes agree as sets)
+    v = fmaxf(v, dpp_f32<DPP_XOR1>(v));
     if (quad == 0 && j < p.n_d) s_e[j] = fast_exp2(v);
   };
   // four loads in flight per lane while there are that many key groups left for the wave, then one at a time
@@ -407,8 +409,7 @@ __device__ __forceinline__ float est_reduce_row(const EstParams& p, float* s_e, 
   // row sum in a fixed order: per-thread strided partials, wave butterfly, four wave partials
   float part = 0.f;
   for (int j = tid; j < p.n_d; j += 256) part += s_e[j];
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) part += __shfl_xor(part, o, 64);
+  part = wave_sum_f32(part);
   if (lane == 0) s_part[wave] = part;
   __syncthreads();
   return (s_part[0] + s_part[1]) + (s_part[2] + s_part[3]);

@@ -1,8 +1,8 @@
 // Scores -> pyramid level map (and the index-list format), plus small map utilities.
 //
 // One workgroup per (b, h, q-block) row.  The row (<= a few thousand fp32 scores) lives in LDS:
-//   1. stable descending order by rank counting on a 64-bit key (inverted order-preserving score
-//      bits, then column index) - keys are unique so ties resolve to the lower column;
+//   1. stable descending order on a 64-bit key (inverted order-preserving score bits, then column
+//      index) - keys are unique so ties resolve to the lower column (sort_row_desc);
 //   2. thresholdbound only: sequential fp64 prefix sums rounded to fp32 (one lane walks the row,
 //      which keeps the additions in exactly the order a serial CPU scan uses), r = c / c[last] with
 //      an IEEE fp32 division, per-threshold counts of r <= thr;
@@ -34,7 +34,7 @@ extern "C" int psa_level_map(const float* scores, void* map_out, int map_elem_by
     hipError_t e = hipFuncSetAttribute((const void*)psa_level_map_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
     PSA_REQUIRE(e == hipSuccess, PSA_ERR_LAUNCH, "psa_level_map: cannot reserve %zu bytes of LDS", shmem);
   }
-  const int nt = Nk >= 256 ? 256 : ((Nk + 63) / 64) * 64;  // one thread per score up to 256: idle waves only take up slots
+  const int nt = Nk > RANK_SORT_MAX ? 256 : ((Nk + 63) / 64) * 64;  // one thread per score of a short row: idle waves only take up slots
   hipLaunchKernelGGL(psa_level_map_kernel, dim3((unsigned)rows), dim3(nt), shmem, (hipStream_t)stream, p);
   return psa_check_launch("psa_level_map");
 }
@@ -64,7 +64,7 @@ extern "C" int psa_level_map_qwen(const float* scores, void* map_out, int map_el
     hipError_t e = hipFuncSetAttribute((const void*)psa_level_map_qwen_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
     PSA_REQUIRE(e == hipSuccess, PSA_ERR_LAUNCH, "psa_level_map_qwen: cannot reserve %zu bytes of LDS", shmem);
   }
-  const int nt = S >= 256 ? 256 : ((S + 63) / 64) * 64;
+  const int nt = S > RANK_SORT_MAX ? 256 : ((S + 63) / 64) * 64;
   hipLaunchKernelGGL(psa_level_map_qwen_kernel, dim3((unsigned)(bh * S)), dim3(nt), shmem, (hipStream_t)stream, p);
   return psa_check_launch("psa_level_map_qwen");
 }

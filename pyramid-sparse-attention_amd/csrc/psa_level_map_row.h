@@ -31,24 +31,32 @@ __device__ __forceinline__ uint32_t desc_key(float s) {
   return ~u;                                   // descending
 }
 
-// Stable descending order of one row of scores: sw[i] / sidx[i] = score and column of sorted position i.
+// Stable descending order of one row of scores: sidx[i] = column of sorted position i, sw[i] its score.
 // The 64-bit keys (inverted score bits, column) are unique, so every correct sort gives the same order.
-// Rows of up to 256 scores are ranked by counting (one pass of N comparisons per score, no barriers inside);
-// longer rows (32-key blocks: 1024 scores) are sorted in place by a bitonic network over key[0 .. Npad), Npad the
-// next power of two, padded with keys that sort last: N/2 compare-exchanges per stage instead of N comparisons
-// per score (1024 scores: 55 stages of 2 exchanges per thread against 4096 comparisons per thread).
-constexpr int RANK_SORT_MAX = 256;
+// Rows of up to RANK_SORT_MAX scores are ranked by counting (one pass of N comparisons per score, no barriers inside).  Longer ones are
+// dealt to SORT_BINS bins, equal steps of the score bits between the row's best and worst (8 bins per octave if that is the whole
+// range of a float, more otherwise), and ranked by counting inside their bin: a few comparisons per score and seven barriers.
+// A bin of more than SORT_CAP scores (equal scores, mostly) sends the row to a bitonic network over key[0 .. sort_pad).
+// Against ranking up to 256 scores by counting and longer rows by the network, reduction + map of estimates by attention mass, us: 40 heads x
+// 10750 tokens of 32-key blocks (336 scores) 102 -> 66, 24 x 13273 (415) 73 -> 53, 12 x 32760 of 128-key blocks (256) 58 -> 46.
+constexpr int RANK_SORT_MAX = 128, SORT_BINS = 1024, SORT_CAP = 128;
 __host__ __device__ inline int sort_pad(int N) {
   if (N <= RANK_SORT_MAX) return N;
   int n = 1;
   while (n < N) n <<= 1;
   return n;
 }
-__device__ __forceinline__ void sort_row_desc(uint64_t* key, float* sw, int* sidx, const float* src, int N, int tid, int nt) {
-  const int Npad = sort_pad(N);
-  for (int j = tid; j < Npad; j += nt) key[j] = j < N ? (((uint64_t)desc_key(src[j]) << 32) | (uint32_t)j) : ~0ull;
-  __syncthreads();
+// LDS, in words of 4 bytes: [hist, later the prefix sums: sort_hist(N)][keys: 2 * sort_pad(N)][sw: N][sidx: N].  Rows longer than
+// RANK_SORT_MAX: 256 threads.
+__host__ __device__ inline int sort_hist(int N) {
+  const int n = (N + 3) & ~3;  // (the histogram and the keys behind it are read 16 bytes at a time)
+  return N > RANK_SORT_MAX && n < SORT_BINS ? SORT_BINS : n;
+}
+__host__ __device__ inline size_t sort_lds_bytes(int N) { return (size_t)sort_hist(N) * 4 + (size_t)sort_pad(N) * 8 + (size_t)N * 8; }
+__device__ __forceinline__ void sort_row_desc(uint64_t* key, float* sw, int* sidx, uint32_t* hist, const float* src, int N, int tid, int nt) {
   if (N <= RANK_SORT_MAX) {
+    for (int j = tid; j < N; j += nt) key[j] = ((uint64_t)desc_key(src[j]) << 32) | (uint32_t)j;
+    __syncthreads();
     for (int j = tid; j < N; j += nt) {
       const uint64_t kj = key[j];
       int rank = 0;
@@ -56,27 +64,105 @@ __device__ __forceinline__ void sort_row_desc(uint64_t* key, float* sw, int* sid
       sw[rank] = src[j];
       sidx[rank] = j;
     }
-  } else {
-    for (int k = 2; k <= Npad; k <<= 1) {
-      for (int j = k >> 1; j > 0; j >>= 1) {
-        for (int e = tid; e < (Npad >> 1); e += nt) {
-          // pair e of this stage: i has bit j clear, its partner is i + j; ascending where bit k of i is clear
-          const int i = ((e & ~(j - 1)) << 1) | (e & (j - 1));
-          const uint64_t a = key[i], b = key[i + j];
-          const bool up = (i & k) == 0;
-          if ((a > b) == up) {
-            key[i] = b;
-            key[i + j] = a;
+    __syncthreads();
+    return;
+  }
+  constexpr int NT = 256, NW = NT / 64;
+  static_assert(SORT_BINS == 4 * NT, "a thread scans four bins");
+  __shared__ uint32_t s_lo[NW], s_hi[NW], s_sum[NW], s_most[NW];
+  const int lane = tid & 63, wave = tid >> 6;
+  ((u32x4*)hist)[tid] = u32x4{0u, 0u, 0u, 0u};
+  uint32_t* kbuf = (uint32_t*)sidx;  // (the score bits, until the columns take their place)
+  uint32_t lo = 0xffffffffu, hi = 0u;
+  for (int j = tid; j < N; j += NT) {
+    const uint32_t k = desc_key(src[j]);
+    kbuf[j] = k;
+    lo = k < lo ? k : lo;
+    hi = k > hi ? k : hi;
+  }
+  lo = wave_min_u32(lo);
+  hi = wave_max_u32(hi);
+  if (lane == 0) {
+    s_lo[wave] = lo;
+    s_hi[wave] = hi;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    lo = s_lo[w] < lo ? s_lo[w] : lo;
+    hi = s_hi[w] > hi ? s_hi[w] : hi;
+  }
+  const int bits = 32 - __builtin_clz((hi - lo) | 1u), shift = bits > 10 ? bits - 10 : 0;
+  static_assert(SORT_BINS == 1 << 10, "bins");
+  for (int j = tid; j < N; j += NT) atomicAdd(&hist[(kbuf[j] - lo) >> shift], 1u);
+  __syncthreads();
+  {
+    u32x4 c = ((const u32x4*)hist)[tid];
+    const uint32_t sum = c[0] + c[1] + c[2] + c[3];
+    uint32_t most = c[0] > c[1] ? c[0] : c[1];
+    most = c[2] > most ? c[2] : most;
+    most = wave_max_u32(c[3] > most ? c[3] : most);
+    uint32_t run = (uint32_t)wave_scan_add((int)sum);
+    if (lane == 63) s_sum[wave] = run;
+    if (lane == 0) s_most[wave] = most;
+    run -= sum;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < NW; ++w) run += w < wave ? s_sum[w] : 0u;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t n = c[e];
+      c[e] = run;
+      run += n;
+    }
+    ((u32x4*)hist)[tid] = c;
+    most = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) most = s_most[w] > most ? s_most[w] : most;
+    if (most > (uint32_t)SORT_CAP) {  // (uniform)
+      const int Npad = sort_pad(N);
+      for (int j = tid; j < Npad; j += NT) key[j] = j < N ? (((uint64_t)kbuf[j] << 32) | (uint32_t)j) : ~0ull;
+      __syncthreads();
+      for (int k = 2; k <= Npad; k <<= 1) {
+        for (int j = k >> 1; j > 0; j >>= 1) {
+          for (int e = tid; e < (Npad >> 1); e += NT) {
+            // pair e of this stage: i has bit j clear, its partner is i + j; ascending where bit k of i is clear
+            const int i = ((e & ~(j - 1)) << 1) | (e & (j - 1));
+            const uint64_t a = key[i], b = key[i + j];
+            const bool up = (i & k) == 0;
+            if ((a > b) == up) {
+              key[i] = b;
+              key[i + j] = a;
+            }
           }
+          __syncthreads();
         }
-        __syncthreads();
       }
+      for (int i = tid; i < N; i += NT) {
+        const int col = (int)(uint32_t)key[i];
+        sidx[i] = col;
+        sw[i] = src[col];
+      }
+      __syncthreads();
+      return;
     }
-    for (int i = tid; i < N; i += nt) {
-      const int col = (int)(uint32_t)key[i];
-      sidx[i] = col;
-      sw[i] = src[col];
-    }
+  }
+  __syncthreads();
+  // hist[b]: the next free place of bin b, in the end the first place of bin b + 1
+  for (int j = tid; j < N; j += NT) {
+    const uint32_t k = kbuf[j];
+    key[atomicAdd(&hist[(k - lo) >> shift], 1u)] = ((uint64_t)k << 32) | (uint32_t)j;
+  }
+  __syncthreads();
+  for (int i = tid; i < N; i += NT) {
+    const uint64_t mine = key[i];
+    const uint32_t bin = ((uint32_t)(mine >> 32) - lo) >> shift;
+    const int first = bin > 0 ? (int)hist[bin - 1] : 0, last = (int)hist[bin];
+    int rank = first;
+    for (int e = first; e < last; ++e) rank += key[e] < mine ? 1 : 0;
+    const int col = (int)(uint32_t)mine;
+    sidx[rank] = col;
+    sw[rank] = src[col];
   }
   __syncthreads();
 }
@@ -93,15 +179,26 @@ __device__ __forceinline__ void row_prefix_sums(double* wide, const float* sw, f
   if (tid == 0) {
     __builtin_amdgcn_s_setprio(3);
     double acc = 0.0;
+    // eight scores at a time, the next eight requested before they are added: the chain is the additions, not the LDS
+    f64x2 w[4], nx[4];
+    const int n8 = N & ~7;
+    if (n8 > 0) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) nx[e] = *(const f64x2*)(wide + 2 * e);
+    }
     int i = 0;
-    for (; i + 4 <= N; i += 4) {
-      const f64x2 w0 = *(const f64x2*)(wide + i), w1 = *(const f64x2*)(wide + i + 2);
-      const double a0 = acc + w0[0];
-      const double a1 = a0 + w0[1];
-      const double a2 = a1 + w1[0];
-      acc = a2 + w1[1];
-      *(f64x2*)(wide + i) = f64x2{a0, a1};
-      *(f64x2*)(wide + i + 2) = f64x2{a2, acc};
+    for (; i < n8; i += 8) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w[e] = nx[e];
+      const int at = i + 8 < n8 ? i + 8 : i;  // (the last one's repeat is not used)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) nx[e] = *(const f64x2*)(wide + at + 2 * e);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        w[e][0] = acc + w[e][0];
+        w[e][1] = acc = w[e][0] + w[e][1];
+        *(f64x2*)(wide + i + 2 * e) = w[e];
+      }
     }
     for (; i < N; ++i) {
       acc += wide[i];
@@ -124,14 +221,14 @@ __device__ __forceinline__ void row_prefix_sums(double* wide, const float* sw, f
 // 0.25: 21 / 26 / 34 / 41, bitonic network 65 to 71 whatever the scores; 3072 rows of 512: 17 / 18 / 20 / 28 against 34; of
 // 2048: 31 / 46 / 58 / 60 against 200.  (Building the cut key bit by bit over the whole row instead of descending: 21 / 58 / 138 /
 // 266 at 1024 scores.)  With the reduction of the estimator's workspace, which the launch also does and which bounds it: 16944
-// rows of 1410 scores 1480 -> 600 us (3.05 GB read, 5.1 TB/s).  Below RANK_SORT_MAX ranking by counting is as fast and also
+// rows of 1410 scores 1480 -> 600 us (3.05 GB read, 5.1 TB/s).  Up to SEL_MIN scores sorting is as fast and also
 // serves the other modes.
 // LDS: (SEL_BINS + 2 * SEL_MAX_CUTS * SEL_CAP + 8 * SEL_MAX_CUTS) 4-byte words.  256 threads.
-constexpr int SEL_BINS = 1024, SEL_SHIFT = 19, SEL_CAP = 64, SEL_MAX_CUTS = 8;
+constexpr int SEL_MIN = 256, SEL_BINS = 1024, SEL_SHIFT = 19, SEL_CAP = 64, SEL_MAX_CUTS = 8;
 constexpr int SEL_COL_BITS = 13;  // columns of a row: at most 6144
 constexpr size_t SEL_LDS_BYTES = (SEL_BINS + 2 * SEL_MAX_CUTS * SEL_CAP + 8 * SEL_MAX_CUTS) * 4;
 __host__ __device__ inline bool level_map_selects(int mode, int n_cuts, int Nk) {
-  return mode == PSA_MODE_TOPK && n_cuts <= SEL_MAX_CUTS && Nk > RANK_SORT_MAX;
+  return mode == PSA_MODE_TOPK && n_cuts <= SEL_MAX_CUTS && Nk > SEL_MIN;
 }
 __device__ __forceinline__ void level_map_row_select(const LevelMapParams& p, const float* src, int64_t row, unsigned char* smem, int tid,
                                                      uint8_t* lds_out) {
@@ -154,11 +251,7 @@ __device__ __forceinline__ void level_map_row_select(const LevelMapParams& p, co
     const uint32_t k = desc_key(src[j]);
     kmin = k < kmin ? k : kmin;
   }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const uint32_t other = (uint32_t)__shfl_xor((int)kmin, o, 64);
-    kmin = other < kmin ? other : kmin;
-  }
+  kmin = wave_min_u32(kmin);
   if (lane == 0) wsum[wave] = (int)kmin;
   __syncthreads();
 #pragma unroll
@@ -180,12 +273,7 @@ __device__ __forceinline__ void level_map_row_select(const LevelMapParams& p, co
       c[e] = hist[tid * PER + e];
       sum += c[e];
     }
-    int incl = sum;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int up = __shfl_up(incl, d, 64);
-      incl += lane >= d ? up : 0;
-    }
+    const int incl = wave_scan_add(sum);
     if (lane == 63) wsum[4 + wave] = incl;
     __syncthreads();
     int run = incl - sum;
@@ -301,13 +389,14 @@ __device__ __forceinline__ void level_map_row(const LevelMapParams& p, const flo
     level_map_row_select(p, src, row, smem, tid, lds_out);
     return;
   }
-  uint64_t* key = (uint64_t*)smem;            // [sort_pad(N)]
+  uint32_t* hist = (uint32_t*)smem;           // [sort_hist(N)]
+  float* c32 = (float*)hist;                  // [N] prefix sums
+  uint64_t* key = (uint64_t*)(hist + sort_hist(N));  // [sort_pad(N)]
   float* sw = (float*)(key + sort_pad(N));    // [N] scores in sorted order
   int* sidx = (int*)(sw + N);                 // [N] column of sorted position
-  float* c32 = (float*)(sidx + N);            // [N] prefix sums
 
   if (tid < PSA_MAX_LEVEL_ITEMS) s_cnt[tid] = 0;
-  sort_row_desc(key, sw, sidx, src, N, tid, nt);
+  sort_row_desc(key, sw, sidx, hist, src, N, tid, nt);
 
   if (p.mode == PSA_MODE_THRESHOLDBOUND) {
     row_prefix_sums((double*)key, sw, c32, N, tid, nt);
@@ -413,18 +502,19 @@ struct QwenMapParams {
   int causal;
 };
 // LDS of a row of n scores
-__host__ __device__ inline size_t qwen_row_lds_bytes(int n) { return (size_t)sort_pad(n) * 8 + (size_t)n * 12; }
+__host__ __device__ inline size_t qwen_row_lds_bytes(int n) { return sort_lds_bytes(n); }
 // Levels of row i_row from its scores `src`, handed to store(column, level).  Only the first n columns are ranked: n = S, or the
 // i_row + 1 columns of a causal row whose other scores are all 0 - those sort last whatever the rest (no score is negative), add
 // nothing to a prefix sum and are skipped above the diagonal anyway.
 template <class Store>
 __device__ __forceinline__ void qwen_map_row(const QwenMapParams& p, const float* src, int i_row, int n, unsigned char* smem, int tid, int nt,
                                              Store store) {
-  uint64_t* key = (uint64_t*)smem;
+  uint32_t* hist = (uint32_t*)smem;
+  float* c32 = (float*)hist;
+  uint64_t* key = (uint64_t*)(hist + sort_hist(n));
   float* sw = (float*)(key + sort_pad(n));
   int* sidx = (int*)(sw + n);
-  float* c32 = (float*)(sidx + n);
-  sort_row_desc(key, sw, sidx, src, n, tid, nt);
+  sort_row_desc(key, sw, sidx, hist, src, n, tid, nt);
   if (p.mode == PSA_MODE_THRESHOLDBOUND) row_prefix_sums((double*)key, sw, c32, n, tid, nt);
   const float total = p.mode == PSA_MODE_THRESHOLDBOUND ? fmaxf(c32[n - 1], 1e-10f) : 1.f;
   const float valid_len = p.causal ? (float)(i_row + 1) : (float)p.S;
@@ -554,5 +644,5 @@ static inline int level_map_fill_params(LevelMapParams& p, int Nk, int mode, int
 // LDS scratch of level_map_row: of the selection where it serves the call (dense maps by quotas), else of the sort
 static inline size_t level_map_lds_bytes(const LevelMapParams& p) {
   if (p.list_out == nullptr && level_map_selects(p.mode, p.n_cuts, p.Nk)) return SEL_LDS_BYTES;
-  return (size_t)sort_pad(p.Nk) * 8 + (size_t)p.Nk * (4 + 4 + 4);
+  return sort_lds_bytes(p.Nk);
 }
