@@ -378,6 +378,47 @@ __global__ __launch_bounds__(256) void psa_bwd_cost_kernel(BwdParams p, int row_
 // ------------------------------------------------------------------------------------------------------
 constexpr int B_ISTR = LT_ISTR;  // bytes between the blocks of a tile
 
+// Gradients of the replicate-pad rows L .. npad - 1, which land on the last real token: over the pooled rows behind it, each counted
+// with its share of pad tokens.  By the 256 threads of the workgroup that owns that token (barriers inside), dK to fold[0 .. D) and dV to
+// fold[D .. 2 D); part: 2048 floats of LDS.  One lane that walks the pad tokens of its channels, three loads each, holds up the whole
+// launch: 16 heads of 3484 x 128 (100 pad tokens) 223 us for a walk of 50.
+template <int D>
+__device__ __forceinline__ void fold_pad_rows(const BwdParams& p, int bhk, int tid, float* part, float* fold) {
+  constexpr int CH = D / 4, NG = 256 / CH;
+  const int c = tid % CH, g = tid / CH;
+  const int64_t BH = (int64_t)p.B * p.Hkv;
+  f32x4 k = {0.f, 0.f, 0.f, 0.f}, v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int l = 1; l < 4; ++l) {
+    const int64_t rows = BH * p.npad + pool_row_offset(l, BH, bhk, p.npad);
+    const int t0 = p.L >> l, t1 = (int)(p.npad >> l);
+#pragma unroll 2
+    for (int t = t0 + g; t < t1; t += NG) {
+      const f32x4 x = *(const f32x4*)(p.wk + (rows + t) * D + c * 4), y = *(const f32x4*)(p.wv + (rows + t) * D + c * 4);
+      const float share = t == t0 ? (float)(((t0 + 1) << l) - p.L) / (float)(1 << l) : 1.f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        k[e] = __builtin_fmaf(x[e], share, k[e]);
+        v[e] = __builtin_fmaf(y[e], share, v[e]);
+      }
+    }
+  }
+  f32x4* const sums = (f32x4*)part;  // [tensor][group][chunk]
+  sums[tid] = k;
+  sums[256 + tid] = v;
+  __syncthreads();
+  if (tid < 2 * CH) {
+    f32x4 a = sums[(tid / CH) * 256 + tid % CH];
+    for (int i = 1; i < NG; ++i) {
+      const f32x4 x = sums[(tid / CH) * 256 + i * CH + tid % CH];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) a[e] += x[e];
+    }
+    ((f32x4*)fold)[tid] = a;
+  }
+  __syncthreads();
+}
+
 // One instantiation per kind of slot (WIDE: the 128-key level-0 slot; else the slots slot_lo .. slot_lo + slot_cnt - 1 of
 // every kv-block); workgroup id = ((b * Hkv + kv head) * Nk + kv-block) * slot_cnt + (slot - slot_lo), optionally
 // re-ordered.
@@ -662,8 +703,14 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
   // ---- 128-key level-0 slot: this workgroup owns 128 tokens of dK / dV outright.  The pooled levels' launch has
   // finished, so the tokens' shares of the pooled gradients (1/l of pooled row n >> level; for the last real token
   // also those of the replicate-pad tokens behind it) are added here and dK, dV leave in the tensors' 16-bit type: no fp32 level-0
-  // buffer, no separate pass.  Same sums in the same order as psa_bwd_unpool_kernel.
+  // buffer, no separate pass.
   if constexpr (WIDE) {
+    float* const fold = (float*)smem;
+    const bool folds = key_row0 + 128 >= L && p.npad > L;  // (this workgroup owns the last token, and there are pad rows)
+    if (folds) {
+      __syncthreads();
+      fold_pad_rows<D>(p, bhk, wave * 64 + ln, fold + 2 * D, fold);
+    }
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) {
       const int64_t n = key_row0 + kh * 32 + (ln & 15) + 16 * kb;
@@ -705,14 +752,12 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
               gv[e] += av[e];
             }
           }
-          if (n == L - 1) {  // gradient of the replicate-pad rows lands on the last real token
-            for (int64_t r = L; r < npad; ++r) {
-              const f32x4 ak = contrib(lk, r, col), av = contrib(lvv, r, col);
+          if (folds && n == L - 1) {
+            const f32x4 ak = *(const f32x4*)(fold + col), av = *(const f32x4*)(fold + D + col);
 #pragma unroll
-              for (int e = 0; e < 4; ++e) {
-                gk[e] += ak[e];
-                gv[e] += av[e];
-              }
+            for (int e = 0; e < 4; ++e) {
+              gk[e] += ak[e];
+              gv[e] += av[e];
             }
           }
           u32x2 ok_, ov_;
@@ -802,11 +847,17 @@ __global__ __launch_bounds__(256) void psa_bwd_unpool_kernel(BwdParams p, int D)
 #pragma unroll
     for (int e = 0; e < 4; ++e) g[e] += a[e];
   }
-  if (n == p.L - 1) {  // gradient of the replicate-pad rows lands on the last real token
-    for (int64_t r = p.L; r < npad; ++r) {
-      const f32x4 a = contrib(r);
+  if (n == p.L - 1) {  // gradient of the replicate-pad rows lands on the last real token (fold_pad_rows)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) g[e] += a[e];
+    for (int lv = 1; lv < 4; ++lv) {
+      const int t0 = p.L >> lv, t1 = (int)(npad >> lv);
+#pragma unroll 4
+      for (int t = t0; t < t1; ++t) {
+        const f32x4 x = *(const f32x4*)(wl[lv - 1] + (int64_t)t * D + c * 4);
+        const float share = t == t0 ? (float)(((t0 + 1) << lv) - p.L) / (float)(1 << lv) : 1.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) g[e] = __builtin_fmaf(x[e], share, g[e]);
+      }
     }
   }
   bf16_t* dst = which == 0 ? p.dk + b * p.dk_sb + hk * p.dk_sh + n * p.dk_sl : p.dv + b * p.dv_sb + hk * p.dv_sh + n * p.dv_sl;
