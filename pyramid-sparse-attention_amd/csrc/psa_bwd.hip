@@ -319,9 +319,9 @@ constexpr int COL_BINS = psa_order::COST_BINS;
 // per list) and two cost launches and three sorts one after the other left the chip nearly idle.  Measured now 9 + 12.5 us;
 // training step of 48 heads x 8776 x 64 1208 -> 1198 us, of 12 heads x 32760 x 128 4549 -> 4543 us.  The first row_wgs workgroups: four rows each, costs of the dQ walk.  The others, one per
 // (kv head, kv-block): per-level counts over the column -> cost of each of its slots.  The
-// costs of the slots slot_lo .. of all blocks form one list per dK/dV launch: with a 128-key slot 0 that slot's list comes first
-// (n_blocks entries), then the list of the slots 1 .. 3.  The 128-key slots' costs are in units of wide_div q-blocks.
-__global__ __launch_bounds__(256) void psa_bwd_cost_kernel(BwdParams p, int row_wgs, int32_t* cost_row, int wide0, int wide_div, int32_t* cost) {
+// costs of the slots slot_lo .. of all blocks form one list per dK/dV launch; with a 128-key slot 0 that slot's costs are a list of their
+// own (cost0, in units of wide_div q-blocks), or its lengths go to count0 and psa_bwd_parts_kernel makes the list.
+__global__ __launch_bounds__(256) void psa_bwd_cost_kernel(BwdParams p, int row_wgs, int32_t* cost_row, int wide0, int wide_div, int32_t* count0, int32_t* cost0, int32_t* cost) {
   __shared__ int s_n[4];
   if ((int)blockIdx.x < row_wgs) {
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -354,10 +354,87 @@ __global__ __launch_bounds__(256) void psa_bwd_cost_kernel(BwdParams p, int row_
   if ((int)threadIdx.x < DKDV_SLOTS) {
     const int lv = (int)threadIdx.x;
     const int c = s_n[lv] < COL_BINS - 1 ? s_n[lv] : COL_BINS - 1;
-    const int64_t n_blocks = (int64_t)p.B * p.Hkv * p.Nk;
     if (!wide0) cost[blk * DKDV_SLOTS + lv] = c;
-    else if (lv == 0) cost[blk] = s_n[0] / wide_div < COL_BINS - 1 ? s_n[0] / wide_div : COL_BINS - 1;
-    else cost[n_blocks + blk * (DKDV_SLOTS - 1) + (lv - 1)] = c;
+    else if (lv == 0) {
+      if (count0 != nullptr) count0[blk] = s_n[0];
+      else cost0[blk] = s_n[0] / wide_div < COL_BINS - 1 ? s_n[0] / wide_div : COL_BINS - 1;
+    }
+    else cost[blk * (DKDV_SLOTS - 1) + (lv - 1)] = c;
+  }
+}
+
+// ------------------------------------------------------------------------------------------------------
+// 128-key slots in parts.  A few key blocks are kept by nearly every q-block, others by one or two, and a launch that the chip holds in
+// one round or little more takes as long as its longest slot (16 heads of 3484 x 128 114 us beside a dQ walk of 55).  A list longer
+// than one and a half units is cut into parts of at most a unit, a workgroup each; the parts leave fp32 sums in the level-0 part of the
+// workspace, which 128-key slots do not use otherwise, and psa_bwd_join_kernel adds them in order.
+// The unit is PART_MEAN times the mean list of the slot's own head, PART_MIN q-blocks of 128 rows at least: the parts follow from the
+// head's map alone, and they fit its share of that buffer (cut slots have fewer than 1.5 * pairs / unit parts).
+// An item: {kv-block | part << 16 | parts << 24, its slot of the buffer}; a head's items are its slots' first parts (even entries) and
+// the other parts, spread over the odd entries.  Unused: parts = 0.
+// Training steps without / with parts, us, fixed quotas and thresholds: 12 heads of 2500 x 128 250 / 184 and 247 / 232, 8 of 5300 x 128 326 /
+// 267 and 334 / 318, 12 of 5300 x 128 360 / 293 and 382 / 355, 24 of 4000 x 128 (768 slots) 370 / 353 and 429 / 430; head dim 64: 8 of
+// 9000 369 / 321 and 379 / 349, 8 of 16000 (1000 slots) 629 / 629 and 627 / 605.  Larger launches lose: slots that walk the same q-blocks
+// at the same time share their rows in L2, parts do not, and the sums cost traffic (12 of 9000 x 128, 852 slots, 604 / 631 and 699 / 739).
+constexpr int PART_MEAN_10 = 17, PART_MIN = 4, PART_MOST = 64;
+constexpr int parts_max_slots(int D) { return D == 128 ? 768 : 1024; }  // (the chip holds 512 / 768 workgroups at once)
+__device__ __forceinline__ int part_at(int n, int part, int parts) { return (int)((int64_t)n * part / parts); }
+
+__global__ __launch_bounds__(256) void psa_bwd_parts_kernel(const int32_t* count0, int Nk, int min_unit, int wide_div, u32x2* items, int32_t* cost) {
+  __shared__ int s_sum[4], s_more[4];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int64_t head = blockIdx.x;
+  const int32_t* n_of = count0 + head * Nk;
+  items += head * 2 * Nk;
+  cost += head * 2 * Nk;
+  auto total = [&](int v, int* sums) __attribute__((always_inline)) {  // over the workgroup
+    v = wave_scan_add(v);
+    if (lane == 63) sums[wave] = v;
+    __syncthreads();
+    return sums[0] + sums[1] + sums[2] + sums[3];
+  };
+  int pairs = 0;
+  for (int j = tid; j < Nk; j += 256) {
+    pairs += n_of[j];
+    items[2 * j + 1] = u32x2{0u, 0u};
+    cost[2 * j + 1] = 0;
+  }
+  pairs = total(pairs, s_sum);
+  const int mean = (int)(((int64_t)PART_MEAN_10 * pairs + 10 * Nk - 1) / (10 * Nk));
+  const int unit = mean > min_unit ? mean : min_unit;
+  auto parts_of = [&](int n) __attribute__((always_inline)) {
+    if (n <= unit + unit / 2) return 1;
+    const int q = (n + unit - 1) / unit;
+    return q < PART_MOST ? q : PART_MOST;
+  };
+  int more = 0;
+  for (int j = tid; j < Nk; j += 256) more += parts_of(n_of[j]) - 1;
+  more = total(more, s_more);
+  int at = 0, slot_at = 0;  // further parts and buffer slots of the columns before this round
+  for (int j0 = 0; j0 < Nk; j0 += 256) {
+    const int j = j0 + tid, n = j < Nk ? n_of[j] : 0, parts = parts_of(n);
+    const int e = parts - 1, sl = parts > 1 ? parts : 0;
+    const int e_to = wave_scan_add(e), sl_to = wave_scan_add(sl);
+    __syncthreads();
+    if (lane == 63) {
+      s_sum[wave] = e_to;
+      s_more[wave] = sl_to;
+    }
+    __syncthreads();
+    int first = at + e_to - e, slot = slot_at + sl_to - sl;
+    for (int w = 0; w < wave; ++w) {
+      first += s_sum[w];
+      slot += s_more[w];
+    }
+    if (j < Nk)
+      for (int part = 0; part < parts; ++part) {
+        const int len = part_at(n, part + 1, parts) - part_at(n, part, parts), c = len / wide_div;
+        const int pos = part == 0 ? 2 * j : 2 * (int)((int64_t)(first + part - 1) * Nk / more) + 1;
+        items[pos] = u32x2{(uint32_t)j | ((uint32_t)part << 16) | ((uint32_t)parts << 24), (uint32_t)(head * Nk + slot + part)};
+        cost[pos] = c < COL_BINS - 1 ? c : COL_BINS - 1;
+      }
+    at += s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3];
+    slot_at += s_more[0] + s_more[1] + s_more[2] + s_more[3];
   }
 }
 
@@ -420,11 +497,11 @@ __device__ __forceinline__ void fold_pad_rows(const BwdParams& p, int bhk, int t
 }
 
 // One instantiation per kind of slot (WIDE: the 128-key level-0 slot; else the slots slot_lo .. slot_lo + slot_cnt - 1 of
-// every kv-block); workgroup id = ((b * Hkv + kv head) * Nk + kv-block) * slot_cnt + (slot - slot_lo), optionally
-// re-ordered.
+// every kv-block); workgroup id = ((b * Hkv + kv head) * Nk + kv-block) * slot_cnt + (slot - slot_lo), or the entry of items (WIDE),
+// optionally re-ordered.
 template <int D, bool WIDE, bool CAUSAL, class ET>
 __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, int slot_lo, int slot_cnt, int n_wg, int chunk,
-                                                                 const int32_t* order) {
+                                                                 const int32_t* order, const u32x2* items) {
   using G = LtGeom<D>;
   using x8 = typename ET::x8;
   constexpr int KK = D / 32, DB = D / 16, RPL = G::RPL;
@@ -440,8 +517,18 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
   if (order != nullptr) wg = order[wg];
   if (wg < 0 || wg >= n_wg) return;
   const int slot = slot_lo + wg % slot_cnt;
-  const int J = (wg / slot_cnt) % p.Nk;
-  const int bhk = wg / (slot_cnt * p.Nk), b = bhk / p.Hkv, hk = bhk % p.Hkv;
+  int J = (wg / slot_cnt) % p.Nk, bhk = wg / (slot_cnt * p.Nk), part = 0, parts = 1, part_slot = 0;
+  if constexpr (WIDE)
+    if (items != nullptr) {
+      const uint32_t it = __builtin_amdgcn_readfirstlane(items[wg][0]);
+      part_slot = __builtin_amdgcn_readfirstlane(items[wg][1]);
+      J = (int)(it & 0xffffu);
+      bhk = wg / (2 * p.Nk);
+      part = (int)((it >> 16) & 255u);
+      parts = (int)(it >> 24);
+      if (parts == 0) return;
+    }
+  const int b = bhk / p.Hkv, hk = bhk % p.Hkv;
   const int n_rep = p.Hq / p.Hkv;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, lg = lane >> 4;
@@ -516,7 +603,12 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
   // last token that the pooled key covers (< npad); block kb: + 16 << lv
   const int key_up = (int)(((key_row0 + key_local + 1) << lv) - 1);
   __syncthreads();
-  const int nq = s_nq;
+  int nq = s_nq;
+  if constexpr (WIDE) {
+    const int from = part_at(nq, part, parts);
+    nq = part_at(nq, part + 1, parts) - from;
+    qlist += from;
+  }
 
   // ---- lane-invariant LDS addressing (tile layout: see the forward kernel) ---------------------------
   // copy: wave w fills the 16-row group w of both tiles; lane (fq = lane / CH, pos = lane % CH) of block n writes
@@ -705,6 +797,17 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
   // also those of the replicate-pad tokens behind it) are added here and dK, dV leave in the tensors' 16-bit type: no fp32 level-0
   // buffer, no separate pass.
   if constexpr (WIDE) {
+    if (parts > 1) {  // fp32 sums of this part, in the accumulators' layout (psa_bwd_join_kernel)
+      const int64_t at = (int64_t)part_slot * (128 * D) + (int64_t)kh * (2 * DB * 256) + ln * 4;
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int db = 0; db < DB; ++db) {
+          *(f32x4*)(p.wk + at + (kb * DB + db) * 256) = dk[kb][db];
+          *(f32x4*)(p.wv + at + (kb * DB + db) * 256) = dv[kb][db];
+        }
+      return;
+    }
     float* const fold = (float*)smem;
     const bool folds = key_row0 + 128 >= L && p.npad > L;  // (this workgroup owns the last token, and there are pad rows)
     if (folds) {
@@ -812,6 +915,82 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
 
 }
 
+// The 128-key slots that were cut: their parts added in order, then what ends such a slot (above), four channels of one token per
+// thread: a wave has 16 tokens and 16 channels.  (The workgroups of the other slots have nothing to do.)
+template <int D, class ET>
+__global__ __launch_bounds__(256) void psa_bwd_join_kernel(BwdParams p, const u32x2* items) {
+  constexpr int PER = D / 8;  // workgroups per slot
+  const int J = (int)blockIdx.x / PER, bhk = (int)blockIdx.y;
+  const u32x2 it = items[((int64_t)bhk * p.Nk + J) * 2];
+  const int parts = (int)(it[0] >> 24);
+  if (parts < 2) return;
+  const int unit = ((int)blockIdx.x % PER) * 256 + (int)threadIdx.x, lane = unit & 63, blk = unit >> 6;  // blk: (key block of 16, channel block of 16)
+  const int64_t n = (int64_t)J * 128 + (blk / (D / 16)) * 16 + (lane & 15), L = p.L;
+  const int col = (blk % (D / 16)) * 16 + (lane >> 4) * 4;
+  const int64_t at = (int64_t)it[1] * (128 * D) + unit * 4;
+  f32x4 gk = *(const f32x4*)(p.wk + at), gv = *(const f32x4*)(p.wv + at);
+  for (int part = 1; part < parts; ++part) {
+    const f32x4 x = *(const f32x4*)(p.wk + at + (int64_t)part * (128 * D)), y = *(const f32x4*)(p.wv + at + (int64_t)part * (128 * D));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      gk[e] += x[e];
+      gv[e] += y[e];
+    }
+  }
+  const int64_t BH = (int64_t)p.B * p.Hkv;
+  f32x4 ak = {0.f, 0.f, 0.f, 0.f}, av = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int l = 1; l < 4; ++l) {
+    const int64_t row = BH * p.npad + pool_row_offset(l, BH, bhk, p.npad) + (n >> l);
+    const f32x4 x = *(const f32x4*)(p.wk + row * D + col), y = *(const f32x4*)(p.wv + row * D + col);
+    const float inv = 1.0f / (float)(1 << l);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      ak[e] += x[e] * inv;
+      av[e] += y[e] * inv;
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    gk[e] = gk[e] * p.scale + ak[e];
+    gv[e] += av[e];
+  }
+  const int64_t first = n - (lane & 15);
+  if (first < L && first + 16 >= L && p.npad > L) {  // (uniform) the wave of the last token: the pad rows' gradients, 16 lanes per chunk
+    f32x4 k = {0.f, 0.f, 0.f, 0.f}, v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int l = 1; l < 4; ++l) {
+      const int64_t rows = BH * p.npad + pool_row_offset(l, BH, bhk, p.npad);
+      const int t0 = p.L >> l, t1 = (int)(p.npad >> l);
+      for (int t = t0 + (lane & 15); t < t1; t += 16) {
+        const f32x4 x = *(const f32x4*)(p.wk + (rows + t) * D + col), y = *(const f32x4*)(p.wv + (rows + t) * D + col);
+        const float share = t == t0 ? (float)(((t0 + 1) << l) - p.L) / (float)(1 << l) : 1.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          k[e] = __builtin_fmaf(x[e], share, k[e]);
+          v[e] = __builtin_fmaf(y[e], share, v[e]);
+        }
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      auto sum16 = [](float a) __attribute__((always_inline)) {
+        a += dpp_f32<DPP_ROW_ROR + 8>(a);
+        a += dpp_f32<DPP_ROW_ROR + 4>(a);
+        a += dpp_f32<DPP_ROW_ROR + 2>(a);
+        return a + dpp_f32<DPP_ROW_ROR + 1>(a);
+      };
+      const float sk = sum16(k[e]), sv = sum16(v[e]);
+      gk[e] += n == L - 1 ? sk : 0.f;
+      gv[e] += n == L - 1 ? sv : 0.f;
+    }
+  }
+  if (n >= L) return;
+  const int b = bhk / p.Hkv, hk = bhk % p.Hkv;
+  *(u32x2*)(p.dk + b * p.dk_sb + hk * p.dk_sh + n * p.dk_sl + col) = u32x2{ET::pack2(gk[0], gk[1]), ET::pack2(gk[2], gk[3])};
+  *(u32x2*)(p.dv + b * p.dv_sb + hk * p.dv_sh + n * p.dv_sl + col) = u32x2{ET::pack2(gv[0], gv[1]), ET::pack2(gv[2], gv[3])};
+}
+
 // ------------------------------------------------------------------------------------------------------
 // un-pool: levels -> dK, dV (the tensors' 16-bit type)
 // ------------------------------------------------------------------------------------------------------
@@ -874,10 +1053,11 @@ extern "C" int64_t psa_bwd_workspace_bytes(int B, int Hq, int Hkv, int L, int D,
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || L <= 0 || D <= 0 || block_n <= 0) return 0;
   const int64_t npad = (int64_t)((L + block_n - 1) / block_n) * block_n;
   const int64_t levels = (int64_t)B * Hkv * D * (npad + npad / 2 + npad / 4 + npad / 8);
-  // + cost and issue order of the dQ rows (block_m >= 64) and of the dK/dV slots (4 per kv-block), padded to whole shares
+  // + cost and issue order of the dQ rows (block_m >= 64) and of the dK/dV slots (4 per kv-block, or lengths, 2 items and 3 slots), padded to
+  // whole shares, and the items
   const int64_t pad = 16 * psa_order::MAX_PHASES;
-  const int64_t n_rows = (int64_t)B * Hq * ((L + 63) / 64), n_slots = (int64_t)B * Hkv * ((L + block_n - 1) / block_n) * DKDV_SLOTS;
-  return (2 * levels + 2 * (int64_t)B * Hq * L + 2 * (n_rows + pad) + 2 * (n_slots + 2 * pad)) * (int64_t)sizeof(float);
+  const int64_t n_rows = (int64_t)B * Hq * ((L + 63) / 64), n_blocks = (int64_t)B * Hkv * ((L + block_n - 1) / block_n);
+  return (2 * levels + 2 * (int64_t)B * Hq * L + 2 * (n_rows + pad) + (6 + 5 + 4) * n_blocks + 4 * pad) * (int64_t)sizeof(float);
 }
 
 extern "C" int psa_bwd(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const void* k_pool, const void* v_pool, const void* map,
@@ -953,8 +1133,10 @@ extern "C" int psa_bwd(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const void* 
   // (if block_n = 128) and the other slots.
   const int64_t total = (int64_t)B * Hq * Mq, n_blocks = (int64_t)B * Hkv * Nk;
   const bool wide0 = block_n > 64;
-  const int64_t n_wide = wide0 ? n_blocks : 0, n_rest = n_blocks * (wide0 ? DKDV_SLOTS - 1 : DKDV_SLOTS);
-  PSA_REQUIRE(total < (1ll << 28) && n_wide + n_rest < (1ll << 28), PSA_ERR_UNSUPPORTED, "psa_bwd: too many workgroups");
+  const bool cols_ordered = map != nullptr && n_blocks > 8;
+  const bool in_parts = cols_ordered && wide0 && n_blocks <= parts_max_slots(D);
+  const int64_t n_wide = wide0 ? (in_parts ? 2 * n_blocks : n_blocks) : 0, n_rest = n_blocks * (wide0 ? DKDV_SLOTS - 1 : DKDV_SLOTS);
+  PSA_REQUIRE(total < (1ll << 28) && 4 * n_blocks < (1ll << 28), PSA_ERR_UNSUPPORTED, "psa_bwd: too many workgroups");
   // shares by the K/V rows (dQ) and the Q/dO rows (dK/dV) that the walks stream
   const double kv_bytes = 2.0 * B * Hkv * (double)p.npad * D * 2.0 * (map != nullptr ? 1.875 : 1.0);
   const double qdo_bytes = 2.0 * B * Hq * (double)L * D * 2.0;
@@ -963,13 +1145,17 @@ extern "C" int psa_bwd(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const void* 
   if (wide0) psa_order::deal(n_wide, qdo_bytes, B * Hkv, chunk_w, groups_w);
   psa_order::deal(n_rest, qdo_bytes, B * Hkv, chunk_r, groups_r);
   const int32_t *order = nullptr, *order_wide = nullptr, *order_rest = nullptr;
-  const bool rows_ordered = map != nullptr && total > 8 * 32, cols_ordered = map != nullptr && n_blocks > 8;
+  const u32x2* items_wide = nullptr;
+  const bool rows_ordered = map != nullptr && total > 8 * 32;
   if (rows_ordered || cols_ordered) {
     int32_t* cost = (int32_t*)(p.nlse2 + (int64_t)B * Hq * L);
     int32_t* ord = cost + total;
-    int32_t* cost_c = cost + 2 * total + 16 * psa_order::MAX_PHASES;
-    int32_t* ord_w = cost_c + (n_wide + n_rest);
+    int32_t* count0 = cost + 2 * total + 16 * psa_order::MAX_PHASES;
+    int32_t* cost_r = count0 + n_blocks;
+    int32_t* cost_w = cost_r + n_rest;
+    int32_t* ord_w = cost_w + n_wide;
     int32_t* ord_r = ord_w + (wide0 ? (int64_t)chunk_w * groups_w : 0);
+    u32x2* items = (u32x2*)(((uintptr_t)(ord_r + (int64_t)chunk_r * groups_r) + 7) & ~(uintptr_t)7);
     const int row_wgs = rows_ordered ? (int)((total + 3) / 4) : 0;
     // Where the Q / dO rows of a head group are about the size of an XCD's L2 (4 MiB), the 128-key slots of a share are issued in
     // classes of a quarter of the longest possible list, head by head inside a class (the sort is stable): an XCD then works on one
@@ -980,14 +1166,19 @@ extern "C" int psa_bwd(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const void* 
     // chip holds at once (512 or 768) only the tail counts: 12 x 4000 x 64 311 / 319; columns of fewer than 32
     // q-blocks leave classes of a few: 48 x 3000 x 128 727 / 740.
     // (shares of about one round, which also keep an XCD on one head, lose 3-5 % at 24 x 12001 x 64 and 32 x 6000 x 128)
-    const bool by_head = wide0 && qdo_bytes / (B * Hkv) <= 5.5 * 1024 * 1024 && n_wide > 768 && Hq / Hkv * Mq >= 32;
+    const bool by_head = wide0 && qdo_bytes / (B * Hkv) <= 5.5 * 1024 * 1024 && n_blocks > 768 && Hq / Hkv * Mq >= 32;
     const int wide_div = by_head ? (Hq / Hkv * Mq + 3) / 4 : 1;
     hipLaunchKernelGGL(psa_bwd_cost_kernel, dim3((unsigned)(row_wgs + (cols_ordered ? n_blocks : 0))), dim3(256), 0, st, p, row_wgs, cost,
-                       wide0 ? 1 : 0, wide_div, cost_c);
+                       wide0 ? 1 : 0, wide_div, in_parts ? count0 : nullptr, cost_w, cost_r);
     if (int e = psa_check_launch("psa_bwd (cost)")) return e;
+    if (in_parts) {
+      hipLaunchKernelGGL(psa_bwd_parts_kernel, dim3((unsigned)(B * Hkv)), dim3(256), 0, st, count0, Nk, PART_MIN * 128 / block_m, wide_div, items, cost_w);
+      if (int e = psa_check_launch("psa_bwd (parts)")) return e;
+      items_wide = items;
+    }
     psa_order::sort_lists<3>({{{cost, ord, (int)total, chunk, rows_ordered ? groups : 0},
-                               {cost_c, ord_w, (int)n_wide, chunk_w, cols_ordered && wide0 ? groups_w : 0},
-                               {cost_c + n_wide, ord_r, (int)n_rest, chunk_r, cols_ordered ? groups_r : 0}}}, st);
+                               {cost_w, ord_w, (int)n_wide, chunk_w, cols_ordered && wide0 ? groups_w : 0},
+                               {cost_r, ord_r, (int)n_rest, chunk_r, cols_ordered ? groups_r : 0}}}, st);
     if (int e = psa_check_launch("psa_bwd (order)")) return e;
     if (rows_ordered) order = ord;
     if (cols_ordered) {
@@ -1023,7 +1214,7 @@ extern "C" int psa_bwd(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const void* 
     PSA_REQUIRE(shmem <= 160 * 1024, PSA_ERR_UNSUPPORTED, "psa_bwd: too many q-blocks for the on-chip lists (LDS)");
     auto launch = [&](auto kern, int64_t n_wg, int chunk, int groups, int slot_lo, int slot_cnt, const int32_t* order) -> int {
       if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem) != hipSuccess) return PSA_ERR_LAUNCH;
-      hipLaunchKernelGGL(kern, dim3((unsigned)(chunk * groups)), dim3(256), shmem, st, p, slot_lo, slot_cnt, (int)n_wg, chunk, order);
+      hipLaunchKernelGGL(kern, dim3((unsigned)(chunk * groups)), dim3(256), shmem, st, p, slot_lo, slot_cnt, (int)n_wg, chunk, order, slot_lo == 0 && slot_cnt == 1 ? items_wide : nullptr);
       return PSA_OK;
     };
     // the pooled levels first: the 128-key level-0 launch adds their rows to its own and writes dK, dV
@@ -1045,7 +1236,13 @@ extern "C" int psa_bwd(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const void* 
         rl = D == 128 ? launch(psa_bwd_dkdv_lds_kernel<128, true, false, ET>, n_wide, chunk_w, groups_w, 0, 1, order_wide)
                       : launch(psa_bwd_dkdv_lds_kernel<64, true, false, ET>, n_wide, chunk_w, groups_w, 0, 1, order_wide);
       PSA_REQUIRE(rl == PSA_OK, rl, "psa_bwd: cannot reserve %zu bytes of LDS", shmem);
-      return psa_check_launch("psa_bwd (dK/dV, 128-key slots)");
+      if (int e = psa_check_launch("psa_bwd (dK/dV, 128-key slots)")) return e;
+      if (items_wide != nullptr) {
+        const dim3 grid((unsigned)(Nk * (D / 8)), (unsigned)(B * Hkv));
+        if (D == 128) hipLaunchKernelGGL((psa_bwd_join_kernel<128, ET>), grid, dim3(256), 0, st, p, items_wide);
+        else hipLaunchKernelGGL((psa_bwd_join_kernel<64, ET>), grid, dim3(256), 0, st, p, items_wide);
+      }
+      return psa_check_launch("psa_bwd (dK/dV, cut slots)");
     }
   }
   // 5. un-pool (blocks of 64 or 32 keys: every level went to the fp32 buffers)
