@@ -320,8 +320,13 @@ constexpr int COL_BINS = psa_order::COST_BINS;
 // training step of 48 heads x 8776 x 64 1208 -> 1198 us, of 12 heads x 32760 x 128 4549 -> 4543 us.  The first row_wgs workgroups: four rows each, costs of the dQ walk.  The others, one per
 // (kv head, kv-block): per-level counts over the column -> cost of each of its slots.  The
 // costs of the slots slot_lo .. of all blocks form one list per dK/dV launch; with a 128-key slot 0 that slot's costs are a list of their
-// own (cost0, in units of wide_div q-blocks), or its lengths go to count0 and psa_bwd_parts_kernel makes the list.
-__global__ __launch_bounds__(256) void psa_bwd_cost_kernel(BwdParams p, int row_wgs, int32_t* cost_row, int wide0, int wide_div, int32_t* count0, int32_t* cost0, int32_t* cost) {
+// own (cost0), or its lengths go to count0 and psa_bwd_parts_kernel makes the list.
+// cost of a 128-key slot of n q-blocks: exact, or the octave of its length (classes, issued head by head)
+__device__ __forceinline__ int wide_cost(int n, bool octaves) {
+  if (octaves) return 32 - __builtin_clz(n | 1);
+  return n < COL_BINS - 1 ? n : COL_BINS - 1;
+}
+__global__ __launch_bounds__(256) void psa_bwd_cost_kernel(BwdParams p, int row_wgs, int32_t* cost_row, int wide0, bool octaves, int32_t* count0, int32_t* cost0, int32_t* cost) {
   __shared__ int s_n[4];
   if ((int)blockIdx.x < row_wgs) {
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -357,7 +362,7 @@ __global__ __launch_bounds__(256) void psa_bwd_cost_kernel(BwdParams p, int row_
     if (!wide0) cost[blk * DKDV_SLOTS + lv] = c;
     else if (lv == 0) {
       if (count0 != nullptr) count0[blk] = s_n[0];
-      else cost0[blk] = s_n[0] / wide_div < COL_BINS - 1 ? s_n[0] / wide_div : COL_BINS - 1;
+      else cost0[blk] = wide_cost(s_n[0], octaves);
     }
     else cost[blk * (DKDV_SLOTS - 1) + (lv - 1)] = c;
   }
@@ -380,7 +385,7 @@ constexpr int PART_MEAN_10 = 17, PART_MIN = 4, PART_MOST = 64;
 constexpr int parts_max_slots(int D) { return D == 128 ? 768 : 1024; }  // (the chip holds 512 / 768 workgroups at once)
 __device__ __forceinline__ int part_at(int n, int part, int parts) { return (int)((int64_t)n * part / parts); }
 
-__global__ __launch_bounds__(256) void psa_bwd_parts_kernel(const int32_t* count0, int Nk, int min_unit, int wide_div, u32x2* items, int32_t* cost) {
+__global__ __launch_bounds__(256) void psa_bwd_parts_kernel(const int32_t* count0, int Nk, int min_unit, bool octaves, u32x2* items, int32_t* cost) {
   __shared__ int s_sum[4], s_more[4];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t head = blockIdx.x;
@@ -428,10 +433,10 @@ __global__ __launch_bounds__(256) void psa_bwd_parts_kernel(const int32_t* count
     }
     if (j < Nk)
       for (int part = 0; part < parts; ++part) {
-        const int len = part_at(n, part + 1, parts) - part_at(n, part, parts), c = len / wide_div;
+        const int len = part_at(n, part + 1, parts) - part_at(n, part, parts);
         const int pos = part == 0 ? 2 * j : 2 * (int)((int64_t)(first + part - 1) * Nk / more) + 1;
         items[pos] = u32x2{(uint32_t)j | ((uint32_t)part << 16) | ((uint32_t)parts << 24), (uint32_t)(head * Nk + slot + part)};
-        cost[pos] = c < COL_BINS - 1 ? c : COL_BINS - 1;
+        cost[pos] = wide_cost(len, octaves);
       }
     at += s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3];
     slot_at += s_more[0] + s_more[1] + s_more[2] + s_more[3];
@@ -1158,21 +1163,23 @@ extern "C" int psa_bwd(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const void* 
     u32x2* items = (u32x2*)(((uintptr_t)(ord_r + (int64_t)chunk_r * groups_r) + 7) & ~(uintptr_t)7);
     const int row_wgs = rows_ordered ? (int)((total + 3) / 4) : 0;
     // Where the Q / dO rows of a head group are about the size of an XCD's L2 (4 MiB), the 128-key slots of a share are issued in
-    // classes of a quarter of the longest possible list, head by head inside a class (the sort is stable): an XCD then works on one
-    // or two heads at a time and finds their rows in L2, where the exact longest-first order mixes all heads of the share, and the
-    // few long columns still go first.  Training steps in exact order / in classes: 48 heads x 8776 x 64 1195 / 1160 us,
+    // classes, an octave of their list's length each, head by head inside a class (the sort is stable): an XCD then works on one
+    // or two heads at a time and finds their rows in L2, where the exact longest-first order mixes all heads of the share; the
+    // few long columns still go first, and what is left for the end is short.  The launch in classes of a quarter of the longest possible list /
+    // of an octave, us: 24 x 21613 x 64 580 / 533, 24 x 12001 x 64 224 / 213 and 312 / 303 (fixed quotas, thresholds), 48 x 8776 x 64 236 / 235
+    // and 380 / 365, 12 x 10700 x 128 302 / 275.  In exact order / classes of a quarter, training steps: 48 heads x 8776 x 64 1195 / 1160 us,
     // 24 x 12001 x 64 1028 / 999, 24 x 9000 x 128 1640 / 1601 (4.4 MiB), 12 x 10700 x 128 1013 / 983 (5.2 MiB).  Past the line the
-    // rows do not fit: 24 x 30000 x 64 (7.3 MiB) 4390 / 4442, 16 x 16000 x 128 (7.8 MiB) 1900 / 1936.  With fewer slots than the
+    // rows do not fit (the launch, exact / octaves): 24 x 23000 x 64 (5.6 MiB) 655 / 669, 24 x 30000 x 64 (7.3 MiB) 962 / 982 and 1118 / 1173,
+    // 16 x 16000 x 128 (7.8 MiB) 404 / 410 and 542 / 557.  With fewer slots than the
     // chip holds at once (512 or 768) only the tail counts: 12 x 4000 x 64 311 / 319; columns of fewer than 32
     // q-blocks leave classes of a few: 48 x 3000 x 128 727 / 740.
     // (shares of about one round, which also keep an XCD on one head, lose 3-5 % at 24 x 12001 x 64 and 32 x 6000 x 128)
     const bool by_head = wide0 && qdo_bytes / (B * Hkv) <= 5.5 * 1024 * 1024 && n_blocks > 768 && Hq / Hkv * Mq >= 32;
-    const int wide_div = by_head ? (Hq / Hkv * Mq + 3) / 4 : 1;
     hipLaunchKernelGGL(psa_bwd_cost_kernel, dim3((unsigned)(row_wgs + (cols_ordered ? n_blocks : 0))), dim3(256), 0, st, p, row_wgs, cost,
-                       wide0 ? 1 : 0, wide_div, in_parts ? count0 : nullptr, cost_w, cost_r);
+                       wide0 ? 1 : 0, by_head, in_parts ? count0 : nullptr, cost_w, cost_r);
     if (int e = psa_check_launch("psa_bwd (cost)")) return e;
     if (in_parts) {
-      hipLaunchKernelGGL(psa_bwd_parts_kernel, dim3((unsigned)(B * Hkv)), dim3(256), 0, st, count0, Nk, PART_MIN * 128 / block_m, wide_div, items, cost_w);
+      hipLaunchKernelGGL(psa_bwd_parts_kernel, dim3((unsigned)(B * Hkv)), dim3(256), 0, st, count0, Nk, PART_MIN * 128 / block_m, by_head, items, cost_w);
       if (int e = psa_check_launch("psa_bwd (parts)")) return e;
       items_wide = items;
     }
