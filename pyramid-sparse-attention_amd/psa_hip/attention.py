@@ -114,9 +114,12 @@ class PSAAttention(nn.Module):
 
     def build_mask(self, q, k, v):
         """estimate -> level mask in the format `attn_impl` selects (no gradient)."""
+        return self._mask(q, k, v, self.sample_offsets)
+
+    def _mask(self, q, k, v, sample_offsets):
         config = self.config
         with torch.no_grad():
-            pooling, sim_cap = _compute_attention_pooling(q, k, v, config, self.sample_offsets)
+            pooling, sim_cap = _compute_attention_pooling(q, k, v, config, sample_offsets)
             mode = config.mask_mode if config.attn_impl == "old_mask_type" else f"{config.mask_mode}_newtype"
             mask = ops.level_map(pooling, config.mask_ratios, 0, mode, blocksize=config.block_n, compute_tile=config.tile_n)
             if config.use_sim_mask and sim_cap is not None:
@@ -136,6 +139,17 @@ class PSAAttention(nn.Module):
             cap = calc_k_similarity(k, config.block_n, config) if config.use_sim_mask else None
             return ops.psa_layer_fwd(q, k, v, off_q, off_k, config.mask_ratios, config.mask_mode, config.block_m,
                                      config.block_n, config.tile_n, level_cap=cap)
+        listed = getattr(self.sparse_attention_fn, "listed", None)
+        if listed is not None and not config.use_sim_mask and getattr(self.build_mask, "__func__", None) is PSAAttention.build_mask:
+            # the module's own mask and attention: levels and the attention's tile list come out of the estimate's reduction
+            offsets = self.sample_offsets
+            if offsets is None:
+                offsets = draw_layer_offsets(q.shape[0], q.shape[1], k.shape[1], config.block_m, config.block_n, q.device)
+            with torch.no_grad():
+                both = ops.estimate_walk(q, k, *offsets, config.mask_ratios, config.mask_mode, config.block_m, config.block_n, config.tile_n)
+            if both is not None:
+                return listed(q, k, v, *both)
+            return self.sparse_attention_fn(q, k, v, self._mask(q, k, v, offsets), None)
         mask = self.build_mask(q, k, v)
         return self.sparse_attention_fn(q, k, v, mask, None)
 

@@ -13,13 +13,13 @@ class _sparse_attention(torch.autograd.Function):
     """Differentiable in q, k, v; the mask carries no gradient."""
 
     @staticmethod
-    def forward(ctx, q, k, v, block_sparse_dense, sm_scale, block_m=128, block_n=128, causal=False):
+    def forward(ctx, q, k, v, block_sparse_dense, sm_scale, block_m=128, block_n=128, causal=False, walk=None):
         sm_scale = sm_scale if sm_scale is not None else q.shape[-1] ** -0.5
         need_backward = q.requires_grad or k.requires_grad or v.requires_grad
         if not need_backward:
-            return ops.sparse_attention_fwd(q, k, v, block_sparse_dense, block_m, block_n, sm_scale, causal=causal)
+            return ops.sparse_attention_fwd(q, k, v, block_sparse_dense, block_m, block_n, sm_scale, causal=causal, _walk=walk)
         o, lse, pools = ops.sparse_attention_fwd(q, k, v, block_sparse_dense, block_m, block_n, sm_scale, causal=causal,
-                                               return_lse=True)
+                                               return_lse=True, _walk=walk)
         ctx.save_for_backward(q, k, v, block_sparse_dense, o, lse, pools[0], pools[1])
         ctx.sm_scale, ctx.causal, ctx.block_m, ctx.block_n = sm_scale, causal, block_m, block_n
         return o
@@ -29,7 +29,7 @@ class _sparse_attention(torch.autograd.Function):
         q, k, v, mask, o, lse, kp, vp = ctx.saved_tensors
         dq, dk, dv = ops.sparse_attention_bwd(q, k, v, mask, o, do, lse, ctx.block_m, ctx.block_n, ctx.sm_scale,
                                               causal=ctx.causal, pools=(kp, vp))
-        return dq, dk, dv, None, None, None, None, None
+        return dq, dk, dv, None, None, None, None, None, None
 
 
 def sparse_attention_factory(BLOCK_M=128, BLOCK_N=32, POOLING_BLOCK_N=128, causal=False, **kwargs):
@@ -57,6 +57,8 @@ def sparse_attention_factory(BLOCK_M=128, BLOCK_N=32, POOLING_BLOCK_N=128, causa
     def _fn(q, k, v, block_sparse_dense, sm_scale=None):
         return _sparse_attention.apply(q, k, v, block_sparse_dense, sm_scale, BLOCK_M, POOLING_BLOCK_N, causal)
 
+    if not causal:  # the same on a map whose tiles are listed already (ops.estimate_walk)
+        _fn.listed = lambda q, k, v, level_map, walk: _sparse_attention.apply(q, k, v, level_map, None, BLOCK_M, POOLING_BLOCK_N, False, walk)
     return _fn
 
 
