@@ -456,7 +456,11 @@ __global__ __launch_bounds__(256) void psa_bwd_parts_kernel(const int32_t* count
 // 381 -> 262, 338 -> 280 us; training steps, with the dQ walk, 4601 -> 4196 us and 1193 -> 1071 us.
 // The four waves of a workgroup split its keys and the 64 query rows of a step: 128 keys (level 0 of a 128-key
 // block) = 4 key quarters, every wave takes both query halves one after the other ("wide": each Q / dO tile that is
-// fetched feeds twice the arithmetic); <= 64 keys = 2 key halves x 2 query halves, combined through LDS at the end.
+// fetched feeds twice the arithmetic); <= 64 keys = 2 key halves x 2 query halves, combined through LDS at the end.  A wave works on 32 keys,
+// two blocks of 16, in slots of more than 32 keys and on one block in smaller ones: all four waves of a 32-key slot have work, and those of
+// a 16-key slot compute nothing for keys that are not there.  The walk is there twice in the kernel for that, one branch at its
+// start (a branch around each step spills).  With 32 keys per wave throughout / now, the launch of the pooled levels, us: 48 heads of 17043 x
+// 128, fixed quotas, 1677 / 1488, 24 of 21613 x 64 693 / 606, 48 of 8776 x 64 282 / 250, 12 of 32760 x 128, thresholds, 660 / 621.
 // ------------------------------------------------------------------------------------------------------
 constexpr int B_ISTR = LT_ISTR;  // bytes between the blocks of a tile
 
@@ -513,9 +517,10 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
   constexpr int B_TILE = G::TILE;
   extern __shared__ __align__(16) unsigned char smem[];
   // stage s: Q tile at 2*s*B_TILE, dO tile at (2*s + 1)*B_TILE
-  float* s_lse = (float*)(smem + 4 * B_TILE);  // [2 stages][64]
-  float* s_del = s_lse + 128;                  // [2 stages][64]
-  uint32_t* qlist = (uint32_t*)(s_del + 128);  // [n_rep * Mq]  (head in group << 16 | q-block)
+  PSA_LDS(float) const s_lse = (PSA_LDS(float))((PSA_LDS(unsigned char))smem + 4 * B_TILE);  // [2 stages][64]
+  PSA_LDS(float) const s_del = s_lse + 128;                                                  // [2 stages][64]
+  PSA_LDS(uint32_t) const qlist = (PSA_LDS(uint32_t))(s_del + 128);                          // [n_rep * Mq]  (head in group << 16 | q-block)
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(PSA_LDS(unsigned char))smem;
   __shared__ int s_nq;
 
   int wg = psa_order::dealt_entry((int)blockIdx.x, chunk);  // shares of slots per XCD, longest lists first (psa_order.h)
@@ -549,12 +554,14 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
     const int64_t rem = (int64_t)L - key_row0;
     key_valid = rem < nkeys ? (rem > 0 ? (int)rem : 0) : nkeys;
   }
-  // <= 64 keys: waves = 2 key halves x 2 query halves.  With at most 32 keys only one key half works: alternate
+  // <= 64 keys: waves = 2 key halves x 2 query halves.  With 16 keys only one key half works: alternate
   // which pair of waves that is from workgroup to workgroup, so that all four SIMDs of a CU get work.
   // 128 keys: waves = 4 key quarters.
-  const int flip = nkeys <= 32 ? (int)((blockIdx.x >> 3) & 1) : 0;
+  const int flip = nkeys <= 16 ? (int)((blockIdx.x >> 3) & 1) : 0;
   const int kh = wide ? wave : ((wave & 1) ^ flip), qh = wide ? 0 : wave >> 1;
-  const bool wave_active = key_valid > kh * 32;
+  const bool narrow = !wide && nkeys <= 32;       // 16 keys per wave
+  const int wave_key0 = narrow ? kh * 16 : kh * 32;
+  const bool wave_active = key_valid > wave_key0;
 
   // ---- list of (head in group, q-block) that retain block J at this level -------------------------
   if (wave == 0) {
@@ -580,11 +587,13 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
     if (lane == 0) s_nq = n;
   }
 
-  // ---- this wave's 32 keys, two blocks of 16: K and V fragments (B operands), lane = key l16, channels 32 * kk + 8 * lg .. + 7 -----
-  const int key_local = kh * 32 + l16;  // block kb: + 16 * kb
-  x8 kf[2][KK], vf[2][KK];
+  auto walk = [&](auto kb_c) __attribute__((always_inline)) {
+  constexpr int KB = decltype(kb_c)::value;
+  // ---- this wave's keys, KB blocks of 16: K and V fragments (B operands), lane = key l16, channels 32 * kk + 8 * lg .. + 7 -----
+  const int key_local = wave_key0 + l16;  // block kb: + 16 * kb
+  x8 kf[KB][KK], vf[KB][KK];
 #pragma unroll
-  for (int kb = 0; kb < 2; ++kb) {
+  for (int kb = 0; kb < KB; ++kb) {
     const int key = key_local + 16 * kb;
     int64_t row = key_row0 + (key < key_valid ? key : 0);
     if (key_valid == 0) row = 0;
@@ -608,11 +617,10 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
   // last token that the pooled key covers (< npad); block kb: + 16 << lv
   const int key_up = (int)(((key_row0 + key_local + 1) << lv) - 1);
   __syncthreads();
-  int nq = s_nq;
+  int nq = s_nq, from = 0;  // (of a slot's list, WIDE: the part of this workgroup)
   if constexpr (WIDE) {
-    const int from = part_at(nq, part, parts);
+    from = part_at(nq, part, parts);
     nq = part_at(nq, part + 1, parts) - from;
-    qlist += from;
   }
 
   // ---- lane-invariant LDS addressing (tile layout: see the forward kernel) ---------------------------
@@ -628,9 +636,9 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
 #pragma unroll
   for (int i = 0; i < 2; ++i) t_off[i] += (uint32_t)(qh * G::HALF);
 
-  f32x4 dk[2][DB], dv[2][DB];  // [key block][channel block]
+  f32x4 dk[KB][DB], dv[KB][DB];  // [key block][channel block]
 #pragma unroll
-  for (int kb = 0; kb < 2; ++kb)
+  for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
     for (int db = 0; db < DB; ++db) dk[kb][db] = dv[kb][db] = f32x4{0.f, 0.f, 0.f, 0.f};
   const float scale_log2 = p.scale_log2;
@@ -641,7 +649,7 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
 
   // step i -> (head, q-block, first query row)
   auto step_of = [&](int i, int& h, int& I, int& q0) __attribute__((always_inline)) {
-    const uint32_t ent = qlist[i >> spb_log2];
+    const uint32_t ent = qlist[from + (i >> spb_log2)];
     h = hk * n_rep + (int)(ent >> 16);
     I = (int)(ent & 0xffff);
     q0 = I * bm + (i & ((1 << spb_log2) - 1)) * 64;
@@ -656,8 +664,8 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
     if (wave == 0) {
       const int64_t at = ((int64_t)b * p.Hq + h) * L + q0;
       if (q0 + ln < L) {
-        psa_tiles::lds_copy4((const char*)(p.nlse2 + at), (uint32_t)ln * 4u, psa_tiles::lds_addr_of(s_lse + stage * 64));
-        psa_tiles::lds_copy4((const char*)(p.ndelta + at), (uint32_t)ln * 4u, psa_tiles::lds_addr_of(s_del + stage * 64));
+        psa_tiles::lds_copy4((const char*)(p.nlse2 + at), (uint32_t)ln * 4u, lds0 + (uint32_t)(4 * B_TILE + stage * 256));
+        psa_tiles::lds_copy4((const char*)(p.ndelta + at), (uint32_t)ln * 4u, lds0 + (uint32_t)(4 * B_TILE + 512 + stage * 256));
       } else {  // rows past L: -lse = -inf makes every p vanish
         s_lse[stage * 64 + ln] = -INFINITY;
         s_del[stage * 64 + ln] = 0.f;
@@ -672,8 +680,8 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
       const uint32_t qo = (uint32_t)r0 * q_strb + f_chunk, oo = (uint32_t)r0 * do_strb + f_chunk;
 #pragma unroll
       for (int n = 0; n < RPL; ++n) {
-        psa_tiles::lds_copy16(qb + (uint64_t)(n * q_strb), qo, psa_tiles::lds_addr_of(smem + 2 * stage * B_TILE + (wave * RPL + n) * B_ISTR));
-        psa_tiles::lds_copy16(ob + (uint64_t)(n * do_strb), oo, psa_tiles::lds_addr_of(smem + (2 * stage + 1) * B_TILE + (wave * RPL + n) * B_ISTR));
+        psa_tiles::lds_copy16(qb + (uint64_t)(n * q_strb), qo, lds0 + (uint32_t)(2 * stage * B_TILE + (wave * RPL + n) * B_ISTR));
+        psa_tiles::lds_copy16(ob + (uint64_t)(n * do_strb), oo, lds0 + (uint32_t)((2 * stage + 1) * B_TILE + (wave * RPL + n) * B_ISTR));
       }
     } else {
 #pragma unroll
@@ -681,8 +689,8 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
         int row = r0 + n;
         row = row < L ? row : L - 1;
         row = row > 0 ? row : 0;
-        psa_tiles::lds_copy16(qb, (uint32_t)row * q_strb + f_chunk, psa_tiles::lds_addr_of(smem + 2 * stage * B_TILE + (wave * RPL + n) * B_ISTR));
-        psa_tiles::lds_copy16(ob, (uint32_t)row * do_strb + f_chunk, psa_tiles::lds_addr_of(smem + (2 * stage + 1) * B_TILE + (wave * RPL + n) * B_ISTR));
+        psa_tiles::lds_copy16(qb, (uint32_t)row * q_strb + f_chunk, lds0 + (uint32_t)(2 * stage * B_TILE + (wave * RPL + n) * B_ISTR));
+        psa_tiles::lds_copy16(ob, (uint32_t)row * do_strb + f_chunk, lds0 + (uint32_t)((2 * stage + 1) * B_TILE + (wave * RPL + n) * B_ISTR));
       }
     }
   };
@@ -692,9 +700,11 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
   // (the key blocks) and is read PD pairs ahead: two are what the registers allow without spilling (one where the causal mask takes
   // two more; one everywhere 1646 us where two take 1583).
   PSA_LDS(const float) rows_base = (PSA_LDS(const float))(smem + 4 * B_TILE) + (qh * 32 + lg * 4);
-  constexpr int NM = 4 * KK, NO = NM / 2, PD = D == 128 && WIDE && CAUSAL ? 1 : 2;  // MFMAs and operands of a run
+  constexpr int PD = D == 128 && WIDE && CAUSAL ? 1 : 2;
+  constexpr int NO = 2 * KK;  // operands of a run
   static_assert(NO == DB, "");
-  constexpr int VPS = 16 / NM;  // logits of a lane per MFMA
+  constexpr int VPS = 4 / KK;  // logits of a lane per MFMA
+  constexpr int NM = NO * KB, NV = 8 * KB;  // MFMAs of a run, logits of a lane
   auto compute_step = [&](int i) __attribute__((always_inline)) {
     int h, I, q0;
     step_of(i, h, I, q0);
@@ -708,8 +718,8 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
       PSA_LDS(unsigned char) Os = (PSA_LDS(unsigned char))(smem) + B_TILE + qi * G::HALF;
       PSA_LDS(const float) rows = rows_base + qi * 32;  // one lane base + immediates (group, lse / delta array)
       // lane = key column, registers = query rows: [16-row group][key block]
-      f32x4 s[2][2], dp[2][2], l4[2];
-      u32x4 pk[2], dsk[2];  // [key block]: P and dS, the B operands of the last two runs
+      f32x4 s[2][KB], dp[2][KB], l4[2];
+      u32x4 pk[KB], dsk[KB];  // [key block]: P and dS, the B operands of the last two runs
       x8 op[4 * NO];
       auto fetch = [&](auto n_c) __attribute__((always_inline)) {
         constexpr int n = decltype(n_c)::value, run = n / NO, j = n % NO;
@@ -725,13 +735,13 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
       // the lane's rows, that sees the lane's key).  Lanes whose key does not exist (the ragged end of the sequence at level 0;
       // lanes beyond the 16 keys of a level-8 block) work on a copy of the block's first key: the columns of dK^T / dV^T are
       // independent of each other and those lanes' columns are never read.
-      int thr[2] = {0, 0};
+      int thr[KB] = {};
       if constexpr (CAUSAL)
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb) thr[kb] = diag ? key_up + ((16 * kb) << lv) - (q0 + qhv * 32 + lg * 4) : -0x40000000;
-      // logit v (0..15) of a lane, in the order in which a run completes them: p = exp2(scale * s + bias - lse)
+        for (int kb = 0; kb < KB; ++kb) thr[kb] = diag ? key_up + ((16 * kb) << lv) - (q0 + qhv * 32 + lg * 4) : -0x40000000;
+      // logit v of a lane, in the order in which a run completes them: p = exp2(scale * s + bias - lse)
       auto prob = [&](auto v_c) __attribute__((always_inline)) {
-        constexpr int v = decltype(v_c)::value, qg = v >> 3, kb = (v >> 2) & 1, e = v & 3;
+        constexpr int v = decltype(v_c)::value, qg = v / (4 * KB), kb = (v >> 2) % KB, e = v & 3;
         float pe = fast_exp2(__builtin_fmaf(s[qg][kb][e], scale_log2, l4[qg][e]));
         if constexpr (CAUSAL) pe = thr[kb] <= qg * 16 + e ? pe : 0.f;
         s[qg][kb][e] = pe;
@@ -739,7 +749,7 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
       };
       // dS = p (dP - delta)
       auto dsv = [&](auto v_c) __attribute__((always_inline)) {
-        constexpr int v = decltype(v_c)::value, qg = v >> 3, kb = (v >> 2) & 1, e = v & 3;
+        constexpr int v = decltype(v_c)::value, qg = v / (4 * KB), kb = (v >> 2) % KB, e = v & 3;
         dp[qg][kb][e] *= s[qg][kb][e];
         if constexpr (e & 1) dsk[kb][qg * 2 + (e >> 1)] = ET::pack2(dp[qg][kb][e - 1], dp[qg][kb][e]);
       };
@@ -748,27 +758,28 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
         constexpr int run = decltype(run_c)::value;
         __builtin_amdgcn_sched_barrier(0);
         static_for<NM>([&](auto st_c) __attribute__((always_inline)) {
-          constexpr int st = decltype(st_c)::value, j = st >> 1, kb = st & 1, qg = j / KK, kk = j % KK, n = run * NO + j;
+          constexpr int st = decltype(st_c)::value, j = st / KB, kb = st % KB, qg = j / KK, kk = j % KK, n = run * NO + j;
           if constexpr (run < 2 && kk == 0 && kb == 0) {
             if constexpr (run == 0) {
-              s[qg][0] = s[qg][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+              static_for<KB>([&](auto x) __attribute__((always_inline)) { s[qg][decltype(x)::value] = f32x4{0.f, 0.f, 0.f, 0.f}; });
               l4[qg] = *(PSA_LDS(const f32x4))(rows + qg * 16);
               if constexpr (!WIDE)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) l4[qg][e] += bias;
             } else {
-              dp[qg][0] = dp[qg][1] = *(PSA_LDS(const f32x4))(rows + 128 + qg * 16);
+              const f32x4 d4 = *(PSA_LDS(const f32x4))(rows + 128 + qg * 16);
+              static_for<KB>([&](auto x) __attribute__((always_inline)) { dp[qg][decltype(x)::value] = d4; });
             }
           }
           if constexpr (run == 0) s[qg][kb] = ET::mfma16(op[n], kf[kb][kk], s[qg][kb]);
           if constexpr (run == 1) dp[qg][kb] = ET::mfma16(op[n], vf[kb][kk], dp[qg][kb]);
           if constexpr (run == 2) dv[kb][j] = ET::mfma16(op[n], __builtin_bit_cast(x8, pk[kb]), dv[kb][j]);
           if constexpr (run == 3) dk[kb][j] = ET::mfma16(op[n], __builtin_bit_cast(x8, dsk[kb]), dk[kb][j]);
-          if constexpr (kb == 1) fetch(IC<n + PD>{});
+          if constexpr (kb == KB - 1) fetch(IC<n + PD>{});
           static_for<VPS>([&](auto u) __attribute__((always_inline)) {
             constexpr int v = (run * NM + st - NM / 2) * VPS + decltype(u)::value;
-            if constexpr (v >= 0 && v < 16) prob(IC<v>{});
-            if constexpr (v >= 16 && v < 32) dsv(IC<v - 16>{});
+            if constexpr (v >= 0 && v < NV) prob(IC<v>{});
+            if constexpr (v >= NV && v < 2 * NV) dsv(IC<v - NV>{});
           });
           __builtin_amdgcn_sched_barrier(0);
         });
@@ -805,7 +816,7 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
     if (parts > 1) {  // fp32 sums of this part, in the accumulators' layout (psa_bwd_join_kernel)
       const int64_t at = (int64_t)part_slot * (128 * D) + (int64_t)kh * (2 * DB * 256) + ln * 4;
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
+      for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
           *(f32x4*)(p.wk + at + (kb * DB + db) * 256) = dk[kb][db];
@@ -820,7 +831,7 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
       fold_pad_rows<D>(p, bhk, wave * 64 + ln, fold + 2 * D, fold);
     }
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
+    for (int kb = 0; kb < KB; ++kb) {
       const int64_t n = key_row0 + kh * 32 + (ln & 15) + 16 * kb;
       if (n >= L) continue;
       const int64_t BH = (int64_t)p.B * p.Hkv, npad = p.npad;
@@ -881,11 +892,11 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
   }
   // ---- combine the two query halves (<= 64 keys) and write this workgroup's rows of the level buffers ----
   __syncthreads();
-  f32x4* red = (f32x4*)smem;  // [2 key halves][2 tensors][2 key blocks][DB][64 lanes]
-  auto red_at = [&](int tensor, int kb, int db) __attribute__((always_inline)) { return red + (((kh * 2 + tensor) * 2 + kb) * DB + db) * 64 + ln; };
+  f32x4* red = (f32x4*)smem;  // [2 key halves][2 tensors][KB key blocks][DB][64 lanes]
+  auto red_at = [&](int tensor, int kb, int db) __attribute__((always_inline)) { return red + (((kh * 2 + tensor) * KB + kb) * DB + db) * 64 + ln; };
   if (qh == 1) {
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
+    for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
       for (int db = 0; db < DB; ++db) {
         *red_at(0, kb, db) = dk[kb][db];
@@ -899,8 +910,8 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
   const int64_t base_rows = lv == 0 ? bhk * p.npad : (int64_t)p.B * p.Hkv * p.npad + lvl_off;
   const float scale = p.scale;
 #pragma unroll
-  for (int kb = 0; kb < 2; ++kb) {
-    const int key = kh * 32 + (ln & 15) + 16 * kb;
+  for (int kb = 0; kb < KB; ++kb) {
+    const int key = wave_key0 + (ln & 15) + 16 * kb;
     if (key >= nkeys) continue;
     float* wk = p.wk + (base_rows + key_row0 + key) * D;
     float* wv = p.wv + (base_rows + key_row0 + key) * D;
@@ -917,7 +928,11 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
       *(f32x4*)(wv + db * 16 + (ln >> 4) * 4) = c2;
     }
   }
-
+  };
+  if constexpr (!WIDE) {
+    if (narrow) return walk(IC<1>{});
+  }
+  walk(IC<2>{});
 }
 
 // The 128-key slots that were cut: their parts added in order, then what ends such a slot (above), four channels of one token per
