@@ -17,6 +17,7 @@
 // group's rows of R - m, exp2, row sum in a fixed order, normalisation.
 #include "psa_common.h"
 #include "psa_level_map_row.h"
+#include "psa_pool_rows.h"
 #include "psa_schedule.h"
 #include "psa_tiles.h"
 
@@ -85,8 +86,47 @@ __device__ __forceinline__ void chunk_max_piece(const f32x16& sc, float (&val)[1
   }
 }
 
-template <int D, int GPC, class ET>
-__global__ __launch_bounds__(256, 2) void psa_est_gemm_lds_kernel(EstParams p) {
+// The pooling pass of a layer as further workgroups of the contraction's launch (which layers: psa_layer.hip, pools_beside).  Both are short,
+// neither needs the other, and the contraction alone leaves most of the chip idle: what goes is the start and the end of a launch, 3 to 6 us.
+// Workgroups below `first` are the contraction's, numbered as its grid is; then nx per (tensor, kv head).  In large layers both draw the
+// board's power: 12 heads x 32760 x 128, re-ordered, 289 us one after the other and 281 to 330 together, by the order of the workgroups.
+struct EstPool {
+  PoolParams p;
+  int first, nx, heads;
+  int mx, bhs;  // first two extents of the contraction's grid
+};
+struct EstAlone {};
+
+// Block coordinates of a workgroup of the contraction; false: it was one of the pooling pass, and is done.
+template <class PT>
+__device__ __forceinline__ bool est_block(const EstAlone&, int& bx, int& bh, int& ks) {
+  bx = blockIdx.x;
+  bh = blockIdx.y;
+  ks = blockIdx.z;
+  return true;
+}
+template <class PT>
+__device__ __forceinline__ bool est_block(const EstPool& b, int& bx, int& bh, int& ks) {
+  const int id = (int)blockIdx.x;
+  if (id >= b.first) {
+    const int px = (id - b.first) % b.nx, ph = (id - b.first) / b.nx, which = ph >= b.heads ? 1 : 0;
+    if constexpr (PT::ES == 2) {
+      if (b.p.cap != nullptr) {
+        pool_rows<false, true, PT>(b.p, px, ph - which * b.heads, which, b.heads);
+        return false;
+      }
+    }
+    pool_rows<false, false, PT>(b.p, px, ph - which * b.heads, which, b.heads);
+    return false;
+  }
+  bx = id % b.mx;
+  bh = id / b.mx % b.bhs;
+  ks = id / (b.mx * b.bhs);
+  return true;
+}
+
+template <int D, int GPC, class ET, class BESIDE>
+__global__ __launch_bounds__(256, 2) void psa_est_gemm_lds_kernel(EstParams p, BESIDE beside) {
   using x8 = typename ET::x8;
   using G = psa_tiles::LtGeom<D>;
   constexpr int KK = D / 16, RS = 2;  // RS sets of 32 query rows per wave
@@ -95,17 +135,18 @@ __global__ __launch_bounds__(256, 2) void psa_est_gemm_lds_kernel(EstParams p) {
   constexpr int PPS = 8 / KK;         // pieces of the first chunk's maxima per k-step of the second chunk
   static_assert(8 % KK == 0 && PPS >= 1, "the maxima of a chunk are 8 pieces");
   __shared__ __align__(16) unsigned char smem[E_STAGES * E_TILE];
+  int bx, bh, ks;
+  if (!est_block<Pool16<ET>>(beside, bx, bh, ks)) return;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, hh = lane >> 5;
-  const int bh = blockIdx.y;
   const int h = bh % p.Hq, b = bh / p.Hq;
   const int hk = h / (p.Hq / p.Hkv);
   const int keep_m = 1 << p.keep_m_log2;
   constexpr int kn_log2 = 5 - GPC, keep_n = 1 << kn_log2;
 
   // Q fragments: lane holds Q[row l32 of set rs][16*kk + 8*hh .. +8]
-  const int row0 = blockIdx.x * (4 * 32 * RS) + wave * (32 * RS);
+  const int row0 = bx * (4 * 32 * RS) + wave * (32 * RS);
   x8 qf[RS][KK];
   {
     const int32_t* oq = p.off_q ? p.off_q + (int64_t)bh * keep_m : nullptr;
@@ -187,7 +228,6 @@ __global__ __launch_bounds__(256, 2) void psa_est_gemm_lds_kernel(EstParams p) {
   };
 
   // this workgroup's share of the key tiles
-  const int ks = blockIdx.z;
   const int t_begin = (int)((int64_t)T * ks / p.ksplit), t_end = (int)((int64_t)T * (ks + 1) / p.ksplit);
   issue_tile(t_begin, t_begin & 1);
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
@@ -256,8 +296,8 @@ __global__ __launch_bounds__(256, 2) void psa_est_gemm_lds_kernel(EstParams p) {
 // consecutive bytes of a row per four k-steps; the next step's rows are requested before the current step's products), so
 // the waves run free of barriers.  Shares (grid z, up to 4) are cut until there are two workgroups per CU.
 // 2 heads x 1024 sampled rows x 1024 keys x 64: 72 us on the vector units (two LDS operands per 4 FMAs), 9 us here.
-template <int D, int GPC>
-__global__ __launch_bounds__(256) void psa_est_gemm_f32_kernel(EstParams p) {
+template <int D, int GPC, class BESIDE>
+__global__ __launch_bounds__(256) void psa_est_gemm_f32_kernel(EstParams p, BESIDE beside) {
   constexpr int SQ = D / 16, RS = 2, NV = 1 << GPC;  // NV key groups per 32 keys
   constexpr int kn_log2 = 5 - GPC, keep_n = 1 << kn_log2;
   __shared__ float s_m[4][RS * 16];
@@ -265,8 +305,10 @@ __global__ __launch_bounds__(256) void psa_est_gemm_f32_kernel(EstParams p) {
   const float* kg = (const float*)p.k;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, g4 = lane >> 4;
-  const int bh = blockIdx.y, h = bh % p.Hq, b = bh / p.Hq, hk = h / (p.Hq / p.Hkv);
-  const int row0 = blockIdx.x * (RS * 16);
+  int bx, bh, ks;
+  if (!est_block<PoolF32>(beside, bx, bh, ks)) return;
+  const int h = bh % p.Hq, b = bh / p.Hq, hk = h / (p.Hq / p.Hkv);
+  const int row0 = bx * (RS * 16);
   const int32_t* oq = p.off_q ? p.off_q + (int64_t)bh * (1 << p.keep_m_log2) : nullptr;
   const int32_t* ok = p.off_k ? p.off_k + ((int64_t)b * p.Hkv + hk) * keep_n : nullptr;
   // operands: step 4 c + j takes channel 16 c + 4 g + j
@@ -289,7 +331,7 @@ __global__ __launch_bounds__(256) void psa_est_gemm_f32_kernel(EstParams p) {
     const int src = r < p.Ns ? (r >> kn_log2) * p.bn + off : ((p.Ns - 1) >> kn_log2) * p.bn + last_off;
     return kb + (int64_t)(src < p.Lk ? src : p.Lk - 1) * p.k_sl;
   };
-  const int steps = p.Ns_pad / 32, ks = blockIdx.z;
+  const int steps = p.Ns_pad / 32;
   const int s_begin = (int)((int64_t)steps * ks / p.ksplit), s_end = (int)((int64_t)steps * (ks + 1) / p.ksplit);
   f32x4 ka[2][SQ];
   auto load = [&](int st) __attribute__((always_inline)) {
@@ -453,7 +495,7 @@ __global__ __launch_bounds__(256, 6) void psa_est_reduce_map_kernel(EstParams p,
 }
 
 template <int D>
-int launch_est(EstParams& p, int B, hipStream_t stream, const LevelMapParams* lp, psa_sched::MapEnd& end, bool* map_done) {
+int launch_est(EstParams& p, int B, hipStream_t stream, const LevelMapParams* lp, psa_sched::MapEnd& end, const PoolParams* pool, bool* map_done) {
   const int rows_needed = p.out_rows << p.keep_m_log2;
   dim3 grid((unsigned)((rows_needed + 255) / 256), (unsigned)(B * p.Hq));
   // 256-row workgroups: cut the key range until about 3 workgroups per CU exist (the kernel's occupancy),
@@ -468,21 +510,39 @@ int launch_est(EstParams& p, int B, hipStream_t stream, const LevelMapParams* lp
     const int64_t wgs32 = (int64_t)(p.Ms_pad / 32) * B * p.Hq;
     p.ksplit = 1;
     while (p.ksplit < EST_MAX_KSPLIT && wgs32 * p.ksplit < 512 && p.Ns_pad / 32 / (p.ksplit * 2) >= 4) p.ksplit *= 2;
-    const dim3 g32((unsigned)(p.Ms_pad / 32), (unsigned)(B * p.Hq), (unsigned)p.ksplit);
-    switch (p.keep_n_log2) {
-      case 5: hipLaunchKernelGGL((psa_est_gemm_f32_kernel<D, 0>), g32, dim3(256), 0, stream, p); break;
-      case 4: hipLaunchKernelGGL((psa_est_gemm_f32_kernel<D, 1>), g32, dim3(256), 0, stream, p); break;
-      default: hipLaunchKernelGGL((psa_est_gemm_f32_kernel<D, 2>), g32, dim3(256), 0, stream, p); break;
-    }
+    grid = dim3((unsigned)(p.Ms_pad / 32), (unsigned)(B * p.Hq), (unsigned)p.ksplit);
   }
-  psa_dispatch16(p.dtype, [&](auto et) {
-    using ET = decltype(et);
-    switch (p.keep_n_log2) {
-      case 5: hipLaunchKernelGGL((psa_est_gemm_lds_kernel<D, 0, ET>), grid, dim3(256), 0, stream, p); break;
-      case 4: hipLaunchKernelGGL((psa_est_gemm_lds_kernel<D, 1, ET>), grid, dim3(256), 0, stream, p); break;
-      default: hipLaunchKernelGGL((psa_est_gemm_lds_kernel<D, 2, ET>), grid, dim3(256), 0, stream, p); break;
+  auto launch = [&](auto beside, dim3 blocks) {
+    using BESIDE = decltype(beside);
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, blocks, dim3(256), 0, stream, p, beside); };
+    if (p.dtype == PSA_DTYPE_F32) {
+      switch (p.keep_n_log2) {
+        case 5: go(psa_est_gemm_f32_kernel<D, 0, BESIDE>); break;
+        case 4: go(psa_est_gemm_f32_kernel<D, 1, BESIDE>); break;
+        default: go(psa_est_gemm_f32_kernel<D, 2, BESIDE>); break;
+      }
     }
-  });
+    psa_dispatch16(p.dtype, [&](auto et) {
+      using ET = decltype(et);
+      switch (p.keep_n_log2) {
+        case 5: go(psa_est_gemm_lds_kernel<D, 0, ET, BESIDE>); break;
+        case 4: go(psa_est_gemm_lds_kernel<D, 1, ET, BESIDE>); break;
+        default: go(psa_est_gemm_lds_kernel<D, 2, ET, BESIDE>); break;
+      }
+    });
+  };
+  if (pool != nullptr) {
+    EstPool b;
+    b.p = *pool;
+    b.first = (int)(grid.x * grid.y * grid.z);
+    b.nx = (int)((pool->npad / 8 * (D / (p.dtype == PSA_DTYPE_F32 ? PoolF32::CH : 8)) + 255) / 256);
+    b.heads = B * p.Hkv;
+    b.mx = (int)grid.x;
+    b.bhs = (int)grid.y;
+    launch(b, dim3((unsigned)(b.first + b.nx * b.heads * 2)));
+  } else {
+    launch(EstAlone{}, grid);
+  }
   const int rc = psa_check_launch("psa_estimate_sampled (contraction)");
   if (rc != PSA_OK) return rc;
   const dim3 rgrid((unsigned)p.out_rows, (unsigned)(B * p.Hq));
@@ -548,7 +608,7 @@ namespace {
 int est_run(psa_tensor4 q, psa_tensor4 k, const int32_t* off_q, const int32_t* off_k, const int32_t* q_index, float* scores,
             void* workspace, int B, int Hq,
             int Hkv, int Lq, int Lk, int D, int block_m, int block_n, int keep_m, int keep_n, float sm_scale, int out_rows,
-            int out_cols, LevelMapParams* lp, psa_sched::MapEnd& end, bool* map_done, psa_stream_t stream) {
+            int out_cols, LevelMapParams* lp, psa_sched::MapEnd& end, bool* map_done, psa_stream_t stream, const PoolParams* pool = nullptr) {
   PSA_REQUIRE(q.ptr && k.ptr && (scores || lp) && workspace, PSA_ERR_ARG, "psa_estimate_sampled: null pointer");
   PSA_REQUIRE(B > 0 && Hq > 0 && Hkv > 0 && Lq > 0 && Lk > 0, PSA_ERR_ARG, "psa_estimate_sampled: sizes must be positive");
   PSA_REQUIRE(Hq % Hkv == 0, PSA_ERR_ARG, "psa_estimate_sampled: Hq must be a multiple of Hkv");
@@ -584,7 +644,7 @@ int est_run(psa_tensor4 q, psa_tensor4 k, const int32_t* off_q, const int32_t* o
     PSA_REQUIRE(lp->Nk == out_cols, PSA_ERR_ARG, "psa_estimate_sampled_map: the map has %d columns, the scores %d", lp->Nk, out_cols);
     lp->scores = nullptr;
   }
-  return D == 128 ? launch_est<128>(p, B, (hipStream_t)stream, lp, end, map_done) : launch_est<64>(p, B, (hipStream_t)stream, lp, end, map_done);
+  return D == 128 ? launch_est<128>(p, B, (hipStream_t)stream, lp, end, pool, map_done) : launch_est<64>(p, B, (hipStream_t)stream, lp, end, pool, map_done);
 }
 }  // namespace
 
@@ -615,7 +675,7 @@ static int est_map_run(psa_tensor4 q, psa_tensor4 k, const int32_t* off_q, const
                        int keep_m, int keep_n, float sm_scale, int out_rows, int out_cols, void* map_out,
                        int map_elem_bytes, int mode, int n_items, const int32_t* item_level, const double* item_hi,
                        int align_div, int text_blocks, double min_full_attn_ratio, psa_stream_t stream, const int32_t* cap = nullptr,
-                       void* walk = nullptr, bool* ended = nullptr) {
+                       void* walk = nullptr, bool* ended = nullptr, const PoolParams* pool = nullptr) {
   PSA_REQUIRE(map_out, PSA_ERR_ARG, "psa_estimate_sampled_map: null pointer");
   PSA_REQUIRE(map_elem_bytes == 1 || map_elem_bytes == 4, PSA_ERR_ARG, "psa_estimate_sampled_map: map_elem_bytes must be 1 or 4");
   PSA_REQUIRE(out_cols > 0, PSA_ERR_ARG, "psa_estimate_sampled_map: out_cols must be positive");
@@ -634,7 +694,7 @@ static int est_map_run(psa_tensor4 q, psa_tensor4 k, const int32_t* off_q, const
   }
   bool map_done = false;
   const int rc2 = est_run(q, k, off_q, off_k, q_index, scores, workspace, B, Hq, Hkv, Lq, Lk, D, block_m, block_n, keep_m, keep_n,
-                          sm_scale, out_rows, out_cols, &lp, end, &map_done, stream);
+                          sm_scale, out_rows, out_cols, &lp, end, &map_done, stream, pool);
   if (ended != nullptr) *ended = map_done && end.map_out != nullptr;
   if (rc2 != PSA_OK || map_done) return rc2;
   return psa_level_map(scores, map_out, map_elem_bytes, nullptr, (int64_t)B * Hq * out_rows, out_cols, mode, n_items, item_level, item_hi,
@@ -664,12 +724,12 @@ extern "C" int psa_estimate_sampled_map_indexed(psa_tensor4 q, const int32_t* q_
 }
 
 // Map, similarity cap and tile records of a layer (psa_layer.hip): where *ended, the cap is applied and the records of `walk` are written
-// (its issue order is not).
+// (its issue order is not).  pool (null: none): the layer's pooling pass, run in the contraction's launch.
 int psa_estimate_layer_map(psa_tensor4 q, psa_tensor4 k, const int32_t* off_q, const int32_t* off_k, const int32_t* q_index, float* scores,
                            void* workspace, int B, int Hq, int Hkv, int L, int D, int block_m, int block_n, float sm_scale, void* map_out, int mode,
                            int n_items, const int32_t* item_level, const double* item_hi, int align_div, int text_blocks,
-                           double min_full_attn_ratio, const int32_t* cap, void* walk, bool* ended, psa_stream_t stream) {
+                           double min_full_attn_ratio, const int32_t* cap, void* walk, bool* ended, const PoolParams* pool, psa_stream_t stream) {
   return est_map_run(q, k, off_q, off_k, q_index, scores, workspace, B, Hq, Hkv, L, L, D, block_m, block_n, block_m / 4, block_n / 4, sm_scale,
                      (L + block_m - 1) / block_m, (L + block_n - 1) / block_n, map_out, 1, mode, n_items, item_level, item_hi, align_div,
-                     text_blocks, min_full_attn_ratio, stream, cap, walk, ended);
+                     text_blocks, min_full_attn_ratio, stream, cap, walk, ended, pool);
 }

@@ -3,6 +3,7 @@
 // work per launch (argument conversion, allocations, stream and device look-ups of five to nine calls), which bounds small
 // layers: 8 heads of 1000 tokens 82 -> 40 us, 2 fp32 heads of 4096 tokens 82 -> 57 us.
 #include "psa_common.h"
+#include "psa_pool_rows.h"
 #include "psa_schedule.h"
 
 // psa_level_map.hip
@@ -14,7 +15,7 @@ int psa_pool_kv_cap(psa_tensor4 k, psa_tensor4 v, const int32_t* index, const ps
 int psa_estimate_layer_map(psa_tensor4 q, psa_tensor4 k, const int32_t* off_q, const int32_t* off_k, const int32_t* q_index, float* scores,
                            void* workspace, int B, int Hq, int Hkv, int L, int D, int block_m, int block_n, float sm_scale, void* map_out, int mode,
                            int n_items, const int32_t* item_level, const double* item_hi, int align_div, int text_blocks,
-                           double min_full_attn_ratio, const int32_t* cap, void* walk, bool* ended, psa_stream_t stream);
+                           double min_full_attn_ratio, const int32_t* cap, void* walk, bool* ended, const PoolParams* pool, psa_stream_t stream);
 int psa_xattn_layer_map(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, void* workspace, void* k_pool, void* v_pool, int32_t* cap,
                         const float* thresholds, void* map, void* walk, int B, int Hq, int Hkv, int L, int D,
                         int block, int stride, int chunk, int mode, int n_items, const int32_t* item_level, const double* item_lo,
@@ -135,6 +136,30 @@ LayerExtra layer_extra(int elem, int B, int Hq, int Hkv, int L, int D, int block
   e.bytes = w.top;
   return e;
 }
+
+// Layers whose pooling pass runs in the launch of the estimate's contraction (psa_estimate.hip) instead of one of its own: up to 32 MiB of K
+// and V, 24 in fp32.  Such a launch is short, and its start and end are what it costs (a pass, us, before and after):
+//   bf16  8 heads x 1000 x 64   41.0  38.4     24 x 5000 x 64   74.7  69.5     12 x 5400 x 128  95.8  90.5     8 x 8192 x 128  121.6 120.7
+//   fp32  2 x 4096 x 64         56.5  52.7     4 x 6000 x 64   157.2 152.8     8 x 6000 x 64   223.8 217.1     8 x 8000 x 64   284.8 290.2
+// Larger ones of 16 bits have the pass on a stream of its own.
+bool pools_beside(int elem, int B, int Hkv, int L, int D) {
+  return (int64_t)B * Hkv * L * D * elem * 2 <= (int64_t)(elem == 4 ? 24 : 32) << 20;
+}
+// The output as the estimate's scratch, which ends before the output is written: large enough, aligned, without gaps, and apart from the
+// rows that are still to be read.  (In the workspace the scratch lies where the pools go.)
+bool overlaps(const psa_tensor4& out, int64_t out_bytes, const psa_tensor4& t, int elem, int B, int H, int L, int D) {
+  if (t.stride_b < 0 || t.stride_h < 0 || t.stride_l < 0) return true;
+  const int64_t bytes = ((B - 1) * t.stride_b + (H - 1) * t.stride_h + (L - 1) * t.stride_l + D) * elem;
+  const uintptr_t o = (uintptr_t)out.ptr, a = (uintptr_t)t.ptr;
+  return o < a + (uintptr_t)bytes && a < o + (uintptr_t)out_bytes;
+}
+bool output_takes_scratch(const psa_tensor4& out, const psa_tensor4& q, const psa_tensor4& k, const psa_tensor4& v, int64_t scratch, int elem, int B,
+                          int Hq, int Hkv, int L, int D) {
+  const int64_t bytes = (int64_t)B * Hq * L * D * elem;
+  const bool dense = (L == 1 || out.stride_l == D) && (Hq == 1 || out.stride_h == (int64_t)L * D) && (B == 1 || out.stride_b == (int64_t)Hq * L * D);
+  return out.ptr != nullptr && (uintptr_t)out.ptr % 256 == 0 && dense && scratch <= bytes && !overlaps(out, bytes, q, elem, B, Hq, L, D) &&
+         !overlaps(out, bytes, k, elem, B, Hkv, L, D) && !overlaps(out, bytes, v, elem, B, Hkv, L, D);
+}
 }  // namespace
 
 extern "C" int64_t psa_layer_extra_bytes(int elem_bytes, int B, int Hq, int Hkv, int L, int D, int block_m, int block_n, int indexed, int walk) {
@@ -171,7 +196,9 @@ extern "C" int psa_layer_fwd_extra(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, 
   char* vp = e.vp >= 0 ? ex + e.vp : ws + p.attn.vp;
   void* const listed = e.walk >= 0 ? ex + e.walk : nullptr;  // the walk, where the map's kernel writes its records
   const int Mq = (L + block_m - 1) / block_m, Nk = (L + block_n - 1) / block_n;
-  bool pooled = false, capped = false;
+  bool pooled = false, capped = false, beside = false;
+  PoolParams pool;
+  char* est_at = ws + p.est;  // the estimate's scratch
   int rc;
   if (token_index != nullptr) {
     psa_tensor4 ko = k, vo = v;
@@ -189,18 +216,28 @@ extern "C" int psa_layer_fwd_extra(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, 
     k = ko;
     v = vo;
   } else if (sim_thresholds != nullptr && extra != nullptr) {
-    rc = psa_pool_kv_cap(k, v, nullptr, nullptr, nullptr, kp, vp, cap_out, sim_thresholds, B, Hkv, L, D, block_n, stream);
+    beside = pools_beside(elem, B, Hkv, L, D);
+    rc = beside ? psa_pool_params(pool, k, v, nullptr, nullptr, nullptr, kp, vp, B, Hkv, L, D, block_n, cap_out, sim_thresholds)
+                : psa_pool_kv_cap(k, v, nullptr, nullptr, nullptr, kp, vp, cap_out, sim_thresholds, B, Hkv, L, D, block_n, stream);
     if (rc != PSA_OK) return rc;
     capped = pooled = true;
+  } else if (p.scores < 0 && pools_beside(elem, B, Hkv, L, D)) {
+    const int64_t scratch = psa_estimate_workspace_bytes(B, Hq, L, L, block_m, block_n, block_m / 4, block_n / 4);
+    if (output_takes_scratch(out, q, k, v, scratch, elem, B, Hq, Hkv, L, D)) {
+      rc = psa_pool_params(pool, k, v, nullptr, nullptr, nullptr, kp, vp, B, Hkv, L, D, block_n, nullptr, nullptr);
+      if (rc != PSA_OK) return rc;
+      est_at = (char*)out.ptr;
+      pooled = beside = true;
+    }
   }
   if (sim_thresholds != nullptr && !capped) {
     rc = psa_ksim(k, cap_out, B, Hkv, L, D, block_n, sim_thresholds[0], sim_thresholds[1], sim_thresholds[2], stream);
     if (rc != PSA_OK) return rc;
   }
   bool ended = false;
-  rc = psa_estimate_layer_map(q, k, off_q, off_k, token_index, p.scores >= 0 ? (float*)(ws + p.scores) : nullptr, ws + p.est, B, Hq, Hkv, L, D, block_m,
+  rc = psa_estimate_layer_map(q, k, off_q, off_k, token_index, p.scores >= 0 ? (float*)(ws + p.scores) : nullptr, est_at, B, Hq, Hkv, L, D, block_m,
                               block_n, sm_scale, map_out, mode, n_items, item_level, item_hi, align_div, text_blocks, min_full_attn_ratio,
-                              sim_thresholds != nullptr ? cap_out : nullptr, listed, &ended, stream);
+                              sim_thresholds != nullptr ? cap_out : nullptr, listed, &ended, beside ? &pool : nullptr, stream);
   if (rc != PSA_OK) return rc;
   if (sim_thresholds != nullptr && !ended) {
     rc = psa_map_min_cap(map_out, 1, cap_out, (int64_t)B * Hq, Mq, Nk, stream);
@@ -229,7 +266,7 @@ extern "C" int psa_estimate_walk(psa_tensor4 q, psa_tensor4 k, const int32_t* of
   PSA_REQUIRE(psa_schedule_geometry(B, Hq, Hkv, L, D, block_m, block_n, g), PSA_ERR_UNSUPPORTED, "psa_estimate_walk: shape out of range");
   bool ended = false;
   int rc = psa_estimate_layer_map(q, k, off_q, off_k, token_index, scores, workspace, B, Hq, Hkv, L, D, block_m, block_n, sm_scale, map_out, mode,
-                                  n_items, item_level, item_hi, align_div, text_blocks, min_full_attn_ratio, cap, walk, &ended, stream);
+                                  n_items, item_level, item_hi, align_div, text_blocks, min_full_attn_ratio, cap, walk, &ended, nullptr, stream);
   if (rc != PSA_OK) return rc;
   if (ended) return psa_walk_order(walk, g, stream);
   if (cap != nullptr) {
