@@ -377,12 +377,18 @@ __global__ __launch_bounds__(256) void psa_bwd_cost_kernel(BwdParams p, int row_
 // head's map alone, and they fit its share of that buffer (cut slots have fewer than 1.5 * pairs / unit parts).
 // An item: {kv-block | part << 16 | parts << 24, its slot of the buffer}; a head's items are its slots' first parts (even entries) and
 // the other parts, spread over the odd entries.  Unused: parts = 0.
-// Training steps without / with parts, us, fixed quotas and thresholds: 12 heads of 2500 x 128 250 / 184 and 247 / 232, 8 of 5300 x 128 326 /
-// 267 and 334 / 318, 12 of 5300 x 128 360 / 293 and 382 / 355, 24 of 4000 x 128 (768 slots) 370 / 353 and 429 / 430; head dim 64: 8 of
-// 9000 369 / 321 and 379 / 349, 8 of 16000 (1000 slots) 629 / 629 and 627 / 605.  Larger launches lose: slots that walk the same q-blocks
-// at the same time share their rows in L2, parts do not, and the sums cost traffic (12 of 9000 x 128, 852 slots, 604 / 631 and 699 / 739).
+// Which launches: training steps without / with parts, us, fixed quotas and thresholds, by the longest possible list (q-blocks of the kv head):
+//   head dim 128   16 q-blocks, 384 slots 205 / 179 and 230 / 231, 768 slots 268 / 281 and 319 / 352;   26, 650 slots 311 / 286 and 372 / 363, 780
+//                  336 / 341 and 416 / 430;   32, 512 slots 295 / 249 and 334 / 322;   48, 768 slots 456 / 427 and 522 / 494;   8, 384 slots 148 / 154 and 175 / 181
+//   head dim 64    16, 384 and more slots, and 26: 1 to 3 % slower (steps that the host bounds: two launches more);   32, 768 slots 243 / 241 and
+//                  279 / 273;   48, 768 slots 311 / 256 and 338 / 313, 1008 slots 331 / 294 and 392 / 389;   125, 1000 slots 629 / 629 and 627 / 605
+// Short lists have little to cut for the two launches and the traffic of the sums; in large launches slots that walk the same q-blocks at the
+// same time share their rows in L2, parts do not (12 heads of 9000 x 128, 852 slots, 604 / 631 and 699 / 739).
 constexpr int PART_MEAN_10 = 17, PART_MIN = 4, PART_MOST = 64;
-constexpr int parts_max_slots(int D) { return D == 128 ? 768 : 1024; }  // (the chip holds 512 / 768 workgroups at once)
+bool slots_in_parts(int D, int64_t slots, int64_t list) {  // (the chip holds 512 / 768 workgroups of the walk at once)
+  const int64_t most = D == 128 ? 768 : 1024;
+  return list >= (D == 128 ? 16 : 32) && slots <= (24 * list < most ? 24 * list : most);
+}
 __device__ __forceinline__ int part_at(int n, int part, int parts) { return (int)((int64_t)n * part / parts); }
 
 __global__ __launch_bounds__(256) void psa_bwd_parts_kernel(const int32_t* count0, int Nk, int min_unit, bool octaves, u32x2* items, int32_t* cost) {
@@ -1154,7 +1160,7 @@ extern "C" int psa_bwd(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const void* 
   const int64_t total = (int64_t)B * Hq * Mq, n_blocks = (int64_t)B * Hkv * Nk;
   const bool wide0 = block_n > 64;
   const bool cols_ordered = map != nullptr && n_blocks > 8;
-  const bool in_parts = cols_ordered && wide0 && n_blocks <= parts_max_slots(D);
+  const bool in_parts = cols_ordered && wide0 && slots_in_parts(D, n_blocks, (int64_t)(Hq / Hkv) * Mq);
   const int64_t n_wide = wide0 ? (in_parts ? 2 * n_blocks : n_blocks) : 0, n_rest = n_blocks * (wide0 ? DKDV_SLOTS - 1 : DKDV_SLOTS);
   PSA_REQUIRE(total < (1ll << 28) && 4 * n_blocks < (1ll << 28), PSA_ERR_UNSUPPORTED, "psa_bwd: too many workgroups");
   // shares by the K/V rows (dQ) and the Q/dO rows (dK/dV) that the walks stream

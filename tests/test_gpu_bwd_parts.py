@@ -18,11 +18,13 @@ def _popular(B, H, Mq, Nk, seed, columns):
 
 
 @pytest.mark.parametrize("B,Hq,Hkv,L,bm", [
-    (1, 3, 3, 1024, 128),      # lists of 8: two parts of a unit of 4
-    (1, 2, 2, 1100, 128),      # a ragged last block among them: pad rows
-    (2, 4, 2, 1000, 128),      # two query heads: lists of 16
+    (1, 2, 2, 4096, 128),      # lists of 32
+    (1, 1, 1, 4300, 128),      # a ragged last block among them: pad rows
+    (2, 8, 2, 1000, 128),      # four query heads: lists of 32
     (1, 2, 1, 1500, 64),       # 64-row q-blocks
     (1, 8, 1, 1300, 128),      # lists of 88, several parts
+    (1, 2, 1, 1024, 128),      # lists of 16: cut at head dim 128
+    (1, 1, 1, 1900, 128),      # lists of 15: not cut
 ])
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("causal", [False, True])
@@ -39,18 +41,18 @@ def test_cut_slots(B, Hq, Hkv, L, bm, D, causal):
 @pytest.mark.parametrize("D", [64, 128])
 def test_every_slot_long(D):
     """All lists equally long: nothing is cut, whatever their length.  And one long list among empty ones."""
-    run_bwd(1, 2, 2, 1300, D, 128, 128, False, seed=1, lmap=np.ones((1, 2, 11, 11), np.int32))
-    m = np.zeros((1, 2, 11, 11), np.int32)
+    run_bwd(1, 2, 2, 4200, D, 128, 128, False, seed=1, lmap=np.ones((1, 2, 33, 33), np.int32))
+    m = np.zeros((1, 2, 33, 33), np.int32)
     m[0, 0, :, 4] = 1
-    m[0, 1, :, 10] = 1
-    run_bwd(1, 2, 2, 1300, D, 128, 128, False, seed=2, lmap=m)
+    m[0, 1, :, 32] = 1
+    run_bwd(1, 2, 2, 4200, D, 128, 128, False, seed=2, lmap=m)
 
 
 @pytest.mark.parametrize("D", [64, 128])
 def test_a_head_has_its_bits_in_any_launch(D):
     from psa_hip import ops
 
-    H, L = 6, 128 * 24 + 40
+    H, L = 6, 128 * 32 + 40
     n = -(-L // 128)
     q, k, v = (rnd(1, H, L, D, seed=i).to(dev()) for i in range(3))
     do = rnd(1, H, L, D, seed=3, scale=0.5).to(dev())
