@@ -3,15 +3,16 @@
 // (psa_tiles.h: the map row is compacted into tiles of 64 pooled keys of one level), same softmax (base 2, +log2(level)
 // bias, online), same masks.
 //
-// One workgroup of 4 waves per QR = 64 / KS query rows; the K and V tile goes straight into LDS and is shared by the waves:
-// wave w works on row group w / KS (16 rows) and the w % KS -th share of the tile's four 16-key blocks, with a softmax state
-// of its own; the KS shares of a row meet once, at the end.  KS = 1, 2 or 4: the smallest that still gives the launch two
-// workgroups per CU (the small layers this path serves have few rows: 2 heads of 4096 tokens are 128 q-blocks of 64).
+// A tile's four 16-key blocks go one to each wave of a workgroup (psa_fwd_f32_direct_kernel: 16 or 32 query rows; a softmax state per
+// wave, joined once at the end) or all to every wave, which then has 16 rows of its own (psa_fwd_f32_kernel: 64 rows).
 // The transposed products S^T = K Q^T and O^T += V^T P^T leave a lane 4 keys of one query in the accumulator, and with
 // k-index g of the i-th PV step taken to be key 4 g + i that register IS the step's B operand: nothing crosses lanes
 // between the two products, and a row maximum is two lane exchanges.  Channels are dealt so that a lane's operands of four
-// steps are 16 consecutive bytes (one ds_read_b128); rows are XOR-swizzled by 16-byte chunks: conflict-free.
-// 2 heads of 4096 tokens x 64, 64-key blocks, 80 % sparse: 109 us on the vector units (two LDS operands per 4 FMAs), 36 us here.
+// steps are 16 consecutive bytes.
+// Bound by the vector units: the fp32 matrix instruction runs on them, 32 cycles of a SIMD for 16 x 16 x 4, and nothing else issues beside
+// it.  What helps is fewer instructions around it.
+// 2 heads of 4096 tokens x 64, 64-key blocks, 80 % sparse: 109 us with plain multiply-adds (two LDS operands per 4 FMAs), 36 with tiles through
+// LDS, 27 here (11 of them products).
 #include <type_traits>
 
 #include "psa_common.h"
@@ -47,10 +48,61 @@ struct F32Geom {
   static constexpr int STAGES = D == 64 ? 2 : 1;  // (128 channels: two workgroups per CU instead of a second buffer)
 };
 
+// The KS shares of a row meet in LDS; results leave as rows.  smem: 64 rows of D + 4 floats.
 template <int D, int KS>
+__device__ __forceinline__ void f32_finish(const F32Params& p, int b, int h, int q0, int wave, int l16, int g4, int tid, const f32x4 (&acc)[D / 16],
+                                           float m_run, float l_run, float* smem, float (*s_m)[16], float (*s_l)[16]) {
+  using G = F32Geom<D>;
+  constexpr int QR = 64 / KS, DB = D / 16;
+  constexpr int OP = D + 4;  // padded row of the staging area (floats)
+  float l_tot = l_run + __shfl_xor(l_run, 16, 64);
+  l_tot += __shfl_xor(l_tot, 32, 64);
+  float* os = smem + wave * 16 * OP;
+#pragma unroll
+  for (int c = 0; c < DB / 4; ++c)
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      *(f32x4*)(os + l16 * OP + 64 * c + 16 * g4 + 4 * i) = f32x4{acc[4 * c][i], acc[4 * c + 1][i], acc[4 * c + 2][i], acc[4 * c + 3][i]};
+  if (g4 == 0) {
+    s_m[wave][l16] = m_run;
+    s_l[wave][l16] = l_tot;
+  }
+  __syncthreads();
+  for (int u = tid; u < QR * G::CH; u += 256) {
+    const int r = u / G::CH, c4 = u % G::CH, w0 = (r >> 4) * KS, r16 = r & 15;
+    const int qi = q0 + r;
+    if (qi >= p.L) continue;
+    const int orow = p.q_index != nullptr ? p.q_index[qi] : qi;
+    if ((unsigned)orow >= (unsigned)p.L) continue;
+    float m = s_m[w0][r16];
+#pragma unroll
+    for (int w = 1; w < KS; ++w) m = fmaxf(m, s_m[w0 + w][r16]);
+    const float m_use = m == -INFINITY ? 0.f : m;
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+    float l = 0.f;
+#pragma unroll
+    for (int w = 0; w < KS; ++w) {
+      const float f = fast_exp2(s_m[w0 + w][r16] - m_use);
+      const f32x4 x = *(const f32x4*)(smem + ((w0 + w) * 16 + r16) * OP + c4 * 4);
+      l = __builtin_fmaf(s_l[w0 + w][r16], f, l);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = __builtin_fmaf(x[e], f, o[e]);
+    }
+    const float l_safe = fmaxf(l, 1e-8f);
+    const float inv = 1.0f / l_safe;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] *= inv;
+    *(f32x4*)(p.o + b * p.o_sb + h * p.o_sh + (int64_t)orow * p.o_sl + c4 * 4) = o;
+    if (p.lse != nullptr && c4 == 0) p.lse[((int64_t)b * p.Hq + h) * p.L + orow] = (m + fast_log2(l_safe)) * 0.6931471805599453f;
+  }
+}
+
+// Large launches at head dim 128, and rows that lie too far apart for 32-bit offsets: 64 rows per workgroup.  The K and V tile goes straight
+// into LDS and is shared by the waves; rows are XOR-swizzled by 16-byte chunks (one ds_read_b128 per four steps): conflict-free.
+template <int D>
 __global__ __launch_bounds__(256, 2) void psa_fwd_f32_kernel(F32Params p) {
   using G = F32Geom<D>;
-  constexpr int QR = 64 / KS, KBW = 4 / KS, SQ = D / 16, DB = D / 16;
+  constexpr int QR = 64, KBW = 4, SQ = D / 16, DB = D / 16;
   extern __shared__ __align__(16) unsigned char smem[];  // [STAGES][K, V] tiles, later the shares of the output
   u32x2* tdesc = (u32x2*)(smem + G::STAGES * 2 * G::TILE);
   uint16_t* ids = (uint16_t*)(tdesc + p.max_tiles);
@@ -59,13 +111,12 @@ __global__ __launch_bounds__(256, 2) void psa_fwd_f32_kernel(F32Params p) {
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l16 = lane & 15, g4 = lane >> 4;
-  const int rg = wave / KS, ks = wave % KS;
   const int unit = blockIdx.x;  // (b, h, q-block, part)
   const int part = unit % p.parts, logical = unit / p.parts;
   const int I = logical % p.Mq, bh = logical / p.Mq, h = bh % p.Hq, b = bh / p.Hq;
   const int hk = h / (p.Hq / p.Hkv);
   const int q0 = I * p.bm + part * QR;  // first query position of this workgroup
-  const int q_idx = q0 + rg * 16 + l16;
+  const int q_idx = q0 + wave * 16 + l16;
   int jmax = p.Nk;
   if (p.causal) {
     const int ce = (int)((((int64_t)(I + 1) * p.bm) + (1 << p.bn_log2) - 1) >> p.bn_log2);
@@ -130,7 +181,7 @@ __global__ __launch_bounds__(256, 2) void psa_fwd_f32_kernel(F32Params p) {
   float m_run = -INFINITY, l_run = 0.f;  // the row's maximum over this wave's keys; this lane's part of its sum
 
   auto compute = [&](int t, int stage) __attribute__((always_inline)) {
-    PSA_LDS(unsigned char) Ts = (PSA_LDS(unsigned char))(smem) + stage * 2 * G::TILE + ks * (KBW * 16 * G::ROW);
+    PSA_LDS(unsigned char) Ts = (PSA_LDS(unsigned char))(smem) + stage * 2 * G::TILE;
     f32x4 s[KBW];
 #pragma unroll
     for (int x = 0; x < KBW; ++x) {
@@ -154,7 +205,7 @@ __global__ __launch_bounds__(256, 2) void psa_fwd_f32_kernel(F32Params p) {
       const int qlim = (q_idx + 1) >> tr.lv;
 #pragma unroll
       for (int x = 0; x < KBW; ++x) {
-        const int r0 = (ks * KBW + x) * 16 + 4 * g4;
+        const int r0 = x * 16 + 4 * g4;
         int keep = tr.nvalid - r0;
         if (p.causal) {
           const int pos = (tr.lt << 6) + r0;
@@ -170,8 +221,7 @@ __global__ __launch_bounds__(256, 2) void psa_fwd_f32_kernel(F32Params p) {
     float mx = fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3]));
 #pragma unroll
     for (int x = 1; x < KBW; ++x) mx = fmaxf(mx, fmaxf(fmaxf(s[x][0], s[x][1]), fmaxf(s[x][2], s[x][3])));
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mx = quarter_wave_max(mx);
     const float m_new = fmaxf(m_run, mx);
     const float m_use = m_new == -INFINITY ? 0.f : m_new;
     const float alpha = fast_exp2(m_run - m_use);
@@ -224,60 +274,255 @@ __global__ __launch_bounds__(256, 2) void psa_fwd_f32_kernel(F32Params p) {
     }
   }
 
-  // ---- the KS shares of a row meet in LDS; results leave as rows ---------------------------------------------------
-  constexpr int OP = D + 4;  // padded row of the staging area (floats)
-  float l_tot = l_run + __shfl_xor(l_run, 16, 64);
-  l_tot += __shfl_xor(l_tot, 32, 64);
-  float* os = (float*)smem + wave * 16 * OP;
+  f32_finish<D, 1>(p, b, h, q0, wave, l16, g4, tid, acc, m_run, l_run, (float*)smem, s_m, s_l);
+}
+
+// 16 RG rows per workgroup, K and V rows straight into the registers of the wave that has their block: no LDS tiles and no barriers between
+// the row's list and the end.  The next block's rows are requested before a block's products (two blocks ahead: more registers, fewer waves, 4 to
+// 8 % slower).  Wave w has keys 16 w .. 16 w + 15 of every tile.  RG = 2 halves the row addresses per product and the number of workgroups.
+// Measured: layers of 80 % sparsity, us, with LDS tiles (16 to 64 rows), RG = 1 and RG = 2:
+//   head dim 64   2 heads x 4096  58 / 51 / 52   4 x 3291  84 / 69 / 71   8 x 2000 (1000 blocks of 16 rows)  64 / 59 / 60
+//                 8 x 3000 (1504)  110 / 89 / 84   8 x 6000 (3000)  228 / 193 / 186   24 x 8000 (12000)  837 / 816 / 784   16 x 16000  1732 / 1734 / 1669
+//   head dim 128  2 x 4096  90 / 77   8 x 6000 (3000)  423 / 395   8 x 8000 (4000)  558 / 570   16 x 4500 (4512)  526 / 533   24 x 4000 (6000)  577 / 613
+// (RG = 2 at head dim 128 would take more than the 256 registers of two waves per SIMD.)
+template <int D, int RG>
+__global__ __launch_bounds__(256, 2) void psa_fwd_f32_direct_kernel(F32Params p) {
+  constexpr int SQ = D / 16, DB = D / 16, NV = D / 16, NB = 2;
+  extern __shared__ __align__(16) unsigned char smem[];  // the shares of the output, then the row's tiles
+  u32x2* tdesc = (u32x2*)(smem + 64 * (D + 4) * 4);
+  uint16_t* ids = (uint16_t*)(tdesc + p.max_tiles);
+  __shared__ int s_cnt[4], s_ioff[4], s_toff[5], s_wcnt[16];
+  __shared__ float s_m[4][16], s_l[4][16];
+  __shared__ __align__(16) u32x4 s_base[4];  // first rows of K and V of every level
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, g4 = lane >> 4;
+  const int unit = blockIdx.x;  // (b, h, q-block, part)
+  const int part = unit % p.parts, logical = unit / p.parts;
+  const int I = logical % p.Mq, bh = logical / p.Mq, h = bh % p.Hq, b = bh / p.Hq;
+  const int hk = h / (p.Hq / p.Hkv);
+  const int q0 = I * p.bm + part * (16 * RG);
+  int jmax = p.Nk;
+  if (p.causal) {
+    const int ce = (int)((((int64_t)(I + 1) * p.bm) + (1 << p.bn_log2) - 1) >> p.bn_log2);
+    jmax = ce < jmax ? ce : jmax;
+  }
+  f32x4 qf[RG][SQ];
 #pragma unroll
-  for (int c = 0; c < DB / 4; ++c)
+  for (int r = 0; r < RG; ++r) {
+    int qr = q0 + r * 16 + l16;
+    qr = qr < p.L ? qr : p.L - 1;
+    if (p.q_index != nullptr) qr = clamp_row(p.q_index[qr], p.L);
+    const float* qp = p.q + b * p.q_sb + h * p.q_sh + (int64_t)qr * p.q_sl + 4 * g4;
+#pragma unroll
+    for (int s = 0; s < SQ; ++s) qf[r][s] = *(const f32x4*)(qp + 16 * s);
+  }
+  if (tid < 4) {
+    const int64_t BHkv = (int64_t)p.B * p.Hkv, bhk = (int64_t)b * p.Hkv + hk, at = psa_tiles::pool_row_offset(tid, BHkv, bhk, p.npad) * D;
+    const uint64_t kb = (uint64_t)(tid == 0 ? p.k + b * p.k_sb + hk * p.k_sh : p.kp + at), vb = (uint64_t)(tid == 0 ? p.v + b * p.v_sb + hk * p.v_sh : p.vp + at);
+    s_base[tid] = u32x4{(uint32_t)kb, (uint32_t)(kb >> 32), (uint32_t)vb, (uint32_t)(vb >> 32)};
+  }
+  const int T = psa_tiles::build_row_schedule<256>(p.map, p.map_elem, ((int64_t)bh * p.Mq + I) * p.Nk, p.Nk, jmax, p.bn_log2, p.L,
+                                                  p.causal != 0, (int64_t)I * p.bm, ids, tdesc, s_cnt, s_ioff, s_toff, s_wcnt);
+
+  // Rows through buffer descriptors: 32-bit offsets (one 24-bit multiply-add per lane and tensor), the four V rows of a lane, which follow
+  // each other in one block, by scalar offsets.
+  auto rows_of = [](uint32_t lo, uint32_t hi) __attribute__((always_inline)) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane(hi) << 32 | (uint32_t)__builtin_amdgcn_readfirstlane(lo)), 0, -1, 0x00020000);
+  };
+
+  // Two look-ups lead from a tile to its rows: its description, then the blocks of this lane's K row and V rows.
+  struct Block {
+    f32x4 k[SQ], v[NV];
+    uint32_t d0, d1;
+  };
+  u32x2 d_next = {0u, 0u};
+  uint32_t d0 = 0, d1 = 0;
+  int k_id = 0, v_id = 0;
+  u32x4 base = {0u, 0u, 0u, 0u};
+  auto look_desc = [&](int t) __attribute__((always_inline)) { d_next = tdesc[t < T ? t : T - 1]; };
+  auto look_ids = [&]() __attribute__((always_inline)) {
+    d0 = __builtin_amdgcn_readfirstlane(d_next[0]);
+    d1 = __builtin_amdgcn_readfirstlane(d_next[1]);
+    const int sbs_log2 = p.bn_log2 - (int)(d0 & 3), last = (int)(d1 >> 16) - 1;
+    const uint16_t* list = ids + (d1 & 0xffff);
+    const int pos = ((int)(d0 >> 10) << 6) + wave * 16;
+    int kb = (pos + l16) >> sbs_log2, vb = (pos + 4 * g4) >> sbs_log2;
+    kb = kb < last ? kb : last;
+    vb = vb < last ? vb : last;
+    k_id = list[kb];
+    v_id = list[vb];
+    base = s_base[d0 & 3];
+  };
+  auto load = [&](Block& w) __attribute__((always_inline)) {
+    const int lv = d0 & 3, sbs_log2 = p.bn_log2 - lv, mask = (1 << sbs_log2) - 1, pos = ((int)(d0 >> 10) << 6) + wave * 16;
+    const uint32_t kstr = lv == 0 ? (uint32_t)p.k_sl * 4u : D * 4u, vstr = lv == 0 ? (uint32_t)p.v_sl * 4u : D * 4u;
+    const auto kr = rows_of(base[0], base[1]), vr = rows_of(base[2], base[3]);
+    const int last = (lv == 0 ? p.L : (int)(p.npad >> lv)) - 1;
+    int ks = (k_id << sbs_log2) + ((pos + l16) & mask);
+    ks = ks < last ? ks : last;
+    const int at = (int)__umul24(ks, kstr) + 16 * g4;
+#pragma unroll
+    for (int s = 0; s < SQ; ++s) w.k[s] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(kr, at + 64 * s, 0, 0));
+    const int vs = (v_id << sbs_log2) + ((pos + 4 * g4) & mask);
+    if (lv == 0 && (d0 >> 3 & 127) < TK32) {  // (the sequence may end among the four rows)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int vat = (int)__umul24(vs + i < last ? vs + i : last, vstr) + 16 * l16;
+#pragma unroll
+        for (int c = 0; c < DB / 4; ++c) w.v[i * (DB / 4) + c] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(vr, vat + 256 * c, 0, 0));
+      }
+    } else {
+      const int vat = (int)__umul24(vs, vstr) + 16 * l16;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int c = 0; c < DB / 4; ++c)
+          w.v[i * (DB / 4) + c] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(vr, vat + 256 * c, (int)(i * vstr), 0));
+    }
+    w.d0 = d0;
+    w.d1 = d1;
+  };
+
+  f32x4 acc[RG][DB];
+  float m_run[RG], l_run[RG];
+#pragma unroll
+  for (int r = 0; r < RG; ++r) {
+#pragma unroll
+    for (int db = 0; db < DB; ++db) acc[r][db] = f32x4{0.f, 0.f, 0.f, 0.f};
+    m_run[r] = -INFINITY;
+    l_run[r] = 0.f;
+  }
+
+  auto compute = [&](Block& w) __attribute__((always_inline)) {
+    const int lv = w.d0 & 3, nvalid = (w.d0 >> 3) & 127;
+    if (wave * 16 >= nvalid) return;
+    f32x4 s[RG];
+#pragma unroll
+    for (int r = 0; r < RG; ++r) s[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < SQ; ++c)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int r = 0; r < RG; ++r) s[r] = __builtin_amdgcn_mfma_f32_16x16x4f32(w.k[c][j], qf[r][c][j], s[r], 0, 0, 0);
+    const float bias = (float)lv;
+#pragma unroll
+    for (int r = 0; r < RG; ++r)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s[r][i] = __builtin_fmaf(s[r][i], p.scale_log2, bias);
+    if (w.d0 & 4) {
+      // (as above; V rows of slots that hold no key are some row of the sequence and become zero)
+      const int r0 = wave * 16 + 4 * g4, full = nvalid - r0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int c = 0; c < DB / 4; ++c)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) w.v[i * (DB / 4) + c][e] = i < full ? w.v[i * (DB / 4) + c][e] : 0.f;
+      int src0 = 0;
+      if (p.causal) {
+        const int pos = ((int)(w.d0 >> 10) << 6) + r0, sbs_log2 = p.bn_log2 - lv, last = (int)(w.d1 >> 16) - 1;
+        int bi = pos >> sbs_log2;
+        bi = bi < last ? bi : last;
+        src0 = ((int)ids[(w.d1 & 0xffff) + bi] << sbs_log2) + (pos & ((1 << sbs_log2) - 1));
+      }
+#pragma unroll
+      for (int r = 0; r < RG; ++r) {
+        const int qlim = (q0 + r * 16 + l16 + 1) >> lv;
+        const int keep = p.causal && qlim - src0 < full ? qlim - src0 : full;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s[r][i] = i < keep ? s[r][i] : -INFINITY;
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < RG; ++r) {
+      const float mx = quarter_wave_max(fmaxf(fmaxf(s[r][0], s[r][1]), fmaxf(s[r][2], s[r][3])));
+      const float m_new = fmaxf(m_run[r], mx);
+      const float m_use = m_new == -INFINITY ? 0.f : m_new;
+      const float alpha = fast_exp2(m_run[r] - m_use);
+      float sum = 0.f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        s[r][i] = fast_exp2(s[r][i] - m_use);
+        sum += s[r][i];
+      }
+      l_run[r] = l_run[r] * alpha + sum;
+      m_run[r] = m_new;
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[r][db][i] *= alpha;
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      *(f32x4*)(os + l16 * OP + 64 * c + 16 * g4 + 4 * i) = f32x4{acc[4 * c][i], acc[4 * c + 1][i], acc[4 * c + 2][i], acc[4 * c + 3][i]};
-  if (g4 == 0) {
-    s_m[wave][l16] = m_run;
-    s_l[wave][l16] = l_tot;
-  }
-  __syncthreads();
-  for (int u = tid; u < QR * G::CH; u += 256) {
-    const int r = u / G::CH, c4 = u % G::CH, w0 = (r >> 4) * KS, r16 = r & 15;
-    const int qi = q0 + r;
-    if (qi >= p.L) continue;
-    const int orow = p.q_index != nullptr ? p.q_index[qi] : qi;
-    if ((unsigned)orow >= (unsigned)p.L) continue;
-    float m = s_m[w0][r16];
 #pragma unroll
-    for (int w = 1; w < KS; ++w) m = fmaxf(m, s_m[w0 + w][r16]);
-    const float m_use = m == -INFINITY ? 0.f : m;
-    f32x4 o = {0.f, 0.f, 0.f, 0.f};
-    float l = 0.f;
+      for (int c = 0; c < DB / 4; ++c)
 #pragma unroll
-    for (int w = 0; w < KS; ++w) {
-      const float f = fast_exp2(s_m[w0 + w][r16] - m_use);
-      const f32x4 x = *(const f32x4*)((const float*)smem + ((w0 + w) * 16 + r16) * OP + c4 * 4);
-      l = __builtin_fmaf(s_l[w0 + w][r16], f, l);
+        for (int r = 0; r < RG; ++r)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) o[e] = __builtin_fmaf(x[e], f, o[e]);
+          for (int e = 0; e < 4; ++e)
+            acc[r][4 * c + e] = __builtin_amdgcn_mfma_f32_16x16x4f32(w.v[i * (DB / 4) + c][e], s[r][i], acc[r][4 * c + e], 0, 0, 0);
+  };
+  if (T > 0) {
+    Block w[NB];
+    look_desc(0);
+    look_ids();
+    look_desc(1);
+#pragma unroll
+    for (int n = 0; n < NB - 1; ++n) {
+      load(w[n]);
+      look_ids();
+      look_desc(n + 2);
     }
-    const float l_safe = fmaxf(l, 1e-8f);
-    const float inv = 1.0f / l_safe;
+    auto step = [&](int t, Block& next, Block& w) __attribute__((always_inline)) {
+      load(next);  // tile t + NB - 1, or the last again
+      look_ids();
+      look_desc(t + NB + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      compute(w);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    for (int t = 0;;) {
+      step(t, w[NB - 1], w[0]);
+      if (++t >= T) break;
+      step(t, w[0], w[1]);
+      if (++t >= T) break;
+    }
+  }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] *= inv;
-    *(f32x4*)(p.o + b * p.o_sb + h * p.o_sh + (int64_t)orow * p.o_sl + c4 * 4) = o;
-    if (p.lse != nullptr && c4 == 0) p.lse[((int64_t)b * p.Hq + h) * p.L + orow] = (m + fast_log2(l_safe)) * 0.6931471805599453f;
+  for (int r = 0; r < RG; ++r) {
+    if (r > 0) __syncthreads();  // the staging area's readers are done
+    f32_finish<D, 4>(p, b, h, q0 + 16 * r, wave, l16, g4, tid, acc[r], m_run[r], l_run[r], (float*)smem, s_m, s_l);
   }
 }
 
-template <int D, int KS>
-int launch_f32(const F32Params& p, hipStream_t stream) {
-  using G = F32Geom<D>;
-  const size_t shmem = (size_t)G::STAGES * 2 * G::TILE + (size_t)p.max_tiles * 8 + (size_t)p.Nk * 2 + 16;
-  if (shmem > 159 * 1024) return PSA_ERR_UNSUPPORTED;
-  if (hipFuncSetAttribute((const void*)psa_fwd_f32_kernel<D, KS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem) != hipSuccess)
+size_t f32_list_bytes(const F32Params& p) { return (size_t)p.max_tiles * 8 + (size_t)p.Nk * 2 + 16; }
+
+template <class K>
+int launch_f32(K kernel, size_t tiles, int64_t grid, const F32Params& p, hipStream_t stream) {
+  const size_t shmem = tiles + f32_list_bytes(p);
+  if (shmem > 48 * 1024 && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem) != hipSuccess)
     return PSA_ERR_LAUNCH;
-  const int64_t units = (int64_t)p.B * p.Hq * p.Mq * p.parts;
-  hipLaunchKernelGGL((psa_fwd_f32_kernel<D, KS>), dim3((unsigned)units), dim3(256), shmem, stream, p);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(256), shmem, stream, p);
   return PSA_OK;
+}
+template <int D>
+int launch_f32(F32Params p, hipStream_t stream) {
+  const int64_t rows16 = (int64_t)p.B * p.Hq * p.Mq * (p.bm / 16);
+  // (sizes in elements: a row's offset in bytes below 2^31, its factors below 2^24)
+  auto near = [&](int64_t stride, int64_t rows) { return stride >= 0 && stride < (1 << 22) && rows < (1 << 24) && rows * (stride > D ? stride : D) < (1ll << 29); };
+  const bool direct = near(p.k_sl, p.L) && near(p.v_sl, p.L) && near(D, p.npad);
+  if (direct && (D == 64 || rows16 <= 3072)) {
+    const int rg = D == 64 && rows16 > 1280 ? 2 : 1;
+    p.parts = p.bm / (16 * rg);
+    const size_t stage = (size_t)64 * (D + 4) * 4;
+    if constexpr (D == 64)
+      if (rg == 2) return launch_f32(psa_fwd_f32_direct_kernel<D, 2>, stage, rows16 / rg, p, stream);
+    return launch_f32(psa_fwd_f32_direct_kernel<D, 1>, stage, rows16 / rg, p, stream);
+  }
+  p.parts = p.bm / 64;
+  return launch_f32(psa_fwd_f32_kernel<D>, (size_t)F32Geom<D>::STAGES * 2 * F32Geom<D>::TILE, rows16 / 4, p, stream);
 }
 
 }  // namespace
@@ -309,19 +554,15 @@ int psa_fwd_f32(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const void* k_pool,
   p.v_sb = v.stride_b; p.v_sh = v.stride_h; p.v_sl = v.stride_l;
   p.o_sb = out.stride_b; p.o_sh = out.stride_h; p.o_sl = out.stride_l;
   p.B = B; p.Hq = Hq; p.Hkv = Hkv; p.L = L; p.Mq = Mq; p.Nk = Nk;
-  // rows per workgroup: 64, or 32 / 16 while the launch would have fewer than two workgroups per CU
-  int ks = 1;
-  while (ks < 4 && (int64_t)B * Hq * Mq * (block_m * ks / 64) < 512) ks *= 2;
-  p.bn_log2 = psa_ilog2(block_n); p.bm = block_m; p.parts = block_m * ks / 64;
+  p.bn_log2 = psa_ilog2(block_n); p.bm = block_m;
   p.npad = (int64_t)Nk * block_n;
   p.scale_log2 = sm_scale * 1.4426950408889634f;
   p.causal = causal ? 1 : 0;
   p.max_tiles = (block_n >= 64 ? Nk * (block_n / 64) : (Nk * block_n + 63) / 64) + 4;
   p.q_index = q_index;
   hipStream_t st = (hipStream_t)stream;
-  int rc;
-  if (D == 128) rc = ks == 1 ? launch_f32<128, 1>(p, st) : ks == 2 ? launch_f32<128, 2>(p, st) : launch_f32<128, 4>(p, st);
-  else rc = ks == 1 ? launch_f32<64, 1>(p, st) : ks == 2 ? launch_f32<64, 2>(p, st) : launch_f32<64, 4>(p, st);
-  PSA_REQUIRE(rc == PSA_OK, rc, "psa_fwd: sequence too long for the fp32 kernel's on-chip schedule (LDS)");
+  PSA_REQUIRE(64 * 1024 + f32_list_bytes(p) <= 159 * 1024, PSA_ERR_UNSUPPORTED, "psa_fwd: sequence too long for the fp32 kernel's on-chip schedule (LDS)");
+  const int rc = D == 128 ? launch_f32<128>(p, st) : launch_f32<64>(p, st);
+  PSA_REQUIRE(rc == PSA_OK, rc, "psa_fwd: cannot reserve the fp32 kernel's LDS");
   return psa_check_launch("psa_fwd (fp32)");
 }
