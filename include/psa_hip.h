@@ -304,7 +304,8 @@ int psa_estimate_walk(psa_tensor4 q, psa_tensor4 k, const int32_t* off_q, const 
  * the separate calls.  token_index (may be NULL): the layer works on the re-ordered tokens (psa_pool_kv_indexed, and the
  * *_indexed forms of the others).  sim_thresholds (may be NULL; 3 floats on the host): psa_ksim of the keys in the layer's order
  * into cap_out (int32 [B, Hkv, Nk]) and psa_map_min_cap; Hq == Hkv.  workspace: psa_layer_workspace_bytes(...) bytes (elem_bytes of
- * q / k / v: 2 or 4), 256-byte aligned; map_out: int8 [B, Hq, ceil(L / block_m), ceil(L / block_n)]. */
+ * q / k / v: 2 or 4), 256-byte aligned; map_out: int8 [B, Hq, ceil(L / block_m), ceil(L / block_n)].  out may hold the estimate's
+ * scratch until the rows are written (only where it overlaps none of q, k, v). */
 int64_t psa_layer_workspace_bytes(int elem_bytes, int B, int Hq, int Hkv, int L, int D, int block_m, int block_n, int indexed, int walk);
 int psa_layer_fwd(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const int32_t* token_index, const int32_t* off_q,
                   const int32_t* off_k, const float* sim_thresholds, int32_t* cap_out, void* workspace, void* map_out,
@@ -350,7 +351,7 @@ int psa_fwd_noalloc(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const void* k_p
 int64_t psa_fwd_noalloc_max_rows(void);
 
 /* Bytes of workspace psa_bwd needs (fp32 dK/dV per pyramid level, delta, lse in log2 units, cost and issue order of
- * the dQ rows and of the dK/dV workgroups). */
+ * the dQ rows and of the dK/dV workgroups, and the parts that long lists of the latter are cut into). */
 int64_t psa_bwd_workspace_bytes(int B, int Hq, int Hkv, int L, int D, int block_n);
 
 /* Backward of psa_fwd w.r.t. q, k, v (the map carries no gradient).  bf16 or fp16 tensors; dq/dk/dv are views like

@@ -6,13 +6,16 @@
 //   dQ_i    += scale sum_t dS_it K_l[t]                                dK_l[t] += scale sum_i dS_it q_i
 //   dK[n]    = dK_1[n] + sum_{l=2,4,8} dK_l[n/l] / l, the part of replicate-pad rows n >= L added to row L-1
 //
-// Four kernels:
+// Kernels:
+//   psa_bwd_cost_kernel    row and column costs of the walks, whose issue orders psa_order.h sorts
 //   psa_bwd_delta_kernel   HBM-bound: -delta and -lse in log2 units (rows without keys get -inf so p = 0)
 //   psa_bwd_dq_lds_kernel  MFMA-bound row walk: the forward's tile schedule; per tile S^T = K Q^T,
 //                          dP^T = V dO^T, dQ^T += K^T dS^T on bf16 / fp16 MFMA, operands pooled K/V read directly
-//   psa_bwd_dkdv_lds_kernel MFMA-bound column walk: one workgroup per (kv head, kv-block, level slot) keeps its
-//                          <= 64 pooled keys in registers and streams the q-blocks that retain this block at
+//   psa_bwd_dkdv_lds_kernel MFMA-bound column walk: one workgroup per (kv head, kv-block, level slot) keeps
+//                          its pooled keys (128 at most) in registers and streams the q-blocks that retain this block at
 //                          this level; dK_l, dV_l go to an fp32 workspace (every row written exactly once)
+//   psa_bwd_parts_kernel   items of the 128-key slots: long lists cut into parts where the launch is short
+//   psa_bwd_join_kernel    adds the parts' sums in order, then as the un-pool pass
 //   psa_bwd_unpool_kernel  HBM-bound: sums the levels, spreads pooled gradients, folds the pad tail, -> the tensors' type
 #include "psa_tiles.h"
 #include "psa_order.h"
