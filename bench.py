@@ -491,7 +491,7 @@ def main():
     pool_bytes = 2.0 * B * H * (Nk * bn) * D * q.element_size() * (1 + 7 / 8)
     est_flops = 2.0 * (Mq * km) * (Nk * kn) * D * B * H
 
-    fwd_kernel = "psa_fwd_f32_kernel" if tdtype == torch.float32 else "psa_fwd_kernel" if D == 128 else "psa_fwd_lds_kernel"
+    fwd_kernel = ("psa_fwd_f32_direct_kernel" if D == 64 else "psa_fwd_f32_kernel") if tdtype == torch.float32 else "psa_fwd_kernel" if D == 128 else "psa_fwd_lds_kernel"
     roofline = {
         "kernel": fwd_kernel,
         "bound": "mfma",  # (fp32: the matrix cores' fp32 instructions and their peak)
