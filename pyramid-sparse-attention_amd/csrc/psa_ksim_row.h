@@ -38,7 +38,17 @@ __device__ __forceinline__ void group_cosines(const float (&v)[15], float& c2, f
   c4 = v[12] / (n[0] * n[3] + 1e-6f) + v[13] / (n[4] * n[7] + 1e-6f);
   c8 = v[14] / (n[0] * n[7] + 1e-6f);
 }
-// cap of a block of bn tokens from the cosines of its bn / 8 groups
+// a > b as IEEE 754 has it, false where either is no number, in every file that includes this: without NaN semantics (psa_estimate.hip)
+// the compiler may turn the comparison round and call a NaN above everything.  The bits go through an empty assembly statement, or
+// the test for a NaN would be dropped as one that never holds.
+__device__ __forceinline__ bool above(float a, float b) {
+  uint32_t x = __builtin_bit_cast(uint32_t, a), y = __builtin_bit_cast(uint32_t, b);
+  asm("" : "+v"(x), "+v"(y));
+  constexpr uint32_t INF = 0x7f800000u, ABS = 0x7fffffffu;
+  return (x & ABS) <= INF && (y & ABS) <= INF && __builtin_bit_cast(float, x) > __builtin_bit_cast(float, y);
+}
+// cap of a block of bn tokens from the cosines of its bn / 8 groups: 1 where a mean cosine is no number (a key that is not finite, or whose
+// squared norm is not)
 __device__ __forceinline__ int block_cap(const float* c2, const float* c4, const float* c8, int bn, float t2, float t4, float t8) {
   const int ng = bn >> 3;
   float s2 = 0.f, s4 = 0.f, s8 = 0.f;
@@ -51,9 +61,9 @@ __device__ __forceinline__ int block_cap(const float* c2, const float* c4, const
   s4 /= (float)(bn >> 2);
   s8 /= (float)(bn >> 3);
   int lv = 1;
-  if (s2 > t2) lv = 2;
-  if (s4 > t4) lv = 4;
-  if (s8 > t8) lv = 8;
+  if (above(s2, t2)) lv = 2;
+  if (above(s4, t4)) lv = 4;
+  if (above(s8, t8)) lv = 8;
   return lv;
 }
 

@@ -66,3 +66,28 @@ def test_scratch_in_the_output(B, Hq, Hkv, L, D, bm, bn, dtype, capped):
     kp, vp = ops.pool_kv(k, v, bn)
     assert torch.equal(mp, ref)
     assert torch.equal(out, ops.sparse_attention_fwd(q, k, v, ref, bm, bn, D ** -0.5, pools=(kp, vp)))
+
+
+@pytest.mark.parametrize("H,L,D,bn", [(4, 700, 64, 64), (3, 1029, 128, 128), (2, 333, 64, 32), (3, 700, 128, 64)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_cap_of_keys_that_are_not_finite(H, L, D, bn, dtype):
+    """A kv-block with a NaN or infinite key, or with keys whose squared norms are above the largest float, has no mean cosine and takes no
+    pooling (cap 1; the thresholds are below all cosines, so every other block has 8): in the contraction's launch as in psa_ksim."""
+    from psa_hip import ops
+
+    q, k, v = (rnd(1, H, L, D, seed=L + i).to(dtype).to(dev()) for i in range(3))
+    expected = torch.full((1, H, -(-L // bn)), 8, dtype=torch.int32)
+    for b, x in enumerate((float("nan"), float("inf"), float("-inf"), 3e19)):
+        if not torch.isfinite(torch.tensor(x)) or dtype == torch.bfloat16:
+            at = b * bn + 8 * b  # (the first or the last of 8 tokens, which pairs of every distance meet; all of them)
+            k[:, b % H, slice(at, at + 8) if x == 3e19 else at + 7 * (b & 1), b] = x
+            expected[:, b % H, b] = 1
+    k[:, H - 1, L - 1, D - 1] = float("nan")  # (and the pad rows behind it)
+    expected[:, H - 1, -1] = 1
+    thr = (-2.0, -2.0, -2.0)
+    off_q, off_k = ops.draw_sample_offsets(1, H, H, 128, 32, bn, bn // 4, dev(), seed=L)
+    _, mp, cap = ops._layer_one_call(q, k, v, off_q, off_k, RATIOS, "topk", 128, bn, bn, D ** -0.5, 0, None, thr)
+    assert torch.equal(ops.k_similarity(k, bn, *thr).cpu(), expected)
+    assert torch.equal(cap.cpu(), expected)
+    ref = ops.estimate_sampled_map(q, k, off_q, off_k, 128, bn, 32, bn // 4, RATIOS, 0, "topk", compute_tile=bn, map_dtype=torch.int8)
+    assert torch.equal(mp, ops.map_min_cap(ref, cap))
