@@ -139,8 +139,11 @@ class PSAAttention(nn.Module):
             cap = calc_k_similarity(k, config.block_n, config) if config.use_sim_mask else None
             return ops.psa_layer_fwd(q, k, v, off_q, off_k, config.mask_ratios, config.mask_mode, config.block_m,
                                      config.block_n, config.tile_n, level_cap=cap)
-        listed = getattr(self.sparse_attention_fn, "listed", None)
-        if listed is not None and not config.use_sim_mask and getattr(self.build_mask, "__func__", None) is PSAAttention.build_mask:
+        fn = self.sparse_attention_fn
+        listed = getattr(fn, "listed", None)
+        # (a wrapper made with functools.wraps carries its function's attributes, but is not the function)
+        own = listed is not None and listed.serves is fn and getattr(self.build_mask, "__func__", None) is _OWN_BUILD_MASK
+        if own and not config.use_sim_mask:
             # the module's own mask and attention: levels and the attention's tile list come out of the estimate's reduction
             offsets = self.sample_offsets
             if offsets is None:
@@ -152,6 +155,9 @@ class PSAAttention(nn.Module):
             return self.sparse_attention_fn(q, k, v, self._mask(q, k, v, offsets), None)
         mask = self.build_mask(q, k, v)
         return self.sparse_attention_fn(q, k, v, mask, None)
+
+
+_OWN_BUILD_MASK = PSAAttention.build_mask  # (held apart: a caller may replace the method in a subclass, an instance or the class itself)
 
 
 def psa_attention(q, k, v, *, config: PSAConfig = None, mask_ratios=None, mask_mode: str = None, block_m: int = None,

@@ -1,5 +1,7 @@
 """PSAAttention with gradients: the level map and its tile list from one launch of the estimate's reduction (ops.estimate_walk) against
 build_mask + the attention function, which the module takes where either is the caller's own: same outputs and gradients, bit for bit."""
+import functools
+
 import pytest
 import torch
 
@@ -52,6 +54,37 @@ def test_a_mask_of_the_callers_own_is_used():
     m = Dense(PSAConfig(block_m=128, block_n=128, attn_impl="old_mask_type"))
     out = m(q, k, v)
     assert torch.equal(out, ops.sparse_attention_fwd(q.detach(), k.detach(), v.detach(), m.build_mask(q, k, v), 128, 128, return_lse=True)[0])
+
+
+def test_a_mask_set_on_the_class_is_used(monkeypatch):
+    from psa_hip import PSAAttention, PSAConfig, ops
+
+    def dense(self, q, k, v):
+        n = -(-q.shape[2] // 128)
+        return torch.ones(q.shape[0], q.shape[1], n, n, dtype=torch.int32, device=q.device)
+
+    q, k, v = (rnd(1, 2, 700, 64, seed=i).to(dev()).requires_grad_(True) for i in range(3))
+    m = PSAAttention(PSAConfig(block_m=128, block_n=128, attn_impl="old_mask_type"))
+    monkeypatch.setattr(PSAAttention, "build_mask", dense)
+    out = m(q, k, v)
+    assert torch.equal(out, ops.sparse_attention_fwd(q.detach(), k.detach(), v.detach(), dense(m, q, k, v), 128, 128, return_lse=True)[0])
+
+
+def test_a_wrapped_attention_function_is_called():
+    from psa_hip import PSAAttention, PSAConfig
+
+    q, k, v = (rnd(1, 2, 300, 64, seed=i).to(dev()).requires_grad_(True) for i in range(3))
+    m = PSAAttention(PSAConfig(block_m=128, block_n=128, attn_impl="old_mask_type"))
+    plain, masks = m.sparse_attention_fn, []
+
+    @functools.wraps(plain)
+    def wrapper(q, k, v, mask, sm_scale):
+        masks.append(mask)
+        return plain(q, k, v, mask, sm_scale)
+
+    m.sparse_attention_fn = wrapper
+    m(q, k, v)
+    assert len(masks) == 1 and masks[0].shape == (1, 2, 3, 3)
 
 
 def test_errors_stay():
