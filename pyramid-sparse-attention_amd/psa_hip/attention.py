@@ -142,7 +142,7 @@ class PSAAttention(nn.Module):
         fn = self.sparse_attention_fn
         listed = getattr(fn, "listed", None)
         # (a wrapper made with functools.wraps carries its function's attributes, but is not the function)
-        own = listed is not None and listed.serves is fn and getattr(self.build_mask, "__func__", None) is _OWN_BUILD_MASK
+        own = listed is not None and listed.serves == (fn, config.block_m, config.block_n) and getattr(self.build_mask, "__func__", None) is _OWN_BUILD_MASK
         if own and not config.use_sim_mask:
             # the module's own mask and attention: levels and the attention's tile list come out of the estimate's reduction
             offsets = self.sample_offsets

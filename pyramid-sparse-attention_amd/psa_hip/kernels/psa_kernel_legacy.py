@@ -59,7 +59,7 @@ def sparse_attention_factory(BLOCK_M=128, BLOCK_N=32, POOLING_BLOCK_N=128, causa
 
     if not causal:  # the same on a map whose tiles are listed already (ops.estimate_walk)
         _fn.listed = lambda q, k, v, level_map, walk: _sparse_attention.apply(q, k, v, level_map, None, BLOCK_M, POOLING_BLOCK_N, False, walk)
-        _fn.listed.serves = _fn
+        _fn.listed.serves = (_fn, BLOCK_M, POOLING_BLOCK_N)
     return _fn
 
 

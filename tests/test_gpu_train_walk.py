@@ -87,6 +87,17 @@ def test_a_wrapped_attention_function_is_called():
     assert len(masks) == 1 and masks[0].shape == (1, 2, 3, 3)
 
 
+def test_a_function_of_other_blocks_than_the_map():
+    """60 tokens are one block of 64 or of 128: the map of a configuration changed later fits, and the function's own block sizes count."""
+    from psa_hip import PSAAttention, PSAConfig, ops
+
+    q, k, v = (rnd(1, 2, 60, 64, seed=i).to(dev()).requires_grad_(True) for i in range(3))
+    m = PSAAttention(PSAConfig(block_m=128, block_n=128, attn_impl="old_mask_type"))
+    m.config.block_m = m.config.block_n = 64
+    m.sample_offsets = ops.draw_sample_offsets(1, 2, 2, 64, 16, 64, 16, dev(), seed=1)
+    assert torch.equal(m(q, k, v), m.sparse_attention_fn(q, k, v, m.build_mask(q, k, v)))
+
+
 def test_errors_stay():
     from psa_hip import PSAAttention, PSAConfig
 
