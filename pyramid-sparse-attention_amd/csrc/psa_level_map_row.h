@@ -34,12 +34,18 @@ __device__ __forceinline__ uint32_t desc_key(float s) {
 // Stable descending order of one row of scores: sidx[i] = column of sorted position i, sw[i] its score.
 // The 64-bit keys (inverted score bits, column) are unique, so every correct sort gives the same order.
 // Rows of up to RANK_SORT_MAX scores are ranked by counting (one pass of N comparisons per score, no barriers inside).  Longer ones are
-// dealt to SORT_BINS bins, equal steps of the score bits between the row's best and worst (8 bins per octave if that is the whole
-// range of a float, more otherwise), and ranked by counting inside their bin: a few comparisons per score and seven barriers.
-// A bin of more than SORT_CAP scores (equal scores, mostly) sends the row to a bitonic network over key[0 .. sort_pad).
+// dealt to SORT_BINS bins, equal steps of the score bits between the row's best and worst (8 bins per octave for scores that reach from 1 down to
+// the smallest floats, more otherwise), and ranked by counting inside their bin: a few comparisons per score and six barriers.
+// A bin of more than SORT_TIES scores is mostly scores equal to the worst (the zeros above a causal diagonal, scores that underflow,
+// rows that are all alike): those are placed in column order, by ballots, and their bin is ranked without them.  If a bin of a row of more than 256
+// still has more than SORT_CAP (scores of a few values), the row goes through a bitonic network over key[0 .. sort_pad).
 // Against ranking up to 256 scores by counting and longer rows by the network, reduction + map of estimates by attention mass, us: 40 heads x
-// 10750 tokens of 32-key blocks (336 scores) 102 -> 66, 24 x 13273 (415) 73 -> 53, 12 x 32760 of 128-key blocks (256) 58 -> 46.
-constexpr int RANK_SORT_MAX = 128, SORT_BINS = 1024, SORT_CAP = 128;
+// 10750 tokens of 32-key blocks (336 scores) 102 -> 66, 24 x 13273 (415) 73 -> 53, 12 x 32760 of 128-key blocks (256) 58 -> 46.  Maps alone, us,
+// then / now, continuous scores and rows of which 84 % are 0: 8192 rows of 129 scores 42 / 39, 42 / 43; of 256 73 / 55, 73 / 61; of 512
+// 149 / 98, 148 / 109; 4096 of 1024 161 / 105, 159 / 115; 1024 of 4096 564 / 360, 562 / 350.  Causal maps of their own (28 heads of
+// 200 x 200, zeros above the diagonal) 39 / 33.  (Without the placing of ties: 67, 90, 156, 171, 592, and 50.)  Rows of nine values pay for the
+// bins in vain: 129 scores 42 / 53, 256 73 / 83, 4096 564 / 599.
+constexpr int RANK_SORT_MAX = 128, SORT_BINS = 1024, SORT_TIES = 32, SORT_CAP = 128;
 __host__ __device__ inline int sort_pad(int N) {
   if (N <= RANK_SORT_MAX) return N;
   int n = 1;
@@ -70,7 +76,7 @@ __device__ __forceinline__ void sort_row_desc(uint64_t* key, float* sw, int* sid
   constexpr int NT = 256, NW = NT / 64;
   static_assert(SORT_BINS == 4 * NT, "a thread scans four bins");
   __shared__ uint32_t s_lo[NW], s_hi[NW], s_sum[NW], s_most[NW];
-  const int lane = tid & 63, wave = tid >> 6;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   ((u32x4*)hist)[tid] = u32x4{0u, 0u, 0u, 0u};
   uint32_t* kbuf = (uint32_t*)sidx;  // (the score bits, until the columns take their place)
   uint32_t lo = 0xffffffffu, hi = 0u;
@@ -93,6 +99,9 @@ __device__ __forceinline__ void sort_row_desc(uint64_t* key, float* sw, int* sid
     hi = s_hi[w] > hi ? s_hi[w] : hi;
   }
   const int bits = 32 - __builtin_clz((hi - lo) | 1u), shift = bits > 10 ? bits - 10 : 0;
+  bool ties = false;                                       // many columns have the worst score: they are placed in column order
+  const int span = ((N + NT - 1) / NT) * 64, c0 = wave * span, c1 = c0 + span < N ? c0 + span : N;  // columns of this wave where there are
+  uint32_t at = 0;                                         // ... and where its tied ones go
   static_assert(SORT_BINS == 1 << 10, "bins");
   for (int j = tid; j < N; j += NT) atomicAdd(&hist[(kbuf[j] - lo) >> shift], 1u);
   __syncthreads();
@@ -119,47 +128,88 @@ __device__ __forceinline__ void sort_row_desc(uint64_t* key, float* sw, int* sid
     most = 0;
 #pragma unroll
     for (int w = 0; w < NW; ++w) most = s_most[w] > most ? s_most[w] : most;
-    if (most > (uint32_t)SORT_CAP) {  // (uniform)
-      const int Npad = sort_pad(N);
-      for (int j = tid; j < Npad; j += NT) key[j] = j < N ? (((uint64_t)kbuf[j] << 32) | (uint32_t)j) : ~0ull;
+    if (most > (uint32_t)SORT_TIES) {  // (uniform)
+      uint32_t n = 0;
+      for (int j0 = c0; j0 < c1; j0 += 64) n += (uint32_t)__popcll(__ballot(j0 + lane < c1 && kbuf[j0 + lane < c1 ? j0 + lane : 0] == hi));
+      if (lane == 0) s_lo[wave] = n;
       __syncthreads();
-      for (int k = 2; k <= Npad; k <<= 1) {
-        for (int j = k >> 1; j > 0; j >>= 1) {
-          for (int e = tid; e < (Npad >> 1); e += NT) {
-            // pair e of this stage: i has bit j clear, its partner is i + j; ascending where bit k of i is clear
-            const int i = ((e & ~(j - 1)) << 1) | (e & (j - 1));
-            const uint64_t a = key[i], b = key[i + j];
-            const bool up = (i & k) == 0;
-            if ((a > b) == up) {
-              key[i] = b;
-              key[i + j] = a;
+      const uint32_t tied = s_lo[0] + s_lo[1] + s_lo[2] + s_lo[3];
+      ties = tied > 1;
+      at = (uint32_t)N;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) at -= w >= wave ? s_lo[w] : 0u;
+      if (N > 256 && most > (uint32_t)SORT_CAP) {  // without the tied columns, which are at the end of the last bin
+        most = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          uint32_t in = (e < 3 ? c[e < 3 ? e + 1 : 3] : run) - c[e];
+          in -= (uint32_t)(4 * tid + e) == (hi - lo) >> shift ? tied : 0u;
+          most = in > most ? in : most;
+        }
+        most = wave_max_u32(most);
+        if (lane == 0) s_hi[wave] = most;
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < NW; ++w) most = s_hi[w] > most ? s_hi[w] : most;
+        if (most > (uint32_t)SORT_CAP) {
+          const int Npad = sort_pad(N);
+          for (int j = tid; j < Npad; j += NT) key[j] = j < N ? (((uint64_t)kbuf[j] << 32) | (uint32_t)j) : ~0ull;
+          __syncthreads();
+          for (int k = 2; k <= Npad; k <<= 1) {
+            for (int j = k >> 1; j > 0; j >>= 1) {
+              for (int e = tid; e < (Npad >> 1); e += NT) {
+                // pair e of this stage: i has bit j clear, its partner is i + j; ascending where bit k of i is clear
+                const int i = ((e & ~(j - 1)) << 1) | (e & (j - 1));
+                const uint64_t a = key[i], b = key[i + j];
+                const bool up = (i & k) == 0;
+                if ((a > b) == up) {
+                  key[i] = b;
+                  key[i + j] = a;
+                }
+              }
+              __syncthreads();
             }
           }
+          for (int i = tid; i < N; i += NT) {
+            const int col = (int)(uint32_t)key[i];
+            sidx[i] = col;
+            sw[i] = src[col];
+          }
           __syncthreads();
+          return;
         }
       }
-      for (int i = tid; i < N; i += NT) {
-        const int col = (int)(uint32_t)key[i];
-        sidx[i] = col;
-        sw[i] = src[col];
-      }
-      __syncthreads();
-      return;
     }
   }
   __syncthreads();
   // hist[b]: the next free place of bin b, in the end the first place of bin b + 1
-  for (int j = tid; j < N; j += NT) {
-    const uint32_t k = kbuf[j];
-    key[atomicAdd(&hist[(k - lo) >> shift], 1u)] = ((uint64_t)k << 32) | (uint32_t)j;
+  if (ties) {
+    for (int j0 = c0; j0 < c1; j0 += 64) {
+      const int j = j0 + lane;
+      const uint32_t k = kbuf[j < c1 ? j : 0];
+      const uint64_t tied = __ballot(j < c1 && k == hi);
+      if (j < c1) {
+        const uint32_t before = __builtin_amdgcn_mbcnt_hi((uint32_t)(tied >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)tied, 0u));
+        key[k == hi ? at + before : atomicAdd(&hist[(k - lo) >> shift], 1u)] = ((uint64_t)k << 32) | (uint32_t)j;
+      }
+      at += (uint32_t)__popcll(tied);
+    }
+  } else {
+    for (int j = tid; j < N; j += NT) {
+      const uint32_t k = kbuf[j];
+      key[atomicAdd(&hist[(k - lo) >> shift], 1u)] = ((uint64_t)k << 32) | (uint32_t)j;
+    }
   }
   __syncthreads();
   for (int i = tid; i < N; i += NT) {
     const uint64_t mine = key[i];
-    const uint32_t bin = ((uint32_t)(mine >> 32) - lo) >> shift;
-    const int first = bin > 0 ? (int)hist[bin - 1] : 0, last = (int)hist[bin];
-    int rank = first;
-    for (int e = first; e < last; ++e) rank += key[e] < mine ? 1 : 0;
+    const uint32_t k = (uint32_t)(mine >> 32), bin = (k - lo) >> shift;
+    int rank = i;
+    if (!ties || k != hi) {
+      const int first = bin > 0 ? (int)hist[bin - 1] : 0, last = (int)hist[bin];
+      rank = first;
+      for (int e = first; e < last; ++e) rank += key[e] < mine ? 1 : 0;
+    }
     const int col = (int)(uint32_t)mine;
     sidx[rank] = col;
     sw[rank] = src[col];
