@@ -491,7 +491,15 @@ def main():
     pool_bytes = 2.0 * B * H * (Nk * bn) * D * q.element_size() * (1 + 7 / 8)
     est_flops = 2.0 * (Mq * km) * (Nk * kn) * D * B * H
 
-    fwd_kernel = ("psa_fwd_f32_direct_kernel" if D == 64 else "psa_fwd_f32_kernel") if tdtype == torch.float32 else "psa_fwd_kernel" if D == 128 else "psa_fwd_lds_kernel"
+    if tdtype == torch.float32:  # (csrc/psa_f32.hip, launch_f32)
+        rows16 = B * H * Mq * (bm // 16)
+        if D == 64:
+            direct = L > 2048 or not (2048 <= rows16 <= 4096 and (rows16 - 1) % 2048 >= 1840)
+        else:
+            direct = rows16 < 1024 or (rows16 <= 1728 and 4096 <= L <= 20480)
+        fwd_kernel = "psa_fwd_f32_direct_kernel" if direct else "psa_fwd_f32_kernel"
+    else:
+        fwd_kernel = "psa_fwd_kernel" if D == 128 else "psa_fwd_lds_kernel"
     roofline = {
         "kernel": fwd_kernel,
         "bound": "mfma",  # (fp32: the matrix cores' fp32 instructions and their peak)

@@ -4,7 +4,8 @@
 // bias, online), same masks.
 //
 // A tile's four 16-key blocks go one to each wave of a workgroup (psa_fwd_f32_direct_kernel: 16 or 32 query rows; a softmax state per
-// wave, joined once at the end) or all to every wave, which then has 16 rows of its own (psa_fwd_f32_kernel: 64 rows).
+// wave, joined once at the end) or all, or two, to every wave, which then has 16 rows of its own or with one other (psa_fwd_f32_kernel: 64 or
+// 32 rows).  Which: launch_f32.
 // The transposed products S^T = K Q^T and O^T += V^T P^T leave a lane 4 keys of one query in the accumulator, and with
 // k-index g of the i-th PV step taken to be key 4 g + i that register IS the step's B operand: nothing crosses lanes
 // between the two products, and a row maximum is two lane exchanges.  Channels are dealt so that a lane's operands of four
@@ -97,12 +98,11 @@ __device__ __forceinline__ void f32_finish(const F32Params& p, int b, int h, int
   }
 }
 
-// Large launches at head dim 128, and rows that lie too far apart for 32-bit offsets: 64 rows per workgroup.  The K and V tile goes straight
-// into LDS and is shared by the waves; rows are XOR-swizzled by 16-byte chunks (one ds_read_b128 per four steps): conflict-free.
-template <int D>
+// 64 / KS rows per workgroup; KS waves share a row's keys.  The K and V tile goes straight into LDS and is shared by the waves; rows are XOR-swizzled by 16-byte chunks (one ds_read_b128 per four steps): conflict-free.
+template <int D, int KS>
 __global__ __launch_bounds__(256, 2) void psa_fwd_f32_kernel(F32Params p) {
   using G = F32Geom<D>;
-  constexpr int QR = 64, KBW = 4, SQ = D / 16, DB = D / 16;
+  constexpr int QR = 64 / KS, KBW = 4 / KS, SQ = D / 16, DB = D / 16;
   extern __shared__ __align__(16) unsigned char smem[];  // [STAGES][K, V] tiles, later the shares of the output
   u32x2* tdesc = (u32x2*)(smem + G::STAGES * 2 * G::TILE);
   uint16_t* ids = (uint16_t*)(tdesc + p.max_tiles);
@@ -116,7 +116,8 @@ __global__ __launch_bounds__(256, 2) void psa_fwd_f32_kernel(F32Params p) {
   const int I = logical % p.Mq, bh = logical / p.Mq, h = bh % p.Hq, b = bh / p.Hq;
   const int hk = h / (p.Hq / p.Hkv);
   const int q0 = I * p.bm + part * QR;  // first query position of this workgroup
-  const int q_idx = q0 + wave * 16 + l16;
+  const int rg = wave / KS, ks = wave % KS;  // this wave's 16 rows and its share of a tile's keys
+  const int q_idx = q0 + rg * 16 + l16;
   int jmax = p.Nk;
   if (p.causal) {
     const int ce = (int)((((int64_t)(I + 1) * p.bm) + (1 << p.bn_log2) - 1) >> p.bn_log2);
@@ -181,7 +182,7 @@ __global__ __launch_bounds__(256, 2) void psa_fwd_f32_kernel(F32Params p) {
   float m_run = -INFINITY, l_run = 0.f;  // the row's maximum over this wave's keys; this lane's part of its sum
 
   auto compute = [&](int t, int stage) __attribute__((always_inline)) {
-    PSA_LDS(unsigned char) Ts = (PSA_LDS(unsigned char))(smem) + stage * 2 * G::TILE;
+    PSA_LDS(unsigned char) Ts = (PSA_LDS(unsigned char))(smem) + stage * 2 * G::TILE + ks * (KBW * 16 * G::ROW);
     f32x4 s[KBW];
 #pragma unroll
     for (int x = 0; x < KBW; ++x) {
@@ -205,7 +206,7 @@ __global__ __launch_bounds__(256, 2) void psa_fwd_f32_kernel(F32Params p) {
       const int qlim = (q_idx + 1) >> tr.lv;
 #pragma unroll
       for (int x = 0; x < KBW; ++x) {
-        const int r0 = x * 16 + 4 * g4;
+        const int r0 = (ks * KBW + x) * 16 + 4 * g4;
         int keep = tr.nvalid - r0;
         if (p.causal) {
           const int pos = (tr.lt << 6) + r0;
@@ -274,16 +275,12 @@ __global__ __launch_bounds__(256, 2) void psa_fwd_f32_kernel(F32Params p) {
     }
   }
 
-  f32_finish<D, 1>(p, b, h, q0, wave, l16, g4, tid, acc, m_run, l_run, (float*)smem, s_m, s_l);
+  f32_finish<D, KS>(p, b, h, q0, wave, l16, g4, tid, acc, m_run, l_run, (float*)smem, s_m, s_l);
 }
 
 // 16 RG rows per workgroup, K and V rows straight into the registers of the wave that has their block: no LDS tiles and no barriers between
 // the row's list and the end.  The next block's rows are requested before a block's products (two blocks ahead: more registers, fewer waves, 4 to
 // 8 % slower).  Wave w has keys 16 w .. 16 w + 15 of every tile.  RG = 2 halves the row addresses per product and the number of workgroups.
-// Measured: layers of 80 % sparsity, us, with LDS tiles (16 to 64 rows), RG = 1 and RG = 2:
-//   head dim 64   2 heads x 4096  58 / 51 / 52   4 x 3291  84 / 69 / 71   8 x 2000 (1000 blocks of 16 rows)  64 / 59 / 60
-//                 8 x 3000 (1504)  110 / 89 / 84   8 x 6000 (3000)  228 / 193 / 186   24 x 8000 (12000)  837 / 816 / 784   16 x 16000  1732 / 1734 / 1669
-//   head dim 128  2 x 4096  90 / 77   8 x 6000 (3000)  423 / 395   8 x 8000 (4000)  558 / 570   16 x 4500 (4512)  526 / 533   24 x 4000 (6000)  577 / 613
 // (RG = 2 at head dim 128 would take more than the 256 registers of two waves per SIMD.)
 template <int D, int RG>
 __global__ __launch_bounds__(256, 2) void psa_fwd_f32_direct_kernel(F32Params p) {
@@ -507,13 +504,29 @@ int launch_f32(K kernel, size_t tiles, int64_t grid, const F32Params& p, hipStre
   hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(256), shmem, stream, p);
   return PSA_OK;
 }
+// Workgroups of 16 or 32 rows without LDS tiles, or of 32 or 64 rows with them.  The former list a row's tiles two to four times as often and
+// fetch K and V as often again; the latter wait at a barrier for every tile and, with 64 rows, leave small launches with too few workgroups.
+// Layers, us, tiles in LDS (16 rows below 1024 blocks of 16 rows, 32 below 2048, 64 from there on) / without (RG = 1 up to 1280 blocks, 2 above;
+// head dim 128: 1) / as chosen here, on keys with a common part, topk (head dim 64: 128-key blocks, and where marked 64):
+//   head dim 64   8 heads x 1000  32 / 29 / 28   12 x 2048  49 / 41 / 41   17 x 2000  63 / 54 / 55   24 x 1536  55 / 51 / 51   12 x 4000  106 / 98 / 99
+//                 8 x 8000  229 / 224 / 223   1 x 30000  449 / 390 / 388.   Short rows in one or two full rounds of 64-row workgroups: 16 x 2000  50 / 54 / 49
+//                 32 x 1000 (64)  46 / 47 / 43   200 x 300 (64)  59 / 66 / 59   512 x 128  59 / 65 / 59
+//   head dim 128  2 x 4096  63 / 56 / 56   8 x 1000  40 / 36 / 35   24 x 640 (960)  44 / 45 / 46   3 x 7000  195 / 183 / 183   1 x 20000  458 / 377 / 377   3 x 9000 (1704 blocks)  298 / 266 / 265
+//                 6 x 4600 (1728)  160 / 152 / 151.   Short rows: 12 x 2048 (1536)  75 / 80 / 71   24 x 1152 (1728)  84 / 92 / 84.   More rows: 16 x 2000 (2000)
+//                 78 / 99 / 76   12 x 4000 (3072)  194 / 220 / 191   8 x 6000 (3008)  270 / 297 / 264   96 x 500 (3072)  88 / 117 / 86.   K and V of a head beyond 20 MiB,
+//                 which rows of 16 fetch from memory: 1 x 24000  567 / 511 / 537   1 x 30000 (1880)  830 / 793 / 830 (forward on a random map of 80 % 726 / 890 / 726)
+// Rounding (relative to float64, random maps): 12 x 1400 x 128 4.3e-7 / 4.0e-7 / 4.3e-7, 32 x 1000 x 64 3.6e-7 / 2.8e-7 / 3.6e-7; without tiles a row's
+// keys are added up in four parts.
 template <int D>
 int launch_f32(F32Params p, hipStream_t stream) {
   const int64_t rows16 = (int64_t)p.B * p.Hq * p.Mq * (p.bm / 16);
   // (sizes in elements: a row's offset in bytes below 2^31, its factors below 2^24)
   auto near = [&](int64_t stride, int64_t rows) { return stride >= 0 && stride < (1 << 22) && rows < (1 << 24) && rows * (stride > D ? stride : D) < (1ll << 29); };
   const bool direct = near(p.k_sl, p.L) && near(p.v_sl, p.L) && near(D, p.npad);
-  if (direct && (D == 64 || rows16 <= 3072)) {
+  // workgroups of 64 rows in one or two full rounds of the chip's 512 places
+  const bool full_rounds = rows16 >= 2048 && rows16 <= 4096 && (rows16 - 1) % 2048 >= 1840;
+  const bool wins = D == 64 ? p.L > 2048 || !full_rounds : rows16 < 1024 || (rows16 <= 1728 && p.L >= 4096 && p.L <= 20480);
+  if (direct && wins) {
     const int rg = D == 64 && rows16 > 1280 ? 2 : 1;
     p.parts = p.bm / (16 * rg);
     const size_t stage = (size_t)64 * (D + 4) * 4;
@@ -521,8 +534,11 @@ int launch_f32(F32Params p, hipStream_t stream) {
       if (rg == 2) return launch_f32(psa_fwd_f32_direct_kernel<D, 2>, stage, rows16 / rg, p, stream);
     return launch_f32(psa_fwd_f32_direct_kernel<D, 1>, stage, rows16 / rg, p, stream);
   }
-  p.parts = p.bm / 64;
-  return launch_f32(psa_fwd_f32_kernel<D>, (size_t)F32Geom<D>::STAGES * 2 * F32Geom<D>::TILE, rows16 / 4, p, stream);
+  const size_t tiles = (size_t)F32Geom<D>::STAGES * 2 * F32Geom<D>::TILE;
+  const int ks = rows16 < 2048 ? 2 : 1;
+  p.parts = p.bm * ks / 64;
+  if (ks == 2) return launch_f32(psa_fwd_f32_kernel<D, 2>, tiles, rows16 / 2, p, stream);
+  return launch_f32(psa_fwd_f32_kernel<D, 1>, tiles, rows16 / 4, p, stream);
 }
 
 }  // namespace

@@ -46,3 +46,14 @@ def xattn_tile(heads, Lq, Lk, block, stride, chunk, causal):
     if (small + 256) * 3 < -(-large // 256) * 2560:
         return "small", 1
     return "large", -(-(-(-large // 8)) // 32)  # 8 XCDs, 32 workgroups each
+
+
+def fp32_kernel(D, B, Hq, L, bm, far=False):
+    """Kernel of the fp32 forward that a call runs (csrc/psa_f32.hip, launch_f32) and its rows per workgroup; far: rows of K or V beyond 32-bit
+    offsets."""
+    rows16 = B * Hq * -(-L // bm) * (bm // 16)
+    full_rounds = 2048 <= rows16 <= 4096 and (rows16 - 1) % 2048 >= 1840
+    wins = L > 2048 or not full_rounds if D == 64 else rows16 < 1024 or (rows16 <= 1728 and 4096 <= L <= 20480)
+    if wins and not far:
+        return "direct", 32 if D == 64 and rows16 > 1280 else 16
+    return "tiles", 32 if rows16 < 2048 else 64
