@@ -14,8 +14,6 @@
 //   psa_bwd_dkdv_lds_kernel MFMA-bound column walk: one workgroup per (kv head, kv-block, level slot) keeps
 //                          its pooled keys (128 at most) in registers and streams the q-blocks that retain this block at
 //                          this level; dK_l, dV_l go to an fp32 workspace (every row written exactly once)
-//   psa_bwd_parts_kernel   items of the 128-key slots: long lists cut into parts where the launch is short
-//   psa_bwd_join_kernel    adds the parts' sums in order, then as the un-pool pass
 //   psa_bwd_unpool_kernel  HBM-bound: sums the levels, spreads pooled gradients, folds the pad tail, -> the tensors' type
 #include "psa_tiles.h"
 #include "psa_order.h"
@@ -318,18 +316,19 @@ constexpr int DKDV_SLOTS = 4;
 // ------------------------------------------------------------------------------------------------------
 constexpr int COL_BINS = psa_order::COST_BINS;
 
-// Costs of every walk in one launch, their sorts in another: both are latency-bound (a sort is one workgroup per share, 8 to 16
-// per list) and two cost launches and three sorts one after the other left the chip nearly idle.  Measured now 9 + 12.5 us;
-// training step of 48 heads x 8776 x 64 1208 -> 1198 us, of 12 heads x 32760 x 128 4549 -> 4543 us.  The first row_wgs workgroups: four rows each, costs of the dQ walk.  The others, one per
-// (kv head, kv-block): per-level counts over the column -> cost of each of its slots.  The
-// costs of the slots slot_lo .. of all blocks form one list per dK/dV launch; with a 128-key slot 0 that slot's costs are a list of their
-// own (cost0), or its lengths go to count0 and psa_bwd_parts_kernel makes the list.
 // cost of a 128-key slot of n q-blocks: exact, or the octave of its length (classes, issued head by head)
 __device__ __forceinline__ int wide_cost(int n, bool octaves) {
   if (octaves) return 32 - __builtin_clz(n | 1);
   return n < COL_BINS - 1 ? n : COL_BINS - 1;
 }
-__global__ __launch_bounds__(256) void psa_bwd_cost_kernel(BwdParams p, int row_wgs, int32_t* cost_row, int wide0, bool octaves, int32_t* count0, int32_t* cost0, int32_t* cost) {
+
+// Costs of every walk in one launch, their sorts in another: both are latency-bound (a sort is one workgroup per share, 8 to 16
+// per list) and two cost launches and three sorts one after the other left the chip nearly idle.  Measured now 9 + 12.5 us;
+// training step of 48 heads x 8776 x 64 1208 -> 1198 us, of 12 heads x 32760 x 128 4549 -> 4543 us.  The first row_wgs workgroups: four rows each, costs of the dQ walk.  The others, one per
+// (kv head, kv-block): per-level counts over the column -> cost of each of its slots.  The
+// costs of the slots slot_lo .. of all blocks form one list per dK/dV launch; with a 128-key slot 0 that slot's costs are a list of their
+// own (cost0): one cost per slot, or (halve > 0) one per half, 0 for the second one of a slot of fewer than halve q-blocks.
+__global__ __launch_bounds__(256) void psa_bwd_cost_kernel(BwdParams p, int row_wgs, int32_t* cost_row, int wide0, bool octaves, int halve, int32_t* cost0, int32_t* cost) {
   __shared__ int s_n[4];
   if ((int)blockIdx.x < row_wgs) {
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -364,92 +363,40 @@ __global__ __launch_bounds__(256) void psa_bwd_cost_kernel(BwdParams p, int row_
     const int c = s_n[lv] < COL_BINS - 1 ? s_n[lv] : COL_BINS - 1;
     if (!wide0) cost[blk * DKDV_SLOTS + lv] = c;
     else if (lv == 0) {
-      if (count0 != nullptr) count0[blk] = s_n[0];
-      else cost0[blk] = wide_cost(s_n[0], octaves);
+      const int n = s_n[0];
+      if (halve > 0) {
+        const bool cut = n >= halve;
+        cost0[2 * blk] = wide_cost(cut ? (n + 1) / 2 : n, octaves);
+        cost0[2 * blk + 1] = cut ? wide_cost((n + 1) / 2, octaves) : 0;
+      } else {
+        cost0[blk] = wide_cost(n, octaves);
+      }
     }
     else cost[blk * (DKDV_SLOTS - 1) + (lv - 1)] = c;
   }
 }
 
 // ------------------------------------------------------------------------------------------------------
-// 128-key slots in parts.  A few key blocks are kept by nearly every q-block, others by one or two, and a launch that the chip holds in
-// one round or little more takes as long as its longest slot (16 heads of 3484 x 128 114 us beside a dQ walk of 55).  A list longer
-// than one and a half units is cut into parts of at most a unit, a workgroup each; the parts leave fp32 sums in the level-0 part of the
-// workspace, which 128-key slots do not use otherwise, and psa_bwd_join_kernel adds them in order.
-// The unit is PART_MEAN times the mean list of the slot's own head, PART_MIN q-blocks of 128 rows at least: the parts follow from the
-// head's map alone, and they fit its share of that buffer (cut slots have fewer than 1.5 * pairs / unit parts).
-// An item: {kv-block | part << 16 | parts << 24, its slot of the buffer}; a head's items are its slots' first parts (even entries) and
-// the other parts, spread over the odd entries.  Unused: parts = 0.
-// Which launches: training steps without / with parts, us, fixed quotas and thresholds, by the longest possible list (q-blocks of the kv head):
-//   head dim 128   16 q-blocks, 384 slots 205 / 179 and 230 / 231, 768 slots 268 / 281 and 319 / 352;   26, 650 slots 311 / 286 and 372 / 363, 780
-//                  336 / 341 and 416 / 430;   32, 512 slots 295 / 249 and 334 / 322;   48, 768 slots 456 / 427 and 522 / 494;   8, 384 slots 148 / 154 and 175 / 181
-//   head dim 64    16, 384 and more slots, and 26: 1 to 3 % slower (steps that the host bounds: two launches more);   32, 768 slots 243 / 241 and
-//                  279 / 273;   48, 768 slots 311 / 256 and 338 / 313, 1008 slots 331 / 294 and 392 / 389;   125, 1000 slots 629 / 629 and 627 / 605
-// Short lists have little to cut for the two launches and the traffic of the sums; in large launches slots that walk the same q-blocks at the
-// same time share their rows in L2, parts do not (12 heads of 9000 x 128, 852 slots, 604 / 631 and 699 / 739).
-constexpr int PART_MEAN_10 = 17, PART_MIN = 4, PART_MOST = 64;
-bool slots_in_parts(int D, int64_t slots, int64_t list) {  // (the chip holds 512 / 768 workgroups of the walk at once)
+// 128-key slots in halves.  A few key blocks are kept by nearly every q-block, others by one or two, and a launch that the chip holds in
+// one round or little more takes as long as its longest slot (16 heads of 3484 x 128 114 us beside a dQ walk of 55).  There a slot that a
+// quarter of the q-blocks and more keep goes to two workgroups of 64 keys each, 16 per wave, which walk the whole list: a key's products are
+// added in the same order wherever it is worked on, so a head's gradients have the same bits in any launch.
+// Which launches: the whole backward with whole / halved slots, us, fixed quotas and thresholds, by the longest possible list (q-blocks of the kv head):
+//   head dim 128   16 q-blocks, 384 slots 148 / 133 and 155 / 141, 640 slots 169 / 156 and 195 / 214;   26, 650 slots 213 / 194 and 242 / 250;
+//                  32, 512 slots 218 / 192 and 230 / 211, 768 slots 243 / 222 and 292 / 293, 1024 slots 284 / 277 and 357 / 386;   48, 384 slots
+//                  273 / 238 and 274 / 246, 768 slots 318 / 290 and 360 / 342, 960 slots 354 / 327 and 416 / 442;   71, 852 slots 449 / 408 and
+//                  478 / 518;   8, 384 slots 82 / 102 and 110 / 108
+//   head dim 64    16, 384 slots 103 / 97 and 107 / 103 (steps that the host bounds);   32, 768 slots 172 / 157 and 185 / 177;   48, 768 slots 232 / 210
+//                  and 234 / 222, 1008 slots 227 / 210 and 261 / 262, 1200 slots 257 / 240 and 301 / 310;   125, 1000 slots 428 / 402 and 423 / 416
+// In larger launches the lists of threshold maps, of which many are that long, lose more by half-filled workgroups than the tail gives.  Cut from a half
+// or an eighth of the q-blocks on: 8 x 9000 x 128 350 and 326 us for 320; elsewhere within 2 %.
+// (Lists cut along the q-blocks with fp32 sums in memory end sooner, 48 q-blocks of 384 slots 186 and 240, but the sums' order is then the launch's
+// business, or, in the order of the parts everywhere, 1 to 12 % of large launches with fixed quotas: 48 x 2583 x 128 240 -> 270.)
+// ------------------------------------------------------------------------------------------------------
+int halved_slots(int D, int64_t slots, int64_t list) {  // shortest list of a halved slot; 0: none.  (The chip holds 512 / 768 workgroups of the walk at once)
   const int64_t most = D == 128 ? 768 : 1024;
-  return list >= (D == 128 ? 16 : 32) && slots <= (24 * list < most ? 24 * list : most);
-}
-__device__ __forceinline__ int part_at(int n, int part, int parts) { return (int)((int64_t)n * part / parts); }
-
-__global__ __launch_bounds__(256) void psa_bwd_parts_kernel(const int32_t* count0, int Nk, int min_unit, bool octaves, u32x2* items, int32_t* cost) {
-  __shared__ int s_sum[4], s_more[4];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int64_t head = blockIdx.x;
-  const int32_t* n_of = count0 + head * Nk;
-  items += head * 2 * Nk;
-  cost += head * 2 * Nk;
-  auto total = [&](int v, int* sums) __attribute__((always_inline)) {  // over the workgroup
-    v = wave_scan_add(v);
-    if (lane == 63) sums[wave] = v;
-    __syncthreads();
-    return sums[0] + sums[1] + sums[2] + sums[3];
-  };
-  int pairs = 0;
-  for (int j = tid; j < Nk; j += 256) {
-    pairs += n_of[j];
-    items[2 * j + 1] = u32x2{0u, 0u};
-    cost[2 * j + 1] = 0;
-  }
-  pairs = total(pairs, s_sum);
-  const int mean = (int)(((int64_t)PART_MEAN_10 * pairs + 10 * Nk - 1) / (10 * Nk));
-  const int unit = mean > min_unit ? mean : min_unit;
-  auto parts_of = [&](int n) __attribute__((always_inline)) {
-    if (n <= unit + unit / 2) return 1;
-    const int q = (n + unit - 1) / unit;
-    return q < PART_MOST ? q : PART_MOST;
-  };
-  int more = 0;
-  for (int j = tid; j < Nk; j += 256) more += parts_of(n_of[j]) - 1;
-  more = total(more, s_more);
-  int at = 0, slot_at = 0;  // further parts and buffer slots of the columns before this round
-  for (int j0 = 0; j0 < Nk; j0 += 256) {
-    const int j = j0 + tid, n = j < Nk ? n_of[j] : 0, parts = parts_of(n);
-    const int e = parts - 1, sl = parts > 1 ? parts : 0;
-    const int e_to = wave_scan_add(e), sl_to = wave_scan_add(sl);
-    __syncthreads();
-    if (lane == 63) {
-      s_sum[wave] = e_to;
-      s_more[wave] = sl_to;
-    }
-    __syncthreads();
-    int first = at + e_to - e, slot = slot_at + sl_to - sl;
-    for (int w = 0; w < wave; ++w) {
-      first += s_sum[w];
-      slot += s_more[w];
-    }
-    if (j < Nk)
-      for (int part = 0; part < parts; ++part) {
-        const int len = part_at(n, part + 1, parts) - part_at(n, part, parts);
-        const int pos = part == 0 ? 2 * j : 2 * (int)((int64_t)(first + part - 1) * Nk / more) + 1;
-        items[pos] = u32x2{(uint32_t)j | ((uint32_t)part << 16) | ((uint32_t)parts << 24), (uint32_t)(head * Nk + slot + part)};
-        cost[pos] = wide_cost(len, octaves);
-      }
-    at += s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3];
-    slot_at += s_more[0] + s_more[1] + s_more[2] + s_more[3];
-  }
+  if (list < (D == 128 ? 16 : 32) || slots > (24 * list < most ? 24 * list : most)) return 0;
+  return (int)(list / 4);
 }
 
 // ------------------------------------------------------------------------------------------------------
@@ -466,9 +413,9 @@ __global__ __launch_bounds__(256) void psa_bwd_parts_kernel(const int32_t* count
 // The four waves of a workgroup split its keys and the 64 query rows of a step: 128 keys (level 0 of a 128-key
 // block) = 4 key quarters, every wave takes both query halves one after the other ("wide": each Q / dO tile that is
 // fetched feeds twice the arithmetic); <= 64 keys = 2 key halves x 2 query halves, combined through LDS at the end.  A wave works on 32 keys,
-// two blocks of 16, in slots of more than 32 keys and on one block in smaller ones: all four waves of a 32-key slot have work, and those of
-// a 16-key slot compute nothing for keys that are not there.  The walk is there twice in the kernel for that, one branch at its
-// start (a branch around each step spills).  With 32 keys per wave throughout / now, the launch of the pooled levels, us: 48 heads of 17043 x
+// two blocks of 16, in slots of more than 32 keys and on one block in smaller ones and in halves of 128: all four waves of a 32-key slot have work,
+// and those of a 16-key slot compute nothing for keys that are not there.  The walk is there twice in the kernel for that, one branch at its
+// start: 14 to 48 scalars are spilled before the walk and come back behind it, few of them in a step (a branch around each step spills there).  With 32 keys per wave throughout / now, the launch of the pooled levels, us: 48 heads of 17043 x
 // 128, fixed quotas, 1677 / 1488, 24 of 21613 x 64 693 / 606, 48 of 8776 x 64 282 / 250, 12 of 32760 x 128, thresholds, 660 / 621.
 // ------------------------------------------------------------------------------------------------------
 constexpr int B_ISTR = LT_ISTR;  // bytes between the blocks of a tile
@@ -476,7 +423,7 @@ constexpr int B_ISTR = LT_ISTR;  // bytes between the blocks of a tile
 // Gradients of the replicate-pad rows L .. npad - 1, which land on the last real token: over the pooled rows behind it, each counted
 // with its share of pad tokens.  By the 256 threads of the workgroup that owns that token (barriers inside), dK to fold[0 .. D) and dV to
 // fold[D .. 2 D); part: 2048 floats of LDS.  One lane that walks the pad tokens of its channels, three loads each, holds up the whole
-// launch: 16 heads of 3484 x 128 (100 pad tokens) 223 us for a walk of 50.
+// launch: 16 heads of 3484 x 128 (100 pad tokens) 223 us, 114 without that.
 template <int D>
 __device__ __forceinline__ void fold_pad_rows(const BwdParams& p, int bhk, int tid, float* part, float* fold) {
   constexpr int CH = D / 4, NG = 256 / CH;
@@ -515,11 +462,12 @@ __device__ __forceinline__ void fold_pad_rows(const BwdParams& p, int bhk, int t
 }
 
 // One instantiation per kind of slot (WIDE: the 128-key level-0 slot; else the slots slot_lo .. slot_lo + slot_cnt - 1 of
-// every kv-block); workgroup id = ((b * Hkv + kv head) * Nk + kv-block) * slot_cnt + (slot - slot_lo), or the entry of items (WIDE),
-// optionally re-ordered.
-template <int D, bool WIDE, bool CAUSAL, class ET>
+// every kv-block); workgroup id = ((b * Hkv + kv head) * Nk + kv-block) * slot_cnt + (slot - slot_lo), or (WIDE, halves: the halves' costs)
+// ((b * Hkv + kv head) * Nk + kv-block) * 2 + half, optionally re-ordered.
+// HALVES: launches with halved slots; the others keep a kernel with the one walk.
+template <int D, bool WIDE, bool CAUSAL, class ET, bool HALVES = false>
 __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, int slot_lo, int slot_cnt, int n_wg, int chunk,
-                                                                 const int32_t* order, const u32x2* items) {
+                                                                 const int32_t* order, const int32_t* halves) {
   using G = LtGeom<D>;
   using x8 = typename ET::x8;
   constexpr int KK = D / 32, DB = D / 16, RPL = G::RPL;
@@ -536,17 +484,15 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
   if (order != nullptr) wg = order[wg];
   if (wg < 0 || wg >= n_wg) return;
   const int slot = slot_lo + wg % slot_cnt;
-  int J = (wg / slot_cnt) % p.Nk, bhk = wg / (slot_cnt * p.Nk), part = 0, parts = 1, part_slot = 0;
-  if constexpr (WIDE)
-    if (items != nullptr) {
-      const uint32_t it = __builtin_amdgcn_readfirstlane(items[wg][0]);
-      part_slot = __builtin_amdgcn_readfirstlane(items[wg][1]);
-      J = (int)(it & 0xffffu);
-      bhk = wg / (2 * p.Nk);
-      part = (int)((it >> 16) & 255u);
-      parts = (int)(it >> 24);
-      if (parts == 0) return;
-    }
+  int blk = wg / slot_cnt, half = 0;
+  bool halved = false;
+  if constexpr (HALVES) {
+    blk = wg >> 1;
+    half = wg & 1;
+    halved = __builtin_amdgcn_readfirstlane(halves[wg | 1]) > 0;
+    if (half > 0 && !halved) return;
+  }
+  const int J = blk % p.Nk, bhk = blk / p.Nk;
   const int b = bhk / p.Hkv, hk = bhk % p.Hkv;
   const int n_rep = p.Hq / p.Hkv;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -568,8 +514,8 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
   // 128 keys: waves = 4 key quarters.
   const int flip = nkeys <= 16 ? (int)((blockIdx.x >> 3) & 1) : 0;
   const int kh = wide ? wave : ((wave & 1) ^ flip), qh = wide ? 0 : wave >> 1;
-  const bool narrow = !wide && nkeys <= 32;       // 16 keys per wave
-  const int wave_key0 = narrow ? kh * 16 : kh * 32;
+  const bool narrow = wide ? halved : nkeys <= 32;  // 16 keys per wave
+  const int wave_key0 = (narrow ? kh * 16 : kh * 32) + half * 64;
   const bool wave_active = key_valid > wave_key0;
 
   // ---- list of (head in group, q-block) that retain block J at this level -------------------------
@@ -626,11 +572,7 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
   // last token that the pooled key covers (< npad); block kb: + 16 << lv
   const int key_up = (int)(((key_row0 + key_local + 1) << lv) - 1);
   __syncthreads();
-  int nq = s_nq, from = 0;  // (of a slot's list, WIDE: the part of this workgroup)
-  if constexpr (WIDE) {
-    from = part_at(nq, part, parts);
-    nq = part_at(nq, part + 1, parts) - from;
-  }
+  const int nq = s_nq;
 
   // ---- lane-invariant LDS addressing (tile layout: see the forward kernel) ---------------------------
   // copy: wave w fills the 16-row group w of both tiles; lane (fq = lane / CH, pos = lane % CH) of block n writes
@@ -658,7 +600,7 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
 
   // step i -> (head, q-block, first query row)
   auto step_of = [&](int i, int& h, int& I, int& q0) __attribute__((always_inline)) {
-    const uint32_t ent = qlist[from + (i >> spb_log2)];
+    const uint32_t ent = qlist[i >> spb_log2];
     h = hk * n_rep + (int)(ent >> 16);
     I = (int)(ent & 0xffff);
     q0 = I * bm + (i & ((1 << spb_log2) - 1)) * 64;
@@ -822,26 +764,16 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
   // also those of the replicate-pad tokens behind it) are added here and dK, dV leave in the tensors' 16-bit type: no fp32 level-0
   // buffer, no separate pass.
   if constexpr (WIDE) {
-    if (parts > 1) {  // fp32 sums of this part, in the accumulators' layout (psa_bwd_join_kernel)
-      const int64_t at = (int64_t)part_slot * (128 * D) + (int64_t)kh * (2 * DB * 256) + ln * 4;
-#pragma unroll
-      for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-        for (int db = 0; db < DB; ++db) {
-          *(f32x4*)(p.wk + at + (kb * DB + db) * 256) = dk[kb][db];
-          *(f32x4*)(p.wv + at + (kb * DB + db) * 256) = dv[kb][db];
-        }
-      return;
-    }
     float* const fold = (float*)smem;
-    const bool folds = key_row0 + 128 >= L && p.npad > L;  // (this workgroup owns the last token, and there are pad rows)
+    const int64_t key_end = key_row0 + (half > 0 || !halved ? 128 : 64);
+    const bool folds = key_end >= L && p.npad > L;  // (this workgroup owns the last token, and there are pad rows)
     if (folds) {
       __syncthreads();
       fold_pad_rows<D>(p, bhk, wave * 64 + ln, fold + 2 * D, fold);
     }
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
-      const int64_t n = key_row0 + kh * 32 + (ln & 15) + 16 * kb;
+      const int64_t n = key_row0 + wave_key0 + (ln & 15) + 16 * kb;
       if (n >= L) continue;
       const int64_t BH = (int64_t)p.B * p.Hkv, npad = p.npad;
       const float* lk[3];
@@ -938,86 +870,10 @@ __global__ __launch_bounds__(256, 2) void psa_bwd_dkdv_lds_kernel(BwdParams p, i
     }
   }
   };
-  if constexpr (!WIDE) {
+  if constexpr (!WIDE || HALVES) {
     if (narrow) return walk(IC<1>{});
   }
   walk(IC<2>{});
-}
-
-// The 128-key slots that were cut: their parts added in order, then what ends such a slot (above), four channels of one token per
-// thread: a wave has 16 tokens and 16 channels.  (The workgroups of the other slots have nothing to do.)
-template <int D, class ET>
-__global__ __launch_bounds__(256) void psa_bwd_join_kernel(BwdParams p, const u32x2* items) {
-  constexpr int PER = D / 8;  // workgroups per slot
-  const int J = (int)blockIdx.x / PER, bhk = (int)blockIdx.y;
-  const u32x2 it = items[((int64_t)bhk * p.Nk + J) * 2];
-  const int parts = (int)(it[0] >> 24);
-  if (parts < 2) return;
-  const int unit = ((int)blockIdx.x % PER) * 256 + (int)threadIdx.x, lane = unit & 63, blk = unit >> 6;  // blk: (key block of 16, channel block of 16)
-  const int64_t n = (int64_t)J * 128 + (blk / (D / 16)) * 16 + (lane & 15), L = p.L;
-  const int col = (blk % (D / 16)) * 16 + (lane >> 4) * 4;
-  const int64_t at = (int64_t)it[1] * (128 * D) + unit * 4;
-  f32x4 gk = *(const f32x4*)(p.wk + at), gv = *(const f32x4*)(p.wv + at);
-  for (int part = 1; part < parts; ++part) {
-    const f32x4 x = *(const f32x4*)(p.wk + at + (int64_t)part * (128 * D)), y = *(const f32x4*)(p.wv + at + (int64_t)part * (128 * D));
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      gk[e] += x[e];
-      gv[e] += y[e];
-    }
-  }
-  const int64_t BH = (int64_t)p.B * p.Hkv;
-  f32x4 ak = {0.f, 0.f, 0.f, 0.f}, av = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int l = 1; l < 4; ++l) {
-    const int64_t row = BH * p.npad + pool_row_offset(l, BH, bhk, p.npad) + (n >> l);
-    const f32x4 x = *(const f32x4*)(p.wk + row * D + col), y = *(const f32x4*)(p.wv + row * D + col);
-    const float inv = 1.0f / (float)(1 << l);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      ak[e] += x[e] * inv;
-      av[e] += y[e] * inv;
-    }
-  }
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    gk[e] = gk[e] * p.scale + ak[e];
-    gv[e] += av[e];
-  }
-  const int64_t first = n - (lane & 15);
-  if (first < L && first + 16 >= L && p.npad > L) {  // (uniform) the wave of the last token: the pad rows' gradients, 16 lanes per chunk
-    f32x4 k = {0.f, 0.f, 0.f, 0.f}, v = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int l = 1; l < 4; ++l) {
-      const int64_t rows = BH * p.npad + pool_row_offset(l, BH, bhk, p.npad);
-      const int t0 = p.L >> l, t1 = (int)(p.npad >> l);
-      for (int t = t0 + (lane & 15); t < t1; t += 16) {
-        const f32x4 x = *(const f32x4*)(p.wk + (rows + t) * D + col), y = *(const f32x4*)(p.wv + (rows + t) * D + col);
-        const float share = t == t0 ? (float)(((t0 + 1) << l) - p.L) / (float)(1 << l) : 1.f;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          k[e] = __builtin_fmaf(x[e], share, k[e]);
-          v[e] = __builtin_fmaf(y[e], share, v[e]);
-        }
-      }
-    }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      auto sum16 = [](float a) __attribute__((always_inline)) {
-        a += dpp_f32<DPP_ROW_ROR + 8>(a);
-        a += dpp_f32<DPP_ROW_ROR + 4>(a);
-        a += dpp_f32<DPP_ROW_ROR + 2>(a);
-        return a + dpp_f32<DPP_ROW_ROR + 1>(a);
-      };
-      const float sk = sum16(k[e]), sv = sum16(v[e]);
-      gk[e] += n == L - 1 ? sk : 0.f;
-      gv[e] += n == L - 1 ? sv : 0.f;
-    }
-  }
-  if (n >= L) return;
-  const int b = bhk / p.Hkv, hk = bhk % p.Hkv;
-  *(u32x2*)(p.dk + b * p.dk_sb + hk * p.dk_sh + n * p.dk_sl + col) = u32x2{ET::pack2(gk[0], gk[1]), ET::pack2(gk[2], gk[3])};
-  *(u32x2*)(p.dv + b * p.dv_sb + hk * p.dv_sh + n * p.dv_sl + col) = u32x2{ET::pack2(gv[0], gv[1]), ET::pack2(gv[2], gv[3])};
 }
 
 // ------------------------------------------------------------------------------------------------------
@@ -1082,11 +938,10 @@ extern "C" int64_t psa_bwd_workspace_bytes(int B, int Hq, int Hkv, int L, int D,
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || L <= 0 || D <= 0 || block_n <= 0) return 0;
   const int64_t npad = (int64_t)((L + block_n - 1) / block_n) * block_n;
   const int64_t levels = (int64_t)B * Hkv * D * (npad + npad / 2 + npad / 4 + npad / 8);
-  // + cost and issue order of the dQ rows (block_m >= 64) and of the dK/dV slots (4 per kv-block, or lengths, 2 items and 3 slots), padded to
-  // whole shares, and the items
+  // + cost and issue order of the dQ rows (block_m >= 64) and of the dK/dV slots (4 per kv-block, or 3 and two halves), padded to whole shares
   const int64_t pad = 16 * psa_order::MAX_PHASES;
   const int64_t n_rows = (int64_t)B * Hq * ((L + 63) / 64), n_blocks = (int64_t)B * Hkv * ((L + block_n - 1) / block_n);
-  return (2 * levels + 2 * (int64_t)B * Hq * L + 2 * (n_rows + pad) + (6 + 5 + 4) * n_blocks + 4 * pad) * (int64_t)sizeof(float);
+  return (2 * levels + 2 * (int64_t)B * Hq * L + 2 * (n_rows + pad) + 2 * (5 * n_blocks + 2 * pad)) * (int64_t)sizeof(float);
 }
 
 extern "C" int psa_bwd(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const void* k_pool, const void* v_pool, const void* map,
@@ -1163,8 +1018,8 @@ extern "C" int psa_bwd(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const void* 
   const int64_t total = (int64_t)B * Hq * Mq, n_blocks = (int64_t)B * Hkv * Nk;
   const bool wide0 = block_n > 64;
   const bool cols_ordered = map != nullptr && n_blocks > 8;
-  const bool in_parts = cols_ordered && wide0 && slots_in_parts(D, n_blocks, (int64_t)(Hq / Hkv) * Mq);
-  const int64_t n_wide = wide0 ? (in_parts ? 2 * n_blocks : n_blocks) : 0, n_rest = n_blocks * (wide0 ? DKDV_SLOTS - 1 : DKDV_SLOTS);
+  const int halve = cols_ordered && wide0 ? halved_slots(D, n_blocks, (int64_t)(Hq / Hkv) * Mq) : 0;
+  const int64_t n_wide = wide0 ? (halve > 0 ? 2 * n_blocks : n_blocks) : 0, n_rest = n_blocks * (wide0 ? DKDV_SLOTS - 1 : DKDV_SLOTS);
   PSA_REQUIRE(total < (1ll << 28) && 4 * n_blocks < (1ll << 28), PSA_ERR_UNSUPPORTED, "psa_bwd: too many workgroups");
   // shares by the K/V rows (dQ) and the Q/dO rows (dK/dV) that the walks stream
   const double kv_bytes = 2.0 * B * Hkv * (double)p.npad * D * 2.0 * (map != nullptr ? 1.875 : 1.0);
@@ -1174,17 +1029,15 @@ extern "C" int psa_bwd(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const void* 
   if (wide0) psa_order::deal(n_wide, qdo_bytes, B * Hkv, chunk_w, groups_w);
   psa_order::deal(n_rest, qdo_bytes, B * Hkv, chunk_r, groups_r);
   const int32_t *order = nullptr, *order_wide = nullptr, *order_rest = nullptr;
-  const u32x2* items_wide = nullptr;
+  const int32_t* halves = nullptr;
   const bool rows_ordered = map != nullptr && total > 8 * 32;
   if (rows_ordered || cols_ordered) {
     int32_t* cost = (int32_t*)(p.nlse2 + (int64_t)B * Hq * L);
     int32_t* ord = cost + total;
-    int32_t* count0 = cost + 2 * total + 16 * psa_order::MAX_PHASES;
-    int32_t* cost_r = count0 + n_blocks;
+    int32_t* cost_r = cost + 2 * total + 16 * psa_order::MAX_PHASES;
     int32_t* cost_w = cost_r + n_rest;
     int32_t* ord_w = cost_w + n_wide;
     int32_t* ord_r = ord_w + (wide0 ? (int64_t)chunk_w * groups_w : 0);
-    u32x2* items = (u32x2*)(((uintptr_t)(ord_r + (int64_t)chunk_r * groups_r) + 7) & ~(uintptr_t)7);
     const int row_wgs = rows_ordered ? (int)((total + 3) / 4) : 0;
     // Where the Q / dO rows of a head group are about the size of an XCD's L2 (4 MiB), the 128-key slots of a share are issued in
     // classes, an octave of their list's length each, head by head inside a class (the sort is stable): an XCD then works on one
@@ -1200,13 +1053,9 @@ extern "C" int psa_bwd(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const void* 
     // (shares of about one round, which also keep an XCD on one head, lose 3-5 % at 24 x 12001 x 64 and 32 x 6000 x 128)
     const bool by_head = wide0 && qdo_bytes / (B * Hkv) <= 5.5 * 1024 * 1024 && n_blocks > 768 && Hq / Hkv * Mq >= 32;
     hipLaunchKernelGGL(psa_bwd_cost_kernel, dim3((unsigned)(row_wgs + (cols_ordered ? n_blocks : 0))), dim3(256), 0, st, p, row_wgs, cost,
-                       wide0 ? 1 : 0, by_head, in_parts ? count0 : nullptr, cost_w, cost_r);
+                       wide0 ? 1 : 0, by_head, halve, cost_w, cost_r);
     if (int e = psa_check_launch("psa_bwd (cost)")) return e;
-    if (in_parts) {
-      hipLaunchKernelGGL(psa_bwd_parts_kernel, dim3((unsigned)(B * Hkv)), dim3(256), 0, st, count0, Nk, PART_MIN * 128 / block_m, by_head, items, cost_w);
-      if (int e = psa_check_launch("psa_bwd (parts)")) return e;
-      items_wide = items;
-    }
+    if (halve > 0) halves = cost_w;
     psa_order::sort_lists<3>({{{cost, ord, (int)total, chunk, rows_ordered ? groups : 0},
                                {cost_w, ord_w, (int)n_wide, chunk_w, cols_ordered && wide0 ? groups_w : 0},
                                {cost_r, ord_r, (int)n_rest, chunk_r, cols_ordered ? groups_r : 0}}}, st);
@@ -1245,7 +1094,7 @@ extern "C" int psa_bwd(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const void* 
     PSA_REQUIRE(shmem <= 160 * 1024, PSA_ERR_UNSUPPORTED, "psa_bwd: too many q-blocks for the on-chip lists (LDS)");
     auto launch = [&](auto kern, int64_t n_wg, int chunk, int groups, int slot_lo, int slot_cnt, const int32_t* order) -> int {
       if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem) != hipSuccess) return PSA_ERR_LAUNCH;
-      hipLaunchKernelGGL(kern, dim3((unsigned)(chunk * groups)), dim3(256), shmem, st, p, slot_lo, slot_cnt, (int)n_wg, chunk, order, slot_lo == 0 && slot_cnt == 1 ? items_wide : nullptr);
+      hipLaunchKernelGGL(kern, dim3((unsigned)(chunk * groups)), dim3(256), shmem, st, p, slot_lo, slot_cnt, (int)n_wg, chunk, order, halves);
       return PSA_OK;
     };
     // the pooled levels first: the 128-key level-0 launch adds their rows to its own and writes dK, dV
@@ -1260,20 +1109,17 @@ extern "C" int psa_bwd(psa_tensor4 q, psa_tensor4 k, psa_tensor4 v, const void* 
     PSA_REQUIRE(rl == PSA_OK, rl, "psa_bwd: cannot reserve %zu bytes of LDS", shmem);
     if (int e = psa_check_launch("psa_bwd (dK/dV)")) return e;
     if (wide0) {
-      if (causal)
-        rl = D == 128 ? launch(psa_bwd_dkdv_lds_kernel<128, true, true, ET>, n_wide, chunk_w, groups_w, 0, 1, order_wide)
-                      : launch(psa_bwd_dkdv_lds_kernel<64, true, true, ET>, n_wide, chunk_w, groups_w, 0, 1, order_wide);
-      else
-        rl = D == 128 ? launch(psa_bwd_dkdv_lds_kernel<128, true, false, ET>, n_wide, chunk_w, groups_w, 0, 1, order_wide)
-                      : launch(psa_bwd_dkdv_lds_kernel<64, true, false, ET>, n_wide, chunk_w, groups_w, 0, 1, order_wide);
+      auto launch_wide = [&](auto halves_c) {
+        constexpr bool H = decltype(halves_c)::value;
+        if (causal)
+          return D == 128 ? launch(psa_bwd_dkdv_lds_kernel<128, true, true, ET, H>, n_wide, chunk_w, groups_w, 0, 1, order_wide)
+                          : launch(psa_bwd_dkdv_lds_kernel<64, true, true, ET, H>, n_wide, chunk_w, groups_w, 0, 1, order_wide);
+        return D == 128 ? launch(psa_bwd_dkdv_lds_kernel<128, true, false, ET, H>, n_wide, chunk_w, groups_w, 0, 1, order_wide)
+                        : launch(psa_bwd_dkdv_lds_kernel<64, true, false, ET, H>, n_wide, chunk_w, groups_w, 0, 1, order_wide);
+      };
+      rl = halves != nullptr ? launch_wide(std::true_type{}) : launch_wide(std::false_type{});
       PSA_REQUIRE(rl == PSA_OK, rl, "psa_bwd: cannot reserve %zu bytes of LDS", shmem);
-      if (int e = psa_check_launch("psa_bwd (dK/dV, 128-key slots)")) return e;
-      if (items_wide != nullptr) {
-        const dim3 grid((unsigned)(Nk * (D / 8)), (unsigned)(B * Hkv));
-        if (D == 128) hipLaunchKernelGGL((psa_bwd_join_kernel<128, ET>), grid, dim3(256), 0, st, p, items_wide);
-        else hipLaunchKernelGGL((psa_bwd_join_kernel<64, ET>), grid, dim3(256), 0, st, p, items_wide);
-      }
-      return psa_check_launch("psa_bwd (dK/dV, cut slots)");
+      return psa_check_launch("psa_bwd (dK/dV, 128-key slots)");
     }
   }
   // 5. un-pool (blocks of 64 or 32 keys: every level went to the fp32 buffers)
