@@ -471,7 +471,7 @@ __global__ __launch_bounds__(256) void psa_est_reduce_kernel(EstParams p) {
 // through memory go away.  With a similarity cap or a list of tiles the row's levels end in LDS too (psa_sched::end_map_row; else
 // end.map_out is null and they go straight to the map: rows of few levels lose 1.5 of 40 us per layer by the way through LDS).
 // LDS: [level-map scratch: lm_bytes][n_d floats][Nk levels, if they end there].  p.scores may be null.
-// (80 registers, six waves per SIMD: at 82, five, 3072 rows of 1024 scores take 109.5 us instead of 104.1)
+// (Six waves per SIMD need at most 80 registers; it takes 52.  When it took 82, five waves, 3072 rows of 1024 scores were 109.5 us instead of 104.1.)
 __global__ __launch_bounds__(256, 6) void psa_est_reduce_map_kernel(EstParams p, LevelMapParams lp, psa_sched::MapEnd end, int lm_bytes) {
   extern __shared__ __align__(16) unsigned char smem_rm[];
   __shared__ float s_part[4];
